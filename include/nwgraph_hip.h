@@ -124,7 +124,7 @@ int nwg_pagerank_f32(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* csc
  * loops, harnesses that forbid hipMalloc).  The CSC, the optional out-degrees and the scores
  * are [device] pointers; the call runs on the context's stream and makes no hipMalloc,
  * hipFree or other allocating call.  Its working memory (contributions, counted degrees, L1
- * partials and accumulators) is one static 48.2 MiB device array per GPU, looked up by
+ * partials and accumulators) is one static 51.7 MiB device array per GPU, looked up by
  * nwg_create and held until the process ends.  Limits: n <= 4194304 vertices and
  * max_iters <= 4096, else NWG_EINVAL; csc_idx 16-byte aligned; NWG_INFO_KERNEL_TIMING is
  * not supported (NWG_EINVAL).  Calls that overlap on one GPU share the array and race

@@ -1,0 +1,97 @@
+"""The item sweep (nwgraph_amd/csrc/items.hip) at the edges of its work items: rows just below,
+at and above an item's span, rows over many items, runs of empty rows, item counts of one and
+just past the switch between 64 and 256 lanes.  Scores are held to float64 sweeps: row sums are
+exact, so a sweep rounds each score three times (x / deg, the row sum, the update) and damps
+what it inherits by d, at most 3 * 2^-24 / (1 - d) of the score vector in all."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+D = 0.85
+SWEEPS = 12
+
+
+def _csc(indeg, seed):
+    indeg = np.asarray(indeg, np.int64)
+    n = indeg.size
+    rng = np.random.default_rng(seed)
+    ptr = np.zeros(n + 1, np.int64)
+    ptr[1:] = np.cumsum(indeg)
+    col = rng.integers(0, n, ptr[-1])
+    return n, ptr.astype(np.uint32), col.astype(np.uint32), np.bincount(col, minlength=n).astype(np.uint32)
+
+
+def _fp64(n, ptr, col, deg, d, sweeps):
+    row = np.repeat(np.arange(n), np.diff(ptr.astype(np.int64)))
+    x = np.full(n, 1.0 / n)
+    err = []
+    for _ in range(sweeps):
+        z = np.bincount(row, weights=x[col] / deg[col], minlength=n)
+        y = (1 - d) / n + d * z
+        err.append(np.abs(y - x).sum())
+        x = y
+    return x, err
+
+
+def _noalloc(ctx, n, ptr, col, deg, d, sweeps):
+    import torch
+    from nwgraph_amd import _lib
+
+    dev = [torch.from_numpy(a.astype(np.int32)).cuda() for a in (ptr, col, deg)]
+    x = torch.full((n,), -1.0, device="cuda")
+    info = _lib.PrInfo()
+    err = np.zeros(sweeps)
+    info.error_trace = err.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    info.error_trace_len = sweeps
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.nwg_pagerank_f32_noalloc(ctx.handle, n, col.size, dev[0].data_ptr(), dev[1].data_ptr(),
+                                               dev[2].data_ptr(), x.data_ptr(), d, 0.0, sweeps, ctypes.byref(info)))
+    assert int(info.iterations) == sweeps
+    return x.cpu().numpy(), err
+
+
+def _degrees(kind):
+    rng = np.random.default_rng(3)
+    if kind == "one vertex":
+        return [5]
+    if kind == "no edges":
+        return [0] * 700
+    if kind == "one long row":
+        return [0] * 40 + [252 * 9 + 1] + [0] * 40
+    if kind == "around the span of 64 lanes":
+        return [252, 251, 253, 0, 0, 504, 503, 505, 1, 252, 252, 0, 2520, 7] * 8
+    if kind == "switch to 256 lanes":  # 2^18 units: the largest graph of 64-lane items
+        return [1] * (1 << 17)
+    if kind == "around the span of 256 lanes":
+        return [1020, 1019, 1021, 0, 2040, 2041, 0, 0, 10200, 3, 1018] * 20 + [2] * (1 << 16)
+    if kind == "empty rows between long ones":
+        return ([0] * 3000 + [1500] + [0] * 17 + [5000]) * 20 + [1] * 130000
+    return np.minimum(rng.zipf(2.0, 90001), 30000)  # skewed
+
+
+KINDS = ["one vertex", "no edges", "one long row", "around the span of 64 lanes", "switch to 256 lanes",
+         "around the span of 256 lanes", "empty rows between long ones", "skewed"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_noalloc_items_match_float64(ctx, kind):
+    n, ptr, col, deg = _csc(_degrees(kind), 5)
+    want, err = _fp64(n, ptr, col, deg, D, SWEEPS)
+    got, trace = _noalloc(ctx, n, ptr, col, deg, D, SWEEPS)
+    bound = 3 * 2.0**-24 / (1 - D) * want.sum()
+    assert np.abs(got - want).sum() <= bound
+    # each sweep's L1 change is off by at most twice the iterates' distance from float64
+    assert np.abs(trace - np.array(err)).max() <= 2 * bound
+
+
+def test_noalloc_damping_above_one_keeps_float_sums(ctx):
+    """Scores leave [0, 1], which the exact sums cover: the float row sums serve this call.  A row of
+    m float terms is off by at most m * 2^-24 of its sum."""
+    n, ptr, col, deg = _csc(_degrees("around the span of 64 lanes"), 5)
+    want, _ = _fp64(n, ptr, col, deg, 6.0, SWEEPS)
+    assert want.min() < 0.0
+    got, _ = _noalloc(ctx, n, ptr, col, deg, 6.0, SWEEPS)
+    assert np.abs(got - want).sum() <= SWEEPS * 2520 * 2.0**-24 * np.abs(want).sum()
