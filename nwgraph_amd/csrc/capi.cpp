@@ -21,14 +21,6 @@ using nwg::stage_in;
 
 namespace {
 
-// validate a host CSC: n+1 monotone pointers ending at nnz, entries < n
-void validate_host_csc(uint32_t n, uint64_t nnz, const uint32_t* ptr, const uint32_t* idx) {
-  NWG_REQUIRE(ptr[0] == 0, "csc_ptr[0] must be 0");
-  NWG_REQUIRE(ptr[n] == nnz, "csc_ptr[n] must equal nnz");
-  for (uint32_t i = 0; i < n; ++i) NWG_REQUIRE(ptr[i] <= ptr[i + 1], "csc_ptr must be non-decreasing");
-  for (uint64_t p = 0; p < nnz; ++p) NWG_REQUIRE(idx[p] < n, "csc_idx holds a vertex id >= n");
-}
-
 nwg_graph* new_graph(nwg_ctx* ctx) {
   nwg_graph* g = new nwg_graph();
   g->ctx = ctx;
@@ -102,7 +94,10 @@ int nwg_graph_create_csc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t*
     NWG_REQUIRE(n >= 1, "graph needs at least one vertex");
     NWG_REQUIRE(csc_ptr && (csc_idx || nnz == 0), "csc arrays must not be null");
     NWG_REQUIRE(nnz < (1ull << 32), "nnz must be below 2^32 (uint32 indices)");
-    if (mem_kind == NWG_MEM_HOST) validate_host_csc(n, nnz, csc_ptr, csc_idx);
+    // a host CSC's ends are looked at here, before nnz entries are read; all else is checked on
+    // the device, before any kernel indexes by the entries
+    if (mem_kind == NWG_MEM_HOST)
+      NWG_REQUIRE(csc_ptr[0] == 0 && csc_ptr[n] == nnz, "csc_ptr must go from 0 to nnz");
     DeviceGuard dg(ctx->device);
     std::unique_ptr<nwg_graph> g(new_graph(ctx));
     hipStream_t s = ctx->stream;
@@ -110,18 +105,12 @@ int nwg_graph_create_csc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t*
     g->nnz = nnz;
     stage_in(s, g->csc_ptr, csc_ptr, (size_t)n + 1, mem_kind);
     stage_in(s, g->csc_idx, csc_idx, nnz, mem_kind);
-    // a device CSC is checked on the device before any kernel indexes by its entries
-    if (mem_kind != NWG_MEM_HOST) nwg::validate_device_csc(s, n, nnz, g->csc_ptr.p, g->csc_idx.p);
-    if (outdeg) {
-      // a smaller out-degree than a vertex's out-edges would let its contributions sum past
-      // its score, out of the range the sweeps' exact fixed-point sums cover
-      stage_in(s, g->outdeg, outdeg, n, mem_kind);
-      nwg::check_outdeg_device(s, n, nnz, g->csc_idx.p, g->outdeg.p);
-    } else {
-      g->outdeg.alloc(n);
-      nwg::out_degrees_device(s, n, nnz, g->csc_idx.p, g->outdeg.p);
-    }
-    NWG_HIP(hipStreamSynchronize(s));
+    // a smaller out-degree than a vertex's out-edges would let its contributions sum past its
+    // score, out of the range the sweeps' exact fixed-point sums cover
+    if (outdeg) stage_in(s, g->outdeg, outdeg, n, mem_kind);
+    else g->outdeg.alloc(n);
+    nwg::check_device_csc(s, n, nnz, g->csc_ptr.p, g->csc_idx.p, outdeg ? g->outdeg.p : nullptr,
+                          outdeg ? nullptr : g->outdeg.p);
     *out = g.release();
   });
 }

@@ -222,14 +222,10 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
   uint32_t* flag = reinterpret_cast<uint32_t*>(base + kOffFlag);
   hipStream_t s = ctx->stream;
 
-  validate_device_csc(s, n, nnz, csc_ptr, csc_idx, flag);
-  const uint32_t* deg = outdeg;
-  if (outdeg) {
-    check_outdeg_device(s, n, nnz, csc_idx, outdeg, cdeg, flag);
-  } else {
-    out_degrees_device(s, n, nnz, csc_idx, cdeg, false);  // build_degrees, common.hpp:110-121
-    deg = cdeg;
-  }
+  // the contribution arrays, not in use yet, take the partial histograms
+  const CscCheckScratch scratch_mem{flag, cdeg, reinterpret_cast<uint32_t*>(c0), kOffDeg - kOffC0};
+  check_device_csc(s, n, nnz, csc_ptr, csc_idx, outdeg, outdeg ? nullptr : cdeg, &scratch_mem);
+  const uint32_t* deg = outdeg ? outdeg : cdeg;  // counted: build_degrees, common.hpp:110-121
 
   NaParams P{};
   P.rp = csc_ptr;

@@ -369,18 +369,21 @@ int key_bits_for(uint32_t n);  // bits of a vertex id field in packed sort keys
 // row pointers + entries from keys (row << b | entry) sorted ascending
 void sorted_keys_to_csx(hipStream_t s, const uint64_t* keys, uint64_t m, uint32_t n, int b, uint32_t* ptr,
                         uint32_t* ent);
-// throws NWG_EINVAL unless ptr is monotone from 0 to nnz and every entry of idx is below n;
-// flag: one device word of scratch, or null to allocate it
-void validate_device_csc(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* ptr, const uint32_t* idx,
-                         uint32_t* flag = nullptr);
-// out-degree histogram of col (ids < n); may_allocate = false keeps to the atomic histogram,
-// which needs no device memory beyond deg
-void out_degrees_device(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* col, uint32_t* deg,
-                        bool may_allocate = true);
-// throws NWG_EINVAL when some outdeg[u] is below the number of entries u has in col;
-// counted (n words) and flag (one word): device scratch, or null to allocate them
-void check_outdeg_device(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* col, const uint32_t* outdeg,
-                         uint32_t* counted = nullptr, uint32_t* flag = nullptr);
+// out-degree histogram of col (ids < n)
+void out_degrees_device(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* col, uint32_t* deg);
+// Device memory check_device_csc works in when its caller cannot allocate.
+struct CscCheckScratch {
+  uint32_t* flags;    // 2 words
+  uint32_t* counted;  // n words
+  uint32_t* part;     // part_bytes of partial histograms
+  uint64_t part_bytes;
+};
+// Checks a CSC in device memory, waiting for the device once: throws NWG_EINVAL unless ptr is
+// monotone from 0 to nnz, every entry of col is below n and (with given) no vertex's given
+// out-degree is below its number of entries; without given, deg receives the counted
+// out-degrees (both null: only the structure is checked).  No scratch: allocates.
+void check_device_csc(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* ptr, const uint32_t* col,
+                      const uint32_t* given, uint32_t* deg, const CscCheckScratch* scratch = nullptr);
 
 // ---- primitives (scan.hip / sort.hip) ----
 // exclusive scan of n values; out has n+1 entries (out[n] = total).
