@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256) void item_init_kernel(ItemParams P, uint32_t c
   const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
   if (i < P.n) {
     P.x[i] = init;
-    c0[i] = init / (float)P.deg[i];
+    if (c0) c0[i] = init / (float)P.deg[i];
   }
   if (i < count) {
     P.hsum[i] = 0ull;

@@ -47,7 +47,7 @@ struct ItemParams {
 ItemShape item_shape(uint32_t n, uint64_t nnz, uint64_t max_items);
 // desc (count entries) from the row pointers
 void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, const ItemShape& sh, uint4* desc);
-// x = init, contrib = init / outdeg, and the solve's counters cleared: acc[0 .. iters), the lanes,
+// x = init, c0 (nullable) = init / outdeg, and the solve's counters cleared: acc[0 .. iters), the lanes,
 // hsum and hcnt (count each)
 void items_enqueue_init(hipStream_t s, const ItemShape& sh, const ItemParams& P, float init, float* c0,
                         uint64_t iters);

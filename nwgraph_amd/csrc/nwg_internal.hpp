@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/nwgraph_hip.h"
+#include "items.hpp"
 
 namespace nwg {
 
@@ -136,6 +137,10 @@ struct BinnedLayout {
 struct Plan {
   nwg_plan_params params{};
   bool built = false;
+  ItemShape ish;          // item sweep (items.hip): its shape (threads 0: not used) and items
+  DevBuf<uint4> idesc;
+  // row classes of the class kernels: built by the first solve that runs them
+  bool classes = false;
   uint32_t n_tiles = 0;
   uint32_t cls_count[kGroupClasses] = {};
   uint32_t cls_off[kGroupClasses + 1] = {};  // offsets of each class in group_rows
@@ -292,6 +297,8 @@ struct PrState {
   DevBuf<float> bvals;             // binned sweep: one value per (bin, source) pair
   DevBuf<unsigned long long> bpart;  // binned sweep: partial rows of split bins
   DevBuf<unsigned long long> bacc;   // binned sweep: per-sweep L1 change, kBinAccLanes lanes
+  DevBuf<unsigned long long> ihsum, ilanes;  // item sweep: long rows' sums, L1 change lanes
+  DevBuf<uint32_t> ihcnt;            // and long rows' pieces counted
   DevBuf<double> tcheck;             // teleport check: sum, invalid-entry flag
   std::vector<std::unique_ptr<Captured>> caps;  // the solve's segments of sweeps
 };

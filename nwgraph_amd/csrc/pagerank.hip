@@ -38,6 +38,10 @@ namespace nwg {
 namespace {
 
 constexpr int kThreads = 256;
+// edges from which plans ask for the binned sweep by default, and from which it runs unless
+// the plan names a bin size (plan_takes_items)
+constexpr uint64_t kBinnedEdges = 1ull << 18;
+constexpr uint64_t kBinnedMinEdges = 3ull << 21;
 // rounding slack allowed above 1 in the sum of a teleport vector
 constexpr double kTeleportSlack = 1e-4;
 
@@ -532,15 +536,17 @@ nwg_plan_params default_plan_params() {
   return p;
 }
 
-// The plan a PageRank solve builds when none was set or tuned.  Measured on MI355X (RMAT,
-// edge factor 16): the binned sweep beats the pull sweep from 2^16 vertices (1M edges: 0.023
-// vs 0.048 ms per sweep) up (RMAT-20: 0.049 vs 0.164; RMAT-25: 0.94 vs 3.65), and on the
-// 4096^2 grid; degree ordering pays from RMAT-19 (8M edges) on and costs a little below.
-// The binned layout indexes entries and pairs with 32 bits (below 2^31 entries and 2^30
-// pairs with pads), so larger graphs keep the pull sweep.
+// The plan a PageRank solve builds when none was set or tuned.  Measured on MI355X (edge
+// factor 16, us per sweep, items / binned): RMAT-12 6.1 / 19.6, RMAT-16 9.1 / 19.5, RMAT-18 (3.9 M
+// edges) 21.7 / 26.8, RMAT-19 (8.0 M) 40.6 / 35.7 degree ordered, RMAT-20 79 / 53, uniform random
+// with 2.1 M edges 14.7 / 21.7, with 8.4 M 45.2 / 43.4.  Degree ordering pays from RMAT-19 on and
+// costs a little below.  The plan asks for the binned sweep from kBinnedEdges, and leaves the bin
+// size, hence the sweep, to the graph's size (plan_takes_items).  The binned layout indexes
+// entries and pairs with 32 bits (below 2^31 entries and 2^30 pairs with pads), so larger
+// graphs keep the pull sweep.
 nwg_plan_params default_plan_for(const nwg_graph* g) {
   nwg_plan_params p = default_plan_params();
-  if (g->nnz >= (1ull << 18) && g->nnz < (1ull << 30) - (1ull << 26)) p.binned = 1;
+  if (g->nnz >= kBinnedEdges && g->nnz < (1ull << 30) - (1ull << 26)) p.binned = 1;
   if (g->nnz >= (1ull << 23)) p.relabel = 1;
   // nontemporal streams: the pair values the chunk pass stores are read once by the bin pass
   // (as cached stores, their write-back landed in the bin pass: RMAT-25 0.81 -> 0.72 ms)
@@ -562,16 +568,52 @@ static void validate_params(const nwg_plan_params& p) {
               "plan: slice_min must be 0 or above both 1 and short_max");
 }
 
+// Whether a plan's sweeps run over items (items.hip).  The pull sweep does unless the plan sets
+// class cutoffs of its own, which ask for the row classes; measured on MI355X, the items are the
+// faster at every size (RMAT-12 6.1 against 27.5 us per sweep, RMAT-18 22 / 105, RMAT-24 2220 /
+// 2495, 4096^2 grid 197 / 199).  A binned plan that leaves the bin size open does from
+// kBinnedEdges to kBinnedMinEdges edges, where the items' one launch a sweep beats the binned
+// sweep's three and the contributions still sit in the L2s (default_plan_for has both sides).
+static bool plan_takes_items(const nwg_plan_params& p, uint64_t nnz) {
+  const nwg_plan_params d = default_plan_params();
+  if (p.short_max != d.short_max || p.group_max != d.group_max || p.hub_min != d.hub_min ||
+      p.hub_segment != d.hub_segment || p.slice_min != d.slice_min)
+    return false;
+  return !p.binned || (p.bin_bits == 0 && nnz >= kBinnedEdges && nnz < kBinnedMinEdges);
+}
+
 void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp) {
   validate_params(pp);
   const uint32_t n = g->n;
   if (pp.relabel) relabel_build(s, g);
-  const uint32_t* rp = g->active(pp.relabel != 0).ptr;
+  const ActiveCsc a = g->active(pp.relabel != 0);
   Plan pl;
   pl.params = pp;
+  pl.n_tiles = (uint32_t)ceil_div(n, kThreads);
+  if (plan_takes_items(pp, g->nnz)) pl.ish = item_shape(n, g->nnz, 1ull << 31);
+  if (pl.ish.threads) {
+    pl.idesc.alloc(pl.ish.count);
+    items_build(s, n, g->nnz, a.ptr, pl.ish, pl.idesc.p);
+  } else if (pp.binned) {
+    binned_build(s, a, n, g->nnz, pl.bl, true, nullptr, (int)pp.bin_bits);
+  }
+  NWG_HIP(hipStreamSynchronize(s));
+  pl.built = true;
+  g->plan = std::move(pl);
+  g->plan_version++;
+}
+
+// the row classes of g's plan, for the schedules that run the class kernels
+static void ensure_classes(hipStream_t s, nwg_graph* g) {
+  Plan& pl = g->plan;
+  if (pl.classes) return;
+  const nwg_plan_params& pp = pl.params;
+  const uint32_t n = g->n;
+  const uint32_t* rp = g->active(pp.relabel != 0).ptr;
   DevBuf<uint32_t> flag(n), pos((uint64_t)n + 1);
   uint32_t counts[kGroupClasses];
   uint32_t total = 0;
+  pl.scls_off[0] = 0;
   for (int c = 0; c < kGroupClasses; ++c) {
     counts[c] = select_class(s, n, rp, pp, 1 + c, flag, pos, nullptr);
     total += counts[c];
@@ -637,12 +679,8 @@ void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp) {
   } else {
     pl.scol.release();
   }
-  pl.n_tiles = (uint32_t)ceil_div(n, kThreads);
-  if (pp.binned) binned_build(s, g->active(pp.relabel != 0), n, g->nnz, pl.bl, true, nullptr, (int)pp.bin_bits);
   NWG_HIP(hipStreamSynchronize(s));
-  pl.built = true;
-  g->plan = std::move(pl);
-  g->plan_version++;
+  pl.classes = true;
 }
 
 static constexpr uint32_t kLanes[kGroupClasses] = {4, 8, 16, 32, 64};
@@ -771,6 +809,32 @@ static BinParams make_bin_params(nwg_graph* g, PrState& st, const SweepParams& P
   return B;
 }
 
+// The item sweep's exact sums cover scores in [0, 1] (damping factors in [0, 1]); the delta
+// schedule's residuals are not normalised.
+static bool runs_items(const Plan& pl, PrSchedule sched, float damping) {
+  return pl.ish.threads && sched != PrSchedule::kDelta && damping >= 0.f && damping <= 1.f;
+}
+
+static ItemParams make_item_params(nwg_graph* g, PrState& st, const SweepParams& P) {
+  ItemParams I{};
+  I.desc = g->plan.idesc.p;
+  I.rp = P.rp;
+  I.col = P.col;
+  I.deg = P.deg;
+  I.x = P.x;
+  I.basev = P.basev;
+  I.base = P.base;
+  I.damp = P.damp;
+  I.n = P.n;
+  I.nnz = (uint32_t)g->nnz;
+  I.hsum = st.ihsum.p;
+  I.hcnt = st.ihcnt.p;
+  I.lanes = st.ilanes.p;
+  I.acc = st.acc.p;
+  I.threshold = P.threshold;
+  return I;
+}
+
 // Sweeps [k0, k1) of an iters-sweep solve: the inits when k0 = 0, and for the binned sweep
 // the fold of these sweeps' residual lanes into acc.
 static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams P, uint64_t iters,
@@ -783,13 +847,23 @@ static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams 
   // stages when it starts.  The delta schedule keeps the pull kernels: the binned sweep's
   // exact fixed-point row sums cover [0, 16), enough for PageRank (a row sum is at most the
   // total score, 1) but not for un-normalised residuals, which reach thousands on hub rows.
-  const bool binned = g->plan.params.binned != 0 && sched != PrSchedule::kDelta;
+  const bool binned = g->plan.bl.built && sched != PrSchedule::kDelta;
   BinParams B{};
   if (binned) {
     B = make_bin_params(g, st, P);
     if (k0 == 0) binned_clear_residuals(s, st.bacc.p, iters);
   }
+  const bool items = runs_items(g->plan, sched, P.damp);
+  ItemParams I{};
+  if (items) I = make_item_params(g, st, P);
   auto sweep = [&](const float* cin, float* cout) {
+    if (items) {
+      I.iter = P.iter;
+      I.cin = cin;
+      I.cout = cout;
+      items_enqueue_sweep(s, g->plan.ish, I);
+      return;
+    }
     if (binned) {
       B.iter = P.iter;
       B.cin = cin;
@@ -833,12 +907,15 @@ static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams 
   if (k0 == 0) {
     if (ev) {
       NWG_HIP(hipEventRecord(ev[2 * iters], s));
-      pr_init_kernel<<<blocks_for(std::max<uint64_t>(n, iters)), kThreads, 0, s>>>(n, P.deg, init, st.x.p, nullptr,
-                                                                                   st.acc.p, iters);
+      if (items) items_enqueue_init(s, g->plan.ish, I, init, nullptr, iters);
+      else pr_init_kernel<<<blocks_for(std::max<uint64_t>(n, iters)), kThreads, 0, s>>>(n, P.deg, init, st.x.p, nullptr,
+                                                                                        st.acc.p, iters);
       NWG_HIP(hipEventRecord(ev[2 * iters + 1], s));
       NWG_HIP(hipEventRecord(ev[2 * iters + 2], s));
       pr_contrib_init_kernel<<<blocks_for(n), kThreads, 0, s>>>(n, P.deg, st.x.p, st.contrib0.p);
       NWG_HIP(hipEventRecord(ev[2 * iters + 3], s));
+    } else if (items) {
+      items_enqueue_init(s, g->plan.ish, I, init, st.contrib0.p, iters);
     } else {
       pr_init_kernel<<<blocks_for(std::max<uint64_t>(n, iters)), kThreads, 0, s>>>(n, P.deg, init, st.x.p,
                                                                                    st.contrib0.p, st.acc.p, iters);
@@ -857,6 +934,7 @@ static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams 
   }
   if (binned && k1 > k0)
     binned_fold_residuals(s, st.bacc.p + k0 * kBinAccStride, st.acc.p + k0, k1 - k0);
+  if (items && k1 > k0) items_enqueue_fold(s, I, (uint32_t)(k1 - 1));
 }
 
 void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float damping, float threshold,
@@ -865,8 +943,15 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   hipStream_t s = ctx->stream;
   NWG_REQUIRE(max_iters < (1ull << 31), "max_iters too large");
   if (!g->plan.built) plan_build(s, g, default_plan_for(g));
+  const bool items = runs_items(g->plan, sched, damping);
+  if (!items && (!g->plan.bl.built || sched == PrSchedule::kDelta)) ensure_classes(s, g);
   if (!g->pr) g->pr.reset(new PrState());
   PrState& st = *g->pr;
+  if (items) {
+    st.ihsum.ensure(g->plan.ish.count);
+    st.ihcnt.ensure(g->plan.ish.count);
+    st.ilanes.ensure(kItemLaneWords);
+  }
   const uint32_t n = g->n;
   st.x.ensure(n);
   st.contrib0.ensure(n);
@@ -875,7 +960,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   st.hub_part.ensure(std::max<uint32_t>(g->plan.n_hub_segs, 1));
   st.blk_err.ensure(std::max<uint64_t>(sweep_workgroups_before_hubs(g->plan), 1));
   st.spart.ensure(std::max<uint64_t>((uint64_t)kSlices * g->plan.n_srows, 1));
-  if (g->plan.params.binned && sched != PrSchedule::kDelta) {
+  if (g->plan.bl.built && sched != PrSchedule::kDelta) {
     const BinnedLayout& L = g->plan.bl;
     st.bvals.ensure(L.pairs);
     st.bpart.ensure(std::max<uint64_t>((uint64_t)L.n_slots << L.bin_bits, 1));
@@ -916,6 +1001,9 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     key.ptrs[9] = st.bvals.p;
     key.ptrs[10] = st.bpart.p;
     key.ptrs[11] = st.bacc.p;
+    key.ptrs[12] = st.ihsum.p;
+    key.ptrs[13] = st.ihcnt.p;
+    key.ptrs[14] = st.ilanes.p;
     key.plan_version = g->plan_version;
     key.iters = max_iters;
     key.damping = damping;

@@ -87,6 +87,46 @@ def test_noalloc_items_match_float64(ctx, kind):
     assert np.abs(trace - np.array(err)).max() <= 2 * bound
 
 
+@pytest.mark.parametrize("relabel", [0, 1])
+@pytest.mark.parametrize("kind", KINDS)
+def test_resident_items_match_float64(ctx, kind, relabel):
+    """The resident solve's pull plan, over two segments of sweeps (20, then 8 at a time)."""
+    n, ptr, col, deg = _csc(_degrees(kind), 5)
+    sweeps = 23
+    want, err = _fp64(n, ptr, col, deg, D, sweeps)
+    g = ctx.graph_from_csc(ptr, col, deg)
+    g.set_plan(binned=0, relabel=relabel)
+    got, info = g.pagerank(D, 0.0, sweeps)
+    bound = 3 * 2.0**-24 / (1 - D) * want.sum()
+    assert info["iterations"] == sweeps
+    assert np.abs(got - want).sum() <= bound
+    assert np.abs(info["error_trace"] - np.array(err)).max() <= 2 * bound
+    g.close()
+
+
+@pytest.mark.parametrize("n", [12007, 70001])  # 64- and 256-lane items
+def test_resident_items_stop_and_personalise(ctx, n):
+    rng = np.random.default_rng(n)
+    n, ptr, col, deg = _csc(np.minimum(rng.zipf(2.0, n), 3000), 6)
+    v = rng.random(n)
+    v = (v / v.sum()).astype(np.float32)
+    row = np.repeat(np.arange(n), np.diff(ptr.astype(np.int64)))
+    x = np.full(n, 1.0 / n)
+    for it in range(1, 60):
+        y = (1 - D) * v.astype(np.float64) + D * np.bincount(row, weights=x[col] / deg[col], minlength=n)
+        done = np.abs(y - x).sum() < 1e-4
+        x = y
+        if done:
+            break
+    g = ctx.graph_from_csc(ptr, col, deg)
+    g.set_plan(binned=0)
+    for _ in range(2):
+        got, info = g.pagerank(D, 1e-4, 100, teleport=v)
+        assert info["iterations"] == it
+        assert np.abs(got - x).sum() <= 3 * 2.0**-24 / (1 - D) * x.sum()
+    g.close()
+
+
 def test_noalloc_damping_above_one_keeps_float_sums(ctx):
     """The exact sums cover damping factors in [0, 1]; above, the float row sums serve the call.  A
     sweep is off by at most m * 2^-24 for a row of m float terms and 3 * 2^-24 for its other
