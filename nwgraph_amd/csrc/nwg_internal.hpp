@@ -114,6 +114,7 @@ constexpr uint32_t kBinAccPad = 8;
 constexpr uint32_t kBinAccStride = kBinAccLanes * kBinAccPad;  // words per sweep
 struct BinnedLayout {
   bool built = false;
+  uint64_t build_id = 0;  // weighted layouts: which build of its graph's this is
   uint32_t n_bins = 0, n_chunks = 0, n_items2 = 0, n_items1 = 0, n_items3 = 0, n_segs = 0, n_slots = 0;
   uint32_t n_items2_live = 0;  // bin-pass items of bins with entries (the others come after them)
   int bin_bits = 13;           // rows per bin: 2^13 (64 KiB of row sums, two bin-pass workgroups per CU) or 2^14
@@ -261,6 +262,7 @@ struct WState {
   // binned sweep: weighted layouts of the CSC (forward) and the CSR (adjoint), built on first
   // use and dropped when the weights change; pair values, split-bin partial rows, L1 partials
   std::unique_ptr<BinnedLayout> bl_csc, bl_csr;
+  uint64_t layouts_built = 0;
   DevBuf<float> bvals;
   DevBuf<unsigned long long> bpart;
   DevBuf<double> wpart, stats;

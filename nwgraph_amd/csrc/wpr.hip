@@ -619,7 +619,9 @@ static uint64_t fixed_point(nwg_ctx* ctx, WState& st, std::vector<std::unique_pt
   key.iters = max_iters;
   key.damping = damping;
   key.threshold = threshold;
-  key.plan_version = n_items;
+  // the layout's device arrays stand behind its build number: a layout made after the weights
+  // changed may sit at the old one's host address
+  key.plan_version = L ? L->build_id : n_items;
   key.extra = (relative ? 1u : 0u) | (y0_uniform ? 2u : 0u);
   // the segments' graphs, captured when missing or stale
   uint64_t nseg = 0;
@@ -750,6 +752,7 @@ static const BinnedLayout* weighted_layout(hipStream_t s, nwg_graph* g, WState& 
                             : ActiveCsc{g->csc_ptr.p, g->csc_idx.p, g->outdeg.p, nullptr};
     try {
       binned_build(s, a, g->n, g->nnz, *L, true, csr ? g->w_csr.p : g->w_csc.p, bits);
+      L->build_id = ++st.layouts_built;
     } catch (...) {
       L.reset();
       throw;
