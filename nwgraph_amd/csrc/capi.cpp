@@ -30,6 +30,13 @@ nwg_graph* new_graph(nwg_ctx* ctx) {
 
 }  // namespace
 
+namespace nwg {
+std::mutex& capture_mutex() {
+  static std::mutex mu;
+  return mu;
+}
+}  // namespace nwg
+
 extern "C" {
 
 int nwg_version(void) { return 10000; }
@@ -53,6 +60,9 @@ int nwg_create(nwg_ctx** out, int device) {
     NWG_HIP(hipEventCreate(&ctx->ev0));
     NWG_HIP(hipEventCreate(&ctx->ev1));
     nwg::noalloc_setup(device);
+    size_t total_bytes = 0;
+    NWG_HIP(hipDeviceTotalMem(&total_bytes, device));
+    ctx->pool = std::make_shared<nwg::DevPool>(total_bytes / 64);
   });
   if (rc != NWG_OK) {
     nwg_destroy(ctx);
@@ -71,6 +81,7 @@ void nwg_destroy(nwg_ctx* ctx) {
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
+  if (ctx->pool) ctx->pool->close();  // graphs that outlive the context free their memory directly
   if (ctx->capture_stream) (void)hipStreamDestroy(ctx->capture_stream);
   if (prev >= 0) (void)hipSetDevice(prev);
   delete ctx;
@@ -139,6 +150,7 @@ void nwg_graph_destroy(nwg_graph* g) {
   int prev = -1;
   (void)hipGetDevice(&prev);
   (void)hipSetDevice(g->device);
+  std::lock_guard<std::mutex> lk(nwg::capture_mutex());
   (void)hipDeviceSynchronize();
   delete g;
   if (prev >= 0) (void)hipSetDevice(prev);

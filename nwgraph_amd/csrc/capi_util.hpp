@@ -10,22 +10,35 @@
 
 namespace nwg {
 
+// A failed call may leave work in flight on memory its unwinding has put back into the
+// context's pool: wait for it before the next call can take that memory.
+inline void wait_after_failure(nwg_ctx* ctx) {
+  if (!ctx || !ctx->stream) return;
+  (void)hipStreamSynchronize(ctx->stream);
+  (void)hipGetLastError();
+}
+
 template <class F>
 int guarded(nwg_ctx* ctx, F&& f) {
+  PoolScope scope(ctx ? ctx->pool : nullptr);
   try {
     f();
     if (ctx) ctx->last_error.clear();
     return NWG_OK;
   } catch (const Error& e) {
+    wait_after_failure(ctx);
     if (ctx) ctx->last_error = e.what();
     return e.code;
   } catch (const std::bad_alloc&) {
+    wait_after_failure(ctx);
     if (ctx) ctx->last_error = "host allocation failed";
     return NWG_ENOMEM;
   } catch (const std::exception& e) {
+    wait_after_failure(ctx);
     if (ctx) ctx->last_error = e.what();
     return NWG_EHIP;
   } catch (...) {
+    wait_after_failure(ctx);
     if (ctx) ctx->last_error = "unknown failure";
     return NWG_EHIP;
   }

@@ -1,0 +1,106 @@
+// devpool.cpp -- the free lists of devpool.hpp.
+#include "devpool.hpp"
+
+#include <hip/hip_runtime.h>
+
+#include <new>
+
+#include "nwg_internal.hpp"
+
+namespace nwg {
+
+namespace {
+
+thread_local std::shared_ptr<DevPool> t_pool;
+
+// below 1 MiB powers of two, from there whole MiB: few sizes, little waste
+size_t block_size(size_t bytes) {
+  constexpr size_t kMiB = 1u << 20;
+  if (bytes >= kMiB) return (bytes + kMiB - 1) / kMiB * kMiB;
+  size_t s = 512;
+  while (s < bytes) s <<= 1;
+  return s;
+}
+
+}  // namespace
+
+const std::shared_ptr<DevPool>& current_pool() { return t_pool; }
+PoolScope::PoolScope(std::shared_ptr<DevPool> p) : prev_(std::move(t_pool)) { t_pool = std::move(p); }
+PoolScope::~PoolScope() { t_pool = std::move(prev_); }
+
+void DevPool::trim_locked() noexcept {
+  for (auto& b : free_) (void)hipFree(b.second);
+  free_.clear();
+  held_ = 0;
+}
+
+void* DevPool::take(size_t bytes, size_t* size) {
+  const size_t want = block_size(bytes);
+  *size = want;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    const auto it = free_.lower_bound(want);
+    if (it != free_.end() && it->first <= want + want / 2) {  // the smallest that does, if not much too large
+      void* p = it->second;
+      *size = it->first;
+      held_ -= it->first;
+      free_.erase(it);
+      return p;
+    }
+  }
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, want);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      trim_locked();
+    }
+    e = hipMalloc(&p, want);
+  }
+  NWG_HIP(e);
+  return p;
+}
+
+void DevPool::give(void* p, size_t size) noexcept {
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (size <= limit_) {
+      // room for it: the largest free blocks go first
+      while (held_ + size > limit_) {
+        const auto it = std::prev(free_.end());
+        (void)hipFree(it->second);
+        held_ -= it->first;
+        free_.erase(it);
+      }
+      try {
+        free_.emplace(size, p);
+        held_ += size;
+        return;
+      } catch (const std::bad_alloc&) {
+      }
+    }
+  }
+  (void)hipFree(p);
+}
+
+void DevPool::close() noexcept {
+  std::lock_guard<std::mutex> lk(mu_);
+  trim_locked();
+  limit_ = 0;
+}
+
+void* dev_alloc(const std::shared_ptr<DevPool>& pool, size_t bytes, size_t* size) {
+  if (pool) return pool->take(bytes, size);
+  void* p = nullptr;
+  NWG_HIP(hipMalloc(&p, bytes));
+  *size = bytes;
+  return p;
+}
+
+void dev_free(const std::shared_ptr<DevPool>& pool, void* p, size_t size) noexcept {
+  if (pool) pool->give(p, size);
+  else (void)hipFree(p);
+}
+
+}  // namespace nwg

@@ -324,6 +324,7 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   key.extra = grid | (mg->binned ? 0x80000000u : 0u);
   if (!mg->cap.valid || !(mg->cap.key == key)) {
     mg->cap.reset();
+    std::lock_guard<std::mutex> capture_lock(capture_mutex());
     hipStream_t cs = ctx->capture_stream;
     NWG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     try {
@@ -403,6 +404,7 @@ void nwg_multigraph_destroy(nwg_multigraph* mg) {
   int prev = -1;
   (void)hipGetDevice(&prev);
   (void)hipSetDevice(mg->device);
+  std::lock_guard<std::mutex> lk(nwg::capture_mutex());
   (void)hipDeviceSynchronize();
   delete mg;
   if (prev >= 0) (void)hipSetDevice(prev);

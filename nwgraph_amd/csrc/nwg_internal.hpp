@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/nwgraph_hip.h"
+#include "devpool.hpp"
 #include "items.hpp"
 
 namespace nwg {
@@ -41,7 +42,7 @@ struct Error : std::runtime_error {
 
 inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
-// Owning device allocation.
+// Owning device allocation, from the running call's pool (devpool.hpp) when there is one.
 template <class T>
 struct DevBuf {
   T* p = nullptr;
@@ -50,15 +51,18 @@ struct DevBuf {
   explicit DevBuf(size_t count) { alloc(count); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+  DevBuf(DevBuf&& o) noexcept { swap(o); }
   DevBuf& operator=(DevBuf&& o) noexcept {
-    if (this != &o) { release(); p = o.p; n = o.n; o.p = nullptr; o.n = 0; }
+    if (this != &o) { release(); swap(o); }
     return *this;
   }
   ~DevBuf() { release(); }
   void alloc(size_t count) {
     release();
-    if (count) NWG_HIP(hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T)));
+    if (count) {
+      pool_ = current_pool();
+      p = static_cast<T*>(dev_alloc(pool_, count * sizeof(T), &bytes_));
+    }
     n = count;
   }
   // grow-only reuse
@@ -66,13 +70,24 @@ struct DevBuf {
     if (count > n) alloc(count);
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) dev_free(pool_, p, bytes_);
     p = nullptr;
     n = 0;
+    bytes_ = 0;
+    pool_.reset();
+  }
+  void swap(DevBuf& o) noexcept {
+    std::swap(p, o.p);
+    std::swap(n, o.n);
+    std::swap(bytes_, o.bytes_);
+    pool_.swap(o.pool_);
   }
   T* get() const { return p; }
-};
 
+ private:
+  size_t bytes_ = 0;  // of the block
+  std::shared_ptr<DevPool> pool_;
+};
 
 // Scheduling plan of the pull sweep over one CSC.
 // Row classes by in-degree d (rows of a CSC are destinations):
@@ -235,6 +250,10 @@ struct CaptureKey {
   }
 };
 
+// Held while a HIP graph is recorded and instantiated, and while the destruction of a graph waits
+// for the device: a hipDeviceSynchronize invalidates the recordings of other threads.
+std::mutex& capture_mutex();
+
 // A captured and instantiated HIP graph.
 struct Captured {
   hipGraph_t graph = nullptr;
@@ -334,6 +353,7 @@ struct nwg_ctx {
   hipStream_t capture_stream = nullptr;  // used only to record HIP graphs
   std::string last_error;
   std::mutex mu;
+  std::shared_ptr<nwg::DevPool> pool;  // device memory kept between this context's calls
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 

@@ -1019,6 +1019,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
       Captured& cap = *st.caps[nseg++];
       if (!cap.valid || !(cap.key == key)) {
         cap.reset();
+        std::lock_guard<std::mutex> capture_lock(capture_mutex());
         hipStream_t cs = ctx->capture_stream;
         NWG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
         try {

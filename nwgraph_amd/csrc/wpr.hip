@@ -632,6 +632,7 @@ static uint64_t fixed_point(nwg_ctx* ctx, WState& st, std::vector<std::unique_pt
     ++nseg;
     if (!cap.valid || !(cap.key == key)) {
       cap.reset();
+      std::lock_guard<std::mutex> capture_lock(capture_mutex());
       hipStream_t cs = ctx->capture_stream;
       NWG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
       try {
