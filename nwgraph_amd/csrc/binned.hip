@@ -829,7 +829,7 @@ void binned_build(hipStream_t s, const ActiveCsc& a, uint32_t n, uint64_t nnz, B
     int kb = ub;
     while (kb < 64 && (1ull << (kb - ub)) < L.n_bins) ++kb;
     // stable: the entries of one (bin, source) keep their CSC order (row ascending)
-    radix_sort_pairs(s, keys.p, keys_tmp.p, low.p, low_tmp.p, nnz, kb);
+    radix_sort_pairs(s, keys, keys_tmp, &low, &low_tmp, nnz, 0, kb);
     // the sort's temporaries now hold the pair flags and their exclusive scan
     uint32_t* flag = low_tmp.p;
     uint32_t* pex = reinterpret_cast<uint32_t*>(keys_tmp.p);  // nnz + 1 <= 2 nnz words

@@ -1,15 +1,16 @@
 // build.hip -- on-device edge list -> CSC / CSR construction.
 //
 // Pipeline (reference semantics in brackets, pnnl/NWGraph):
-//   1. pack key = (row << b) | entry, b = bits(n-1); with clean=1 drop u == v
-//      [remove_self_loops, build.hpp:404-410] -- dropping before the sort gives the
-//      same edge set as the reference's sort -> uniq -> remove order (tc.cpp:66-68)
+//   1. the first pass of the sort reads the edges, packs key = (row << b) | entry, b =
+//      bits(n-1), and with clean=1 drops u == v [remove_self_loops, build.hpp:404-410] --
+//      dropping before the sort gives the same edge set as the reference's sort -> uniq ->
+//      remove order (tc.cpp:66-68)
 //   2. stable LSD radix sort of the 2b-bit keys [lexical_sort_by, build.hpp:57-70]
-//   3. with clean=1 drop adjacent equal keys [uniq, build.hpp:392-402]
-//   4. row pointers from the sorted keys and entries = low bits
+//   3. row pointers from the sorted keys and entries = low bits
 //      [fill_directed<idx> + sort_to_be_indexed, build.hpp:209-232,
-//       compressed.hpp:491-502: each row ascending makes the layout unique]
-//   5. out-degree = histogram of sources [build_degrees, bench/gapbs/common.hpp:110-121]
+//       compressed.hpp:491-502: each row ascending makes the layout unique]; with clean=1 of
+//      equal keys only the first [uniq, build.hpp:392-402]
+//   4. out-degree = histogram of sources [build_degrees, bench/gapbs/common.hpp:110-121]
 #include <algorithm>
 
 #include "device_utils.hpp"
@@ -25,63 +26,88 @@ inline int bits_for(uint32_t n) {
   return b;
 }
 
-// flag[i] = keep edge i; also records an id out of range.
-__global__ __launch_bounds__(256) void edge_flag_kernel(const uint32_t* __restrict__ src,
-                                                        const uint32_t* __restrict__ dst, uint64_t ne, uint32_t n,
-                                                        int clean, uint32_t* __restrict__ flag,
-                                                        uint32_t* __restrict__ bad) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ne) return;
-  const uint32_t u = src[i], v = dst[i];
-  const bool self = (u == v);
-  uint32_t keep = 1;
-  if (clean && self) keep = 0;
-  if (keep && (u >= n || v >= n)) {
-    atomicOr(bad, 1u);
-    keep = 0;
+// Sorted keys (row << b | entry) -> row pointers and entries, in tiles of kCsxTile keys; with
+// uniq, equal neighbours count once [uniq, build.hpp:392-402].  A wave takes kCsxItems x 64
+// consecutive keys, 64 at a time.  One pass counts a tile's distinct keys, a scan places the
+// tiles, the second pass writes: 20 bytes moved per key (flags, their scan, a compacted copy and
+// the row pointers as passes of their own moved 56: 0.86 ms for 67 M keys on MI355X, against
+// 0.29 ms now).
+constexpr int kCsxItems = 8;
+constexpr int kCsxTile = 256 * kCsxItems;
+
+// key q is the first of its run of equal keys
+__device__ __forceinline__ bool csx_first(const uint64_t* __restrict__ keys, uint64_t q, bool uniq) {
+  return !uniq || q == 0 || keys[q] != keys[q - 1];
+}
+
+__global__ __launch_bounds__(256) void csx_count_kernel(const uint64_t* __restrict__ keys, uint64_t m,
+                                                        uint32_t* __restrict__ count) {
+  __shared__ uint32_t red[4];
+  const uint64_t base = (uint64_t)blockIdx.x * kCsxTile + threadIdx.x;
+  uint32_t c = 0;
+#pragma unroll
+  for (int j = 0; j < kCsxItems; ++j) {
+    const uint64_t q = base + (uint64_t)j * 256;
+    if (q < m && csx_first(keys, q, true)) ++c;
   }
-  flag[i] = keep;
+  c = block_sum<256>(c, red);
+  if (threadIdx.x == 0) count[blockIdx.x] = c;
 }
 
-// keys[pos[i]] = (row << b) | entry for kept edges (row = dst for idx=1, src for idx=0)
-__global__ __launch_bounds__(256) void pack_kernel(const uint32_t* __restrict__ src, const uint32_t* __restrict__ dst,
-                                                   uint64_t ne, int b, int idx, const uint32_t* __restrict__ flag,
-                                                   const uint32_t* __restrict__ pos, uint64_t* __restrict__ keys) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ne || !flag[i]) return;
-  const uint64_t r = idx ? dst[i] : src[i];
-  const uint64_t e = idx ? src[i] : dst[i];
-  keys[pos[i]] = (r << b) | e;
+// before: distinct keys before each tile (null without uniq: the keys before it).  Rows up to the
+// last key's get their pointer here, the rows after it in csx_tail_kernel.
+__global__ __launch_bounds__(256) void csx_write_kernel(const uint64_t* __restrict__ keys, uint64_t m, int b,
+                                                        const uint32_t* __restrict__ before,
+                                                        uint32_t* __restrict__ ptr, uint32_t* __restrict__ ent) {
+  __shared__ uint32_t wave_total[4];
+  const uint32_t w = threadIdx.x >> 6, lane = lane_id();
+  const uint64_t base = (uint64_t)blockIdx.x * kCsxTile + w * (kCsxItems * 64) + lane;
+  uint64_t k[kCsxItems], prev[kCsxItems], first[kCsxItems];
+#pragma unroll
+  for (int j = 0; j < kCsxItems; ++j) {
+    const uint64_t q = base + 64 * j;
+    k[j] = q < m ? keys[q] : 0ull;
+    prev[j] = q < m && q ? keys[q - 1] : ~0ull;  // no key: ids take fewer than 64 bits
+  }
+  uint32_t total = 0;
+#pragma unroll
+  for (int j = 0; j < kCsxItems; ++j) {
+    first[j] = __ballot(base + 64 * j < m && (!before || k[j] != prev[j]));
+    total += (uint32_t)__popcll(first[j]);
+  }
+  if (lane == 0) wave_total[w] = total;
+  __syncthreads();
+  uint32_t pos = before ? before[blockIdx.x] : blockIdx.x * (uint32_t)kCsxTile;
+  for (uint32_t q = 0; q < w; ++q) pos += wave_total[q];
+  const uint64_t lt = __lanemask_lt();
+#pragma unroll
+  for (int j = 0; j < kCsxItems; ++j) {
+    const bool mine = (first[j] >> lane) & 1ull;
+    const uint32_t at = pos + (uint32_t)__popcll(first[j] & lt);
+    pos += (uint32_t)__popcll(first[j]);
+    // rows (row of the key before, row of this key] begin here
+    const uint32_t row = (uint32_t)(k[j] >> b);
+    const uint32_t lo = prev[j] == ~0ull ? 0u : (uint32_t)(prev[j] >> b) + 1u;
+    if (mine) ent[at] = (uint32_t)(k[j] & ((1ull << b) - 1));
+    const bool wide = mine && row >= lo && row - lo >= 32u;  // a long run of empty rows: by the whole wave
+    if (mine && !wide && row >= lo)
+      for (uint32_t r = lo; r <= row; ++r) ptr[r] = at;
+    uint64_t todo = __ballot(wide);
+    while (todo) {
+      const int l = __builtin_ctzll(todo);
+      todo &= todo - 1;
+      const uint32_t r0 = (uint32_t)__shfl((int)lo, l), r1 = (uint32_t)__shfl((int)row, l),
+                     v = (uint32_t)__shfl((int)at, l);
+      for (uint64_t r = (uint64_t)r0 + lane; r <= r1; r += 64) ptr[r] = v;
+    }
+  }
 }
 
-__global__ __launch_bounds__(256) void uniq_flag_kernel(const uint64_t* __restrict__ keys, uint64_t m,
-                                                        uint32_t* __restrict__ flag) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  flag[i] = (i == 0 || keys[i] != keys[i - 1]) ? 1u : 0u;
-}
-
-__global__ __launch_bounds__(256) void compact_keys_kernel(const uint64_t* __restrict__ in, uint64_t m,
-                                                           const uint32_t* __restrict__ flag,
-                                                           const uint32_t* __restrict__ pos,
-                                                           uint64_t* __restrict__ out) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < m && flag[i]) out[pos[i]] = in[i];
-}
-
-// Row pointers: every key i fills ptr[r] for rows (row(i-1), row(i)]; the last key
-// also fills rows (row(m-1), n].  entries = low b bits.
-__global__ __launch_bounds__(256) void csx_kernel(const uint64_t* __restrict__ keys, uint64_t m, uint32_t n, int b,
-                                                  uint32_t* __restrict__ ptr, uint32_t* __restrict__ ent) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const uint64_t k = keys[i];
-  const uint64_t r = k >> b;
-  ent[i] = (uint32_t)(k & ((1ull << b) - 1));
-  const int64_t prev = i ? (int64_t)(keys[i - 1] >> b) : -1;
-  for (int64_t rr = prev + 1; rr <= (int64_t)r; ++rr) ptr[rr] = (uint32_t)i;
-  if (i == m - 1)
-    for (uint64_t rr = r + 1; rr <= n; ++rr) ptr[rr] = (uint32_t)m;
+// ptr[r] = m_out for the rows after the last key's, and the end
+__global__ __launch_bounds__(256) void csx_tail_kernel(const uint64_t* __restrict__ keys, uint64_t m, uint32_t n, int b,
+                                                       uint32_t m_out, uint32_t* __restrict__ ptr) {
+  const uint64_t r = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (r <= n && r > (keys[m - 1] >> b)) ptr[r] = m_out;
 }
 
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* __restrict__ p, uint64_t n, uint32_t v) {
@@ -203,16 +229,21 @@ __global__ __launch_bounds__(256) void hist_add_kernel(uint32_t n, uint32_t word
 }
 
 // Out-degrees of a large CSC without global atomics: the ids are grouped by id range
-// (2^kDegRangeBits ids per range) with a radix sort of a copy over the range bits only,
-// then every range is counted in an LDS histogram by the workgroups of its work items
-// (kDegItem entries each); a range held by one item stores its counts, the items of a range
-// split over several add theirs.  At RMAT-25 (5.3e8 ids) the global-atomic histogram is
-// bound by the device's atomic rate (~1.3e10 per second); this path streams.
+// (2^kDegRangeBits ids per range) with a radix sort of the range bits only, then every range is
+// counted in LDS histograms.  With at most 256 ranges the sort is one pass that keeps just the
+// ids' low 16 bits and knows where every range starts (12 bytes moved per id); with more, a sort of
+// whole ids, whose range starts are then looked up.  A range's entries are shared by kDegSplit
+// workgroups; when one of them gets all, it stores its counts, else they are added.  At RMAT-22
+// (65 M ids on MI355X) 0.58 ms, against 1.29 ms for sorting whole ids, read-back starts and items of
+// 2^20 entries read two bytes at a time, of which the count alone took 0.71 ms; shares below 2^19
+// entries pay more for their flushes than they save (2^16: 0.84 ms).  The global-atomic
+// histogram is bound by the device's atomic rate (~1.3e10 per second).
 constexpr int kDegRangeBits = 14;
 constexpr uint32_t kDegRange = 1u << kDegRangeBits;
 constexpr uint64_t kDegSortMin = 1ull << 24;  // entries from which the range path is taken
-constexpr uint32_t kDegItem = 1u << 20;
-constexpr uint32_t kDegCountThreads = 512;
+constexpr uint32_t kDegSplit = 32;            // most workgroups of a range
+constexpr uint32_t kDegMin = 1u << 19;        // entries that one workgroup takes alone
+constexpr uint32_t kDegCountThreads = 1024;
 
 // start[r] = first position whose id's range is >= r, r in [0, nr]; every r written once
 __global__ __launch_bounds__(256) void range_start_kernel(const uint32_t* __restrict__ ids, uint64_t nnz, uint32_t nr,
@@ -225,31 +256,47 @@ __global__ __launch_bounds__(256) void range_start_kernel(const uint32_t* __rest
   for (uint32_t r = a; r <= b; ++r) start[r] = (uint32_t)p;
 }
 
-// one work item {range, first, end, split}: LDS counts of the range's ids in [first, end)
-__global__ __launch_bounds__(kDegCountThreads) void range_count_kernel(const uint32_t* __restrict__ ids,
-                                                                       const uint4* __restrict__ items, uint32_t n,
+// workgroup (r, y): LDS counts of its share of range r's ids
+template <class Id>
+__global__ __launch_bounds__(kDegCountThreads) void range_count_kernel(const Id* __restrict__ ids,
+                                                                       const uint32_t* __restrict__ start, uint32_t n,
                                                                        uint32_t* __restrict__ deg) {
   __shared__ uint32_t h[kDegRange];
-  const uint4 it = items[blockIdx.x];
+  const uint32_t e0 = start[blockIdx.x], e1 = start[blockIdx.x + 1];
+  const uint32_t share = max(kDegMin, (uint32_t)(((uint64_t)(e1 - e0) + kDegSplit - 1) / kDegSplit));
+  const uint64_t p0 = e0 + (uint64_t)blockIdx.y * share;
+  if (blockIdx.y && p0 >= e1) return;
+  const uint64_t p1 = p0 + share < e1 ? p0 + share : e1;
   for (uint32_t q = threadIdx.x; q < kDegRange; q += kDegCountThreads) h[q] = 0u;
   __syncthreads();
-  constexpr uint32_t kU = 4;
-  for (uint32_t p = it.y + threadIdx.x; p < it.z; p += kDegCountThreads * kU) {
-    uint32_t u[kU];
+  // 16-byte loads: a workgroup alone on a range has its CU's bandwidth only with enough in flight
+  constexpr uint32_t kPer = 16 / sizeof(Id);
+  const uint64_t a0 = (p0 + kPer - 1) / kPer * kPer, a1 = p1 / kPer * kPer;  // whole 16-byte groups of [p0, p1)
+  auto count = [&](uint32_t u) { atomicAdd(&h[u & (kDegRange - 1)], 1u); };
+  auto ends = [&](uint64_t q0, uint64_t q1) {
+    if (q0 + threadIdx.x < q1) count(ids[q0 + threadIdx.x]);
+  };
+  if (a0 >= a1) {
+    ends(p0, p1);  // fewer than 2 kPer ids
+  } else {
+    ends(p0, a0);
+    ends(a1, p1);
+  }
+  for (uint64_t p = a0 + (uint64_t)threadIdx.x * kPer; p < a1; p += (uint64_t)kDegCountThreads * kPer) {
+    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ids + p));
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (uint32_t t = 0; t < kU; ++t) {
-      const uint32_t q = p + t * kDegCountThreads;
-      u[t] = q < it.z ? __builtin_nontemporal_load(ids + q) : 0u;
+    for (int t = 0; t < 4; ++t) {
+      count(w[t]);
+      if constexpr (sizeof(Id) == 2) count(w[t] >> 16);
     }
-#pragma unroll
-    for (uint32_t t = 0; t < kU; ++t)
-      if (p + t * kDegCountThreads < it.z) atomicAdd(&h[u[t] & (kDegRange - 1)], 1u);
   }
   __syncthreads();
-  const uint32_t v0 = it.x << kDegRangeBits;
+  const uint32_t v0 = blockIdx.x << kDegRangeBits;
   const uint32_t cnt = n - v0 < kDegRange ? n - v0 : kDegRange;
+  const bool split = e1 - e0 > share;
   for (uint32_t q = threadIdx.x; q < cnt; q += kDegCountThreads) {
-    if (!it.w) deg[v0 + q] = h[q];
+    if (!split) deg[v0 + q] = h[q];
     else if (h[q]) atomicAdd(&deg[v0 + q], h[q]);
   }
 }
@@ -290,14 +337,21 @@ static const char* const kBadCsc = "CSC: row pointers not monotone from 0 to nnz
 
 int key_bits_for(uint32_t n) { return bits_for(n); }
 
-void sorted_keys_to_csx(hipStream_t s, const uint64_t* keys, uint64_t m, uint32_t n, int b, uint32_t* ptr,
-                        uint32_t* ent) {
+// row pointers and entries from m sorted keys; before (nullable): distinct keys before each tile
+static void csx_write(hipStream_t s, const uint64_t* keys, uint64_t m, const uint32_t* before, uint32_t m_out,
+                      uint32_t n, int b, uint32_t* ptr, uint32_t* ent) {
   if (m) {
-    csx_kernel<<<grid_for(m), 256, 0, s>>>(keys, m, n, b, ptr, ent);
+    csx_write_kernel<<<(uint32_t)ceil_div(m, kCsxTile), 256, 0, s>>>(keys, m, b, before, ptr, ent);
+    csx_tail_kernel<<<grid_for((uint64_t)n + 1), 256, 0, s>>>(keys, m, n, b, m_out, ptr);
   } else {
     fill_u32_kernel<<<grid_for((uint64_t)n + 1), 256, 0, s>>>(ptr, (uint64_t)n + 1, 0u);
   }
   NWG_LAUNCH_CHECK();
+}
+
+void sorted_keys_to_csx(hipStream_t s, const uint64_t* keys, uint64_t m, uint32_t n, int b, uint32_t* ptr,
+                        uint32_t* ent) {
+  csx_write(s, keys, m, nullptr, (uint32_t)m, n, b, ptr, ent);
 }
 
 // bad[0] = 1 for a CSC in device memory whose row pointers are not monotone from 0 to nnz or
@@ -337,31 +391,25 @@ static void hist_enqueue(hipStream_t s, const HistShape& h, uint32_t n, uint64_t
   NWG_LAUNCH_CHECK();
 }
 
-// The range path for a large CSC (ids below n < 2^32 assumed checked): a sorted copy, range
-// starts read back, work items built on the host.
+// The range path for a large CSC (ids below n < 2^32 assumed checked).
 static void out_degrees_by_range(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* col, uint32_t* deg) {
   const uint32_t nr = (uint32_t)ceil_div(n, kDegRange);
-  DevBuf<uint32_t> ids(nnz), tmp(nnz), start((uint64_t)nr + 1);
-  NWG_HIP(hipMemcpyAsync(ids.p, col, nnz * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
-  radix_sort_keys_u32(s, ids.p, tmp.p, nnz, kDegRangeBits, std::max(kDegRangeBits, bits_for(n)));
-  range_start_kernel<<<grid_for(nnz + 1), 256, 0, s>>>(ids.p, nnz, nr, start.p);
+  fill_u32_kernel<<<grid_for(n), 256, 0, s>>>(deg, n, 0u);
   NWG_LAUNCH_CHECK();
-  std::vector<uint32_t> hs((size_t)nr + 1);
-  NWG_HIP(hipMemcpyAsync(hs.data(), start.p, hs.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  NWG_HIP(hipStreamSynchronize(s));
-  std::vector<uint4> items;
-  for (uint32_t r = 0; r < nr; ++r) {
-    const uint32_t a = hs[r], b = hs[r + 1];
-    const uint32_t split = b - a > kDegItem ? 1u : 0u;
-    for (uint64_t q = a; q < b; q += kDegItem)
-      items.push_back(make_uint4(r, (uint32_t)q, (uint32_t)std::min<uint64_t>(b, q + kDegItem), split));
+  const int bits = std::max(1, bits_for(n) - kDegRangeBits);
+  const dim3 grid(nr, kDegSplit);
+  if (bits <= 8) {
+    DevBuf<uint16_t> low(nnz);
+    DevBuf<uint32_t> start((1u << bits) + 1);
+    radix_partition_low16(s, col, nnz, kDegRangeBits, bits, low.p, start.p);
+    range_count_kernel<uint16_t><<<grid, kDegCountThreads, 0, s>>>(low.p, start.p, n, deg);
+  } else {
+    DevBuf<uint32_t> ids(nnz), tmp(nnz), start((uint64_t)nr + 1);
+    radix_sort_keys_u32(s, ids, tmp, col, nnz, kDegRangeBits, bits_for(n));
+    range_start_kernel<<<grid_for(nnz + 1), 256, 0, s>>>(ids.p, nnz, nr, start.p);
+    range_count_kernel<uint32_t><<<grid, kDegCountThreads, 0, s>>>(ids.p, start.p, n, deg);
   }
-  if (items.empty()) return;
-  DevBuf<uint4> ditems(items.size());
-  NWG_HIP(hipMemcpyAsync(ditems.p, items.data(), items.size() * sizeof(uint4), hipMemcpyHostToDevice, s));
-  range_count_kernel<<<(uint32_t)items.size(), kDegCountThreads, 0, s>>>(ids.p, ditems.p, n, deg);
   NWG_LAUNCH_CHECK();
-  NWG_HIP(hipStreamSynchronize(s));  // the temporaries are freed on return
 }
 
 static void degrees_aligned(const uint32_t* col) {
@@ -392,12 +440,9 @@ void out_degrees_device(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t*
   if (h.chunks) {
     DevBuf<uint32_t> part((uint64_t)h.chunks * h.words);
     hist_enqueue(s, h, n, nnz, col, part.p, deg, nullptr, nullptr);
-    NWG_HIP(hipStreamSynchronize(s));  // before part is freed
     return;
   }
   if (nnz >= kDegSortMin && nnz < (1ull << 32)) {
-    fill_u32_kernel<<<grid_for(n), 256, 0, s>>>(deg, n, 0u);
-    NWG_LAUNCH_CHECK();
     out_degrees_by_range(s, n, nnz, col, deg);
     return;
   }
@@ -440,55 +485,29 @@ void check_device_csc(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* p
   if (bad[1]) throw Error(NWG_EINVAL, "outdeg: some vertex's out-degree is below its number of entries in the CSC");
 }
 
-// Sorted compressed structure from packed keys (consumes keys/tmp).
-static void keys_to_compressed(hipStream_t s, uint32_t n, int b, DevBuf<uint64_t>& keys, DevBuf<uint64_t>& tmp,
-                               uint64_t m, bool clean, DevBuf<uint32_t>& ptr, DevBuf<uint32_t>& ent,
-                               uint64_t* nnz_out) {
-  radix_sort_pairs(s, keys.p, tmp.p, nullptr, nullptr, m, 2 * b);
-  if (clean && m) {
-    DevBuf<uint32_t> flag(m), pos(m + 1);
-    uniq_flag_kernel<<<grid_for(m), 256, 0, s>>>(keys.p, m, flag.p);
-    NWG_LAUNCH_CHECK();
-    exclusive_scan_u32(s, flag.p, pos.p, m);
-    const uint32_t mu = read_back_u32(s, pos.p + m);
-    compact_keys_kernel<<<grid_for(m), 256, 0, s>>>(keys.p, m, flag.p, pos.p, tmp.p);
-    NWG_LAUNCH_CHECK();
-    std::swap(keys, tmp);
-    m = mu;
-    NWG_HIP(hipStreamSynchronize(s));
-  }
-  ptr.alloc((uint64_t)n + 1);
-  ent.alloc(m ? m : 1);
-  if (m) {
-    csx_kernel<<<grid_for(m), 256, 0, s>>>(keys.p, m, n, b, ptr.p, ent.p);
-  } else {
-    fill_u32_kernel<<<grid_for((uint64_t)n + 1), 256, 0, s>>>(ptr.p, (uint64_t)n + 1, 0u);
-  }
-  NWG_LAUNCH_CHECK();
-  *nnz_out = m;
-}
-
-void build_csc_device(hipStream_t s, uint32_t n, uint64_t ne, uint32_t* src, uint32_t* dst, bool clean,
+void build_csc_device(hipStream_t s, uint32_t n, uint64_t ne, const uint32_t* src, const uint32_t* dst, bool clean,
                       nwg_graph* g) {
   NWG_REQUIRE(n >= 1, "graph needs at least one vertex");
   NWG_REQUIRE(ne < (1ull << 32), "edge count must be below 2^32 (uint32 indices)");
   const int b = bits_for(n);
-  uint64_t m = 0;
   DevBuf<uint64_t> keys(ne ? ne : 1), tmp(ne ? ne : 1);
-  if (ne) {
-    DevBuf<uint32_t> flag(ne), pos(ne + 1), bad(1);
-    fill_u32_kernel<<<1, 256, 0, s>>>(bad.p, 1, 0u);
-    edge_flag_kernel<<<grid_for(ne), 256, 0, s>>>(src, dst, ne, n, clean ? 1 : 0, flag.p, bad.p);
+  DevBuf<uint32_t> bad(1);
+  fill_u32_kernel<<<1, 256, 0, s>>>(bad.p, 1, 0u);
+  const uint64_t m = radix_sort_edges(s, EdgeKeySource{src, dst, n, b, clean, bad.p}, ne, keys, tmp);
+  uint64_t nnz = m;
+  const uint32_t tiles = (uint32_t)ceil_div(m, kCsxTile);
+  DevBuf<uint32_t> count, before;
+  if (clean && m) {
+    count.alloc(tiles);
+    before.alloc((uint64_t)tiles + 1);
+    csx_count_kernel<<<tiles, 256, 0, s>>>(keys.p, m, count.p);
     NWG_LAUNCH_CHECK();
-    exclusive_scan_u32(s, flag.p, pos.p, ne);
-    if (read_back_u32(s, bad.p)) throw Error(NWG_EINVAL, "edge list holds a vertex id >= n");
-    m = read_back_u32(s, pos.p + ne);
-    pack_kernel<<<grid_for(ne), 256, 0, s>>>(src, dst, ne, b, 1, flag.p, pos.p, keys.p);
-    NWG_LAUNCH_CHECK();
-    NWG_HIP(hipStreamSynchronize(s));
+    exclusive_scan_u32(s, count.p, before.p, tiles);
+    nnz = read_back_u32(s, before.p + tiles);
   }
-  uint64_t nnz = 0;
-  keys_to_compressed(s, n, b, keys, tmp, m, clean, g->csc_ptr, g->csc_idx, &nnz);
+  g->csc_ptr.alloc((uint64_t)n + 1);
+  g->csc_idx.alloc(nnz ? nnz : 1);
+  csx_write(s, keys.p, m, before.p, (uint32_t)nnz, n, b, g->csc_ptr.p, g->csc_idx.p);
   g->n = n;
   g->nnz = nnz;
   g->outdeg.alloc(n);
@@ -506,16 +525,12 @@ void build_csr_device(hipStream_t s, nwg_graph* g) {
   if (nnz) {
     transpose_keys_kernel<<<grid_for(n), 256, 0, s>>>(n, g->csc_ptr.p, g->csc_idx.p, b, keys.p, pos.p);
     NWG_LAUNCH_CHECK();
-    radix_sort_pairs(s, keys.p, tmp.p, pos.p, pos_tmp.p, nnz, 2 * b);
+    // the CSC's positions ascend by target, and the sort is stable: by source is enough
+    radix_sort_pairs(s, keys, tmp, &pos, &pos_tmp, nnz, b, 2 * b);
   }
   g->csr_ptr.alloc((uint64_t)n + 1);
   g->csr_idx.alloc(nnz ? nnz : 1);
-  if (nnz) {
-    csx_kernel<<<grid_for(nnz), 256, 0, s>>>(keys.p, nnz, n, b, g->csr_ptr.p, g->csr_idx.p);
-  } else {
-    fill_u32_kernel<<<grid_for((uint64_t)n + 1), 256, 0, s>>>(g->csr_ptr.p, (uint64_t)n + 1, 0u);
-  }
-  NWG_LAUNCH_CHECK();
+  csx_write(s, keys.p, nnz, nullptr, (uint32_t)nnz, n, b, g->csr_ptr.p, g->csr_idx.p);
   g->csr_to_csc = std::move(pos);
   NWG_HIP(hipStreamSynchronize(s));
   g->has_csr = true;

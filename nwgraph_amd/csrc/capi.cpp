@@ -18,6 +18,7 @@ using nwg::DeviceGuard;
 using nwg::Error;
 using nwg::guarded;
 using nwg::stage_in;
+using nwg::Staged;
 
 namespace {
 
@@ -136,11 +137,10 @@ int nwg_graph_build_from_edges(nwg_ctx* ctx, uint32_t n, uint64_t ne, const uint
     NWG_REQUIRE((src && dst) || ne == 0, "edge arrays must not be null");
     DeviceGuard dg(ctx->device);
     hipStream_t s = ctx->stream;
-    DevBuf<uint32_t> ds, dd;
-    stage_in(s, ds, src, ne, mem_kind);
-    stage_in(s, dd, dst, ne, mem_kind);
+    Staged<uint32_t> ds(s, const_cast<uint32_t*>(src), ne, mem_kind, true);
+    Staged<uint32_t> dd(s, const_cast<uint32_t*>(dst), ne, mem_kind, true);
     std::unique_ptr<nwg_graph> g(new_graph(ctx));
-    nwg::build_csc_device(s, n, ne, ds.p, dd.p, clean != 0, g.get());
+    nwg::build_csc_device(s, n, ne, ds.dev, dd.dev, clean != 0, g.get());
     *out = g.release();
   });
 }

@@ -389,9 +389,8 @@ struct nwg_graph {
 namespace nwg {
 
 // ---- builder (build.hip) ----
-// Sort-based CSC/CSR construction on the device.  src/dst are device arrays of ne
-// raw edges (they are consumed: contents are undefined afterwards).
-void build_csc_device(hipStream_t s, uint32_t n, uint64_t ne, uint32_t* src, uint32_t* dst,
+// Sort-based CSC/CSR construction on the device.  src/dst are device arrays of ne raw edges.
+void build_csc_device(hipStream_t s, uint32_t n, uint64_t ne, const uint32_t* src, const uint32_t* dst,
                       bool clean, nwg_graph* g);
 void build_csr_device(hipStream_t s, nwg_graph* g);
 int key_bits_for(uint32_t n);  // bits of a vertex id field in packed sort keys
@@ -417,13 +416,31 @@ void check_device_csc(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* p
 // ---- primitives (scan.hip / sort.hip) ----
 // exclusive scan of n values; out has n+1 entries (out[n] = total).
 void exclusive_scan_u32(hipStream_t s, const uint32_t* in, uint32_t* out, uint64_t n);
-// stable LSD radix sort of 64-bit keys over bits [0, key_bits), optional 32-bit payload.
-// Sorted result ends in keys/vals (tmp buffers must have n entries).
-void radix_sort_pairs(hipStream_t s, uint64_t* keys, uint64_t* keys_tmp, uint32_t* vals,
-                      uint32_t* vals_tmp, uint64_t n, int key_bits);
-// stable LSD radix sort of 32-bit keys by their bits [first_bit, end_bit) (the others are
-// carried along unsorted); result in keys (keys_tmp: n entries of scratch).
-void radix_sort_keys_u32(hipStream_t s, uint32_t* keys, uint32_t* keys_tmp, uint64_t n, int first_bit, int end_bit);
+// Stable LSD radix sorts by the key bits [first_bit, end_bit); the result is in keys (and vals),
+// tmp of the same length is scratch: the buffers trade places.
+void radix_sort_pairs(hipStream_t s, DevBuf<uint64_t>& keys, DevBuf<uint64_t>& keys_tmp, DevBuf<uint32_t>* vals,
+                      DevBuf<uint32_t>* vals_tmp, uint64_t n, int first_bit, int end_bit);
+// of the 32-bit keys `in` (left as they are) into keys
+void radix_sort_keys_u32(hipStream_t s, DevBuf<uint32_t>& keys, DevBuf<uint32_t>& keys_tmp, const uint32_t* in,
+                         uint64_t n, int first_bit, int end_bit);
+// Edges as sort keys (dst << bits) | src; self-loops are dropped when asked, and *bad set for an
+// edge with an id >= n.
+struct EdgeKeySource {
+  const uint32_t* src;
+  const uint32_t* dst;
+  uint32_t n;
+  int bits;
+  bool drop_loops;
+  uint32_t* bad;  // device word, 0
+};
+// the sorted keys of ne edges (keys, keys_tmp: ne each); returns how many were kept, throws
+// NWG_EINVAL for an id out of range
+uint64_t radix_sort_edges(hipStream_t s, const EdgeKeySource& e, uint64_t ne, DevBuf<uint64_t>& keys,
+                          DevBuf<uint64_t>& keys_tmp);
+// stable partition of the keys `in` by their bits [shift, shift + bits), of which the low 16 bits are
+// written; start[d] (2^bits + 1): where digit d begins
+void radix_partition_low16(hipStream_t s, const uint32_t* in, uint64_t n, int shift, int bits, uint16_t* low,
+                           uint32_t* start);
 
 // ---- generators (gen.hip) ----
 void rmat_edges_device(hipStream_t s, uint32_t scale, uint32_t a, uint32_t b, uint32_t c, uint64_t seed,

@@ -657,7 +657,7 @@ static void ensure_classes(hipStream_t s, nwg_graph* g) {
       DevBuf<uint32_t> vals_tmp(nnz);
       slice_key_kernel<<<blocks_for(nnz), kThreads, 0, s>>>(n, nnz, rp, a.idx, pp, keys.p, pl.scol.p);
       NWG_LAUNCH_CHECK();
-      radix_sort_pairs(s, keys.p, keys_tmp.p, pl.scol.p, vals_tmp.p, nnz, key_bits_for(n) + 3);
+      radix_sort_pairs(s, keys, keys_tmp, &pl.scol, &vals_tmp, nnz, 0, key_bits_for(n) + 3);
     }
     sseg_kernel<<<blocks_for((uint64_t)ns * (kSlices + 1)), kThreads, 0, s>>>(ns, pl.srows.p, rp, pl.scol.p,
                                                                               pl.sseg.p);

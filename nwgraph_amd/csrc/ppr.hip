@@ -577,7 +577,7 @@ static void build_heavy_slices(hipStream_t s, const ActiveCsc& a, uint32_t n, ui
       NWG_LAUNCH_CHECK();
       int kb = 3;
       while (kb < 64 && (1ull << kb) < (uint64_t)nh * 8) ++kb;
-      radix_sort_pairs(s, keys.p, keys_tmp.p, st.hcol.p, vals_tmp.p, eh, kb);  // stable: sources stay ascending
+      radix_sort_pairs(s, keys, keys_tmp, &st.hcol, &vals_tmp, eh, 0, kb);  // stable: sources stay ascending
       DevBuf<uint32_t> gp((uint64_t)nh * 8 + 1);
       group_ptr_kernel<<<grid1((uint64_t)nh * 8 + 1), kThreads, 0, s>>>(eh, keys.p, (uint64_t)nh * 8, gp.p);
       NWG_LAUNCH_CHECK();

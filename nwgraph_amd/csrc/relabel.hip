@@ -82,7 +82,7 @@ void relabel_build(hipStream_t s, nwg_graph* g) {
     DevBuf<uint64_t> keys(n), tmp(n);
     degree_key_kernel<<<grid1(n), kThreads, 0, s>>>(n, g->outdeg.p, g->csc_ptr.p, b, keys.p);
     NWG_LAUNCH_CHECK();
-    radix_sort_pairs(s, keys.p, tmp.p, nullptr, nullptr, n, 33 + b);
+    radix_sort_pairs(s, keys, tmp, nullptr, nullptr, n, 0, 33 + b);
     order_kernel<<<grid1(n), kThreads, 0, s>>>(n, keys.p, b, g->outdeg.p, rl->order.p, rl->rank.p, rl->outdeg.p);
     NWG_LAUNCH_CHECK();
     NWG_HIP(hipStreamSynchronize(s));
@@ -94,7 +94,7 @@ void relabel_build(hipStream_t s, nwg_graph* g) {
     if (nnz) {
       edge_key_kernel<<<grid1(nnz), kThreads, 0, s>>>(n, nnz, g->csc_ptr.p, g->csc_idx.p, rl->rank.p, b, keys.p);
       NWG_LAUNCH_CHECK();
-      radix_sort_pairs(s, keys.p, tmp.p, nullptr, nullptr, nnz, 2 * b);
+      radix_sort_pairs(s, keys, tmp, nullptr, nullptr, nnz, 0, 2 * b);
     }
     sorted_keys_to_csx(s, keys.p, nnz, n, b, rl->csc_ptr.p, rl->csc_idx.p);
     NWG_HIP(hipStreamSynchronize(s));
