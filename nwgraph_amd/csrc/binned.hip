@@ -186,9 +186,20 @@ __device__ __forceinline__ void finish_rows(const BinParams& P, uint32_t r0, uin
 // 16-byte value store: consecutive lanes then store consecutive 16 bytes, whole lines, which
 // the nontemporal stores of the plan's stream_hints 2 need (a lane storing a whole group
 // with two 16-byte stores wrote every line in two halves, 343 against 315 us at RMAT-25).
+// Weighted: workgroup 0 first folds the previous sweep's L1 partials into werr (a launch of its own
+// took 5 of a sweep's 70 us at RMAT-20), so the bin pass is the first that knows whether the solve
+// has ended with that sweep; the chunk pass stops a sweep later, its values then go unread.
+__device__ __forceinline__ void wfold(const BinParams& P, uint32_t k, double* red);
 template <int NT, bool W = false>
 __global__ __launch_bounds__(kBT) void pr_chunk_kernel(BinParams P) {
-  if (converged_before<W>(P)) return;
+  if constexpr (W) {
+    if (P.iter > 1 && P.werr[P.iter - 2] < P.threshold * (P.thr_scale ? *P.thr_scale : 1.0)) return;
+    __shared__ double red[kBT / 64];
+    if (P.iter > 0 && blockIdx.x == 0) wfold(P, P.iter - 1, red);
+    if (blockIdx.x >= P.n_items1) return;  // launched for the fold alone
+  } else {
+    if (converged_before<W>(P)) return;
+  }
   __shared__ float4 cst4[kChunkSrc / 4];
   float* cst = reinterpret_cast<float*>(cst4);
   __shared__ uint32_t sstart[kBinMaxSegs];
@@ -638,16 +649,19 @@ __global__ __launch_bounds__(256) void pr_bin_combine_kernel(BinParams P) {
       red, gerr, P.n_items2 + blockIdx.x);
 }
 
-// weighted sweep: the sweep's L1 change, the bin items' and combine units' partials added in
-// a fixed order (strided per lane, then a fixed tree)
-__global__ __launch_bounds__(256) void pr_wfold_kernel(BinParams P) {
-  if (converged_before<true>(P)) return;
-  __shared__ double red[4];
+// weighted sweep: the L1 change of sweep k, the bin items' and combine units' partials added in a
+// fixed order (strided per lane, then a fixed tree) by a workgroup of kBT lanes
+__device__ __forceinline__ void wfold(const BinParams& P, uint32_t k, double* red) {
   const uint32_t m = P.n_items2 + P.n_items3;
   double e = 0.0;
-  for (uint32_t q = threadIdx.x; q < m; q += 256) e += P.wpart[q];
-  e = block_sum<256>(e, red);
-  if (threadIdx.x == 0) P.werr[P.iter] = e;
+  for (uint32_t q = threadIdx.x; q < m; q += kBT) e += P.wpart[q];
+  e = block_sum<kBT>(e, red);
+  if (threadIdx.x == 0) P.werr[k] = e;
+}
+__global__ __launch_bounds__(kBT) void pr_wfold_kernel(BinParams P) {
+  if (converged_before<true>(P)) return;
+  __shared__ double red[kBT / 64];
+  wfold(P, P.iter, red);
 }
 
 // ---- layout construction ----
@@ -1103,10 +1117,14 @@ static void enqueue_weighted_bits(hipStream_t s, const BinParams& P) {
 void binned_enqueue_weighted_sweep(hipStream_t s, const BinParams& P) {
   NWG_REQUIRE(P.bw && P.wpart && P.werr && P.basev, "weighted sweep needs weights, partials and a base");
   NWG_REQUIRE(P.bin_bits == 13 || P.bin_bits == 14, "binned sweep: bins of 2^13 or 2^14 rows");
-  if (P.n_items1) pr_chunk_kernel<0, true><<<P.n_items1, kBT, 0, s>>>(P);
+  pr_chunk_kernel<0, true><<<std::max<uint32_t>(P.n_items1, 1), kBT, 0, s>>>(P);
   if (P.bin_bits == 14) enqueue_weighted_bits<14>(s, P);
   else enqueue_weighted_bits<13>(s, P);
-  pr_wfold_kernel<<<1, 256, 0, s>>>(P);
+  NWG_LAUNCH_CHECK();
+}
+
+void binned_enqueue_weighted_fold(hipStream_t s, const BinParams& P) {
+  pr_wfold_kernel<<<1, kBT, 0, s>>>(P);
   NWG_LAUNCH_CHECK();
 }
 

@@ -91,35 +91,50 @@ __device__ __forceinline__ unsigned long long item_update(const ItemParams& P, u
 // the next lane's do not fall on the same banks
 __device__ __forceinline__ uint32_t pos(uint32_t q) { return q + (q >> 3); }
 
-// K values per lane: inclusive fixed-point prefix of the edges [e0, e1), entry q of it for edge
-// b0 + q (b0 = e0 rounded down to 4; entries before e0 are 0)
-template <int NT, int K>
-__device__ __forceinline__ void item_prefix(const ItemParams& P, uint32_t b0, uint32_t e0, uint32_t e1,
-                                            unsigned long long* pre, unsigned long long* wsum) {
-  const uint32_t q0 = threadIdx.x * K;
-  uint32_t u[K];
+// ids of the K entries p0 .. p0 + K of a lane (p0 a multiple of 4): 16-byte loads where whole
+// groups lie in the array, 0 for entries from e1 on
+template <int K>
+__device__ __forceinline__ void item_ids(const uint32_t* __restrict__ ids, uint32_t nnz, uint32_t p0, uint32_t e1,
+                                         uint32_t (&u)[K]) {
 #pragma unroll
   for (int h = 0; h < K; h += 4) {
-    const uint32_t p = b0 + q0 + h;
-    if ((uint64_t)p + 4 <= P.nnz && p < e1) {  // a whole 16-byte group inside the array
-      const u32x4 v = *reinterpret_cast<const u32x4*>(P.col + p);
+    const uint32_t p = p0 + h;
+    if ((uint64_t)p + 4 <= nnz && p < e1) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(ids + p);
       u[h] = v.x;
       u[h + 1] = v.y;
       u[h + 2] = v.z;
       u[h + 3] = v.w;
     } else {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) u[h + t] = p + t < e1 ? P.col[p + t] : 0u;
+      for (int t = 0; t < 4; ++t) u[h + t] = p + t < e1 ? ids[p + t] : 0u;
     }
   }
+}
+
+// K values per lane: inclusive fixed-point prefix of the edges [e0, e1), entry q of it for edge
+// b0 + q (b0 = e0 rounded down to 4; entries before e0 are 0).  w null: value cin[id]; else
+// w * cin[id] scaled by 2^qs.
+template <int NT, int K, bool W>
+__device__ __forceinline__ void item_prefix(const uint32_t* __restrict__ col, const float* w, int qs,
+                                            const float* cin, uint32_t nnz, uint32_t b0, uint32_t e0, uint32_t e1,
+                                            unsigned long long* pre, unsigned long long* wsum) {
+  const uint32_t q0 = threadIdx.x * K;
+  uint32_t u[K];
+  item_ids<K>(col, nnz, b0 + q0, e1, u);
+  uint32_t wt[W ? K : 1];
+  if constexpr (W) item_ids<K>(reinterpret_cast<const uint32_t*>(w), nnz, b0 + q0, e1, wt);
   float c[K];
 #pragma unroll
-  for (int t = 0; t < K; ++t) c[t] = P.cin[u[t]];  // ids outside [e0, e1) are ids too, or 0
+  for (int t = 0; t < K; ++t) c[t] = cin[u[t]];  // ids outside [e0, e1) are ids too, or 0
   unsigned long long v[K], s = 0;
 #pragma unroll
   for (int t = 0; t < K; ++t) {
     const uint32_t p = b0 + q0 + t;
-    s += (p >= e0 && p < e1) ? quantize(c[t]) : 0ull;
+    unsigned long long q;
+    if constexpr (W) q = quantize_signed(__uint_as_float(wt[t]) * c[t], qs);
+    else q = quantize(c[t]);
+    s += (p >= e0 && p < e1) ? q : 0ull;
     v[t] = s;
   }
   unsigned long long inc = wave_inclusive_scan(s);
@@ -128,11 +143,38 @@ __device__ __forceinline__ void item_prefix(const ItemParams& P, uint32_t b0, ui
     if (lane_id() == 63) wsum[threadIdx.x >> 6] = inc;
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < NT / 64 - 1; ++w) off += (uint32_t)w < (threadIdx.x >> 6) ? wsum[w] : 0ull;
+    for (int w2 = 0; w2 < NT / 64 - 1; ++w2) off += (uint32_t)w2 < (threadIdx.x >> 6) ? wsum[w2] : 0ull;
   }
 #pragma unroll
   for (int t = 0; t < K; ++t) pre[pos(q0 + t)] = off + v[t];
   __syncthreads();
+}
+
+// exact sum of the edges [a, b) of an item
+__device__ __forceinline__ unsigned long long item_sum(const unsigned long long* pre, uint32_t b0, uint32_t a,
+                                                       uint32_t b) {
+  if (a >= b) return 0ull;
+  const unsigned long long hi = pre[pos(b - 1 - b0)];
+  return a == b0 ? hi : hi - pre[pos(a - 1 - b0)];
+}
+
+// Adds a piece of long row h (entries [hp0, hp1), this piece's sum `mine`) to the row's counter, that
+// of the item it starts in; true for the last piece, which gets the row's sum and leaves the
+// counters at 0 for the next sweep.  *start: the item the row starts in.
+template <uint32_t S>
+__device__ __forceinline__ bool add_piece(unsigned long long* hsum, uint32_t* hcnt, uint32_t h, uint32_t hp0,
+                                          uint32_t hp1, unsigned long long mine, unsigned long long* z,
+                                          uint32_t* start) {
+  // the row's pieces are those of the items its edges' units lie in
+  const uint32_t a = (uint32_t)(((uint64_t)h + hp0) / S), b = (uint32_t)(((uint64_t)h + hp1 - 1) / S);
+  *start = a;
+  unsigned long long old = __hip_atomic_fetch_add(hsum + a, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // the sum has been added (its old value is back) before the piece is counted
+  asm volatile("s_waitcnt vmcnt(0)" : "+v"(old) : : "memory");
+  if (__hip_atomic_fetch_add(hcnt + a, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != b - a) return false;
+  *z = __hip_atomic_exchange(hsum + a, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(hcnt + a, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
 }
 
 template <int NT>
@@ -168,8 +210,8 @@ __global__ __launch_bounds__(NT) void pr_item_kernel(ItemParams P) {
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * NT) item_prefix<NT, 4>(P, b0, e0, e1, pre, wsum);
-  else item_prefix<NT, 8>(P, b0, e0, e1, pre, wsum);
+  if (e1 - b0 <= 4u * NT) item_prefix<NT, 4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
+  else item_prefix<NT, 8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) ch += __shfl_xor(ch, m, 64);
   if (blockIdx.x == 0) {
@@ -177,11 +219,7 @@ __global__ __launch_bounds__(NT) void pr_item_kernel(ItemParams P) {
     if (threadIdx.x == 0 && P.iter > 0) P.acc[P.iter - 1] = ch;
   }
   if (P.iter > 0 && fixed_to_err(ch) < P.threshold) return;
-  auto sum = [&](uint32_t a, uint32_t b) -> unsigned long long {  // edges [a, b)
-    if (a >= b) return 0ull;
-    const unsigned long long hi = pre[pos(b - 1 - b0)];
-    return a == b0 ? hi : hi - pre[pos(a - 1 - b0)];
-  };
+  auto sum = [&](uint32_t a, uint32_t b) { return item_sum(pre, b0, a, b); };
   unsigned long long err = 0ull;
   if (threadIdx.x < rows) err = item_update(P, r0 + threadIdx.x, dequantize(sum(ra, rb)), xo, bv, dg);
   for (uint32_t q = threadIdx.x + NT; q < rows; q += NT) {
@@ -189,19 +227,10 @@ __global__ __launch_bounds__(NT) void pr_item_kernel(ItemParams P) {
     err += item_update(P, i, dequantize(sum(P.rp[i], P.rp[i + 1])), P.x[i], P.basev ? P.basev[i] : P.base, P.deg[i]);
   }
   if (piece) {
-    // the row's pieces are those of the items its edges' units lie in
-    const uint32_t a = (uint32_t)(((uint64_t)h + hp0) / S), b = (uint32_t)(((uint64_t)h + hp1 - 1) / S);
-    const unsigned long long mine = sum(max(hp0, e0), min(hp1, e1));
-    unsigned long long old = __hip_atomic_fetch_add(P.hsum + a, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // the sum has been added (its old value is back) before the piece is counted
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(old) : : "memory");
-    if (__hip_atomic_fetch_add(P.hcnt + a, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b - a) {
-      // every piece is in: take the sum and leave both counters at 0 for the next sweep
-      const unsigned long long z =
-          __hip_atomic_exchange(P.hsum + a, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(P.hcnt + a, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long z;
+    uint32_t a;
+    if (add_piece<S>(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a))
       err += item_update(P, h, dequantize(z), P.x[h], P.basev ? P.basev[h] : P.base, P.deg[h]);
-    }
   }
   err = wave_sum(err);
   if constexpr (NT > 64) {
@@ -212,6 +241,234 @@ __global__ __launch_bounds__(NT) void pr_item_kernel(ItemParams P) {
   }
   if (threadIdx.x == 0 && err)
     atomicAdd(P.lanes + (P.iter % 3) * kItemLaneSlot + (blockIdx.x % kItemLanes) * kItemLanePad, err);
+}
+
+// ---- weighted ----
+// The L1 changes of a weighted sweep have no bound (fixed_point.hpp's scale covers row sums), so
+// they stay doubles: every item stores its own and, where a long row starts in it, that row's; every
+// workgroup of the next sweep adds them all in one fixed order and stops or goes on, which takes
+// the place of a launch that folds them.
+constexpr uint32_t kWNT = 256;
+
+__device__ __forceinline__ double witem_stop(const WItemParams& P) {
+  return P.thr_scale ? P.threshold * *P.thr_scale : P.threshold;
+}
+
+// L1 change of sweep k from its items' parts; the whole workgroup, result in every lane
+__device__ __forceinline__ double witem_change(const WItemParams& P, uint32_t k, double* red) {
+  const double* part = P.part + (uint64_t)(k & 1u) * 2 * P.count;
+  double e = 0.0;
+  for (uint32_t q = threadIdx.x; q < 2 * P.count; q += kWNT) e += part[q];
+  e = wave_sum(e);
+  if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = e;
+  __syncthreads();
+  return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+__global__ __launch_bounds__(kWNT) void wpr_item_kernel(WItemParams P) {
+  constexpr uint32_t S = item_span(kWNT);
+  static_assert(kWNT == 256, "four waves");
+  __shared__ unsigned long long pre[9 * kWNT];
+  __shared__ unsigned long long wsum[kWNT / 64];
+  __shared__ double red[kWNT / 64], red2[kWNT / 64];
+  const double stop = witem_stop(P);
+  // a solve that stopped before the previous sweep: that sweep stored no parts
+  if (P.iter > 1 && P.err[P.iter - 2] < stop) return;
+  const uint4 d = P.desc[blockIdx.x];
+  const uint32_t e0 = d.x, e1 = d.y, r0 = d.z, rows = d.w & kRowMask;
+  const int qs = *P.qshift;
+  uint32_t ra = 0, rb = 0;
+  float xo = 0.f, bv = 0.f;
+  if (threadIdx.x < rows) {
+    const uint32_t i = r0 + threadIdx.x;
+    ra = P.rp[i];
+    rb = P.rp[i + 1];
+    xo = P.xin[i];
+    bv = P.basev[i];
+  }
+  const bool piece = (threadIdx.x == 0 && (d.w & kHeadPiece)) || (threadIdx.x == 1 && (d.w & kTailPiece));
+  uint32_t h = 0, hp0 = 0, hp1 = 0;
+  if (piece) {
+    h = threadIdx.x == 0 ? r0 - 1 : r0 + rows;
+    hp0 = P.rp[h];
+    hp1 = P.rp[h + 1];
+  }
+  const uint32_t b0 = e0 & ~3u;
+  if (e1 - b0 <= 4u * kWNT) item_prefix<kWNT, 4, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
+  else item_prefix<kWNT, 8, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
+  if (P.iter > 0) {
+    const double ch = witem_change(P, P.iter - 1, red);
+    if (blockIdx.x == 0 && threadIdx.x == 0) P.err[P.iter - 1] = ch;
+    if (ch < stop) return;
+  }
+  auto update = [&](uint32_t i, unsigned long long z, float old, float b) -> double {
+    const float xn = __builtin_fmaf(P.damp, dequantize_signed(z, qs), b);
+    P.xout[i] = xn;
+    return (double)fabsf(xn - old);
+  };
+  double e = 0.0;
+  if (threadIdx.x < rows) e = update(r0 + threadIdx.x, item_sum(pre, b0, ra, rb), xo, bv);
+  for (uint32_t q = threadIdx.x + kWNT; q < rows; q += kWNT) {
+    const uint32_t i = r0 + q;
+    e += update(i, item_sum(pre, b0, P.rp[i], P.rp[i + 1]), P.xin[i], P.basev[i]);
+  }
+  double* part = P.part + (uint64_t)(P.iter & 1u) * 2 * P.count;
+  if (piece) {
+    unsigned long long z;
+    uint32_t a;
+    if (add_piece<S>(P.hsum, P.hcnt, h, hp0, hp1, item_sum(pre, b0, max(hp0, e0), min(hp1, e1)), &z, &a))
+      part[P.count + a] = update(h, z, P.xin[h], P.basev[h]);
+  }
+  e = wave_sum(e);
+  if ((threadIdx.x & 63u) == 0) red2[threadIdx.x >> 6] = e;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = (red2[0] + red2[1]) + (red2[2] + red2[3]);
+}
+
+__global__ __launch_bounds__(256) void witem_init_kernel(WItemParams P, const float* __restrict__ src, float v,
+                                                         float* __restrict__ dst, uint64_t iters) {
+  const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < P.n) dst[i] = src ? src[i] : v;
+  if (i < P.count) {
+    P.hsum[i] = 0ull;
+    P.hcnt[i] = 0u;
+  }
+  if (i < 4ull * P.count) P.part[i] = 0.0;
+  if (i < iters) P.err[i] = 0.0;
+}
+
+__global__ __launch_bounds__(kWNT) void witem_fold_kernel(WItemParams P, uint32_t k) {
+  __shared__ double red[kWNT / 64];
+  if (k > 0 && P.err[k - 1] < witem_stop(P)) return;  // sweep k did nothing
+  const double ch = witem_change(P, k, red);
+  if (threadIdx.x == 0) P.err[k] = ch;
+}
+
+// ---- row sums ----
+// Sums in double, with no value of one row ever added to another's (signed values of any magnitude: a
+// running prefix would cancel): lane t adds its 4 or 8 consecutive values up to the row starts
+// among them, and a segmented scan over the lanes carries what is open.
+__device__ __forceinline__ void seg_scan_step(double& v, uint32_t& f, double pv, uint32_t pf) {
+  if (!f) v += pv;
+  f |= pf;
+}
+
+template <int K>
+__device__ __forceinline__ void item_row_sums(const RowSumParams& P, uint32_t b0, uint32_t e0, uint32_t e1,
+                                              const uint8_t* start, double* pre, double* wv, uint32_t* wf) {
+  const uint32_t q0 = threadIdx.x * K;
+  uint32_t u[K];
+  item_ids<K>(P.idx, P.nnz, b0 + q0, e1, u);
+  double val[K];
+  if (P.gather) {
+    uint32_t wt[K];
+    item_ids<K>(reinterpret_cast<const uint32_t*>(P.src), P.nnz, b0 + q0, e1, wt);
+#pragma unroll
+    for (int t = 0; t < K; ++t) val[t] = (double)P.gather[u[t]] * (double)__uint_as_float(wt[t]);
+  } else {
+#pragma unroll
+    for (int t = 0; t < K; ++t) val[t] = (double)P.src[u[t]];
+  }
+  double run = 0.0;
+  uint32_t open = 0;  // a row starts in the lane's values
+#pragma unroll
+  for (int t = 0; t < K; ++t) {
+    const uint32_t p = b0 + q0 + t;
+    const bool in = p >= e0 && p < e1;
+    if (in && start[q0 + t]) {
+      run = 0.0;
+      open = 1u;
+    }
+    run += in ? val[t] : 0.0;
+    val[t] = run;
+  }
+  // inclusive segmented scan of (run, open) over the wave, then the waves
+  double v = run;
+  uint32_t f = open;
+  const uint32_t lane = lane_id(), w = threadIdx.x >> 6;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double pv = __shfl_up(v, o, 64);
+    const uint32_t pf = (uint32_t)__shfl_up((int)f, o, 64);
+    if (lane >= (uint32_t)o) seg_scan_step(v, f, pv, pf);
+  }
+  if (lane == 63) {
+    wv[w] = v;
+    wf[w] = f;
+  }
+  double cv = __shfl_up(v, 1, 64);
+  uint32_t cf = (uint32_t)__shfl_up((int)f, 1, 64);
+  if (lane == 0) {
+    cv = 0.0;
+    cf = 0u;
+  }
+  __syncthreads();
+  double ov = 0.0;  // open sum before this wave
+  for (uint32_t q = 0; q < w; ++q) ov = wf[q] ? wv[q] : ov + wv[q];
+  const double carry = cf ? cv : ov + cv;  // open sum before this lane
+  bool fresh = false;
+#pragma unroll
+  for (int t = 0; t < K; ++t) {
+    const uint32_t p = b0 + q0 + t;
+    fresh |= p >= e0 && p < e1 && start[q0 + t];
+    pre[pos(q0 + t)] = fresh ? val[t] : carry + val[t];
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ void row_sum_out(const RowSumParams& P, const RowSumOut& o, uint32_t u, double s) {
+  if (!P.gather) {
+    o.out[u] = (float)s;
+    return;
+  }
+  const double x = (double)o.x[u], norm = (double)o.norm[u];
+  // a source without out-edges has no edge that reads its pair
+  o.ab[u] = make_float2((float)(x / norm), (float)(x * ((double)o.d * s) / norm));
+  if (o.gv) o.gv[u] = o.omd * P.gather[u];
+}
+
+__global__ __launch_bounds__(kWNT) void row_sum_kernel(RowSumParams P, RowSumOut o) {
+  __shared__ double pre[9 * kWNT];
+  __shared__ uint8_t start[8 * kWNT];
+  __shared__ double wv[kWNT / 64];
+  __shared__ uint32_t wf[kWNT / 64];
+  const uint4 d = P.desc[blockIdx.x];
+  const uint32_t e0 = d.x, e1 = d.y, r0 = d.z, rows = d.w & kRowMask, b0 = e0 & ~3u;
+  for (uint32_t q = threadIdx.x; q < 2 * kWNT; q += kWNT) reinterpret_cast<uint32_t*>(start)[q] = 0u;
+  __syncthreads();
+  // rows with entries mark their first; the tail piece's row too (r0 + rows)
+  const uint32_t marks = rows + ((d.w & kTailPiece) ? 1u : 0u);
+  for (uint32_t q = threadIdx.x; q < marks; q += kWNT) {
+    const uint32_t a = P.rp[r0 + q];
+    if (P.rp[r0 + q + 1] > a) start[a - b0] = 1;
+  }
+  __syncthreads();
+  if (e1 - b0 <= 4u * kWNT) item_row_sums<4>(P, b0, e0, e1, start, pre, wv, wf);
+  else item_row_sums<8>(P, b0, e0, e1, start, pre, wv, wf);
+  for (uint32_t q = threadIdx.x; q < rows; q += kWNT) {
+    const uint32_t a = P.rp[r0 + q], b = P.rp[r0 + q + 1];
+    row_sum_out(P, o, r0 + q, b > a ? pre[pos(b - 1 - b0)] : 0.0);
+  }
+  if (threadIdx.x == 0 && (d.w & kHeadPiece)) {
+    const uint32_t end = rows || (d.w & kTailPiece) ? P.rp[r0] : e1;
+    P.head[blockIdx.x] = pre[pos(end - 1 - b0)];
+  }
+  if (threadIdx.x == 1 && (d.w & kTailPiece)) P.tail[blockIdx.x] = pre[pos(e1 - 1 - b0)];
+}
+
+// One wave per item: the long row that starts in it, if any, from its pieces (lane-strided, then a
+// fixed tree).
+__global__ __launch_bounds__(256) void row_sum_long_kernel(RowSumParams P, RowSumOut o) {
+  const uint32_t a = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  if (a >= P.count) return;
+  const uint4 d = P.desc[a];
+  if (!(d.w & kTailPiece)) return;
+  const uint32_t h = d.z + (d.w & kRowMask);
+  const uint32_t b = (uint32_t)(((uint64_t)h + P.rp[h + 1] - 1) / item_span(kWNT));
+  double s = lane == 0 ? P.tail[a] : 0.0;
+  for (uint32_t c = a + 1 + lane; c <= b; c += 64) s += P.head[c];
+  s = wave_sum(s);
+  if (lane == 0) row_sum_out(P, o, h, s);
 }
 
 __global__ __launch_bounds__(256) void item_init_kernel(ItemParams P, uint32_t count, float init, float* __restrict__ c0,
@@ -243,9 +500,41 @@ ItemShape item_shape(uint32_t n, uint64_t nnz, uint64_t max_items) {
   ItemShape sh;
   sh.threads = units <= (1ull << 18) ? 64u : 256u;
   const uint64_t count = ceil_div(units, item_span(sh.threads));
-  if (nnz >= (1ull << 31) || count > max_items) sh.threads = 0;
+  if (nnz >= (1ull << 32) || count > max_items) sh.threads = 0;
   else sh.count = (uint32_t)count;
   return sh;
+}
+
+ItemShape item_shape_wide(uint32_t n, uint64_t nnz, uint64_t max_items) {
+  ItemShape sh;
+  sh.threads = kWNT;
+  const uint64_t count = ceil_div((uint64_t)n + nnz, item_span(kWNT));
+  if (nnz >= (1ull << 32) || count > max_items) sh.threads = 0;
+  else sh.count = (uint32_t)count;
+  return sh;
+}
+
+void witems_enqueue_init(hipStream_t s, const WItemParams& P, const float* src, float v, float* dst, uint64_t iters) {
+  const uint64_t m = std::max<uint64_t>({P.n, 4ull * P.count, iters});
+  witem_init_kernel<<<(uint32_t)ceil_div(m, 256), 256, 0, s>>>(P, src, v, dst, iters);
+  NWG_LAUNCH_CHECK();
+}
+
+void witems_enqueue_sweep(hipStream_t s, const WItemParams& P) {
+  wpr_item_kernel<<<P.count, kWNT, 0, s>>>(P);
+  NWG_LAUNCH_CHECK();
+}
+
+void witems_enqueue_fold(hipStream_t s, const WItemParams& P, uint32_t k) {
+  witem_fold_kernel<<<1, kWNT, 0, s>>>(P, k);
+  NWG_LAUNCH_CHECK();
+}
+
+void row_sums_enqueue(hipStream_t s, const RowSumParams& P, const RowSumOut& o) {
+  if (!P.count) return;
+  row_sum_kernel<<<P.count, kWNT, 0, s>>>(P, o);
+  row_sum_long_kernel<<<(P.count + 3) / 4, 256, 0, s>>>(P, o);
+  NWG_LAUNCH_CHECK();
 }
 
 void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, const ItemShape& sh, uint4* desc) {

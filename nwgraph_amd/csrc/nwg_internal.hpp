@@ -270,14 +270,24 @@ struct Captured {
   ~Captured() { reset(); }
 };
 
+// Items of the CSC or CSR of a weighted graph (items.hip).
+struct WItems {
+  ItemShape shape;
+  DevBuf<uint4> desc;
+};
+
 // Cached buffers of the weighted forward / adjoint (wpr.hip).
 struct WState {
-  DevBuf<float> y0, y1, base, lambda, t;
+  DevBuf<float> y0, y1, base, lambda;
   DevBuf<double> part, err;  // per-workgroup L1 partials; per-sweep L1 change
-  DevBuf<double> scale;      // relative threshold: ||b||_1 / (1 - d)
-  DevBuf<uint32_t> scale_done;
+  DevBuf<double> scale;      // the solve's WScale, made on the device and read by its sweeps
   DevBuf<uint32_t> done;     // per sweep: workgroups finished
   DevBuf<uint32_t> row_of;  // CSC position -> row
+  DevBuf<float2> ab;        // per source: x / s and t / s of the raw-weight gradient
+  // item sweep: long rows' sums and pieces, L1 parts
+  DevBuf<unsigned long long> ihsum;
+  DevBuf<uint32_t> ihcnt;
+  DevBuf<double> ipart;
   // binned sweep: weighted layouts of the CSC (forward) and the CSR (adjoint), built on first
   // use and dropped when the weights change; pair values, split-bin partial rows, L1 partials
   std::unique_ptr<BinnedLayout> bl_csc, bl_csr;
@@ -285,13 +295,10 @@ struct WState {
   DevBuf<float> bvals;
   DevBuf<unsigned long long> bpart;
   DevBuf<double> wpart, stats;
-  // captured solve loops (init + max_iters sweeps) of the forward and the adjoint; a call's
-  // varying inputs go to fixed buffers first: the adjoint's grad_x to gin, the binned sweep's
-  // scale exponent to qs
-  std::vector<std::unique_ptr<Captured>> cap_fwd, cap_adj;  // one per segment of sweeps
+  // captured solve loops (init + max_iters sweeps) of the forward and the adjoint, one per segment of
+  // sweeps; the adjoint's grad_x goes to a fixed buffer, gin, first
+  std::vector<std::unique_ptr<Captured>> cap_fwd, cap_adj;
   DevBuf<float> gin;
-  DevBuf<int> qs;
-  int qs_host = 0;
 };
 
 // Degree-ordered copy of a CSC (relabel.hip): new id r is original vertex order[r].
@@ -374,6 +381,7 @@ struct nwg_graph {
   // work items of the weighted sweeps over the CSC (forward) and the CSR (adjoint)
   nwg::DevBuf<uint32_t> w_items_csc_r0, w_items_csc_r1, w_items_csr_r0, w_items_csr_r1;
   uint32_t w_items_csc_n = 0, w_items_csr_n = 0;
+  nwg::WItems wi_csc, wi_csr;
   nwg::Plan plan;
   uint64_t plan_version = 1;
   std::unique_ptr<nwg::Relabeled> rl;  // built when a plan asks for relabel=1
@@ -473,8 +481,10 @@ nwg_plan_params default_plan_for(const nwg_graph* g);
 void binned_build(hipStream_t s, const ActiveCsc& a, uint32_t n, uint64_t nnz, BinnedLayout& L, bool hot,
                   const float* w = nullptr, int bin_bits = 0);
 void binned_enqueue_sweep(hipStream_t s, const BinParams& P);
-// one weighted sweep (P.bw set): chunk, bin and combine passes, then the fold of the L1 partials
+// one weighted sweep (P.bw set): chunk, bin and combine passes; the L1 change is folded by the chunk
+// pass of the next sweep, or by the fold after the last one launched
 void binned_enqueue_weighted_sweep(hipStream_t s, const BinParams& P);
+void binned_enqueue_weighted_fold(hipStream_t s, const BinParams& P);
 // lane counters of iters sweeps cleared / summed into acc[0 .. iters)
 void binned_clear_residuals(hipStream_t s, unsigned long long* lanes, uint64_t iters);
 void binned_fold_residuals(hipStream_t s, const unsigned long long* lanes, unsigned long long* acc, uint64_t iters);

@@ -201,147 +201,28 @@ __global__ __launch_bounds__(kThreads) void winit_kernel(uint32_t n, const float
   }
 }
 
-// base_i = (float)((1-d) * v_i) (v null: uniform 1/n)
-__global__ __launch_bounds__(kThreads) void wbase_kernel(uint32_t n, const float* __restrict__ v, double omd,
-                                                         float* __restrict__ base) {
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  if (i < n) base[i] = v ? (float)(omd * (double)v[i]) : (float)(omd / (double)n);
-}
-
-// Per-row sums over the CSR of v[q] = a[perm[q]] * (b ? b[perm[q]] : 1), in CSR order
-// (deterministic), on the same LDS work items as the sweep.  FP32 with Kahan compensation:
-// the error stays within a few ulp of the sum whatever the row length.
-struct Kahan {
-  float s = 0.f, c = 0.f;
-  __device__ __forceinline__ void add(float v) {
-    const float y = v - c;
-    const float t = s + y;
-    c = (t - s) - y;
-    s = t;
-  }
+// What a solve scales its stop and its fixed point by, made on the device before its sweeps.
+struct WScale {
+  double scale;  // of a relative threshold: ||b||_1 / (1 - d), 1 for the uniform teleport and for b = 0
+  int qshift;    // products are summed in units of 2^(-60 - qshift)
+  int finite;    // b is finite
 };
 
-__global__ __launch_bounds__(kThreads) void csr_rowsum_kernel(const uint32_t* __restrict__ rp,
-                                                              const uint32_t* __restrict__ perm,
-                                                              const float* __restrict__ a,
-                                                              const float* __restrict__ b,
-                                                              const uint32_t* __restrict__ item_r0,
-                                                              const uint32_t* __restrict__ item_r1, uint32_t n_items,
-                                                              float* __restrict__ out) {
-  __shared__ float vals[kItemNnz];
-  __shared__ uint32_t lrows[kItemRows];   // an item's long rows (offsets from its first row)
-  __shared__ uint32_t wlong[kThreads / 64];
-  __shared__ float red_f[kThreads / 64];
-  for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
-    const uint32_t r0 = item_r0[it], r1 = item_r1[it];
-    const uint32_t p0 = rp[r0], p1 = rp[r1];
-    if (p1 - p0 > kItemNnz) {
-      // a single long row: strided compensated partial sums, fixed-tree reduction of the
-      // partials and of their compensations
-      Kahan k;
-      for (uint32_t q = p0 + threadIdx.x; q < p1; q += kThreads) {
-        const uint32_t e = perm[q];
-        k.add(b ? a[e] * b[e] : a[e]);
-      }
-      const float hi = block_sum<kThreads>(k.s, red_f);
-      __syncthreads();
-      const float lo = block_sum<kThreads>(-k.c, red_f);
-      if (threadIdx.x == 0) out[r0] = hi + lo;
-    } else {
-      for (uint32_t q = threadIdx.x; q < p1 - p0; q += kThreads) {
-        const uint32_t e = perm[p0 + q];
-        vals[q] = b ? a[e] * b[e] : a[e];
-      }
-      __syncthreads();
-      // rows of up to kLaneRow entries: one lane each; longer rows: one wave each (lane-strided
-      // compensated partial sums, butterfly sums of the partials and of their compensations),
-      // listed in row order through a ballot
-      const uint32_t u = r0 + threadIdx.x;
-      uint32_t ra = 0, rb = 0;
-      if (u < r1) {
-        ra = rp[u] - p0;
-        rb = rp[u + 1] - p0;
-      }
-      const bool longrow = rb - ra > kLaneRow;
-      if (u < r1 && !longrow) {
-        Kahan k;
-        for (uint32_t q = ra; q < rb; ++q) k.add(vals[q]);
-        out[u] = k.s - k.c;
-      }
-      const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-      const unsigned long long lm = __ballot(longrow);
-      if (lane == 0) wlong[wv] = (uint32_t)__popcll(lm);
-      __syncthreads();
-      uint32_t off = 0, nlong = 0;
-      for (uint32_t q = 0; q < kThreads / 64; ++q) {
-        off += q < wv ? wlong[q] : 0u;
-        nlong += wlong[q];
-      }
-      if (longrow)
-        lrows[off + __builtin_amdgcn_mbcnt_hi((uint32_t)(lm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)lm, 0u))] =
-            threadIdx.x;
-      __syncthreads();
-      for (uint32_t k2 = wv; k2 < nlong; k2 += kThreads / 64) {
-        const uint32_t ri = r0 + lrows[k2];
-        const uint32_t la = rp[ri] - p0, lb = rp[ri + 1] - p0;
-        Kahan k;
-        for (uint32_t q = la + lane; q < lb; q += 64) k.add(vals[q]);
-        float hi = k.s, lo = -k.c;
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-          hi += __shfl_xor(hi, o, 64);
-          lo += __shfl_xor(lo, o, 64);
-        }
-        if (lane == 0) out[ri] = hi + lo;
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// Scale of a relative threshold, ||b||_1 / (1 - d) for the fixed point's constant term b
-// (1 when b is null: the uniform teleport (1 - d) / n summing to 1 - d), or 1 when b is 0.
-// Contiguous ranges per workgroup, partials added in workgroup order by the last workgroup
-// to finish: deterministic.
+// The fixed point's constant term b into dst -- (float)((1-d) * v_i) for a forward solve (v null:
+// uniform 1/n), v itself for an adjoint -- and per workgroup, over a contiguous range, the sum and
+// the largest of |b| (NaN or infinity shows in the sum).
 constexpr uint32_t kNormBlocks = 256;
-__global__ __launch_bounds__(kThreads) void l1_scale_kernel(uint32_t n, const float* __restrict__ b, double inv_omd,
-                                                            double* __restrict__ part, uint32_t* __restrict__ done,
-                                                            double* __restrict__ scale) {
-  __shared__ double red_d[kThreads / 64];
-  __shared__ uint32_t last;
-  double e = 0.0;
-  if (b) {
-    const uint64_t per = ((uint64_t)n + gridDim.x - 1) / gridDim.x;
-    const uint64_t i0 = (uint64_t)blockIdx.x * per, i1 = i0 + per < n ? i0 + per : n;
-    for (uint64_t i = i0 + threadIdx.x; i < i1; i += kThreads) e += (double)fabsf(b[i]);
-  }
-  e = block_sum<kThreads>(e, red_d);
-  if (threadIdx.x == 0) {
-    part[blockIdx.x] = e;
-    __threadfence();
-    last = atomicAdd(done, 1u) == gridDim.x - 1 ? 1u : 0u;
-  }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (uint32_t q = 0; q < gridDim.x; ++q) s += __hip_atomic_load(part + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *scale = !b ? 1.0 : (s > 0.0 ? s * inv_omd : 1.0);
-    *done = 0u;
-  }
-}
-
-// Per workgroup over a contiguous range: sum and max of |b| (the bound a binned weighted sweep
-// scales its fixed point by); NaN or infinity shows in the sum.
-__global__ __launch_bounds__(kThreads) void abs_stats_kernel(uint32_t n, const float* __restrict__ b,
-                                                             double* __restrict__ out) {
+__global__ __launch_bounds__(kThreads) void wprep_kernel(uint32_t n, const float* __restrict__ v, bool forward,
+                                                         double omd, float* __restrict__ dst,
+                                                         double* __restrict__ out) {
   __shared__ double red_d[kThreads / 64];
   const uint64_t per = ((uint64_t)n + gridDim.x - 1) / gridDim.x;
   const uint64_t i0 = (uint64_t)blockIdx.x * per, i1 = i0 + per < n ? i0 + per : n;
   double sum = 0.0, mx = 0.0;
   for (uint64_t i = i0 + threadIdx.x; i < i1; i += kThreads) {
-    const double a = (double)fabsf(b[i]);
+    const float b = !forward ? v[i] : v ? (float)(omd * (double)v[i]) : (float)(omd / (double)n);
+    dst[i] = b;
+    const double a = (double)fabsf(b);
     sum += a;
     mx = a > mx ? a : mx;
   }
@@ -360,11 +241,65 @@ __global__ __launch_bounds__(kThreads) void abs_stats_kernel(uint32_t n, const f
   }
 }
 
-// *bad = 1 when some weight is negative or not finite
-__global__ __launch_bounds__(kThreads) void weight_check_kernel(uint64_t nnz, const float* __restrict__ w,
-                                                                uint32_t* __restrict__ bad) {
+// Scale of the fixed point: 2^t with 2^t * 2M in [1/2, 1), M a bound of every product and partial
+// row sum, from b (the constant term) in exact arithmetic:
+//   forward  x' = b + d A x, x0 = 1/n: |sum_u w(u->i) x_u| <= ||x||_1 <= max(1, ||b||_1 / (1-d))
+//            (A is column-stochastic: ||A x||_1 <= ||x||_1);
+//   adjoint  l' = b + d A^T l, l0 = b: |sum_i w(u->i) l_i| <= ||l||_inf <= ||b||_inf / (1-d)
+//            (each row of A^T sums to 1).
+// The factor 2 covers the FP32 rounding of the iterates.  One workgroup, a fixed tree.
+__global__ __launch_bounds__(kNormBlocks) void wscale_kernel(const double* __restrict__ stats, bool forward,
+                                                             bool uniform, double omd, WScale* __restrict__ out) {
+  __shared__ double red_d[kNormBlocks / 64];
+  double mx = stats[2 * threadIdx.x + 1];
+  const double sum = block_sum<kNormBlocks>(stats[2 * threadIdx.x], red_d);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    const double y = __shfl_xor(mx, o, 64);
+    mx = y > mx ? y : mx;
+  }
+  if ((threadIdx.x & 63) == 0) red_d[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (uint32_t q = 0; q < kNormBlocks / 64; ++q) mx = red_d[q] > mx ? red_d[q] : mx;
+    const double M = forward ? fmax(1.0, sum / omd) : mx / omd;
+    int t = 0;
+    if (M > 0.0 && isfinite(M)) (void)frexp(2.0 * M, &t);
+    out->scale = uniform || !(sum > 0.0) ? 1.0 : sum / omd;
+    out->qshift = -t;
+    out->finite = isfinite(sum) ? 1 : 0;
+  }
+}
+
+// out = the iterate of the solve's last sweep: sweep k leaves it in y[(k + 1) & 1], and the solve ended
+// with the first sweep whose change is below the threshold, or after iters
+__global__ __launch_bounds__(kThreads) void wout_kernel(uint32_t n, const float* __restrict__ y0,
+                                                        const float* __restrict__ y1, const double* __restrict__ err,
+                                                        uint32_t iters, double threshold,
+                                                        const double* __restrict__ thr_scale,
+                                                        float* __restrict__ out) {
+  const double stop = thr_scale ? threshold * *thr_scale : threshold;
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t ended = iters;
+  for (uint32_t k = 0; k < iters; k += 64) {
+    const unsigned long long m = __ballot(k + lane < iters && err[k + lane] < stop);
+    if (m) {
+      ended = k + (uint32_t)__builtin_ctzll(m) + 1;
+      break;
+    }
+  }
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i < n) out[i] = (ended & 1u) ? y1[i] : y0[i];
+}
+
+// the raw weights kept, and *bad = 1 when some weight is negative or not finite
+__global__ __launch_bounds__(kThreads) void weight_copy_kernel(uint64_t nnz, const float* __restrict__ w,
+                                                               float* __restrict__ raw, uint32_t* __restrict__ bad) {
   const uint64_t p = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (p < nnz && !(w[p] >= 0.f && w[p] <= 3.402823466e38f)) *bad = 1u;
+  if (p >= nnz) return;
+  const float v = w[p];
+  raw[p] = v;
+  if (!(v >= 0.f && v <= 3.402823466e38f)) *bad = 1u;
 }
 
 // row of every CSC position (upper bound in the row pointers)
@@ -379,6 +314,10 @@ __global__ __launch_bounds__(kThreads) void row_of_kernel(uint32_t n, uint64_t n
     else hi = mid;
   }
   row[p] = lo;
+}
+
+__global__ __launch_bounds__(64) void wclear_kernel(uint32_t* __restrict__ p) {
+  if (threadIdx.x == 0) *p = 0u;
 }
 
 __global__ __launch_bounds__(kThreads) void normalise_kernel(uint64_t nnz, const uint32_t* __restrict__ col,
@@ -403,14 +342,21 @@ __global__ __launch_bounds__(kThreads) void edge_grad_kernel(uint64_t nnz, const
   if (p < nnz) gw[p] = (d * lambda[row[p]]) * x[col[p]];
 }
 
-__global__ __launch_bounds__(kThreads) void chain_apply_kernel(uint64_t nnz, const uint32_t* __restrict__ col,
-                                                               const float* __restrict__ t,
-                                                               const float* __restrict__ s, float* __restrict__ gw) {
+// The raw-weight gradient of edge p from u = col[p]:
+//   (d lambda_row x_u - t_u) / s_u,  t_u = sum_j d lambda_j x_u w(u->j),
+// as d lambda_row * (x_u / s_u) - t_u / s_u with both quotients made once per source (ab): one
+// gather of 8 bytes per edge.  Edge gradient, row sums over a gathered copy and chain rule as
+// three passes took 885 us for 16 M edges on MI355X (the row sums 647: two scattered reads per edge,
+// long rows one load at a time); row sums over items with the products made in place and this
+// pass take GRAD_US.
+__global__ __launch_bounds__(kThreads) void raw_grad_kernel(uint64_t nnz, const uint32_t* __restrict__ row,
+                                                            const uint32_t* __restrict__ col, float d,
+                                                            const float* __restrict__ lambda,
+                                                            const float2* __restrict__ ab, float* __restrict__ gw) {
   const uint64_t p = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (p < nnz) {
-    const uint32_t u = col[p];
-    gw[p] = (gw[p] - t[u]) / s[u];
-  }
+  if (p >= nnz) return;
+  const float2 q = ab[col[p]];
+  gw[p] = __builtin_fmaf(d * lambda[row[p]], q.x, -q.y);
 }
 
 __global__ __launch_bounds__(kThreads) void scale_kernel(uint32_t n, float a, const float* __restrict__ src,
@@ -456,42 +402,71 @@ static uint32_t persistent_grid(uint32_t n_items) {
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(n_items, (uint64_t)cus * 8));
 }
 
-static void ensure_csr_items(hipStream_t s, nwg_graph* g) {
-  build_csr_device(s, g);
-  if (!g->w_items_csr_n && g->n) build_items(s, g->csr_ptr.p, g->n, g->w_items_csr_r0, g->w_items_csr_r1, &g->w_items_csr_n);
+// the class items of the pull sweep over a compressed structure, built on first use
+static void ensure_pull_items(hipStream_t s, nwg_graph* g, bool csr) {
+  uint32_t& count = csr ? g->w_items_csr_n : g->w_items_csc_n;
+  if (count || !g->n) return;
+  if (csr) build_items(s, g->csr_ptr.p, g->n, g->w_items_csr_r0, g->w_items_csr_r1, &count);
+  else build_items(s, g->csc_ptr.p, g->n, g->w_items_csc_r0, g->w_items_csc_r1, &count);
+}
+
+// 256-lane items (items.hip) of the CSC or CSR, built on first use
+static const WItems& ensure_items(hipStream_t s, nwg_graph* g, bool csr) {
+  WItems& it = csr ? g->wi_csr : g->wi_csc;
+  if (!it.desc.n) {
+    it.shape = item_shape_wide(g->n, g->nnz, 1ull << 31);
+    NWG_REQUIRE(it.shape.threads, "weighted solves take fewer than 2^31 edges");
+    it.desc.alloc(std::max<uint32_t>(it.shape.count, 1));
+    items_build(s, g->n, g->nnz, csr ? g->csr_ptr.p : g->csc_ptr.p, it.shape, it.desc.p);
+  }
+  return it;
+}
+
+// s_u over the CSR's rows (items.hip, RowSumParams)
+static void csr_row_sums(hipStream_t s, nwg_graph* g, const uint32_t* idx, const float* src, const float* gather,
+                         const RowSumOut& out) {
+  const WItems& it = ensure_items(s, g, true);
+  DevBuf<double> pieces(2ull * std::max<uint32_t>(it.shape.count, 1));
+  RowSumParams R{};
+  R.desc = it.desc.p;
+  R.rp = g->csr_ptr.p;
+  R.idx = idx;
+  R.src = src;
+  R.gather = gather;
+  R.n = g->n;
+  R.nnz = (uint32_t)g->nnz;
+  R.count = it.shape.count;
+  R.head = pieces.p;
+  R.tail = pieces.p + it.shape.count;
+  row_sums_enqueue(s, R, out);
 }
 
 void weights_set(hipStream_t s, nwg_graph* g, const float* w_dev, bool normalize) {
   const uint64_t nnz = g->nnz;
-  ensure_csr_items(s, g);
+  build_csr_device(s, g);
   g->w_raw.ensure(nnz ? nnz : 1);
   g->w_csc.ensure(nnz ? nnz : 1);
   g->w_csr.ensure(nnz ? nnz : 1);
   g->w_rowsum.ensure(g->n);
-  if (nnz) NWG_HIP(hipMemcpyAsync(g->w_raw.p, w_dev, nnz * 4, hipMemcpyDeviceToDevice, s));
+  // raw weights all finite and >= 0: the fixed-point bound of the exact weighted sweeps holds
+  DevBuf<uint32_t> bad(1);
+  wclear_kernel<<<1, 64, 0, s>>>(bad.p);
+  if (nnz) weight_copy_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, w_dev, g->w_raw.p, bad.p);
+  NWG_LAUNCH_CHECK();
   if (normalize) {
-    if (g->w_items_csr_n) {
-      csr_rowsum_kernel<<<persistent_grid(g->w_items_csr_n), kThreads, 0, s>>>(
-          g->csr_ptr.p, g->csr_to_csc.p, g->w_raw.p, nullptr, g->w_items_csr_r0.p, g->w_items_csr_r1.p,
-          g->w_items_csr_n, g->w_rowsum.p);
-      NWG_LAUNCH_CHECK();
-    }
-    normalise_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csc_idx.p, g->w_raw.p, g->w_rowsum.p, g->w_csc.p);
+    RowSumOut o{};
+    o.out = g->w_rowsum.p;
+    csr_row_sums(s, g, g->csr_to_csc.p, g->w_raw.p, nullptr, o);
+    if (nnz) normalise_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csc_idx.p, g->w_raw.p, g->w_rowsum.p, g->w_csc.p);
     NWG_LAUNCH_CHECK();
   } else {
     std::vector<float> ones(g->n, 1.0f);
     NWG_HIP(hipMemcpyAsync(g->w_rowsum.p, ones.data(), (size_t)g->n * 4, hipMemcpyHostToDevice, s));
     if (nnz) NWG_HIP(hipMemcpyAsync(g->w_csc.p, w_dev, nnz * 4, hipMemcpyDeviceToDevice, s));
+    NWG_HIP(hipStreamSynchronize(s));  // before ones goes
   }
-  gather_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csr_to_csc.p, g->w_csc.p, g->w_csr.p);
+  if (nnz) gather_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csr_to_csc.p, g->w_csc.p, g->w_csr.p);
   NWG_LAUNCH_CHECK();
-  // raw weights all finite and >= 0: the binned weighted sweep's fixed-point bound holds
-  DevBuf<uint32_t> bad(1);
-  NWG_HIP(hipMemsetAsync(bad.p, 0, sizeof(uint32_t), s));
-  if (nnz) {
-    weight_check_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->w_raw.p, bad.p);
-    NWG_LAUNCH_CHECK();
-  }
   uint32_t hb = 0;
   NWG_HIP(hipMemcpyAsync(&hb, bad.p, sizeof hb, hipMemcpyDeviceToHost, s));
   NWG_HIP(hipStreamSynchronize(s));
@@ -504,68 +479,102 @@ void weights_set(hipStream_t s, nwg_graph* g, const float* w_dev, bool normalize
   }
 }
 
-// Runs the fixed point y <- fma(d, sum w y, base) from y0 over (rp, col, w) in the cached
-// buffers of `st`; returns the sweeps executed and leaves the result in `out`.
-// rhs: the constant term b whose L1 norm scales a relative threshold (null: the uniform
-// teleport).  L (nullable): run the binned weighted sweep over this layout, its products
-// scaled by 2^qshift.  The init and the max_iters sweeps run as one HIP graph captured into
-// cap (re-captured when a buffer, the layout or a parameter changes), so the host launches
-// one graph per solve instead of up to four kernels per sweep; base, y0 and rhs must be
-// buffers that stay the same from call to call.
-static uint64_t fixed_point(nwg_ctx* ctx, WState& st, std::vector<std::unique_ptr<Captured>>& caps,
-                            const uint32_t* rp, const uint32_t* col,
-                            const float* w, const DevBuf<uint32_t>& r0, const DevBuf<uint32_t>& r1, uint32_t n_items,
-                            uint32_t n, const float* base, const float* y0, bool y0_uniform, float damping,
-                            float threshold, uint64_t max_iters, float* out, nwg_pr_info* info, const float* rhs,
-                            const BinnedLayout* L = nullptr, int qshift = 0) {
+// The sweep a weighted solve runs.  The exact sweeps (items, binned) need the weights normalised per
+// source from non-negative raw weights: then every weight is in [0, 1] and each source's out-weights
+// sum to 1, which the fixed-point bound (wscale_kernel) relies on.
+enum class WSweep { kPull, kItems, kBinned };
+
+// One fixed point y <- fma(d, sum w y, b) to solve: over the CSC (forward) or the CSR (adjoint).
+struct WSolve {
+  bool csr;
+  const uint32_t* rp;
+  const uint32_t* col;
+  const float* w;
+  const float* base;  // b
+  const float* y0;    // first iterate; null: uniform 1/n
+  bool uniform;       // b is the uniform teleport's (a relative threshold is then absolute)
+  float damping, threshold;
+  uint64_t max_iters;
+  float* out;
+};
+
+// Runs the fixed point in the cached buffers of `st` and leaves the last iterate in q.out.  L: the layout
+// of a binned sweep.  The init and the max_iters sweeps run as HIP graphs of a segment of sweeps each,
+// captured into caps (again when a buffer, the layout or a parameter changes), so the host launches
+// one graph per segment; base and y0 must be buffers that stay the same from call to call.  st.scale
+// holds the solve's WScale.  Between segments the host reads the sweeps' changes.  `then` queues
+// what follows the solve; with eager it is queued behind every segment before the changes are
+// read, so that a solve that ends in its first segment waits for the device once.  False when b
+// was not finite (an exact sweep is then no answer).
+template <class F>
+static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std::unique_ptr<Captured>>& caps,
+                        const WSolve& q, WSweep kind, const BinnedLayout* L, nwg_pr_info* info, bool eager, F&& then) {
   hipStream_t s = ctx->stream;
+  const uint32_t n = g->n;
+  const uint64_t max_iters = q.max_iters;
   st.y0.ensure(n);
   st.y1.ensure(n);
   st.done.ensure(std::max<uint64_t>(max_iters, 1));
   st.err.ensure(std::max<uint64_t>(max_iters, 1));
   float* y[2] = {st.y0.p, st.y1.p};
-  const uint32_t grid = persistent_grid(n_items);
-  st.part.ensure(std::max<uint32_t>(grid, kNormBlocks));
   const bool relative = info && (info->flags & NWG_INFO_RELATIVE_THRESHOLD);
-  if (relative) {
-    st.scale.ensure(1);
-    st.scale_done.ensure(1);
-    NWG_HIP(hipMemsetAsync(st.scale_done.p, 0, sizeof(uint32_t), s));
-    l1_scale_kernel<<<kNormBlocks, kThreads, 0, s>>>(n, rhs, 1.0 / (1.0 - (double)damping), st.part.p,
-                                                    st.scale_done.p, st.scale.p);
-    NWG_LAUNCH_CHECK();
-  }
-  if (L) {
-    st.qs.ensure(1);
-    st.qs_host = qshift;
-    NWG_HIP(hipMemcpyAsync(st.qs.p, &st.qs_host, sizeof(int), hipMemcpyHostToDevice, s));
+  const double* thr_scale = relative ? &reinterpret_cast<const WScale*>(st.scale.p)->scale : nullptr;
+  const int* qshift = &reinterpret_cast<const WScale*>(st.scale.p)->qshift;
+  const WItems* it = nullptr;
+  uint32_t grid = 0;
+  if (kind == WSweep::kItems) {
+    it = &ensure_items(s, g, q.csr);
+    st.ihsum.ensure(it->shape.count);
+    st.ihcnt.ensure(it->shape.count);
+    st.ipart.ensure(4ull * it->shape.count);
+  } else if (kind == WSweep::kBinned) {
     st.bvals.ensure(L->pairs);
     st.bpart.ensure(std::max<uint64_t>((uint64_t)L->n_slots << L->bin_bits, 1));
     st.wpart.ensure(std::max<uint64_t>((uint64_t)L->n_items2 + L->n_items3, 1));
+  } else {
+    ensure_pull_items(s, g, q.csr);
+    grid = persistent_grid(q.csr ? g->w_items_csr_n : g->w_items_csc_n);
+    st.part.ensure(grid);
   }
-  WParams P{};
-  P.rp = rp;
-  P.col = col;
-  P.w = w;
-  P.item_r0 = r0.p;
-  P.item_r1 = r1.p;
-  P.n_items = n_items;
-  P.base = base;
-  P.damp = damping;
-  P.part = st.part.p;
-  P.done = st.done.p;
-  P.err = st.err.p;
-  P.threshold = (double)threshold;
-  P.thr_scale = relative ? st.scale.p : nullptr;
-  // sweeps [k0, k1) (and the init with k0 = 0) on stream q
-  auto enqueue = [&](hipStream_t q, uint64_t k0, uint64_t k1) {
+  // sweeps [k0, k1) (and the init with k0 = 0) on stream t
+  auto enqueue = [&](hipStream_t t, uint64_t k0, uint64_t k1) {
+    const float* src = q.y0;
+    const float uniform = (float)(1.0 / n);
+    if (kind == WSweep::kItems) {
+      WItemParams I{};
+      I.desc = it->desc.p;
+      I.rp = q.rp;
+      I.col = q.col;
+      I.w = q.w;
+      I.basev = q.base;
+      I.damp = q.damping;
+      I.n = n;
+      I.nnz = (uint32_t)g->nnz;
+      I.count = it->shape.count;
+      I.qshift = qshift;
+      I.hsum = st.ihsum.p;
+      I.hcnt = st.ihcnt.p;
+      I.part = st.ipart.p;
+      I.err = st.err.p;
+      I.threshold = (double)q.threshold;
+      I.thr_scale = thr_scale;
+      if (k0 == 0) witems_enqueue_init(t, I, src, uniform, y[0], max_iters);
+      for (uint64_t k = k0; k < k1; ++k) {
+        I.iter = (uint32_t)k;
+        I.xin = y[k & 1];
+        I.xout = y[(k + 1) & 1];
+        witems_enqueue_sweep(t, I);
+      }
+      if (k1 > k0) witems_enqueue_fold(t, I, (uint32_t)(k1 - 1));
+      return;
+    }
     if (k0 == 0) {
-      winit_kernel<<<grid1(std::max<uint64_t>(n, max_iters)), kThreads, 0, q>>>(
-          n, y0_uniform ? nullptr : y0, (float)(1.0 / n), y[0], st.done.p, st.err.p, max_iters);
+      winit_kernel<<<grid1(std::max<uint64_t>(n, max_iters)), kThreads, 0, t>>>(n, src, uniform, y[0], st.done.p,
+                                                                               st.err.p, max_iters);
       NWG_LAUNCH_CHECK();
     }
-    if (L) {
-      // binned sweep: x double-buffered as y[k & 1] -> y[(k + 1) & 1]; its L1 change goes to st.err
+    if (kind == WSweep::kBinned) {
+      // x double-buffered as y[k & 1] -> y[(k + 1) & 1]; the L1 change goes to st.err
       BinParams B{};
       B.brow = L->brow.p;
       B.bsrc = L->bsrc.p;
@@ -581,48 +590,63 @@ static uint64_t fixed_point(nwg_ctx* ctx, WState& st, std::vector<std::unique_pt
       B.item_hd = L->item_hd.p;
       B.hsrc = L->hsrc.p;
       B.n_hot = L->n_hot;
-      B.basev = base;
-      B.damp = damping;
+      B.basev = q.base;
+      B.damp = q.damping;
       B.n = n;
       B.n_items1 = L->n_items1;
       B.n_items2 = L->n_items2;
       B.bin_bits = L->bin_bits;
       B.n_items3 = L->n_items3;
-      B.threshold = (double)threshold;
-      B.thr_scale = P.thr_scale;
+      B.threshold = (double)q.threshold;
+      B.thr_scale = thr_scale;
       B.bw = L->bw.p;
-      B.qshift = st.qs.p;
+      B.qshift = qshift;
       B.wpart = st.wpart.p;
       B.werr = st.err.p;
       for (uint64_t k = k0; k < k1; ++k) {
         B.iter = (uint32_t)k;
         B.cin = y[k & 1];
         B.x = y[(k + 1) & 1];
-        binned_enqueue_weighted_sweep(q, B);
+        binned_enqueue_weighted_sweep(t, B);
       }
-    } else {
-      for (uint64_t k = k0; k < k1; ++k) {
-        P.iter = (uint32_t)k;
-        P.xin = y[k & 1];
-        P.xout = y[(k + 1) & 1];
-        wsweep_kernel<<<grid, kThreads, 0, q>>>(P);
-        NWG_LAUNCH_CHECK();
-      }
+      if (k1 > k0) binned_enqueue_weighted_fold(t, B);
+      return;
+    }
+    WParams P{};
+    P.rp = q.rp;
+    P.col = q.col;
+    P.w = q.w;
+    P.item_r0 = q.csr ? g->w_items_csr_r0.p : g->w_items_csc_r0.p;
+    P.item_r1 = q.csr ? g->w_items_csr_r1.p : g->w_items_csc_r1.p;
+    P.n_items = q.csr ? g->w_items_csr_n : g->w_items_csc_n;
+    P.base = q.base;
+    P.damp = q.damping;
+    P.part = st.part.p;
+    P.done = st.done.p;
+    P.err = st.err.p;
+    P.threshold = (double)q.threshold;
+    P.thr_scale = thr_scale;
+    for (uint64_t k = k0; k < k1; ++k) {
+      P.iter = (uint32_t)k;
+      P.xin = y[k & 1];
+      P.xout = y[(k + 1) & 1];
+      wsweep_kernel<<<grid, kThreads, 0, t>>>(P);
+      NWG_LAUNCH_CHECK();
     }
   };
   CaptureKey key;
-  const void* ptrs[CaptureKey::kPtrs] = {st.y0.p, st.y1.p, base, y0, st.err.p, st.done.p, st.part.p, rp, col, w,
-                                         L, L ? st.bvals.p : nullptr, L ? st.bpart.p : nullptr,
-                                         L ? st.wpart.p : nullptr, L ? st.qs.p : nullptr,
-                                         relative ? st.scale.p : nullptr};
-  for (int q = 0; q < CaptureKey::kPtrs; ++q) key.ptrs[q] = ptrs[q];
+  const void* ptrs[CaptureKey::kPtrs] = {st.y0.p, st.y1.p, q.base, q.y0, st.err.p, st.done.p, q.rp, q.col, q.w,
+                                         st.scale.p, kind == WSweep::kPull ? (void*)st.part.p : nullptr,
+                                         L ? st.bvals.p : nullptr, L ? st.bpart.p : nullptr, L ? st.wpart.p : nullptr,
+                                         it ? st.ihsum.p : nullptr, it ? (void*)st.ipart.p : nullptr};
+  for (int k = 0; k < CaptureKey::kPtrs; ++k) key.ptrs[k] = ptrs[k];
   key.iters = max_iters;
-  key.damping = damping;
-  key.threshold = threshold;
+  key.damping = q.damping;
+  key.threshold = q.threshold;
   // the layout's device arrays stand behind its build number: a layout made after the weights
   // changed may sit at the old one's host address
-  key.plan_version = L ? L->build_id : n_items;
-  key.extra = (relative ? 1u : 0u) | (y0_uniform ? 2u : 0u);
+  key.plan_version = L ? L->build_id : grid;
+  key.extra = (relative ? 1u : 0u) | (q.y0 ? 0u : 2u) | ((uint32_t)kind << 2);
   // the segments' graphs, captured when missing or stale
   uint64_t nseg = 0;
   for (uint64_t k0 = 0; k0 < max_iters || (k0 == 0 && nseg == 0); k0 = segment_end(k0, max_iters)) {
@@ -650,46 +674,40 @@ static uint64_t fixed_point(nwg_ctx* ctx, WState& st, std::vector<std::unique_pt
     }
     if (k1 >= max_iters) break;
   }
-  double scale_now = 1.0;
-  if (relative) {
-    NWG_HIP(hipMemcpyAsync(&scale_now, st.scale.p, sizeof(double), hipMemcpyDeviceToHost, s));
-    NWG_HIP(hipStreamSynchronize(s));
-  }
-  const double stop_now = relative ? (double)threshold * scale_now : (double)threshold;
+  std::vector<double> h(std::max<uint64_t>(max_iters, 1), 0.0);
+  WScale sc{1.0, 0, 1};
+  double stop = (double)q.threshold;
+  uint64_t iters = max_iters, seg = 0;
   NWG_HIP(hipEventRecord(ctx->ev0, s));
-  uint64_t seg = 0;
   for (uint64_t k0 = 0;; k0 = segment_end(k0, max_iters), ++seg) {
     const uint64_t k1 = segment_end(k0, max_iters);
     NWG_HIP(hipGraphLaunch(caps[seg]->exec, s));
-    if (k1 >= max_iters) break;
-    double last_err = 0.0;  // the segment's last sweep: stop when it converged
-    NWG_HIP(hipMemcpyAsync(&last_err, st.err.p + (k1 - 1), sizeof(double), hipMemcpyDeviceToHost, s));
+    NWG_HIP(hipEventRecord(ctx->ev1, s));
+    wout_kernel<<<grid1(n), kThreads, 0, s>>>(n, y[0], y[1], st.err.p, (uint32_t)k1, (double)q.threshold, thr_scale,
+                                             q.out);
+    NWG_LAUNCH_CHECK();
+    if (eager) then();
+    if (k0 == 0) NWG_HIP(hipMemcpyAsync(&sc, st.scale.p, sizeof sc, hipMemcpyDeviceToHost, s));
+    if (k1 > k0)
+      NWG_HIP(hipMemcpyAsync(h.data() + k0, st.err.p + k0, (k1 - k0) * sizeof(double), hipMemcpyDeviceToHost, s));
     NWG_HIP(hipStreamSynchronize(s));
-    if (last_err < stop_now) break;
+    if (kind != WSweep::kPull && !sc.finite) return false;
+    if (relative) stop = (double)q.threshold * sc.scale;
+    bool ended = k1 >= max_iters;
+    for (uint64_t k = k0; k < k1; ++k)
+      if (h[k] < stop) {
+        iters = k + 1;
+        ended = true;
+        break;
+      }
+    if (ended) break;
   }
-  NWG_HIP(hipEventRecord(ctx->ev1, s));
-  std::vector<double> h(std::max<uint64_t>(max_iters, 1));
-  NWG_HIP(hipMemcpyAsync(h.data(), st.err.p, max_iters * sizeof(double), hipMemcpyDeviceToHost, s));
-  double scale = 1.0;
-  if (relative) NWG_HIP(hipMemcpyAsync(&scale, st.scale.p, sizeof(double), hipMemcpyDeviceToHost, s));
-  NWG_HIP(hipStreamSynchronize(s));
-  const double stop = relative ? (double)threshold * scale : (double)threshold;
-  uint64_t iters = max_iters;
-  double last = 0.0;
-  for (uint64_t k = 0; k < max_iters; ++k) {
-    last = h[k];
-    if (last < stop) {
-      iters = k + 1;
-      break;
-    }
-  }
-  NWG_HIP(hipMemcpyAsync(out, y[iters & 1], (size_t)n * 4, hipMemcpyDeviceToDevice, s));
-  NWG_HIP(hipStreamSynchronize(s));
+  if (!eager) then();
   if (info) {
     float ms = 0.f;
     NWG_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     info->iterations = iters;
-    info->final_error = max_iters ? last : 0.0;
+    info->final_error = iters ? h[iters - 1] : 0.0;
     info->ms_total = ms;
     info->ms_per_iter = iters ? ms / (double)iters : 0.0;
     info->sweep_ms_avg = 0.0;
@@ -697,7 +715,7 @@ static uint64_t fixed_point(nwg_ctx* ctx, WState& st, std::vector<std::unique_pt
     if (info->error_trace)
       for (uint64_t k = 0; k < iters && k < info->error_trace_len; ++k) info->error_trace[k] = h[k];
   }
-  return iters;
+  return true;
 }
 
 static WState& wstate(nwg_graph* g) {
@@ -705,42 +723,17 @@ static WState& wstate(nwg_graph* g) {
   return *g->wst;
 }
 
-// The binned weighted sweep runs when the graph's plan (or, before any plan, the size-based
-// default) asks for the binned sweep and the weights are normalised per source from
-// non-negative raw weights: then every weight is in [0, 1] and each source's out-weights sum
-// to 1, which the fixed-point bound below relies on.
-static bool weighted_binned(const nwg_graph* g) {
+// Weighted sweeps over items up to kItemsWeighted items (about a million rows and edges), which every
+// workgroup's sum of the previous sweep's parts still hides behind its gathers; measured on MI355X
+// (RMAT, edge factor 16, us per sweep, items / binned): WEIGHTED_CROSS.  Above, and where the plan
+// names a bin size, the binned sweep when the plan (or, before any plan, its size) asks for it.
+constexpr uint32_t kItemsWeighted = 1024;
+static WSweep weighted_sweep(const nwg_graph* g, float damping) {
+  if (!g->w_normalized || !g->w_nonneg || g->nnz == 0) return WSweep::kPull;
   const nwg_plan_params pp = g->plan.built ? g->plan.params : default_plan_for(g);
-  return pp.binned != 0 && g->w_normalized && g->w_nonneg && g->nnz > 0;
-}
-
-// Scale of the binned weighted sweep's fixed point: 2^t with 2^t * 2M in [1/2, 1), M a bound
-// of every product and partial row sum, from b (the constant term) in exact arithmetic:
-//   forward  x' = b + d A x, x0 = 1/n: |sum_u w(u->i) x_u| <= ||x||_1 <= max(1, ||b||_1 / (1-d))
-//            (A is column-stochastic: ||A x||_1 <= ||x||_1);
-//   adjoint  l' = b + d A^T l, l0 = b: |sum_i w(u->i) l_i| <= ||l||_inf <= ||b||_inf / (1-d)
-//            (each row of A^T sums to 1).
-// The factor 2 covers the FP32 rounding of the iterates.  False when b is not finite (the
-// pull sweep then runs and shows the NaN / infinity as the reference would).
-static bool fixed_point_scale(hipStream_t s, WState& st, uint32_t n, const float* b, bool forward, float damping,
-                              int* t) {
-  st.stats.ensure(2 * kNormBlocks);
-  abs_stats_kernel<<<kNormBlocks, kThreads, 0, s>>>(n, b, st.stats.p);
-  NWG_LAUNCH_CHECK();
-  std::vector<double> h(2 * kNormBlocks);
-  NWG_HIP(hipMemcpyAsync(h.data(), st.stats.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-  NWG_HIP(hipStreamSynchronize(s));
-  double sum = 0.0, mx = 0.0;
-  for (uint32_t q = 0; q < kNormBlocks; ++q) {
-    sum += h[2 * q];
-    mx = std::max(mx, h[2 * q + 1]);
-  }
-  if (!std::isfinite(sum)) return false;
-  const double omd = 1.0 - (double)damping;
-  const double M = forward ? std::max(1.0, sum / omd) : mx / omd;
-  *t = 0;
-  if (M > 0.0) std::frexp(2.0 * M, t), *t = -*t;
-  return true;
+  if (pp.binned && pp.bin_bits) return WSweep::kBinned;
+  if (item_shape_wide(g->n, g->nnz, kItemsWeighted).threads && damping >= 0.f && damping < 1.f) return WSweep::kItems;
+  return pp.binned ? WSweep::kBinned : WSweep::kPull;
 }
 
 static const BinnedLayout* weighted_layout(hipStream_t s, nwg_graph* g, WState& st, bool csr) {
@@ -762,24 +755,49 @@ static const BinnedLayout* weighted_layout(hipStream_t s, nwg_graph* g, WState& 
   return L.get();
 }
 
+// b, its scale and statistics, on the device
+static void prepare_scale(hipStream_t s, WState& st, uint32_t n, const float* v, bool forward, float damping,
+                          float* b) {
+  const double omd = 1.0 - (double)damping;
+  st.stats.ensure(2 * kNormBlocks);
+  st.scale.ensure(sizeof(WScale) / sizeof(double));
+  wprep_kernel<<<kNormBlocks, kThreads, 0, s>>>(n, v, forward, omd, b, st.stats.p);
+  wscale_kernel<<<1, kNormBlocks, 0, s>>>(st.stats.p, forward, forward && !v, omd,
+                                          reinterpret_cast<WScale*>(st.scale.p));
+  NWG_LAUNCH_CHECK();
+}
+
+// solves q with the graph's sweep, or with the pull sweep when b was not finite (which shows the NaN /
+// infinity as the reference would)
+template <class F>
+static void weighted_solve(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std::unique_ptr<Captured>>& caps,
+                           const WSolve& q, nwg_pr_info* info, F&& then) {
+  const WSweep kind = weighted_sweep(g, q.damping);
+  const BinnedLayout* L = kind == WSweep::kBinned ? weighted_layout(ctx->stream, g, st, q.csr) : nullptr;
+  if (!fixed_point(ctx, g, st, caps, q, kind, L, info, kind == WSweep::kItems, then))
+    (void)fixed_point(ctx, g, st, caps, q, WSweep::kPull, nullptr, info, false, then);
+}
+
 void wpr_forward(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float* x_dev, float damping, float threshold,
                  uint64_t max_iters, nwg_pr_info* info) {
   hipStream_t s = ctx->stream;
   NWG_REQUIRE(g->has_weights, "graph has no weights (nwg_graph_set_weights)");
   NWG_REQUIRE(max_iters < (1ull << 31), "max_iters too large");
-  if (!g->w_items_csc_n && g->n)
-    build_items(s, g->csc_ptr.p, g->n, g->w_items_csc_r0, g->w_items_csc_r1, &g->w_items_csc_n);
   WState& st = wstate(g);
   st.base.ensure(g->n);
-  wbase_kernel<<<grid1(g->n), kThreads, 0, s>>>(g->n, teleport_dev, 1.0 - (double)damping, st.base.p);
-  NWG_LAUNCH_CHECK();
-  const BinnedLayout* L = nullptr;
-  int t = 0;
-  if (weighted_binned(g) && fixed_point_scale(s, st, g->n, st.base.p, true, damping, &t))
-    L = weighted_layout(s, g, st, false);
-  fixed_point(ctx, st, st.cap_fwd, g->csc_ptr.p, g->csc_idx.p, g->w_csc.p, g->w_items_csc_r0, g->w_items_csc_r1,
-              g->w_items_csc_n, g->n, st.base.p, nullptr, true, damping, threshold, max_iters, x_dev, info,
-              teleport_dev ? st.base.p : nullptr, L, t);
+  prepare_scale(s, st, g->n, teleport_dev, true, damping, st.base.p);
+  WSolve q{};
+  q.rp = g->csc_ptr.p;
+  q.col = g->csc_idx.p;
+  q.w = g->w_csc.p;
+  q.base = st.base.p;
+  q.uniform = !teleport_dev;
+  q.damping = damping;
+  q.threshold = threshold;
+  q.max_iters = max_iters;
+  q.out = x_dev;
+  weighted_solve(ctx, g, st, st.cap_fwd, q, info, [] {});
+  NWG_HIP(hipStreamSynchronize(s));
 }
 
 void wpr_backward(nwg_ctx* ctx, nwg_graph* g, const float* x_dev, const float* gx_dev, float* gw_dev, float* gv_dev,
@@ -788,47 +806,53 @@ void wpr_backward(nwg_ctx* ctx, nwg_graph* g, const float* x_dev, const float* g
   NWG_REQUIRE(g->has_weights, "graph has no weights (nwg_graph_set_weights)");
   NWG_REQUIRE(max_iters < (1ull << 31), "max_iters too large");
   NWG_REQUIRE(!raw || g->w_normalized, "raw-weight gradients need weights set with normalize=1");
-  ensure_csr_items(s, g);
+  build_csr_device(s, g);
   const uint32_t n = g->n;
   const uint64_t nnz = g->nnz;
   WState& st = wstate(g);
   st.lambda.ensure(n);
-  // adjoint fixed point: lambda = g + d A^T lambda, started from g
-  // grad_x into a fixed buffer, so that the captured loop serves every call
+  // adjoint fixed point: lambda = g + d A^T lambda, started from g; grad_x in a fixed buffer, so
+  // that the captured loop serves every call
   st.gin.ensure(n);
-  NWG_HIP(hipMemcpyAsync(st.gin.p, gx_dev, (size_t)n * sizeof(float), hipMemcpyDeviceToDevice, s));
-  const BinnedLayout* L = nullptr;
-  int t = 0;
-  if (weighted_binned(g) && fixed_point_scale(s, st, n, st.gin.p, false, damping, &t))
-    L = weighted_layout(s, g, st, true);
-  fixed_point(ctx, st, st.cap_adj, g->csr_ptr.p, g->csr_idx.p, g->w_csr.p, g->w_items_csr_r0, g->w_items_csr_r1,
-              g->w_items_csr_n, n, st.gin.p, st.gin.p, false, damping, threshold, max_iters, st.lambda.p, info,
-              st.gin.p, L, t);
-  if (gw_dev && nnz) {
-    if (!st.row_of.n) {
-      st.row_of.alloc(nnz);
-      row_of_kernel<<<grid1(nnz), kThreads, 0, s>>>(n, nnz, g->csc_ptr.p, st.row_of.p);
-      NWG_LAUNCH_CHECK();
-    }
-    edge_grad_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, st.row_of.p, g->csc_idx.p, damping, st.lambda.p, x_dev,
-                                                     gw_dev);
-    NWG_LAUNCH_CHECK();
-    if (raw) {
-      st.t.ensure(n);
-      if (g->w_items_csr_n) {
-        csr_rowsum_kernel<<<persistent_grid(g->w_items_csr_n), kThreads, 0, s>>>(
-            g->csr_ptr.p, g->csr_to_csc.p, gw_dev, g->w_csc.p, g->w_items_csr_r0.p, g->w_items_csr_r1.p,
-            g->w_items_csr_n, st.t.p);
-        NWG_LAUNCH_CHECK();
-      }
-      chain_apply_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csc_idx.p, st.t.p, g->w_rowsum.p, gw_dev);
-      NWG_LAUNCH_CHECK();
-    }
-  }
-  if (gv_dev) {
-    scale_kernel<<<grid1(n), kThreads, 0, s>>>(n, 1.0f - damping, st.lambda.p, gv_dev);
+  prepare_scale(s, st, n, gx_dev, false, damping, st.gin.p);
+  WSolve q{};
+  q.csr = true;
+  q.rp = g->csr_ptr.p;
+  q.col = g->csr_idx.p;
+  q.w = g->w_csr.p;
+  q.base = st.gin.p;
+  q.y0 = st.gin.p;
+  q.damping = damping;
+  q.threshold = threshold;
+  q.max_iters = max_iters;
+  q.out = st.lambda.p;
+  const bool edges = gw_dev && nnz;
+  if (edges && !st.row_of.n) {
+    st.row_of.alloc(nnz);
+    row_of_kernel<<<grid1(nnz), kThreads, 0, s>>>(n, nnz, g->csc_ptr.p, st.row_of.p);
     NWG_LAUNCH_CHECK();
   }
+  if (edges && raw) st.ab.ensure(n);
+  weighted_solve(ctx, g, st, st.cap_adj, q, info, [&] {
+    if (edges && raw) {
+      RowSumOut o{};
+      o.x = x_dev;
+      o.norm = g->w_rowsum.p;
+      o.ab = st.ab.p;
+      o.gv = gv_dev;
+      o.d = damping;
+      o.omd = 1.0f - damping;
+      csr_row_sums(s, g, g->csr_idx.p, g->w_csr.p, st.lambda.p, o);
+      raw_grad_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, st.row_of.p, g->csc_idx.p, damping, st.lambda.p, st.ab.p,
+                                                      gw_dev);
+    } else {
+      if (edges)
+        edge_grad_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, st.row_of.p, g->csc_idx.p, damping, st.lambda.p, x_dev,
+                                                         gw_dev);
+      if (gv_dev) scale_kernel<<<grid1(n), kThreads, 0, s>>>(n, 1.0f - damping, st.lambda.p, gv_dev);
+    }
+    NWG_LAUNCH_CHECK();
+  });
   NWG_HIP(hipStreamSynchronize(s));
 }
 

@@ -127,6 +127,49 @@ def test_resident_items_stop_and_personalise(ctx, n):
     g.close()
 
 
+@pytest.mark.parametrize("side", ["in", "out"])  # the degrees are those of the CSC's or the CSR's rows
+@pytest.mark.parametrize("kind", KINDS)
+def test_weighted_items_match_float64(ctx, kind, side):
+    """Weighted forward and adjoint over items, and the raw-weight gradient over the CSR's items.  With
+    u = 2^-24: a forward sweep rounds each (positive) score six times at most, weight normalisation
+    included, so 12 of them stay within 72 u of every score; an adjoint sweep is off by at most 6 u of
+    the largest |lambda|, damped by d; the gradient's two terms are at most d |lambda| x_u / s_u."""
+    deg = np.asarray(_degrees(kind), np.int64)
+    n, m = deg.size, int(deg.sum())
+    rng = np.random.default_rng(8)
+    a, b = np.repeat(np.arange(n), deg), rng.integers(0, n, m)
+    src, dst = (b, a) if side == "in" else (a, b)
+    g = ctx.graph_from_edges(n, src.astype(np.uint32), dst.astype(np.uint32), clean=False)
+    ptr, col, _ = g.csc()
+    row = np.repeat(np.arange(n), np.diff(ptr.astype(np.int64)))
+    w = rng.uniform(0.1, 1.0, m).astype(np.float32)
+    c = rng.normal(size=n).astype(np.float32)
+    g.set_weights(w)
+    x, fi = g.wpr_forward(None, D, 0.0, SWEEPS)
+    gw, gv, bi = g.wpr_backward(x, c, D, 0.0, SWEEPS)
+    assert fi["iterations"] == bi["iterations"] == SWEEPS
+    u = 2.0**-24
+    total = np.bincount(col, weights=w.astype(np.float64), minlength=n)
+    wn = w / total[col]
+    want = np.full(n, 1.0 / n)
+    ferr = []
+    for _ in range(SWEEPS):
+        y = (1 - D) / n + D * np.bincount(row, weights=wn * want[col], minlength=n)
+        ferr.append(np.abs(y - want).sum())
+        want = y
+    assert np.all(np.abs(x - want) <= 72 * u * want)
+    assert np.abs(fi["error_trace"] - np.array(ferr)).max() <= 2 * 72 * u * max(want.sum(), 1.0)
+    lam, lmax = c.astype(np.float64), np.abs(c).max()
+    for _ in range(SWEEPS):
+        lam = c + D * np.bincount(col, weights=wn * lam[row], minlength=n)
+        lmax = max(lmax, np.abs(lam).max())
+    assert np.abs(gv - (1 - D) * lam).max() <= (6 / (1 - D) + 2) * u * lmax
+    t = want * np.bincount(col, weights=D * lam[row] * wn, minlength=n)
+    ge = (D * lam[row] * want[col] - t[col]) / total[col] if m else np.zeros(0)
+    assert np.all(np.abs(gw - ge) <= 2 * (72 + 6 / (1 - D) + 8) * u * D * lmax * (want / np.maximum(total, 0.1))[col])
+    g.close()
+
+
 def test_noalloc_damping_above_one_keeps_float_sums(ctx):
     """The exact sums cover damping factors in [0, 1]; above, the float row sums serve the call.  A
     sweep is off by at most m * 2^-24 for a row of m float terms and 3 * 2^-24 for its other
