@@ -189,13 +189,13 @@ __device__ __forceinline__ void finish_rows(const BinParams& P, uint32_t r0, uin
 // Weighted: workgroup 0 first folds the previous sweep's L1 partials into werr (a launch of its own
 // took 5 of a sweep's 70 us at RMAT-20), so the bin pass is the first that knows whether the solve
 // has ended with that sweep; the chunk pass stops a sweep later, its values then go unread.
-__device__ __forceinline__ void wfold(const BinParams& P, uint32_t k, double* red);
+__device__ __forceinline__ double wfold(const BinParams& P, uint32_t k, double* red);
 template <int NT, bool W = false>
 __global__ __launch_bounds__(kBT) void pr_chunk_kernel(BinParams P) {
   if constexpr (W) {
     if (P.iter > 1 && P.werr[P.iter - 2] < P.threshold * (P.thr_scale ? *P.thr_scale : 1.0)) return;
     __shared__ double red[kBT / 64];
-    if (P.iter > 0 && blockIdx.x == 0) wfold(P, P.iter - 1, red);
+    if (P.iter > 0 && blockIdx.x == 0) (void)wfold(P, P.iter - 1, red);
     if (blockIdx.x >= P.n_items1) return;  // launched for the fold alone
   } else {
     if (converged_before<W>(P)) return;
@@ -651,17 +651,19 @@ __global__ __launch_bounds__(256) void pr_bin_combine_kernel(BinParams P) {
 
 // weighted sweep: the L1 change of sweep k, the bin items' and combine units' partials added in a
 // fixed order (strided per lane, then a fixed tree) by a workgroup of kBT lanes
-__device__ __forceinline__ void wfold(const BinParams& P, uint32_t k, double* red) {
+__device__ __forceinline__ double wfold(const BinParams& P, uint32_t k, double* red) {
   const uint32_t m = P.n_items2 + P.n_items3;
   double e = 0.0;
   for (uint32_t q = threadIdx.x; q < m; q += kBT) e += P.wpart[q];
   e = block_sum<kBT>(e, red);
   if (threadIdx.x == 0) P.werr[k] = e;
+  return e;
 }
-__global__ __launch_bounds__(kBT) void pr_wfold_kernel(BinParams P) {
-  if (converged_before<true>(P)) return;
+__global__ __launch_bounds__(kBT) void pr_wfold_kernel(BinParams P, WMail mail) {
   __shared__ double red[kBT / 64];
-  wfold(P, P.iter, red);
+  double e = 0.0;
+  if (!converged_before<true>(P)) e = wfold(P, P.iter, red);  // else the sweep did nothing
+  wmail_post(mail, P.werr, P.iter, e);
 }
 
 // ---- layout construction ----
@@ -799,12 +801,14 @@ __global__ __launch_bounds__(256) void residual_clear_kernel(unsigned long long*
 
 // acc[k] = sum of sweep k's lane counters (exact integer sum); one thread per sweep
 __global__ __launch_bounds__(256) void residual_fold_kernel(const unsigned long long* __restrict__ lanes,
-                                                            unsigned long long* __restrict__ acc, uint64_t iters) {
+                                                            unsigned long long* __restrict__ acc, uint64_t iters,
+                                                            unsigned long long* __restrict__ mail) {
   const uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x;
   if (k >= iters) return;
   unsigned long long t = 0ull;
   for (uint32_t l = 0; l < kBinAccLanes; ++l) t += lanes[k * kBinAccStride + (uint64_t)l * kBinAccPad];
   acc[k] = t;
+  if (mail) mail[k] = t;
 }
 
 }  // namespace
@@ -1123,8 +1127,8 @@ void binned_enqueue_weighted_sweep(hipStream_t s, const BinParams& P) {
   NWG_LAUNCH_CHECK();
 }
 
-void binned_enqueue_weighted_fold(hipStream_t s, const BinParams& P) {
-  pr_wfold_kernel<<<1, kBT, 0, s>>>(P);
+void binned_enqueue_weighted_fold(hipStream_t s, const BinParams& P, const WMail& mail) {
+  pr_wfold_kernel<<<1, kBT, 0, s>>>(P, mail);
   NWG_LAUNCH_CHECK();
 }
 
@@ -1135,9 +1139,10 @@ void binned_clear_residuals(hipStream_t s, unsigned long long* lanes, uint64_t i
   NWG_LAUNCH_CHECK();
 }
 
-void binned_fold_residuals(hipStream_t s, const unsigned long long* lanes, unsigned long long* acc, uint64_t iters) {
+void binned_fold_residuals(hipStream_t s, const unsigned long long* lanes, unsigned long long* acc, uint64_t iters,
+                           unsigned long long* mail) {
   if (!iters) return;
-  residual_fold_kernel<<<(uint32_t)((iters + 255) / 256), 256, 0, s>>>(lanes, acc, iters);
+  residual_fold_kernel<<<(uint32_t)((iters + 255) / 256), 256, 0, s>>>(lanes, acc, iters, mail);
   NWG_LAUNCH_CHECK();
 }
 

@@ -61,6 +61,7 @@ int nwg_create(nwg_ctx** out, int device) {
     NWG_HIP(hipEventCreate(&ctx->ev0));
     NWG_HIP(hipEventCreate(&ctx->ev1));
     nwg::noalloc_setup(device);
+    NWG_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->mail), nwg::kMailWords * 8, hipHostMallocDefault));
     size_t total_bytes = 0;
     NWG_HIP(hipDeviceTotalMem(&total_bytes, device));
     ctx->pool = std::make_shared<nwg::DevPool>(total_bytes / 64);
@@ -82,6 +83,7 @@ void nwg_destroy(nwg_ctx* ctx) {
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
+  if (ctx->mail) (void)hipHostFree(ctx->mail);
   if (ctx->pool) ctx->pool->close();  // graphs that outlive the context free their memory directly
   if (ctx->capture_stream) (void)hipStreamDestroy(ctx->capture_stream);
   if (prev >= 0) (void)hipSetDevice(prev);

@@ -7,6 +7,8 @@
 
 #include <cstdint>
 
+#include "items.hpp"
+
 namespace nwg {
 
 // Native 4 x 32-bit vector (one 16-byte load or store); the nontemporal builtins take it.
@@ -78,6 +80,15 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T* lds /* NT/64 + 1 entri
   *total = lds[NW];
   __syncthreads();
   return r;
+}
+
+// One workgroup leaves a segment's L1 changes and the solve's scales for the host (items.hpp, WMail):
+// err[first .. k), and last for sweep k, whose own store it may just have made.
+__device__ __forceinline__ void wmail_post(const WMail& m, const double* err, uint32_t k, double last) {
+  if (!m.words) return;
+  if (threadIdx.x < 2) m.words[threadIdx.x] = m.scale[threadIdx.x];
+  for (uint32_t q = m.first + threadIdx.x; q < k; q += blockDim.x) m.words[2 + q] = __double_as_longlong(err[q]);
+  if (threadIdx.x == 0) m.words[2 + k] = __double_as_longlong(last);
 }
 
 // Fixed-point accumulation of the L1 change: integer atomics make the sum

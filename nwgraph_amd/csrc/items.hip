@@ -7,7 +7,7 @@
 // thousands of in-edges outlasts everything else.
 //
 // Row i starts at unit D(i) = i + rp[i] of n + nnz units (one per edge, one per row), and item c
-// owns the units [c S, (c + 1) S), S = 4 * threads:
+// owns the units [c S, (c + 1) S), S = kSpan = 1020:
 //   * every row of at most S in-edges that starts in the window, whole (its edges may reach
 //     into the next window: at most 2 S edges are staged);
 //   * of a longer row, the edges whose units fall in the window.  Its pieces lie in consecutive
@@ -34,13 +34,18 @@ namespace nwg {
 
 namespace {
 
+// Lanes of an item.  Measured on MI355X, us per sweep with 128 / 256 / 512 / 1024 lanes: RMAT-12
+// 6.0 / 5.4 / 5.7 / 7.2, RMAT-16 8.9 / 8.8 / 9.5 / 9.7, RMAT-18 21.8 / 21.3 / 21.6 / 30.6; with 64 RMAT-12
+// took 6.1: its span of 252 units cuts more rows into pieces, whose sums meet in atomics.
+constexpr uint32_t kNT = 256;
+
 constexpr uint32_t kHeadPiece = 1u << 30;  // the item's first edges belong to a long row begun before it
 constexpr uint32_t kTailPiece = 1u << 31;  // its last edges to a long row that goes on after it
 constexpr uint32_t kRowMask = kHeadPiece - 1;
 
-// units per item; an item stages at most 2 span - 2 edges, and 3 before them for alignment, in
-// the 8 NT places it has
-__host__ __device__ constexpr uint32_t item_span(uint32_t threads) { return 4u * threads - 4u; }
+// units per item; an item stages at most 2 kSpan - 2 edges, and 3 before them for alignment, in
+// the 8 kNT places it has
+constexpr uint32_t kSpan = 4u * kNT - 4u;
 
 // first row i in [0, n] with i + rp[i] >= unit (n if none)
 __device__ __forceinline__ uint32_t first_row_from(const uint32_t* __restrict__ rp, uint32_t n, uint64_t unit) {
@@ -57,20 +62,20 @@ __device__ __forceinline__ uint32_t first_row_from(const uint32_t* __restrict__ 
 // the item, their edges lie in [e0, e1) after the head piece (of row r0 - 1) and before the
 // tail piece (of row r0 + rows).
 __global__ __launch_bounds__(256) void item_desc_kernel(uint32_t n, uint64_t nnz, const uint32_t* __restrict__ rp,
-                                                        uint32_t span, uint32_t count, uint4* __restrict__ desc) {
+                                                        uint32_t count, uint4* __restrict__ desc) {
   const uint32_t c = blockIdx.x * 256 + threadIdx.x;
   if (c >= count) return;
-  const uint64_t u0 = (uint64_t)c * span, u1 = u0 + span;
+  const uint64_t u0 = (uint64_t)c * kSpan, u1 = u0 + kSpan;
   const uint32_t r0 = first_row_from(rp, n, u0), r1 = first_row_from(rp, n, u1);
   const uint32_t p0 = rp[r0], p1 = rp[r1];
   uint32_t e0 = p0, e1 = p1, rows = r1 - r0, flags = 0;
   // row r0 - 1: a long one whose last edge (unit r0 - 1 + p0 - 1) is not before the window
-  if (r0 > 0 && p0 - rp[r0 - 1] > span && (uint64_t)(r0 - 1) + p0 > u0) {
+  if (r0 > 0 && p0 - rp[r0 - 1] > kSpan && (uint64_t)(r0 - 1) + p0 > u0) {
     flags |= kHeadPiece;
     e0 = (uint32_t)(u0 - (r0 - 1));
     if (!rows) e1 = (uint32_t)min((uint64_t)p0, u1 - (r0 - 1));  // no row starts here: it may go on after the window
   }
-  if (rows && p1 - rp[r1 - 1] > span) {  // the last row that starts here is a long one
+  if (rows && p1 - rp[r1 - 1] > kSpan) {  // the last row that starts here is a long one
     --rows;
     flags |= kTailPiece;
     e1 = (uint32_t)(u1 - (r1 - 1));
@@ -115,7 +120,7 @@ __device__ __forceinline__ void item_ids(const uint32_t* __restrict__ ids, uint3
 // K values per lane: inclusive fixed-point prefix of the edges [e0, e1), entry q of it for edge
 // b0 + q (b0 = e0 rounded down to 4; entries before e0 are 0).  w null: value cin[id]; else
 // w * cin[id] scaled by 2^qs.
-template <int NT, int K, bool W>
+template <int K, bool W>
 __device__ __forceinline__ void item_prefix(const uint32_t* __restrict__ col, const float* w, int qs,
                                             const float* cin, uint32_t nnz, uint32_t b0, uint32_t e0, uint32_t e1,
                                             unsigned long long* pre, unsigned long long* wsum) {
@@ -139,12 +144,10 @@ __device__ __forceinline__ void item_prefix(const uint32_t* __restrict__ col, co
   }
   unsigned long long inc = wave_inclusive_scan(s);
   unsigned long long off = inc - s;
-  if constexpr (NT > 64) {
-    if (lane_id() == 63) wsum[threadIdx.x >> 6] = inc;
-    __syncthreads();
+  if (lane_id() == 63) wsum[threadIdx.x >> 6] = inc;
+  __syncthreads();
 #pragma unroll
-    for (int w2 = 0; w2 < NT / 64 - 1; ++w2) off += (uint32_t)w2 < (threadIdx.x >> 6) ? wsum[w2] : 0ull;
-  }
+  for (uint32_t w2 = 0; w2 < kNT / 64 - 1; ++w2) off += w2 < (threadIdx.x >> 6) ? wsum[w2] : 0ull;
 #pragma unroll
   for (int t = 0; t < K; ++t) pre[pos(q0 + t)] = off + v[t];
   __syncthreads();
@@ -161,12 +164,11 @@ __device__ __forceinline__ unsigned long long item_sum(const unsigned long long*
 // Adds a piece of long row h (entries [hp0, hp1), this piece's sum `mine`) to the row's counter, that
 // of the item it starts in; true for the last piece, which gets the row's sum and leaves the
 // counters at 0 for the next sweep.  *start: the item the row starts in.
-template <uint32_t S>
 __device__ __forceinline__ bool add_piece(unsigned long long* hsum, uint32_t* hcnt, uint32_t h, uint32_t hp0,
                                           uint32_t hp1, unsigned long long mine, unsigned long long* z,
                                           uint32_t* start) {
   // the row's pieces are those of the items its edges' units lie in
-  const uint32_t a = (uint32_t)(((uint64_t)h + hp0) / S), b = (uint32_t)(((uint64_t)h + hp1 - 1) / S);
+  const uint32_t a = (uint32_t)(((uint64_t)h + hp0) / kSpan), b = (uint32_t)(((uint64_t)h + hp1 - 1) / kSpan);
   *start = a;
   unsigned long long old = __hip_atomic_fetch_add(hsum + a, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // the sum has been added (its old value is back) before the piece is counted
@@ -177,12 +179,10 @@ __device__ __forceinline__ bool add_piece(unsigned long long* hsum, uint32_t* hc
   return true;
 }
 
-template <int NT>
-__global__ __launch_bounds__(NT) void pr_item_kernel(ItemParams P) {
-  constexpr uint32_t S = item_span(NT);
-  static_assert(kItemLanes == 64, "one lane counter per wavefront lane");
-  __shared__ unsigned long long pre[9 * NT];
-  __shared__ unsigned long long wsum[NT / 64];
+__global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
+  static_assert(kItemLanes == 64 && kNT == 256, "one lane counter per wavefront lane, four waves");
+  __shared__ unsigned long long pre[9 * kNT];
+  __shared__ unsigned long long wsum[kNT / 64];
   const uint32_t lane = threadIdx.x & 63u;
   const uint4 d = P.desc[blockIdx.x];
   // the previous sweep's L1 change: loaded now, looked at once the gathers are done (a check
@@ -210,8 +210,8 @@ __global__ __launch_bounds__(NT) void pr_item_kernel(ItemParams P) {
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * NT) item_prefix<NT, 4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
-  else item_prefix<NT, 8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
+  else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) ch += __shfl_xor(ch, m, 64);
   if (blockIdx.x == 0) {
@@ -222,23 +222,20 @@ __global__ __launch_bounds__(NT) void pr_item_kernel(ItemParams P) {
   auto sum = [&](uint32_t a, uint32_t b) { return item_sum(pre, b0, a, b); };
   unsigned long long err = 0ull;
   if (threadIdx.x < rows) err = item_update(P, r0 + threadIdx.x, dequantize(sum(ra, rb)), xo, bv, dg);
-  for (uint32_t q = threadIdx.x + NT; q < rows; q += NT) {
+  for (uint32_t q = threadIdx.x + kNT; q < rows; q += kNT) {
     const uint32_t i = r0 + q;
     err += item_update(P, i, dequantize(sum(P.rp[i], P.rp[i + 1])), P.x[i], P.basev ? P.basev[i] : P.base, P.deg[i]);
   }
   if (piece) {
     unsigned long long z;
     uint32_t a;
-    if (add_piece<S>(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a))
+    if (add_piece(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a))
       err += item_update(P, h, dequantize(z), P.x[h], P.basev ? P.basev[h] : P.base, P.deg[h]);
   }
   err = wave_sum(err);
-  if constexpr (NT > 64) {
-    if (lane == 0) wsum[threadIdx.x >> 6] = err;
-    __syncthreads();
-    err = 0ull;
-    for (int w = 0; w < NT / 64; ++w) err += wsum[w];
-  }
+  if (lane == 0) wsum[threadIdx.x >> 6] = err;
+  __syncthreads();
+  err = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
   if (threadIdx.x == 0 && err)
     atomicAdd(P.lanes + (P.iter % 3) * kItemLaneSlot + (blockIdx.x % kItemLanes) * kItemLanePad, err);
 }
@@ -248,7 +245,6 @@ __global__ __launch_bounds__(NT) void pr_item_kernel(ItemParams P) {
 // they stay doubles: every item stores its own and, where a long row starts in it, that row's; every
 // workgroup of the next sweep adds them all in one fixed order and stops or goes on, which takes
 // the place of a launch that folds them.
-constexpr uint32_t kWNT = 256;
 
 __device__ __forceinline__ double witem_stop(const WItemParams& P) {
   return P.thr_scale ? P.threshold * *P.thr_scale : P.threshold;
@@ -258,19 +254,17 @@ __device__ __forceinline__ double witem_stop(const WItemParams& P) {
 __device__ __forceinline__ double witem_change(const WItemParams& P, uint32_t k, double* red) {
   const double* part = P.part + (uint64_t)(k & 1u) * 2 * P.count;
   double e = 0.0;
-  for (uint32_t q = threadIdx.x; q < 2 * P.count; q += kWNT) e += part[q];
+  for (uint32_t q = threadIdx.x; q < 2 * P.count; q += kNT) e += part[q];
   e = wave_sum(e);
   if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = e;
   __syncthreads();
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ __launch_bounds__(kWNT) void wpr_item_kernel(WItemParams P) {
-  constexpr uint32_t S = item_span(kWNT);
-  static_assert(kWNT == 256, "four waves");
-  __shared__ unsigned long long pre[9 * kWNT];
-  __shared__ unsigned long long wsum[kWNT / 64];
-  __shared__ double red[kWNT / 64], red2[kWNT / 64];
+__global__ __launch_bounds__(kNT) void wpr_item_kernel(WItemParams P) {
+  __shared__ unsigned long long pre[9 * kNT];
+  __shared__ unsigned long long wsum[kNT / 64];
+  __shared__ double red[kNT / 64], red2[kNT / 64];
   const double stop = witem_stop(P);
   // a solve that stopped before the previous sweep: that sweep stored no parts
   if (P.iter > 1 && P.err[P.iter - 2] < stop) return;
@@ -294,8 +288,8 @@ __global__ __launch_bounds__(kWNT) void wpr_item_kernel(WItemParams P) {
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * kWNT) item_prefix<kWNT, 4, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
-  else item_prefix<kWNT, 8, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
+  else item_prefix<8, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
   if (P.iter > 0) {
     const double ch = witem_change(P, P.iter - 1, red);
     if (blockIdx.x == 0 && threadIdx.x == 0) P.err[P.iter - 1] = ch;
@@ -308,7 +302,7 @@ __global__ __launch_bounds__(kWNT) void wpr_item_kernel(WItemParams P) {
   };
   double e = 0.0;
   if (threadIdx.x < rows) e = update(r0 + threadIdx.x, item_sum(pre, b0, ra, rb), xo, bv);
-  for (uint32_t q = threadIdx.x + kWNT; q < rows; q += kWNT) {
+  for (uint32_t q = threadIdx.x + kNT; q < rows; q += kNT) {
     const uint32_t i = r0 + q;
     e += update(i, item_sum(pre, b0, P.rp[i], P.rp[i + 1]), P.xin[i], P.basev[i]);
   }
@@ -316,7 +310,7 @@ __global__ __launch_bounds__(kWNT) void wpr_item_kernel(WItemParams P) {
   if (piece) {
     unsigned long long z;
     uint32_t a;
-    if (add_piece<S>(P.hsum, P.hcnt, h, hp0, hp1, item_sum(pre, b0, max(hp0, e0), min(hp1, e1)), &z, &a))
+    if (add_piece(P.hsum, P.hcnt, h, hp0, hp1, item_sum(pre, b0, max(hp0, e0), min(hp1, e1)), &z, &a))
       part[P.count + a] = update(h, z, P.xin[h], P.basev[h]);
   }
   e = wave_sum(e);
@@ -337,11 +331,14 @@ __global__ __launch_bounds__(256) void witem_init_kernel(WItemParams P, const fl
   if (i < iters) P.err[i] = 0.0;
 }
 
-__global__ __launch_bounds__(kWNT) void witem_fold_kernel(WItemParams P, uint32_t k) {
-  __shared__ double red[kWNT / 64];
-  if (k > 0 && P.err[k - 1] < witem_stop(P)) return;  // sweep k did nothing
-  const double ch = witem_change(P, k, red);
-  if (threadIdx.x == 0) P.err[k] = ch;
+__global__ __launch_bounds__(kNT) void witem_fold_kernel(WItemParams P, uint32_t k, WMail mail) {
+  __shared__ double red[kNT / 64];
+  double ch = 0.0;
+  if (k == 0 || !(P.err[k - 1] < witem_stop(P))) {  // else sweep k did nothing
+    ch = witem_change(P, k, red);
+    if (threadIdx.x == 0) P.err[k] = ch;
+  }
+  wmail_post(mail, P.err, k, ch);
 }
 
 // ---- row sums ----
@@ -427,25 +424,25 @@ __device__ __forceinline__ void row_sum_out(const RowSumParams& P, const RowSumO
   if (o.gv) o.gv[u] = o.omd * P.gather[u];
 }
 
-__global__ __launch_bounds__(kWNT) void row_sum_kernel(RowSumParams P, RowSumOut o) {
-  __shared__ double pre[9 * kWNT];
-  __shared__ uint8_t start[8 * kWNT];
-  __shared__ double wv[kWNT / 64];
-  __shared__ uint32_t wf[kWNT / 64];
+__global__ __launch_bounds__(kNT) void row_sum_kernel(RowSumParams P, RowSumOut o) {
+  __shared__ double pre[9 * kNT];
+  __shared__ uint8_t start[8 * kNT];
+  __shared__ double wv[kNT / 64];
+  __shared__ uint32_t wf[kNT / 64];
   const uint4 d = P.desc[blockIdx.x];
   const uint32_t e0 = d.x, e1 = d.y, r0 = d.z, rows = d.w & kRowMask, b0 = e0 & ~3u;
-  for (uint32_t q = threadIdx.x; q < 2 * kWNT; q += kWNT) reinterpret_cast<uint32_t*>(start)[q] = 0u;
+  for (uint32_t q = threadIdx.x; q < 2 * kNT; q += kNT) reinterpret_cast<uint32_t*>(start)[q] = 0u;
   __syncthreads();
   // rows with entries mark their first; the tail piece's row too (r0 + rows)
   const uint32_t marks = rows + ((d.w & kTailPiece) ? 1u : 0u);
-  for (uint32_t q = threadIdx.x; q < marks; q += kWNT) {
+  for (uint32_t q = threadIdx.x; q < marks; q += kNT) {
     const uint32_t a = P.rp[r0 + q];
     if (P.rp[r0 + q + 1] > a) start[a - b0] = 1;
   }
   __syncthreads();
-  if (e1 - b0 <= 4u * kWNT) item_row_sums<4>(P, b0, e0, e1, start, pre, wv, wf);
+  if (e1 - b0 <= 4u * kNT) item_row_sums<4>(P, b0, e0, e1, start, pre, wv, wf);
   else item_row_sums<8>(P, b0, e0, e1, start, pre, wv, wf);
-  for (uint32_t q = threadIdx.x; q < rows; q += kWNT) {
+  for (uint32_t q = threadIdx.x; q < rows; q += kNT) {
     const uint32_t a = P.rp[r0 + q], b = P.rp[r0 + q + 1];
     row_sum_out(P, o, r0 + q, b > a ? pre[pos(b - 1 - b0)] : 0.0);
   }
@@ -464,21 +461,21 @@ __global__ __launch_bounds__(256) void row_sum_long_kernel(RowSumParams P, RowSu
   const uint4 d = P.desc[a];
   if (!(d.w & kTailPiece)) return;
   const uint32_t h = d.z + (d.w & kRowMask);
-  const uint32_t b = (uint32_t)(((uint64_t)h + P.rp[h + 1] - 1) / item_span(kWNT));
+  const uint32_t b = (uint32_t)(((uint64_t)h + P.rp[h + 1] - 1) / kSpan);
   double s = lane == 0 ? P.tail[a] : 0.0;
   for (uint32_t c = a + 1 + lane; c <= b; c += 64) s += P.head[c];
   s = wave_sum(s);
   if (lane == 0) row_sum_out(P, o, h, s);
 }
 
-__global__ __launch_bounds__(256) void item_init_kernel(ItemParams P, uint32_t count, float init, float* __restrict__ c0,
+__global__ __launch_bounds__(256) void item_init_kernel(ItemParams P, float init, float* __restrict__ c0,
                                                         uint64_t iters) {
   const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
   if (i < P.n) {
     P.x[i] = init;
     if (c0) c0[i] = init / (float)P.deg[i];
   }
-  if (i < count) {
+  if (i < P.count) {
     P.hsum[i] = 0ull;
     P.hcnt[i] = 0u;
   }
@@ -487,31 +484,20 @@ __global__ __launch_bounds__(256) void item_init_kernel(ItemParams P, uint32_t c
 }
 
 __global__ __launch_bounds__(64) void item_fold_kernel(const unsigned long long* __restrict__ lanes,
-                                                       unsigned long long* __restrict__ acc, uint32_t k) {
+                                                       unsigned long long* __restrict__ acc, uint32_t first,
+                                                       uint32_t k, unsigned long long* __restrict__ mail) {
   unsigned long long v = lanes[(k % 3) * kItemLaneSlot + threadIdx.x * kItemLanePad];
   v = wave_sum(v);
   if (threadIdx.x == 0) acc[k] = v;
+  if (!mail) return;
+  for (uint32_t q = first + threadIdx.x; q < k; q += 64) mail[q] = acc[q];
+  if (threadIdx.x == 0) mail[k] = v;
 }
 
 }  // namespace
 
-ItemShape item_shape(uint32_t n, uint64_t nnz, uint64_t max_items) {
-  const uint64_t units = (uint64_t)n + nnz;
-  ItemShape sh;
-  sh.threads = units <= (1ull << 18) ? 64u : 256u;
-  const uint64_t count = ceil_div(units, item_span(sh.threads));
-  if (nnz >= (1ull << 32) || count > max_items) sh.threads = 0;
-  else sh.count = (uint32_t)count;
-  return sh;
-}
-
-ItemShape item_shape_wide(uint32_t n, uint64_t nnz, uint64_t max_items) {
-  ItemShape sh;
-  sh.threads = kWNT;
-  const uint64_t count = ceil_div((uint64_t)n + nnz, item_span(kWNT));
-  if (nnz >= (1ull << 32) || count > max_items) sh.threads = 0;
-  else sh.count = (uint32_t)count;
-  return sh;
+uint32_t item_count(uint32_t n, uint64_t nnz) {
+  return (uint32_t)ceil_div((uint64_t)n + nnz, kSpan);
 }
 
 void witems_enqueue_init(hipStream_t s, const WItemParams& P, const float* src, float v, float* dst, uint64_t iters) {
@@ -521,42 +507,41 @@ void witems_enqueue_init(hipStream_t s, const WItemParams& P, const float* src, 
 }
 
 void witems_enqueue_sweep(hipStream_t s, const WItemParams& P) {
-  wpr_item_kernel<<<P.count, kWNT, 0, s>>>(P);
+  wpr_item_kernel<<<P.count, kNT, 0, s>>>(P);
   NWG_LAUNCH_CHECK();
 }
 
-void witems_enqueue_fold(hipStream_t s, const WItemParams& P, uint32_t k) {
-  witem_fold_kernel<<<1, kWNT, 0, s>>>(P, k);
+void witems_enqueue_fold(hipStream_t s, const WItemParams& P, uint32_t k, const WMail& mail) {
+  witem_fold_kernel<<<1, kNT, 0, s>>>(P, k, mail);
   NWG_LAUNCH_CHECK();
 }
 
 void row_sums_enqueue(hipStream_t s, const RowSumParams& P, const RowSumOut& o) {
   if (!P.count) return;
-  row_sum_kernel<<<P.count, kWNT, 0, s>>>(P, o);
+  row_sum_kernel<<<P.count, kNT, 0, s>>>(P, o);
   row_sum_long_kernel<<<(P.count + 3) / 4, 256, 0, s>>>(P, o);
   NWG_LAUNCH_CHECK();
 }
 
-void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, const ItemShape& sh, uint4* desc) {
-  item_desc_kernel<<<(uint32_t)ceil_div(sh.count, 256), 256, 0, s>>>(n, nnz, rp, item_span(sh.threads), sh.count, desc);
+void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, uint4* desc) {
+  const uint32_t count = item_count(n, nnz);
+  item_desc_kernel<<<(uint32_t)ceil_div(count, 256), 256, 0, s>>>(n, nnz, rp, count, desc);
   NWG_LAUNCH_CHECK();
 }
 
-void items_enqueue_init(hipStream_t s, const ItemShape& sh, const ItemParams& P, float init, float* c0,
-                        uint64_t iters) {
-  const uint64_t m = std::max<uint64_t>({P.n, sh.count, kItemLaneWords, iters});
-  item_init_kernel<<<(uint32_t)ceil_div(m, 256), 256, 0, s>>>(P, sh.count, init, c0, iters);
+void items_enqueue_init(hipStream_t s, const ItemParams& P, float init, float* c0, uint64_t iters) {
+  const uint64_t m = std::max<uint64_t>({P.n, P.count, kItemLaneWords, iters});
+  item_init_kernel<<<(uint32_t)ceil_div(m, 256), 256, 0, s>>>(P, init, c0, iters);
   NWG_LAUNCH_CHECK();
 }
 
-void items_enqueue_sweep(hipStream_t s, const ItemShape& sh, const ItemParams& P) {
-  if (sh.threads == 64) pr_item_kernel<64><<<sh.count, 64, 0, s>>>(P);
-  else pr_item_kernel<256><<<sh.count, 256, 0, s>>>(P);
+void items_enqueue_sweep(hipStream_t s, const ItemParams& P) {
+  pr_item_kernel<<<P.count, kNT, 0, s>>>(P);
   NWG_LAUNCH_CHECK();
 }
 
-void items_enqueue_fold(hipStream_t s, const ItemParams& P, uint32_t k) {
-  item_fold_kernel<<<1, 64, 0, s>>>(P.lanes, P.acc, k);
+void items_enqueue_fold(hipStream_t s, const ItemParams& P, uint32_t first, uint32_t k, unsigned long long* mail) {
+  item_fold_kernel<<<1, 64, 0, s>>>(P.lanes, P.acc, first, k, mail);
   NWG_LAUNCH_CHECK();
 }
 

@@ -15,12 +15,6 @@ constexpr uint32_t kItemLanePad = 8;
 constexpr uint32_t kItemLaneSlot = kItemLanes * kItemLanePad;
 constexpr uint32_t kItemLaneWords = 3 * kItemLaneSlot;
 
-// Work items of one CSC: `threads` lanes per item (64 or 256), count items.
-struct ItemShape {
-  uint32_t threads = 0;
-  uint32_t count = 0;
-};
-
 struct ItemParams {
   const uint4* desc;         // per item: {first edge, end edge, first row, rows | flags} (items.hip)
   const uint32_t* rp;
@@ -34,12 +28,21 @@ struct ItemParams {
   float damp;
   uint32_t n;
   uint32_t nnz;
+  uint32_t count;            // items
   unsigned long long* hsum;  // per item: fixed-point sum of the long row that starts in it
   uint32_t* hcnt;            // per item: pieces of that row added so far
   unsigned long long* lanes; // kItemLaneWords
   unsigned long long* acc;   // per sweep: L1 change, fixed point
   uint32_t iter;
   double threshold;
+};
+
+// Where a segment of weighted sweeps leaves what the host reads: the solve's two words of scales, then
+// err[k] at words[2 + k], k in [first, last] of the segment (words null: nowhere).
+struct WMail {
+  unsigned long long* words = nullptr;
+  const unsigned long long* scale = nullptr;
+  uint32_t first = 0;
 };
 
 // The weighted sweep over items: x' = fma(d, sum w * xin, basev), products scaled by 2^(*qshift) and
@@ -92,25 +95,22 @@ struct RowSumOut {
   float d, omd;
 };
 
-// Shape for a CSC of n rows and nnz entries; threads is 0 when it takes more than max_items items
-// (or 2^32 entries or more).
-ItemShape item_shape(uint32_t n, uint64_t nnz, uint64_t max_items);
-// desc (count entries) from the row pointers
-// The same with 256-lane items whatever the size.
-ItemShape item_shape_wide(uint32_t n, uint64_t nnz, uint64_t max_items);
-void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, const ItemShape& sh, uint4* desc);
+// items of a CSC of n rows and nnz entries
+uint32_t item_count(uint32_t n, uint64_t nnz);
+// their descriptions (item_count of them) from the row pointers
+void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, uint4* desc);
 // x = init, c0 (nullable) = init / outdeg, and the solve's counters cleared: acc[0 .. iters), the lanes,
 // hsum and hcnt (count each)
-void items_enqueue_init(hipStream_t s, const ItemShape& sh, const ItemParams& P, float init, float* c0,
-                        uint64_t iters);
-void items_enqueue_sweep(hipStream_t s, const ItemShape& sh, const ItemParams& P);
+void items_enqueue_init(hipStream_t s, const ItemParams& P, float init, float* c0, uint64_t iters);
+void items_enqueue_sweep(hipStream_t s, const ItemParams& P);
 // Weighted: xin[0] = src (null: v), err[0 .. iters) and the items' counters cleared; a sweep; err[k]
 // of sweep k, the last one launched.
 void witems_enqueue_init(hipStream_t s, const WItemParams& P, const float* src, float v, float* dst, uint64_t iters);
 void witems_enqueue_sweep(hipStream_t s, const WItemParams& P);
-void witems_enqueue_fold(hipStream_t s, const WItemParams& P, uint32_t k);
+void witems_enqueue_fold(hipStream_t s, const WItemParams& P, uint32_t k, const WMail& mail);
 void row_sums_enqueue(hipStream_t s, const RowSumParams& P, const RowSumOut& o);
-// acc[k] of sweep k, the last one launched (the others' are stored by the sweep after them)
-void items_enqueue_fold(hipStream_t s, const ItemParams& P, uint32_t k);
+// acc[k] of sweep k, the last one launched (the others' are stored by the sweep after them); with mail,
+// acc[first .. k] there too
+void items_enqueue_fold(hipStream_t s, const ItemParams& P, uint32_t first, uint32_t k, unsigned long long* mail);
 
 }  // namespace nwg

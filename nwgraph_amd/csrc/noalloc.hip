@@ -40,6 +40,7 @@ constexpr uint32_t kNaUnroll = 4;    // gathers in flight per lane
 constexpr uint32_t kNaFoldChunk = 2048;  // workgroup partials folded by one workgroup
 constexpr uint32_t kNaMaxN = 1u << 22;
 constexpr uint64_t kNaMaxIters = 4096;
+static_assert(kNaMaxIters <= kMailWords, "a solve's changes fit the context's mail");
 constexpr uint32_t kNaMaxBlocks = kNaMaxN / kNaThreads;
 // Work items of the item sweep (items.hip): 1020 rows and edges each, so 134 M in all.
 constexpr uint64_t kNaMaxItems = 1u << 17;
@@ -243,8 +244,7 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
 
   // The item sweep's exact fixed-point sums cover scores in [0, 1]: damping factors in [0, 1].
   // Others, and CSCs of more items than the scratch holds, keep the float row sums.
-  const ItemShape sh = item_shape(n, nnz, kNaMaxItems);
-  const bool items = sh.threads && damping >= 0.f && damping <= 1.f;
+  const bool items = item_count(n, nnz) <= kNaMaxItems && damping >= 0.f && damping <= 1.f;
   const float init = (float)(1.0 / n);  // page_rank.hpp:93
   if (items) {
     ItemParams I{};
@@ -258,21 +258,22 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
     I.damp = damping;
     I.n = n;
     I.nnz = (uint32_t)nnz;
+    I.count = item_count(n, nnz);
     I.hsum = reinterpret_cast<unsigned long long*>(base + kOffHsum);
     I.hcnt = reinterpret_cast<uint32_t*>(base + kOffHcnt);
     I.lanes = reinterpret_cast<unsigned long long*>(base + kOffLanes);
     I.acc = acc;
     I.threshold = P.threshold;
-    items_build(s, n, nnz, csc_ptr, sh, desc);
+    items_build(s, n, nnz, csc_ptr, desc);
     NWG_HIP(hipEventRecord(ctx->ev0, s));
-    items_enqueue_init(s, sh, I, init, c0, max_iters);
+    items_enqueue_init(s, I, init, c0, max_iters);
     for (uint64_t k = 0; k < max_iters; ++k) {
       I.iter = (uint32_t)k;
       I.cin = (k & 1) ? c1 : c0;
       I.cout = (k & 1) ? c0 : c1;
-      items_enqueue_sweep(s, sh, I);
+      items_enqueue_sweep(s, I);
     }
-    if (max_iters) items_enqueue_fold(s, I, (uint32_t)(max_iters - 1));
+    if (max_iters) items_enqueue_fold(s, I, 0, (uint32_t)(max_iters - 1), ctx->mail);
     NWG_HIP(hipEventRecord(ctx->ev1, s));
   } else {
     NWG_HIP(hipEventRecord(ctx->ev0, s));
@@ -298,10 +299,10 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
   bool stopped = false;
   for (uint64_t k0 = 0; k0 < max_iters && !stopped; k0 += kPiece) {
     const uint64_t cnt = std::min<uint64_t>(kPiece, max_iters - k0);
-    NWG_HIP(hipMemcpyAsync(h, acc + k0, cnt * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    if (!items) NWG_HIP(hipMemcpyAsync(h, acc + k0, cnt * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     NWG_HIP(hipStreamSynchronize(s));
     for (uint64_t q = 0; q < cnt; ++q) {
-      const double e = fixed_to_err(h[q]);
+      const double e = fixed_to_err(items ? ctx->mail[k0 + q] : h[q]);
       last = e;
       if (info && info->error_trace && k0 + q < info->error_trace_len) info->error_trace[k0 + q] = e;
       if (e < (double)threshold) {

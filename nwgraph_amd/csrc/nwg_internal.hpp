@@ -153,7 +153,7 @@ struct BinnedLayout {
 struct Plan {
   nwg_plan_params params{};
   bool built = false;
-  ItemShape ish;          // item sweep (items.hip): its shape (threads 0: not used) and items
+  uint32_t n_items = 0;   // item sweep (items.hip): its items (0: not used)
   DevBuf<uint4> idesc;
   // row classes of the class kernels: built by the first solve that runs them
   bool classes = false;
@@ -234,6 +234,8 @@ inline uint64_t segment_end(uint64_t start, uint64_t max_iters) {
   return start + len < max_iters ? start + len : max_iters;
 }
 
+constexpr uint64_t kMailWords = 8192;  // of nwg_ctx::mail; longer solves copy
+
 // Identity of a captured sweep loop: re-capture when any of it changes.
 struct CaptureKey {
   static constexpr int kPtrs = 16;
@@ -272,7 +274,7 @@ struct Captured {
 
 // Items of the CSC or CSR of a weighted graph (items.hip).
 struct WItems {
-  ItemShape shape;
+  uint32_t count = 0;
   DevBuf<uint4> desc;
 };
 
@@ -360,6 +362,9 @@ struct nwg_ctx {
   hipStream_t capture_stream = nullptr;  // used only to record HIP graphs
   std::string last_error;
   std::mutex mu;
+  // host memory the device writes: a solve's last kernels leave its L1 changes here, so that the host
+  // reads them after the wait it makes anyway, with no copy
+  unsigned long long* mail = nullptr;
   std::shared_ptr<nwg::DevPool> pool;  // device memory kept between this context's calls
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -484,10 +489,11 @@ void binned_enqueue_sweep(hipStream_t s, const BinParams& P);
 // one weighted sweep (P.bw set): chunk, bin and combine passes; the L1 change is folded by the chunk
 // pass of the next sweep, or by the fold after the last one launched
 void binned_enqueue_weighted_sweep(hipStream_t s, const BinParams& P);
-void binned_enqueue_weighted_fold(hipStream_t s, const BinParams& P);
-// lane counters of iters sweeps cleared / summed into acc[0 .. iters)
+void binned_enqueue_weighted_fold(hipStream_t s, const BinParams& P, const WMail& mail);
+// lane counters of iters sweeps cleared / summed into acc[0 .. iters) (and mail, nullable)
 void binned_clear_residuals(hipStream_t s, unsigned long long* lanes, uint64_t iters);
-void binned_fold_residuals(hipStream_t s, const unsigned long long* lanes, unsigned long long* acc, uint64_t iters);
+void binned_fold_residuals(hipStream_t s, const unsigned long long* lanes, unsigned long long* acc, uint64_t iters,
+                           unsigned long long* mail);
 // Schedules of pagerank_run:
 //   kJacobi   page_rank_v10: double-buffered contributions (pull sweep or binned sweep)
 //   kInPlace  page_rank (v11): one contribution array updated during the sweep

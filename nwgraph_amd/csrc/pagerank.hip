@@ -357,12 +357,12 @@ __global__ __launch_bounds__(kThreads) void pr_base_kernel(uint32_t n, const flo
   if (i < n) base[i] = (float)(omd * (double)v[order ? order[i] : i]);
 }
 
-// scores back to the original numbering: out[v] = x[rank[v]] (rank: original -> new id).
+// scores out, back to the original numbering with rank (original -> new id): out[v] = x[rank[v]].
 // A gather: the writes are whole lines, and the reads of x come mostly from MALL.
-__global__ __launch_bounds__(kThreads) void pr_unpermute_kernel(uint32_t n, const uint32_t* __restrict__ rank,
-                                                                const float* __restrict__ x, float* __restrict__ out) {
+__global__ __launch_bounds__(kThreads) void pr_out_kernel(uint32_t n, const uint32_t* __restrict__ rank,
+                                                          const float* __restrict__ x, float* __restrict__ out) {
   const uint32_t v = blockIdx.x * kThreads + threadIdx.x;
-  if (v < n) out[v] = x[rank[v]];
+  if (v < n) out[v] = x[rank ? rank[v] : v];
 }
 
 // ---------------------------------------------------------------------------
@@ -590,10 +590,10 @@ void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp) {
   Plan pl;
   pl.params = pp;
   pl.n_tiles = (uint32_t)ceil_div(n, kThreads);
-  if (plan_takes_items(pp, g->nnz)) pl.ish = item_shape(n, g->nnz, 1ull << 31);
-  if (pl.ish.threads) {
-    pl.idesc.alloc(pl.ish.count);
-    items_build(s, n, g->nnz, a.ptr, pl.ish, pl.idesc.p);
+  if (plan_takes_items(pp, g->nnz)) {
+    pl.n_items = item_count(n, g->nnz);
+    pl.idesc.alloc(pl.n_items);
+    items_build(s, n, g->nnz, a.ptr, pl.idesc.p);
   } else if (pp.binned) {
     binned_build(s, a, n, g->nnz, pl.bl, true, nullptr, (int)pp.bin_bits);
   }
@@ -812,7 +812,7 @@ static BinParams make_bin_params(nwg_graph* g, PrState& st, const SweepParams& P
 // The item sweep's exact sums cover scores in [0, 1] (damping factors in [0, 1]); the delta
 // schedule's residuals are not normalised.
 static bool runs_items(const Plan& pl, PrSchedule sched, float damping) {
-  return pl.ish.threads && sched != PrSchedule::kDelta && damping >= 0.f && damping <= 1.f;
+  return pl.n_items && sched != PrSchedule::kDelta && damping >= 0.f && damping <= 1.f;
 }
 
 static ItemParams make_item_params(nwg_graph* g, PrState& st, const SweepParams& P) {
@@ -827,6 +827,7 @@ static ItemParams make_item_params(nwg_graph* g, PrState& st, const SweepParams&
   I.damp = P.damp;
   I.n = P.n;
   I.nnz = (uint32_t)g->nnz;
+  I.count = g->plan.n_items;
   I.hsum = st.ihsum.p;
   I.hcnt = st.ihcnt.p;
   I.lanes = st.ilanes.p;
@@ -836,9 +837,10 @@ static ItemParams make_item_params(nwg_graph* g, PrState& st, const SweepParams&
 }
 
 // Sweeps [k0, k1) of an iters-sweep solve: the inits when k0 = 0, and for the binned sweep
-// the fold of these sweeps' residual lanes into acc.
+// the fold of these sweeps' residual lanes into acc.  mail (nullable; item and binned sweeps): where
+// their L1 changes go for the host.
 static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams P, uint64_t iters,
-                          hipEvent_t* ev, PrSchedule sched, uint64_t k0, uint64_t k1) {
+                          hipEvent_t* ev, PrSchedule sched, uint64_t k0, uint64_t k1, unsigned long long* mail) {
   const uint32_t n = g->n;
   const uint32_t nt = g->plan.params.stream_hints;
   // In place, the binned sweep reads and writes one contribution array: its chunk pass stages
@@ -861,7 +863,7 @@ static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams 
       I.iter = P.iter;
       I.cin = cin;
       I.cout = cout;
-      items_enqueue_sweep(s, g->plan.ish, I);
+      items_enqueue_sweep(s, I);
       return;
     }
     if (binned) {
@@ -907,7 +909,7 @@ static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams 
   if (k0 == 0) {
     if (ev) {
       NWG_HIP(hipEventRecord(ev[2 * iters], s));
-      if (items) items_enqueue_init(s, g->plan.ish, I, init, nullptr, iters);
+      if (items) items_enqueue_init(s, I, init, nullptr, iters);
       else pr_init_kernel<<<blocks_for(std::max<uint64_t>(n, iters)), kThreads, 0, s>>>(n, P.deg, init, st.x.p, nullptr,
                                                                                         st.acc.p, iters);
       NWG_HIP(hipEventRecord(ev[2 * iters + 1], s));
@@ -915,7 +917,7 @@ static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams 
       pr_contrib_init_kernel<<<blocks_for(n), kThreads, 0, s>>>(n, P.deg, st.x.p, st.contrib0.p);
       NWG_HIP(hipEventRecord(ev[2 * iters + 3], s));
     } else if (items) {
-      items_enqueue_init(s, g->plan.ish, I, init, st.contrib0.p, iters);
+      items_enqueue_init(s, I, init, st.contrib0.p, iters);
     } else {
       pr_init_kernel<<<blocks_for(std::max<uint64_t>(n, iters)), kThreads, 0, s>>>(n, P.deg, init, st.x.p,
                                                                                    st.contrib0.p, st.acc.p, iters);
@@ -933,8 +935,8 @@ static void enqueue_solve(hipStream_t s, nwg_graph* g, PrState& st, SweepParams 
     if (ev) NWG_HIP(hipEventRecord(ev[2 * k + 1], s));
   }
   if (binned && k1 > k0)
-    binned_fold_residuals(s, st.bacc.p + k0 * kBinAccStride, st.acc.p + k0, k1 - k0);
-  if (items && k1 > k0) items_enqueue_fold(s, I, (uint32_t)(k1 - 1));
+    binned_fold_residuals(s, st.bacc.p + k0 * kBinAccStride, st.acc.p + k0, k1 - k0, mail ? mail + k0 : nullptr);
+  if (items && k1 > k0) items_enqueue_fold(s, I, (uint32_t)k0, (uint32_t)(k1 - 1), mail);
 }
 
 void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float damping, float threshold,
@@ -948,8 +950,8 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   if (!g->pr) g->pr.reset(new PrState());
   PrState& st = *g->pr;
   if (items) {
-    st.ihsum.ensure(g->plan.ish.count);
-    st.ihcnt.ensure(g->plan.ish.count);
+    st.ihsum.ensure(g->plan.n_items);
+    st.ihcnt.ensure(g->plan.n_items);
     st.ilanes.ensure(kItemLaneWords);
   }
   const uint32_t n = g->n;
@@ -986,7 +988,17 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   const bool timing = info && (info->flags & NWG_INFO_KERNEL_TIMING);
   float ms_total = 0.f;
   double sweep_ms = 0.0;
+  uint64_t launched = max_iters;
   std::vector<hipEvent_t> evs;
+  const bool class_kernels = !items && (!g->plan.bl.built || sched == PrSchedule::kDelta);
+  unsigned long long* const mail = !class_kernels && max_iters <= kMailWords ? ctx->mail : nullptr;
+  // scores in the caller's numbering
+  auto copy_out = [&] {
+    if (!scores_dev) return;
+    const uint32_t* rank = g->plan.params.relabel ? g->rl->rank.p : nullptr;
+    pr_out_kernel<<<blocks_for(n), kThreads, 0, s>>>(n, rank, st.x.p, scores_dev);
+    NWG_LAUNCH_CHECK();
+  };
   if (!timing) {
     CaptureKey key;
     key.ptrs[0] = st.x.p;
@@ -1004,6 +1016,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     key.ptrs[12] = st.ihsum.p;
     key.ptrs[13] = st.ihcnt.p;
     key.ptrs[14] = st.ilanes.p;
+    key.ptrs[15] = mail;
     key.plan_version = g->plan_version;
     key.iters = max_iters;
     key.damping = damping;
@@ -1023,7 +1036,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
         hipStream_t cs = ctx->capture_stream;
         NWG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
         try {
-          enqueue_solve(cs, g, st, P, max_iters, nullptr, sched, k0, k1);
+          enqueue_solve(cs, g, st, P, max_iters, nullptr, sched, k0, k1, mail);
         } catch (...) {
           hipGraph_t tmp = nullptr;
           (void)hipStreamEndCapture(cs, &tmp);
@@ -1044,12 +1057,16 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
       NWG_HIP(hipGraphLaunch(st.caps[seg++]->exec, s));
       if (k1 >= max_iters) break;
       unsigned long long last = 0ull;
-      NWG_HIP(hipMemcpyAsync(&last, st.acc.p + (k1 - 1), sizeof last, hipMemcpyDeviceToHost, s));
+      if (!mail) NWG_HIP(hipMemcpyAsync(&last, st.acc.p + (k1 - 1), sizeof last, hipMemcpyDeviceToHost, s));
       NWG_HIP(hipStreamSynchronize(s));
+      if (mail) last = mail[k1 - 1];
       // stopped: delta schedule, nothing pushed (page_rank.hpp:616-620); else the L1 change
       // below the threshold (page_rank.hpp:144) -- or the solve stopped earlier and this
       // sweep's accumulator kept the 0 it was cleared to
-      if (sched == PrSchedule::kDelta ? last == 0ull : fixed_to_err(last) < (double)threshold) break;
+      if (sched == PrSchedule::kDelta ? last == 0ull : fixed_to_err(last) < (double)threshold) {
+        launched = k1;
+        break;
+      }
     }
     NWG_HIP(hipEventRecord(ctx->ev1, s));
   } else {
@@ -1057,7 +1074,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     for (auto& e : evs) NWG_HIP(hipEventCreate(&e));
     NWG_HIP(hipEventRecord(ctx->ev0, s));
     try {
-      enqueue_solve(s, g, st, P, max_iters, evs.data(), sched, 0, max_iters);
+      enqueue_solve(s, g, st, P, max_iters, evs.data(), sched, 0, max_iters, mail);
     } catch (...) {
       for (auto& e : evs) (void)hipEventDestroy(e);
       throw;
@@ -1065,17 +1082,12 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     NWG_HIP(hipEventRecord(ctx->ev1, s));
   }
   std::vector<unsigned long long> acc(std::max<uint64_t>(max_iters, 1));
-  NWG_HIP(hipMemcpyAsync(acc.data(), st.acc.p, max_iters * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-  if (scores_dev) {
-    const uint32_t* order = g->active(g->plan.params.relabel != 0).order;
-    if (order) {
-      pr_unpermute_kernel<<<blocks_for(n), kThreads, 0, s>>>(n, g->rl->rank.p, st.x.p, scores_dev);
-      NWG_LAUNCH_CHECK();
-    } else {
-      NWG_HIP(hipMemcpyAsync(scores_dev, st.x.p, (size_t)n * sizeof(float), hipMemcpyDeviceToDevice, s));
-    }
-  }
+  if (!mail)
+    NWG_HIP(hipMemcpyAsync(acc.data(), st.acc.p, max_iters * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+  copy_out();
   NWG_HIP(hipStreamSynchronize(s));
+  // sweeps that were not launched changed nothing
+  if (mail) std::copy(mail, mail + launched, acc.begin());
   NWG_HIP(hipEventElapsedTime(&ms_total, ctx->ev0, ctx->ev1));
   uint64_t iters = max_iters;
   double last = 0.0;

@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "device_utils.hpp"
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(kThreads) void edge_grad_kernel(uint64_t nnz, const
 // gather of 8 bytes per edge.  Edge gradient, row sums over a gathered copy and chain rule as
 // three passes took 885 us for 16 M edges on MI355X (the row sums 647: two scattered reads per edge,
 // long rows one load at a time); row sums over items with the products made in place and this
-// pass take GRAD_US.
+// pass take 206 us.
 __global__ __launch_bounds__(kThreads) void raw_grad_kernel(uint64_t nnz, const uint32_t* __restrict__ row,
                                                             const uint32_t* __restrict__ col, float d,
                                                             const float* __restrict__ lambda,
@@ -410,14 +411,13 @@ static void ensure_pull_items(hipStream_t s, nwg_graph* g, bool csr) {
   else build_items(s, g->csc_ptr.p, g->n, g->w_items_csc_r0, g->w_items_csc_r1, &count);
 }
 
-// 256-lane items (items.hip) of the CSC or CSR, built on first use
+// items (items.hip) of the CSC or CSR, built on first use
 static const WItems& ensure_items(hipStream_t s, nwg_graph* g, bool csr) {
   WItems& it = csr ? g->wi_csr : g->wi_csc;
   if (!it.desc.n) {
-    it.shape = item_shape_wide(g->n, g->nnz, 1ull << 31);
-    NWG_REQUIRE(it.shape.threads, "weighted solves take fewer than 2^31 edges");
-    it.desc.alloc(std::max<uint32_t>(it.shape.count, 1));
-    items_build(s, g->n, g->nnz, csr ? g->csr_ptr.p : g->csc_ptr.p, it.shape, it.desc.p);
+    it.count = item_count(g->n, g->nnz);
+    it.desc.alloc(it.count);
+    items_build(s, g->n, g->nnz, csr ? g->csr_ptr.p : g->csc_ptr.p, it.desc.p);
   }
   return it;
 }
@@ -426,7 +426,7 @@ static const WItems& ensure_items(hipStream_t s, nwg_graph* g, bool csr) {
 static void csr_row_sums(hipStream_t s, nwg_graph* g, const uint32_t* idx, const float* src, const float* gather,
                          const RowSumOut& out) {
   const WItems& it = ensure_items(s, g, true);
-  DevBuf<double> pieces(2ull * std::max<uint32_t>(it.shape.count, 1));
+  DevBuf<double> pieces(2ull * it.count);
   RowSumParams R{};
   R.desc = it.desc.p;
   R.rp = g->csr_ptr.p;
@@ -435,9 +435,9 @@ static void csr_row_sums(hipStream_t s, nwg_graph* g, const uint32_t* idx, const
   R.gather = gather;
   R.n = g->n;
   R.nnz = (uint32_t)g->nnz;
-  R.count = it.shape.count;
+  R.count = it.count;
   R.head = pieces.p;
-  R.tail = pieces.p + it.shape.count;
+  R.tail = pieces.p + it.count;
   row_sums_enqueue(s, R, out);
 }
 
@@ -524,9 +524,9 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
   uint32_t grid = 0;
   if (kind == WSweep::kItems) {
     it = &ensure_items(s, g, q.csr);
-    st.ihsum.ensure(it->shape.count);
-    st.ihcnt.ensure(it->shape.count);
-    st.ipart.ensure(4ull * it->shape.count);
+    st.ihsum.ensure(it->count);
+    st.ihcnt.ensure(it->count);
+    st.ipart.ensure(4ull * it->count);
   } else if (kind == WSweep::kBinned) {
     st.bvals.ensure(L->pairs);
     st.bpart.ensure(std::max<uint64_t>((uint64_t)L->n_slots << L->bin_bits, 1));
@@ -536,6 +536,10 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
     grid = persistent_grid(q.csr ? g->w_items_csr_n : g->w_items_csc_n);
     st.part.ensure(grid);
   }
+  unsigned long long* const mail = kind != WSweep::kPull && max_iters && max_iters + 2 <= kMailWords ? ctx->mail : nullptr;
+  auto segment_mail = [&](uint64_t k0) {
+    return WMail{mail, reinterpret_cast<const unsigned long long*>(st.scale.p), (uint32_t)k0};
+  };
   // sweeps [k0, k1) (and the init with k0 = 0) on stream t
   auto enqueue = [&](hipStream_t t, uint64_t k0, uint64_t k1) {
     const float* src = q.y0;
@@ -550,7 +554,7 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
       I.damp = q.damping;
       I.n = n;
       I.nnz = (uint32_t)g->nnz;
-      I.count = it->shape.count;
+      I.count = it->count;
       I.qshift = qshift;
       I.hsum = st.ihsum.p;
       I.hcnt = st.ihcnt.p;
@@ -565,7 +569,7 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
         I.xout = y[(k + 1) & 1];
         witems_enqueue_sweep(t, I);
       }
-      if (k1 > k0) witems_enqueue_fold(t, I, (uint32_t)(k1 - 1));
+      if (k1 > k0) witems_enqueue_fold(t, I, (uint32_t)(k1 - 1), segment_mail(k0));
       return;
     }
     if (k0 == 0) {
@@ -609,7 +613,7 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
         B.x = y[(k + 1) & 1];
         binned_enqueue_weighted_sweep(t, B);
       }
-      if (k1 > k0) binned_enqueue_weighted_fold(t, B);
+      if (k1 > k0) binned_enqueue_weighted_fold(t, B, segment_mail(k0));
       return;
     }
     WParams P{};
@@ -636,7 +640,7 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
   };
   CaptureKey key;
   const void* ptrs[CaptureKey::kPtrs] = {st.y0.p, st.y1.p, q.base, q.y0, st.err.p, st.done.p, q.rp, q.col, q.w,
-                                         st.scale.p, kind == WSweep::kPull ? (void*)st.part.p : nullptr,
+                                         st.scale.p, kind == WSweep::kPull ? (void*)st.part.p : (void*)mail,
                                          L ? st.bvals.p : nullptr, L ? st.bpart.p : nullptr, L ? st.wpart.p : nullptr,
                                          it ? st.ihsum.p : nullptr, it ? (void*)st.ipart.p : nullptr};
   for (int k = 0; k < CaptureKey::kPtrs; ++k) key.ptrs[k] = ptrs[k];
@@ -687,10 +691,14 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
                                              q.out);
     NWG_LAUNCH_CHECK();
     if (eager) then();
-    if (k0 == 0) NWG_HIP(hipMemcpyAsync(&sc, st.scale.p, sizeof sc, hipMemcpyDeviceToHost, s));
-    if (k1 > k0)
+    if (!mail && k0 == 0) NWG_HIP(hipMemcpyAsync(&sc, st.scale.p, sizeof sc, hipMemcpyDeviceToHost, s));
+    if (!mail && k1 > k0)
       NWG_HIP(hipMemcpyAsync(h.data() + k0, st.err.p + k0, (k1 - k0) * sizeof(double), hipMemcpyDeviceToHost, s));
     NWG_HIP(hipStreamSynchronize(s));
+    if (mail) {
+      std::memcpy(&sc, mail, sizeof sc);
+      std::memcpy(h.data() + k0, mail + 2 + k0, (k1 - k0) * sizeof(double));
+    }
     if (kind != WSweep::kPull && !sc.finite) return false;
     if (relative) stop = (double)q.threshold * sc.scale;
     bool ended = k1 >= max_iters;
@@ -732,7 +740,7 @@ static WSweep weighted_sweep(const nwg_graph* g, float damping) {
   if (!g->w_normalized || !g->w_nonneg || g->nnz == 0) return WSweep::kPull;
   const nwg_plan_params pp = g->plan.built ? g->plan.params : default_plan_for(g);
   if (pp.binned && pp.bin_bits) return WSweep::kBinned;
-  if (item_shape_wide(g->n, g->nnz, kItemsWeighted).threads && damping >= 0.f && damping < 1.f) return WSweep::kItems;
+  if (item_count(g->n, g->nnz) <= kItemsWeighted && damping >= 0.f && damping < 1.f) return WSweep::kItems;
   return pp.binned ? WSweep::kBinned : WSweep::kPull;
 }
 
