@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
 // The L1 changes of a weighted sweep have no bound (fixed_point.hpp's scale covers row sums), so
 // they stay doubles: every item stores its own and, where a long row starts in it, that row's; every
 // workgroup of the next sweep adds them all in one fixed order and stops or goes on, which takes
-// the place of a launch that folds them.
+// the place of a launch that folds them (with more items than that is worth, the launch does).
 
 __device__ __forceinline__ double witem_stop(const WItemParams& P) {
   return P.thr_scale ? P.threshold * *P.thr_scale : P.threshold;
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(kNT) void wpr_item_kernel(WItemParams P) {
   __shared__ double red[kNT / 64], red2[kNT / 64];
   const double stop = witem_stop(P);
   // a solve that stopped before the previous sweep: that sweep stored no parts
-  if (P.iter > 1 && P.err[P.iter - 2] < stop) return;
+  if (P.folded ? P.iter > 0 && P.err[P.iter - 1] < stop : P.iter > 1 && P.err[P.iter - 2] < stop) return;
   const uint4 d = P.desc[blockIdx.x];
   const uint32_t e0 = d.x, e1 = d.y, r0 = d.z, rows = d.w & kRowMask;
   const int qs = *P.qshift;
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kNT) void wpr_item_kernel(WItemParams P) {
   const uint32_t b0 = e0 & ~3u;
   if (e1 - b0 <= 4u * kNT) item_prefix<4, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
   else item_prefix<8, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
-  if (P.iter > 0) {
+  if (P.iter > 0 && !P.folded) {
     const double ch = witem_change(P, P.iter - 1, red);
     if (blockIdx.x == 0 && threadIdx.x == 0) P.err[P.iter - 1] = ch;
     if (ch < stop) return;

@@ -67,6 +67,7 @@ struct WItemParams {
   uint32_t iter;
   double threshold;
   const double* thr_scale;  // relative threshold: the stop compares with threshold * *thr_scale
+  uint32_t folded;        // err[iter - 1] is folded by a launch between the sweeps, else by the sweep
 };
 
 // Row sums of a compressed structure over its items, s_u = sum of a value per entry q:

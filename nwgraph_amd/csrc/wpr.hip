@@ -479,6 +479,10 @@ void weights_set(hipStream_t s, nwg_graph* g, const float* w_dev, bool normalize
   }
 }
 
+// Items up to which every workgroup adds the previous sweep's parts itself (16 KiB of them, behind
+// its gathers).
+constexpr uint32_t kItemsFolding = 1024;
+
 // The sweep a weighted solve runs.  The exact sweeps (items, binned) need the weights normalised per
 // source from non-negative raw weights: then every weight is in [0, 1] and each source's out-weights
 // sum to 1, which the fixed-point bound (wscale_kernel) relies on.
@@ -563,11 +567,13 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
       I.threshold = (double)q.threshold;
       I.thr_scale = thr_scale;
       if (k0 == 0) witems_enqueue_init(t, I, src, uniform, y[0], max_iters);
+      I.folded = it->count > kItemsFolding;
       for (uint64_t k = k0; k < k1; ++k) {
         I.iter = (uint32_t)k;
         I.xin = y[k & 1];
         I.xout = y[(k + 1) & 1];
         witems_enqueue_sweep(t, I);
+        if (I.folded && k + 1 < k1) witems_enqueue_fold(t, I, (uint32_t)k, WMail{});
       }
       if (k1 > k0) witems_enqueue_fold(t, I, (uint32_t)(k1 - 1), segment_mail(k0));
       return;
@@ -731,11 +737,12 @@ static WState& wstate(nwg_graph* g) {
   return *g->wst;
 }
 
-// Weighted sweeps over items up to kItemsWeighted items (about a million rows and edges), which every
-// workgroup's sum of the previous sweep's parts still hides behind its gathers; measured on MI355X
-// (RMAT, edge factor 16, us per sweep, items / binned): WEIGHTED_CROSS.  Above, and where the plan
-// names a bin size, the binned sweep when the plan (or, before any plan, its size) asks for it.
-constexpr uint32_t kItemsWeighted = 1024;
+// Weighted sweeps over items up to kItemsWeighted items (2.6 M rows and edges).  Measured on MI355X
+// (RMAT, us per sweep, items / binned): 53 K edges 5.9 / 19.9, 228 K 7.2 / 23.1, 842 K 9.9 / 20.3, 1.9 M 17.7 / 23.5,
+// 3.9 M 32.1 / 26.2.
+// Above, and where the plan names a bin size, the binned sweep when the plan (or, before any plan,
+// its size) asks for it.
+constexpr uint32_t kItemsWeighted = 2560;
 static WSweep weighted_sweep(const nwg_graph* g, float damping) {
   if (!g->w_normalized || !g->w_nonneg || g->nnz == 0) return WSweep::kPull;
   const nwg_plan_params pp = g->plan.built ? g->plan.params : default_plan_for(g);

@@ -127,6 +127,29 @@ def test_resident_items_stop_and_personalise(ctx, n):
     g.close()
 
 
+def test_weighted_items_with_a_fold_launch(ctx):
+    """More than 1024 items: the L1 change is folded by a launch between the sweeps; stops as the change
+    of float64 sweeps says, away from the threshold."""
+    rng = np.random.default_rng(4)
+    n, m = 400001, 900000
+    src, dst = rng.integers(0, n, m).astype(np.uint32), rng.integers(0, n, m).astype(np.uint32)
+    g = ctx.graph_from_edges(n, src, dst, clean=False)
+    ptr, col, _ = g.csc()
+    row = np.repeat(np.arange(n), np.diff(ptr.astype(np.int64)))
+    w = rng.uniform(0.1, 1.0, m).astype(np.float32)
+    wn = w / np.bincount(col, weights=w.astype(np.float64), minlength=n)[col]
+    x, err = np.full(n, 1.0 / n), []
+    for _ in range(40):
+        y = (1 - D) / n + D * np.bincount(row, weights=wn * x[col], minlength=n)
+        err.append(np.abs(y - x).sum())
+        x = y
+    g.set_weights(w)
+    for it in (3, 20, 21, 30):  # the geometric mean of two changes: a factor of about 1 / sqrt(d) away
+        got, info = g.wpr_forward(None, D, float(np.sqrt(err[it - 1] * err[it - 2])), 40)
+        assert info["iterations"] == it
+    g.close()
+
+
 @pytest.mark.parametrize("side", ["in", "out"])  # the degrees are those of the CSC's or the CSR's rows
 @pytest.mark.parametrize("kind", KINDS)
 def test_weighted_items_match_float64(ctx, kind, side):
