@@ -180,6 +180,20 @@ __device__ __forceinline__ void finish_rows(const BinParams& P, uint32_t r0, uin
 }
 
 
+// Several graphs: whether rows [r0, r0 + nrows) are of one graph, whose base is then one value and
+// whose L1 change one sum.  Nearly every bin of a union of graphs above 2^13 vertices is: per row, the
+// graph, its frozen flag, its base and an LDS atomic on its one slot (64 lanes on one address) took
+// 252 us of a sweep's 347 at 256 graphs of 2^10 to 2^18 vertices (MI355X); this form takes 225 us
+// of 320.
+struct OneGraph {
+  bool one;
+  uint32_t g;
+};
+__device__ __forceinline__ OneGraph one_graph(const BinParams& P, uint32_t r0, uint32_t nrows) {
+  if (!nrows) return {false, 0u};
+  const uint32_t a = P.row_graph[r0], b = P.row_graph[r0 + nrows - 1];
+  return {a == b, a};
+}
 // chunk pass: vals[p] = contrib[src(p)] over the pairs of the tiles of one item.  Tiles are
 // padded to multiples of 8 pairs (pads have source kPadSrc and get 0), whole groups of 8 pairs
 // never cross a tile, and a lane moves half a group (4 pairs) with one 8-byte id load and one
@@ -492,22 +506,24 @@ struct FinishIn {
   uint32_t dg[bin_rows<BB>() / kBT];
 };
 template <int NT, int BB>
-__device__ __forceinline__ void finish_load(const BinParams& P, uint32_t r0, uint32_t nrows, FinishIn<BB>& in) {
+__device__ __forceinline__ void finish_load(const BinParams& P, const float* basev, float base, uint32_t r0,
+                                            uint32_t nrows, FinishIn<BB>& in) {
 #pragma unroll
   for (uint32_t k = 0; k < bin_rows<BB>() / kBT; ++k) {
     const uint32_t v = threadIdx.x + k * kBT;
     if (v < nrows) {
       in.xo[k] = bld<NT>(P.x + r0 + v);
       in.dg[k] = bld<NT>(P.deg + r0 + v);
-      in.bv[k] = P.basev ? bld<NT>(P.basev + r0 + v) : P.base;
+      in.bv[k] = basev ? bld<NT>(basev + r0 + v) : base;
     }
   }
 }
 // the reference's row update (page_rank.hpp:133-135) on the prefetched rows, and the
-// workgroup's L1 change into a lane counter of the sweep (as finish_rows)
+// workgroup's L1 change into *change (as finish_rows)
 template <int NT, int BB>
 __device__ __forceinline__ void finish_apply(const BinParams& P, uint32_t r0, uint32_t nrows, const FinishIn<BB>& in,
-                                             const unsigned long long* lacc, double* red) {
+                                             const unsigned long long* lacc, double* red,
+                                             unsigned long long* change) {
   double e = 0.0;
 #pragma unroll
   for (uint32_t k = 0; k < bin_rows<BB>() / kBT; ++k) {
@@ -525,7 +541,7 @@ __device__ __forceinline__ void finish_apply(const BinParams& P, uint32_t r0, ui
   if (threadIdx.x == 0) {
     double t = 0.0;
     for (uint32_t q = 0; q < kBT / 64; ++q) t += red[q];
-    if (t > 0.0) atomicAdd(residual_lane(P), err_to_fixed(t));
+    if (t > 0.0) atomicAdd(change, err_to_fixed(t));
   }
 }
 
@@ -548,6 +564,13 @@ __global__ __launch_bounds__(kBT, (BB >= 14) ? 4 : 8) void pr_bin_kernel(BinPara
   __shared__ uint32_t next;  // the range's next block to hand out
   const uint4 it = P.items2[blockIdx.x];  // {bin, first entry, end entry, partial slot or kNoSlot}
   const uint32_t b = it.x;
+  const uint32_t r0 = b << BB;
+  const uint32_t nrows = r0 < P.n ? min(kBinRows, P.n - r0) : 0u;
+  OneGraph og{false, 0u};
+  if constexpr (MULTI) {
+    og = one_graph(P, r0, nrows);
+    if (og.one && graph_frozen(P, og.g)) return;  // as do the bin's other items and its combine units
+  }
   // end of the hot part of [it.y, it.z); the hot contributions' loads are issued first, then
   // the first blocks' loads, and the contributions are written to LDS once the row sums are
   // cleared (bin_range's sync)
@@ -579,14 +602,19 @@ __global__ __launch_bounds__(kBT, (BB >= 14) ? 4 : 8) void pr_bin_kernel(BinPara
     }
     __syncthreads();
   });
-  const uint32_t r0 = b << BB;
-  const uint32_t nrows = r0 < P.n ? min(kBinRows, P.n - r0) : 0u;
-  if constexpr (!MULTI && !W) {
-    if (it.w == kNoSlot) {  // one graph, a bin that is one item: prefetch the rows, then finish
+  if constexpr (!W) {
+    if (it.w == kNoSlot && (!MULTI || og.one)) {  // one graph, a bin that is one item: prefetch the rows, then finish
       FinishIn<BB> in;
-      finish_load<NT, BB>(P, r0, nrows, in);
+      unsigned long long* change;
+      if constexpr (MULTI) {
+        finish_load<NT, BB>(P, nullptr, P.basev[r0], r0, nrows, in);
+        change = P.acc + (uint64_t)P.iter * P.ngraphs + og.g;
+      } else {
+        finish_load<NT, BB>(P, P.basev, P.base, r0, nrows, in);
+        change = residual_lane(P);
+      }
       __syncthreads();
-      finish_apply<NT, BB>(P, r0, nrows, in, lacc, red);
+      finish_apply<NT, BB>(P, r0, nrows, in, lacc, red, change);
       return;
     }
   }
@@ -623,6 +651,11 @@ __global__ __launch_bounds__(256) void pr_bin_combine_kernel(BinParams P) {
   const uint32_t v0 = it.w & 0xFFFFu;
   const uint32_t r0 = (it.x << BB) + v0;
   const uint32_t nrows = r0 < P.n ? min(rows, P.n - r0) : 0u;
+  OneGraph og{false, 0u};
+  if constexpr (MULTI) {
+    og = one_graph(P, r0, nrows);
+    if (og.one && graph_frozen(P, og.g)) return;
+  }
   {
     const uint32_t row = threadIdx.x % rows, lane = threadIdx.x / rows;
     const unsigned long long* src = P.part + (uint64_t)it.y * kBinRows + v0 + row;
@@ -638,15 +671,29 @@ __global__ __launch_bounds__(256) void pr_bin_combine_kernel(BinParams P) {
     psum[threadIdx.x] = (s0 + s1) + (s2 + s3);
   }
   __syncthreads();
-  finish_rows<256, 256, MULTI, NT, W>(
-      P, r0, nrows,
-      [&](uint32_t v) {
-        unsigned long long t = 0ull;
-        for (uint32_t q = 0; q < lanes; ++q) t += psum[q * rows + v];
-        if constexpr (W) return dequantize_signed(t, *P.qshift);
-        else return dequantize(t);
-      },
-      red, gerr, P.n_items2 + blockIdx.x);
+  auto z = [&](uint32_t v) {
+    unsigned long long t = 0ull;
+    for (uint32_t q = 0; q < lanes; ++q) t += psum[q * rows + v];
+    if constexpr (W) return dequantize_signed(t, *P.qshift);
+    else return dequantize(t);
+  };
+  if constexpr (MULTI) {
+    if (og.one) {
+      const float base = P.basev[r0];
+      double e = 0.0;
+      if (threadIdx.x < nrows) {
+        const uint32_t i = r0 + threadIdx.x;
+        const float xo = bld<NT>(P.x + i), xn = __builtin_fmaf(P.damp, z(threadIdx.x), base);
+        bst<NT>(P.x + i, xn);
+        bst<NT>(P.cout + i, xn / (float)bld<NT>(P.deg + i));
+        e = (double)fabsf(xn - xo);
+      }
+      e = block_sum<256>(e, red);
+      if (threadIdx.x == 0 && e > 0.0) atomicAdd(P.acc + (uint64_t)P.iter * P.ngraphs + og.g, err_to_fixed(e));
+      return;
+    }
+  }
+  finish_rows<256, 256, MULTI, NT, W>(P, r0, nrows, z, red, gerr, P.n_items2 + blockIdx.x);
 }
 
 // weighted sweep: the L1 change of sweep k, the bin items' and combine units' partials added in a
