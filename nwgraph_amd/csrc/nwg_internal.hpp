@@ -136,7 +136,7 @@ struct BinnedLayout {
   uint32_t n_hot = 0;            // sources [0, n_hot) form each bin's hot tile (0: no hot tiles)
   uint64_t nnz = 0, padded = 0;  // entries, and the length of the per-entry array (pads included)
   uint64_t pairs = 0;            // length of the per-pair arrays (tiles padded to 8 pairs)
-  DevBuf<uint16_t> brow;         // per entry: row & (2^bin_bits - 1), | kPairStart on a pair's first entry
+  DevBuf<uint16_t> brow;         // per entry: row & (2^bin_bits - 1), permuted (bin_perm), | kPairStart on a pair's first entry
   DevBuf<uint16_t> bsrc;         // per pair: source & (2^kChunkBits - 1), or the source in a hot tile
   DevBuf<uint32_t> bpid;         // per kBinBlock entries: pair of the block's first entry
   DevBuf<uint32_t> item_he;      // per bin-pass item: end of its part of the bin's hot tile (its first tile)
