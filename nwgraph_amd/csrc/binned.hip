@@ -878,10 +878,11 @@ void binned_build(hipStream_t s, const ActiveCsc& a, uint32_t n, uint64_t nnz, B
   L = BinnedLayout();
   // Bins of 2^14 rows have fewer pairs per entry (0.35 against 0.43 at RMAT-25, so 17 % fewer
   // pair values to store and read), but their 128 KiB of row sums leave one bin-pass
-  // workgroup per CU.  That pays for the largest graphs only: measured on MI355X, RMAT-25
-  // (529 M entries) 0.67 against 0.72 ms per sweep, while the 256-graph union (213 M) and
-  // smaller graphs were slower with them.
-  L.bin_bits = bin_bits ? bin_bits : nnz >= (1ull << 28) ? 14 : 13;
+  // workgroup per CU, which pays once there are enough of them.  Measured on MI355X, us per sweep
+  // with 2^14 / 2^13 rows: RMAT-20 (16 M entries) 50.8 / 43.8, uniform random with 24 M 91.7 / 95.3,
+  // RMAT-22 (65 M) 93.7 / 104.2, 236 M RMAT edges 259 / 289, RMAT-25 (529 M) 622 / 724; the 256-graph
+  // union (213 M, no hot tiles) 390 / 290.
+  L.bin_bits = bin_bits ? bin_bits : nnz >= (hot ? 5ull << 22 : 1ull << 28) ? 14 : 13;
   const uint32_t bin_rows_ = 1u << L.bin_bits;
   L.n_bins = (uint32_t)ceil_div(n, bin_rows_);
   L.n_chunks = (uint32_t)ceil_div(n, kChunkSrc);

@@ -115,6 +115,15 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* __restrict__ p,
   if (i < n) p[i] = v;
 }
 
+__global__ __launch_bounds__(256) void max_u32_kernel(const uint32_t* __restrict__ v, uint64_t n,
+                                                      uint32_t* __restrict__ out) {
+  uint32_t m = 0;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) m = max(m, v[i]);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
+  if (lane_id() == 0) atomicMax(out, m);
+}
+
 // Out-degree histogram of the CSC's source ids [build_degrees, common.hpp:110-121].  A
 // grid of 2 workgroups per CU walks contiguous ranges of the ids with 16-byte loads, four
 // in flight per lane (16 ids), and adds one per id with a non-returning atomic.  Ids below
@@ -512,7 +521,17 @@ void build_csc_device(hipStream_t s, uint32_t n, uint64_t ne, const uint32_t* sr
   g->nnz = nnz;
   g->outdeg.alloc(n);
   out_degrees_device(s, n, nnz, g->csc_idx.p, g->outdeg.p);
+  note_max_outdeg(s, g);
   NWG_HIP(hipStreamSynchronize(s));
+}
+
+void note_max_outdeg(hipStream_t s, nwg_graph* g) {
+  if (g->nnz < kOrderEdges) return;
+  DevBuf<uint32_t> m(1);
+  fill_u32_kernel<<<1, 256, 0, s>>>(m.p, 1, 0u);
+  max_u32_kernel<<<(uint32_t)std::min<uint64_t>(grid_for(g->n), 1024), 256, 0, s>>>(g->outdeg.p, g->n, m.p);
+  NWG_LAUNCH_CHECK();
+  g->max_outdeg = read_back_u32(s, m.p);
 }
 
 void build_csr_device(hipStream_t s, nwg_graph* g) {

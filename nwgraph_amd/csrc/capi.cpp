@@ -125,6 +125,7 @@ int nwg_graph_create_csc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t*
     else g->outdeg.alloc(n);
     nwg::check_device_csc(s, n, nnz, g->csc_ptr.p, g->csc_idx.p, outdeg ? g->outdeg.p : nullptr,
                           outdeg ? nullptr : g->outdeg.p);
+    nwg::note_max_outdeg(s, g.get());
     *out = g.release();
   });
 }

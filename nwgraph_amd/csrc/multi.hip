@@ -313,6 +313,7 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
     B.threshold = (double)threshold;
     B.row_graph = mg->row_graph.p;
     B.ngraphs = G;
+    B.hints = 1;  // nontemporal loads: 256 graphs (213 M edges) 5.55 ms, without hints 6.04, stores too 5.94
   }
 
   CaptureKey key;

@@ -375,6 +375,7 @@ struct nwg_graph {
   uint32_t n = 0;
   uint64_t nnz = 0;
   nwg::DevBuf<uint32_t> csc_ptr, csc_idx, outdeg;
+  uint32_t max_outdeg = 0;  // largest out-degree, of graphs of kOrderEdges edges and more
   // optional transposed structure for the adjoint
   bool has_csr = false;
   nwg::DevBuf<uint32_t> csr_ptr, csr_idx, csr_to_csc;
@@ -478,6 +479,10 @@ void build_segments(hipStream_t s, const uint32_t* rp, uint32_t n, uint32_t min_
                     DevBuf<uint32_t>& rows, DevBuf<uint32_t>& seg_ptr, DevBuf<uint32_t>& seg_row, uint32_t* nrows,
                     uint32_t* nsegs);
 nwg_plan_params default_plan_params();
+// edges from which a default plan may order the vertices by degree
+constexpr uint64_t kOrderEdges = 1ull << 23;
+// g->max_outdeg, when the graph is large enough for a plan to look at it; waits for the device
+void note_max_outdeg(hipStream_t s, nwg_graph* g);
 // the plan a PageRank solve of g builds on first use (binned sweep and degree ordering by size)
 nwg_plan_params default_plan_for(const nwg_graph* g);
 // binned sweep (binned.hip)

@@ -539,18 +539,25 @@ nwg_plan_params default_plan_params() {
 // The plan a PageRank solve builds when none was set or tuned.  Measured on MI355X (edge
 // factor 16, us per sweep, items / binned): RMAT-12 6.1 / 19.6, RMAT-16 9.1 / 19.5, RMAT-18 (3.9 M
 // edges) 21.7 / 26.8, RMAT-19 (8.0 M) 40.6 / 35.7 degree ordered, RMAT-20 79 / 53, uniform random
-// with 2.1 M edges 14.7 / 21.7, with 8.4 M 45.2 / 43.4.  Degree ordering pays from RMAT-19 on and
-// costs a little below.  The plan asks for the binned sweep from kBinnedEdges, and leaves the bin
+// with 2.1 M edges 14.7 / 21.7, with 8.4 M 45.2 / 43.4.  Degree ordering pays from RMAT-19 on where
+// degrees are skewed, and costs where they are not and the numbering has locality of its own
+// (ordered / as given: RMAT-20 43.8 / 51.1, RMAT-22 93.7 / 129.9, uniform random with 79 M edges
+// 241 / 233, the 4096^2 lattice 171 / 151).  Nontemporal loads pay once
+// the pair values (some 4 bytes per entry or, with skewed degrees, per three entries) compete with the
+// streams for the last-level cache, nontemporal stores once they no longer stay there either (us per
+// sweep with hints 0 / 1 / 2: uniform random with 24 M edges 92 / 103 / 111, 67 M 242 / 217 / 234, 79 M
+// 253 / 227 / 234, the lattice with 57 M 159 / 141 / 152, RMAT-22 with 65 M 95 / 104 / 103, RMAT with
+// 236 M 279 / 238 / 256, RMAT-25 with 529 M 666 / 694 / 628).  The plan asks for the binned sweep from kBinnedEdges, and leaves the bin
 // size, hence the sweep, to the graph's size (plan_takes_items).  The binned layout indexes
 // entries and pairs with 32 bits (below 2^31 entries and 2^30 pairs with pads), so larger
 // graphs keep the pull sweep.
 nwg_plan_params default_plan_for(const nwg_graph* g) {
   nwg_plan_params p = default_plan_params();
   if (g->nnz >= kBinnedEdges && g->nnz < (1ull << 30) - (1ull << 26)) p.binned = 1;
-  if (g->nnz >= (1ull << 23)) p.relabel = 1;
-  // nontemporal streams: the pair values the chunk pass stores are read once by the bin pass
-  // (as cached stores, their write-back landed in the bin pass: RMAT-25 0.81 -> 0.72 ms)
-  if (p.binned && g->nnz >= (1ull << 23)) p.stream_hints = 2;
+  const bool skewed = (double)g->max_outdeg > 64.0 + 8.0 * (double)g->nnz / (double)std::max<uint32_t>(g->n, 1);
+  if (g->nnz >= kOrderEdges && skewed) p.relabel = 1;
+  const uint64_t pairs = skewed ? g->nnz / 3 : g->nnz;  // about
+  if (p.binned) p.stream_hints = pairs >= 3ull << 25 ? 2 : pairs >= 1ull << 25 ? 1 : 0;
   return p;
 }
 
