@@ -226,15 +226,19 @@ struct BinParams {
 // A solve's sweeps run as captured HIP graphs of kSegFirst sweeps, then kSegNext at a time,
 // with the host checking the last sweep's L1 change between segments: sweeps after
 // convergence still launch (and exit at once), and at a few microseconds per launch, 80 of
-// them cost more than the check.
+// them cost more than the check.  A check costs about 12 us, an empty sweep 3 with one launch
+// and 7 to 9 with the binned sweeps' three: those are checked from the 8th sweep on
+// (uniform random with 24 M edges, 8 sweeps: 0.75 to 0.63 ms).
 constexpr uint64_t kSegFirst = 20;
+constexpr uint64_t kSegFirstBinned = 8;
 constexpr uint64_t kSegNext = 8;
-inline uint64_t segment_end(uint64_t start, uint64_t max_iters) {
-  const uint64_t len = start == 0 ? kSegFirst : kSegNext;
+inline uint64_t segment_end(uint64_t start, uint64_t max_iters, uint64_t first) {
+  const uint64_t len = start == 0 ? first : kSegNext;
   return start + len < max_iters ? start + len : max_iters;
 }
 
-constexpr uint64_t kMailWords = 8192;  // of nwg_ctx::mail; longer solves copy
+constexpr uint64_t kMailWords = 8192;  // of nwg_ctx::mail for L1 changes; longer solves copy.  Two
+                                       // more words take the teleport check
 
 // Identity of a captured sweep loop: re-capture when any of it changes.
 struct CaptureKey {
@@ -261,7 +265,8 @@ struct Captured {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   CaptureKey key;
-  bool valid = false;
+  bool seen = false;   // a segment was run under key
+  bool valid = false;  // and exec holds it
   void reset() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -329,7 +334,7 @@ struct PrState {
   DevBuf<unsigned long long> bacc;   // binned sweep: per-sweep L1 change, kBinAccLanes lanes
   DevBuf<unsigned long long> ihsum, ilanes;  // item sweep: long rows' sums, L1 change lanes
   DevBuf<uint32_t> ihcnt;            // and long rows' pieces counted
-  DevBuf<double> tcheck;             // teleport check: sum, invalid-entry flag
+  DevBuf<double> tcheck;             // teleport check: partials, result
   std::vector<std::unique_ptr<Captured>> caps;  // the solve's segments of sweeps
 };
 
@@ -401,6 +406,43 @@ struct nwg_graph {
 };
 
 namespace nwg {
+
+// Segment seg of a solve, made of the launches of enqueue(stream): launched one by one the first
+// time, captured into caps[seg] when asked for again under the same key, replayed from then on.
+// Capturing and instantiating 20 sweeps takes the host longer than launching them, so a solve that
+// is not repeated (a graph loaded, solved and dropped; a layout rebuilt after the weights changed)
+// captures nothing, and a segment that no solve reaches is never captured (edge list of 200,000
+// vertices to scores: 1.04 to 0.99 ms; first solve of an R-MAT scale-12 graph 0.93 to 0.14 ms with the rest).
+template <class F>
+void run_segment(nwg_ctx* ctx, std::vector<std::unique_ptr<Captured>>& caps, uint64_t seg, const CaptureKey& key,
+                 F&& enqueue) {
+  while (caps.size() <= seg) caps.emplace_back(new Captured());
+  Captured& cap = *caps[seg];
+  if (!cap.seen || !(cap.key == key)) {
+    cap.reset();
+    cap.key = key;
+    cap.seen = true;
+    enqueue(ctx->stream);
+    return;
+  }
+  if (!cap.valid) {
+    std::lock_guard<std::mutex> capture_lock(capture_mutex());
+    hipStream_t cs = ctx->capture_stream;
+    NWG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
+    try {
+      enqueue(cs);
+    } catch (...) {
+      hipGraph_t tmp = nullptr;
+      (void)hipStreamEndCapture(cs, &tmp);
+      if (tmp) (void)hipGraphDestroy(tmp);
+      throw;
+    }
+    NWG_HIP(hipStreamEndCapture(cs, &cap.graph));
+    NWG_HIP(hipGraphInstantiate(&cap.exec, cap.graph, nullptr, nullptr, 0));
+    cap.valid = true;
+  }
+  NWG_HIP(hipGraphLaunch(cap.exec, ctx->stream));
+}
 
 // ---- builder (build.hip) ----
 // Sort-based CSC/CSR construction on the device.  src/dst are device arrays of ne raw edges.

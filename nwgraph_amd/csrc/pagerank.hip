@@ -328,39 +328,70 @@ __global__ __launch_bounds__(kThreads) void pr_delta_push_kernel(SweepParams P, 
   if (__syncthreads_or(pushed) && threadIdx.x == 0) flags[(uint64_t)P.iter * stride] = 1ull;
 }
 
-// Teleport check: out[0] += sum of v (double), out[1] = 1 when some entry is negative, above
-// 1 or not finite.  The sweeps assume scores stay in [0, 1] (the binned sweep's exact row
+// Teleport check: a sum of v (double), and whether some entry is negative, above 1 or not finite, per
+// workgroup (part), then over all of them (out).  The sweeps assume scores stay in [0, 1] (the binned sweep's exact row
 // sums cover [0, 16), the fixed-point L1 change of a sweep [0, 32)), which holds for every
 // teleport with entries >= 0 summing to at most 1.
+// The host does not wait for the check: the kernels that make the base and write the scores look at it
+// (teleport_ok), and the host after the solve.  (One workgroup per 256 entries adding to one double
+// took 74 us for 1.5 M vertices on MI355X, and the wait some 20.)
+constexpr uint32_t kTeleBlocks = 512;
+struct TeleCheck {
+  double sum;
+  double bad;
+};
+__host__ __device__ __forceinline__ bool teleport_ok(const TeleCheck& c) {
+  return c.bad == 0.0 && c.sum <= 1.0 + kTeleportSlack;
+}
 __global__ __launch_bounds__(kThreads) void pr_teleport_check_kernel(uint32_t n, const float* __restrict__ v,
-                                                                     double* __restrict__ out) {
+                                                                     TeleCheck* __restrict__ part) {
   __shared__ double red_d[kThreads / 64];
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   double t = 0.0;
   bool bad = false;
-  if (i < n) {
+  for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kThreads) {
     const float x = v[i];
-    bad = !(x >= 0.f && x <= 1.f);  // also catches NaN
-    t = bad ? 0.0 : (double)x;
+    if (x >= 0.f && x <= 1.f) t += (double)x;
+    else bad = true;  // NaN too
   }
-  if (__syncthreads_or(bad) && threadIdx.x == 0) out[1] = 1.0;
+  const int any = __syncthreads_or(bad);
   t = block_sum<kThreads>(t, red_d);
-  if (threadIdx.x == 0 && t > 0.0) atomicAdd(out, t);
+  if (threadIdx.x == 0) part[blockIdx.x] = TeleCheck{t, any ? 1.0 : 0.0};
 }
 
-// personalised base (1-d) * v rounded once from double; with a relabelled CSC row i
-// is original vertex order[i]
+// personalised base (1-d) * v rounded once from double, with a relabelled CSC row i is original
+// vertex order[i]; zeros when the check failed, so that no sweep sees a value that it was not made
+// for.  Every workgroup adds up the check's m <= kTeleBlocks partials, the first one leaves the result.
 __global__ __launch_bounds__(kThreads) void pr_base_kernel(uint32_t n, const float* __restrict__ v,
                                                            const uint32_t* __restrict__ order, double omd,
+                                                           const TeleCheck* __restrict__ part, uint32_t m,
+                                                           TeleCheck* __restrict__ out, TeleCheck* __restrict__ mail,
                                                            float* __restrict__ base) {
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  if (i < n) base[i] = (float)(omd * (double)v[order ? order[i] : i]);
+  __shared__ double red_d[kThreads / 64];
+  __shared__ double sum;
+  double t = 0.0, bad = 0.0;
+  for (uint32_t i = threadIdx.x; i < m; i += kThreads) {
+    t += part[i].sum;
+    bad += part[i].bad;
+  }
+  const int any = __syncthreads_or(bad != 0.0);
+  t = block_sum<kThreads>(t, red_d);
+  if (threadIdx.x == 0) sum = t;
+  __syncthreads();
+  const TeleCheck c{sum, any ? 1.0 : 0.0};
+  if (blockIdx.x == 0 && threadIdx.x == 0) *out = *mail = c;
+  const bool ok = teleport_ok(c);
+  for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kThreads)
+    base[i] = ok ? (float)(omd * (double)v[order ? order[i] : i]) : 0.f;
 }
 
 // scores out, back to the original numbering with rank (original -> new id): out[v] = x[rank[v]].
 // A gather: the writes are whole lines, and the reads of x come mostly from MALL.
+// tele (nullable): the teleport's check; nothing is written when it failed.
 __global__ __launch_bounds__(kThreads) void pr_out_kernel(uint32_t n, const uint32_t* __restrict__ rank,
-                                                          const float* __restrict__ x, float* __restrict__ out) {
+                                                          const float* __restrict__ x,
+                                                          const TeleCheck* __restrict__ tele,
+                                                          float* __restrict__ out) {
+  if (tele && !teleport_ok(*tele)) return;
   const uint32_t v = blockIdx.x * kThreads + threadIdx.x;
   if (v < n) out[v] = x[rank ? rank[v] : v];
 }
@@ -977,18 +1008,14 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   }
   const bool personalised = teleport_dev != nullptr;
   if (personalised) {
-    st.tcheck.ensure(2);
-    NWG_HIP(hipMemsetAsync(st.tcheck.p, 0, 2 * sizeof(double), s));
-    pr_teleport_check_kernel<<<blocks_for(n), kThreads, 0, s>>>(n, teleport_dev, st.tcheck.p);
-    NWG_LAUNCH_CHECK();
-    double chk[2] = {0.0, 0.0};
-    NWG_HIP(hipMemcpyAsync(chk, st.tcheck.p, sizeof chk, hipMemcpyDeviceToHost, s));
-    NWG_HIP(hipStreamSynchronize(s));
-    NWG_REQUIRE(chk[1] == 0.0, "teleport entries must be finite and in [0, 1]");
-    NWG_REQUIRE(chk[0] <= 1.0 + kTeleportSlack, "teleport entries must sum to at most 1");
+    st.tcheck.ensure(2 * (kTeleBlocks + 1));
     st.base.ensure(n);
-    pr_base_kernel<<<blocks_for(n), kThreads, 0, s>>>(n, teleport_dev, g->active(g->plan.params.relabel != 0).order,
-                                                      1.0 - (double)damping, st.base.p);
+    const uint32_t blocks = std::min(blocks_for(n), kTeleBlocks);
+    TeleCheck* part = reinterpret_cast<TeleCheck*>(st.tcheck.p);
+    pr_teleport_check_kernel<<<blocks, kThreads, 0, s>>>(n, teleport_dev, part);
+    pr_base_kernel<<<blocks, kThreads, 0, s>>>(n, teleport_dev, g->active(g->plan.params.relabel != 0).order,
+                                               1.0 - (double)damping, part, blocks, part + kTeleBlocks,
+                                               reinterpret_cast<TeleCheck*>(ctx->mail + kMailWords), st.base.p);
     NWG_LAUNCH_CHECK();
   }
   const SweepParams P = make_params(g, st, personalised, damping, threshold);
@@ -1003,8 +1030,18 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   auto copy_out = [&] {
     if (!scores_dev) return;
     const uint32_t* rank = g->plan.params.relabel ? g->rl->rank.p : nullptr;
-    pr_out_kernel<<<blocks_for(n), kThreads, 0, s>>>(n, rank, st.x.p, scores_dev);
+    pr_out_kernel<<<blocks_for(n), kThreads, 0, s>>>(
+        n, rank, st.x.p, personalised ? reinterpret_cast<const TeleCheck*>(st.tcheck.p) + kTeleBlocks : nullptr,
+        scores_dev);
     NWG_LAUNCH_CHECK();
+  };
+  // after a wait for the device
+  auto check_teleport = [&] {
+    if (!personalised) return;
+    TeleCheck c;
+    std::memcpy(&c, ctx->mail + kMailWords, sizeof c);
+    NWG_REQUIRE(c.bad == 0.0, "teleport entries must be finite and in [0, 1]");
+    NWG_REQUIRE(teleport_ok(c), "teleport entries must sum to at most 1");
   };
   if (!timing) {
     CaptureKey key;
@@ -1029,43 +1066,22 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     key.damping = damping;
     key.threshold = threshold;
     key.extra = (uint32_t)sched;
-    // the solve's segments (kSegFirst sweeps, then kSegNext at a time), each one captured
-    // graph; between segments the host reads the last sweep's L1 change and stops once the
-    // solve has converged, so sweeps after convergence launch only up to a segment's end
-    uint64_t nseg = 0;
-    for (uint64_t k0 = 0;; k0 = segment_end(k0, max_iters)) {
-      const uint64_t k1 = segment_end(k0, max_iters);
-      if (st.caps.size() <= nseg) st.caps.emplace_back(new Captured());
-      Captured& cap = *st.caps[nseg++];
-      if (!cap.valid || !(cap.key == key)) {
-        cap.reset();
-        std::lock_guard<std::mutex> capture_lock(capture_mutex());
-        hipStream_t cs = ctx->capture_stream;
-        NWG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-        try {
-          enqueue_solve(cs, g, st, P, max_iters, nullptr, sched, k0, k1, mail);
-        } catch (...) {
-          hipGraph_t tmp = nullptr;
-          (void)hipStreamEndCapture(cs, &tmp);
-          if (tmp) (void)hipGraphDestroy(tmp);
-          throw;
-        }
-        NWG_HIP(hipStreamEndCapture(cs, &cap.graph));
-        NWG_HIP(hipGraphInstantiate(&cap.exec, cap.graph, nullptr, nullptr, 0));
-        cap.key = key;
-        cap.valid = true;
-      }
-      if (k1 >= max_iters) break;
-    }
+    const uint64_t first = items || class_kernels ? kSegFirst : kSegFirstBinned;
+    // the solve runs in segments (first sweeps, then kSegNext at a time); between segments the host
+    // reads the last sweep's L1 change and stops once the solve has converged, so sweeps after
+    // convergence launch only up to a segment's end
     NWG_HIP(hipEventRecord(ctx->ev0, s));
     uint64_t seg = 0;
-    for (uint64_t k0 = 0;; k0 = segment_end(k0, max_iters)) {
-      const uint64_t k1 = segment_end(k0, max_iters);
-      NWG_HIP(hipGraphLaunch(st.caps[seg++]->exec, s));
+    for (uint64_t k0 = 0;; k0 = segment_end(k0, max_iters, first)) {
+      const uint64_t k1 = segment_end(k0, max_iters, first);
+      run_segment(ctx, st.caps, seg++, key, [&](hipStream_t t) {
+        enqueue_solve(t, g, st, P, max_iters, nullptr, sched, k0, k1, mail);
+      });
       if (k1 >= max_iters) break;
       unsigned long long last = 0ull;
       if (!mail) NWG_HIP(hipMemcpyAsync(&last, st.acc.p + (k1 - 1), sizeof last, hipMemcpyDeviceToHost, s));
       NWG_HIP(hipStreamSynchronize(s));
+      check_teleport();
       if (mail) last = mail[k1 - 1];
       // stopped: delta schedule, nothing pushed (page_rank.hpp:616-620); else the L1 change
       // below the threshold (page_rank.hpp:144) -- or the solve stopped earlier and this
@@ -1093,6 +1109,15 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     NWG_HIP(hipMemcpyAsync(acc.data(), st.acc.p, max_iters * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   copy_out();
   NWG_HIP(hipStreamSynchronize(s));
+  if (timing && personalised) {
+    try {
+      check_teleport();
+    } catch (...) {
+      for (auto& e : evs) (void)hipEventDestroy(e);
+      throw;
+    }
+  }
+  check_teleport();
   // sweeps that were not launched changed nothing
   if (mail) std::copy(mail, mail + launched, acc.begin());
   NWG_HIP(hipEventElapsedTime(&ms_total, ctx->ev0, ctx->ev1));

@@ -657,41 +657,15 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
   // changed may sit at the old one's host address
   key.plan_version = L ? L->build_id : grid;
   key.extra = (relative ? 1u : 0u) | (q.y0 ? 0u : 2u) | ((uint32_t)kind << 2);
-  // the segments' graphs, captured when missing or stale
-  uint64_t nseg = 0;
-  for (uint64_t k0 = 0; k0 < max_iters || (k0 == 0 && nseg == 0); k0 = segment_end(k0, max_iters)) {
-    const uint64_t k1 = segment_end(k0, max_iters);
-    if (caps.size() <= nseg) caps.emplace_back(new Captured());
-    Captured& cap = *caps[nseg];
-    ++nseg;
-    if (!cap.valid || !(cap.key == key)) {
-      cap.reset();
-      std::lock_guard<std::mutex> capture_lock(capture_mutex());
-      hipStream_t cs = ctx->capture_stream;
-      NWG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-      try {
-        enqueue(cs, k0, k1);
-      } catch (...) {
-        hipGraph_t tmp = nullptr;
-        (void)hipStreamEndCapture(cs, &tmp);
-        if (tmp) (void)hipGraphDestroy(tmp);
-        throw;
-      }
-      NWG_HIP(hipStreamEndCapture(cs, &cap.graph));
-      NWG_HIP(hipGraphInstantiate(&cap.exec, cap.graph, nullptr, nullptr, 0));
-      cap.key = key;
-      cap.valid = true;
-    }
-    if (k1 >= max_iters) break;
-  }
+  const uint64_t first = kind == WSweep::kBinned ? kSegFirstBinned : kSegFirst;
   std::vector<double> h(std::max<uint64_t>(max_iters, 1), 0.0);
   WScale sc{1.0, 0, 1};
   double stop = (double)q.threshold;
   uint64_t iters = max_iters, seg = 0;
   NWG_HIP(hipEventRecord(ctx->ev0, s));
-  for (uint64_t k0 = 0;; k0 = segment_end(k0, max_iters), ++seg) {
-    const uint64_t k1 = segment_end(k0, max_iters);
-    NWG_HIP(hipGraphLaunch(caps[seg]->exec, s));
+  for (uint64_t k0 = 0;; k0 = segment_end(k0, max_iters, first), ++seg) {
+    const uint64_t k1 = segment_end(k0, max_iters, first);
+    run_segment(ctx, caps, seg, key, [&](hipStream_t t) { enqueue(t, k0, k1); });
     NWG_HIP(hipEventRecord(ctx->ev1, s));
     wout_kernel<<<grid1(n), kThreads, 0, s>>>(n, y[0], y[1], st.err.p, (uint32_t)k1, (double)q.threshold, thr_scale,
                                              q.out);
