@@ -86,7 +86,7 @@ typedef struct nwg_plan_params {
   uint32_t stream_hints; /* non-temporal hints.  Pull sweep: 0 none, 1 the column-id stream, 2 every
                             streamed array.  Binned sweep: 0 none, 1 loads of the streams read once
                             per sweep, 2 also the stores of pair values, partial rows and scores */
-  uint32_t ppr_tile;     /* k-tile of the batched solve: 8, 16, 32 or 64 vectors per lane group (0 = widest <= k) */
+  uint32_t ppr_tile;     /* k-tile of the batched solve: 8, 16, 32 or 64 vectors per lane group (0 = narrowest >= k, at most 64) */
   uint32_t relabel;      /* 1: sweep a copy of the CSC renumbered by out-degree (results returned in original ids) */
   uint32_t binned;       /* 1: binned sweep (propagation blocking over a tiled copy of the CSC, 8 bytes per
                             entry; row sums exact in fixed point) instead of the degree-binned pull sweep */

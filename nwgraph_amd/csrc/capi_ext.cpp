@@ -61,9 +61,11 @@ int nwg_ppr_batched(nwg_ctx* ctx, nwg_graph* g, uint32_t k, const uint32_t* seed
     hipStream_t s = ctx->stream;
     std::vector<uint32_t> sp(seed_ptr, seed_ptr + k + 1), sd(seeds, seeds + seed_ptr[k]);
     // the k-tile: the plan's (set by nwg_ppr_autotune or nwg_graph_set_plan), else the
-    // widest tile that does not exceed k
+    // narrowest one that holds all k vectors, up to 64: an edge costs one gather per tile, of nearly
+    // the same time for 32 to 128 bytes (RMAT-20, ms for T = 8 / 16 / 32 / 64: k = 10 4.8 / 2.8 / 4.4 / 7.5,
+    // k = 24 7.1 / 6.2 / 4.8 / 7.7, k = 33 13.8 / 9.4 / 9.5 / 8.1), and the padding is that of two narrower tiles
     const uint32_t req = g->plan.built ? g->plan.params.ppr_tile : 0;
-    const uint32_t tile = req ? req : (k >= 64 ? 64 : k >= 32 ? 32 : k >= 16 ? 16 : 8);
+    const uint32_t tile = req ? req : (k > 32 ? 64 : k > 16 ? 32 : k > 8 ? 16 : 8);
     Staged<float> sc(s, scores, (size_t)g->n * k, mem_kind, false);
     nwg::ppr_run(ctx, g, k, sp, sd, damping, threshold, max_iters, tile, sc.dev, iterations, info);
     sc.finish(s);
