@@ -240,6 +240,121 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
     atomicAdd(P.lanes + (P.iter % 3) * kItemLaneSlot + (blockIdx.x % kItemLanes) * kItemLanePad, err);
 }
 
+// ---- many graphs ----
+// L1 change of graph g in sweep k
+__device__ __forceinline__ unsigned long long many_change(const ItemParams& P, const ManyParams& M, uint32_t k,
+                                                          uint32_t g) {
+  const unsigned long long* l = P.lanes + (uint64_t)(k % 3) * kManyLanes * M.ngraphs + g;
+  unsigned long long s = 0ull;
+#pragma unroll
+  for (uint32_t q = 0; q < kManyLanes; ++q) s += l[(uint64_t)q * M.ngraphs];
+  return s;
+}
+
+// The sweep over the union of many graphs: items are cut from it as from one graph, so one may hold rows
+// of several.  The L1 changes of its first kManyLocal graphs meet in LDS, those of further ones
+// (graphs of a few vertices) go to memory row by row.  Measured on MI355X, ms for 20 sweeps here / with
+// workgroups of up to 4096 edges that add up a row per lane / binned: 63 graphs of 256 to 1024
+// vertices (0.4 M edges) 0.17 / 0.42 / 0.39, 12 of 2^12 to 2^18 (9.5 M) 0.87 / 4.7 / 1.53, 80 of 2^12 to 2^16
+// (18.7 M) 1.47 / 4.5 / 1.63.
+constexpr uint32_t kManyLocal = 64;
+__global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyParams M) {
+  __shared__ unsigned long long pre[9 * kNT];
+  __shared__ unsigned long long wsum[kNT / 64];
+  __shared__ unsigned long long errs[kManyLocal];
+  __shared__ uint32_t done[kManyLocal];
+  // the previous sweep's changes, for the host, and the next sweep's lanes
+  if (P.iter > 0)
+    for (uint32_t q = blockIdx.x * kNT + threadIdx.x; q < M.ngraphs; q += gridDim.x * kNT)
+      P.acc[(uint64_t)(P.iter - 1) * M.ngraphs + q] = many_change(P, M, P.iter - 1, q);
+  for (uint64_t q = blockIdx.x * kNT + threadIdx.x; q < (uint64_t)kManyLanes * M.ngraphs; q += gridDim.x * kNT)
+    P.lanes[(uint64_t)((P.iter + 1) % 3) * kManyLanes * M.ngraphs + q] = 0ull;
+  const uint4 d = P.desc[blockIdx.x];
+  const uint32_t e0 = d.x, e1 = d.y, r0 = d.z, rows = d.w & kRowMask;
+  const bool head = d.w & kHeadPiece, tail = d.w & kTailPiece;
+  if (!rows && !head && !tail) return;
+  uint32_t ra = 0, rb = 0, dg = 0, rg = 0;
+  float xo = 0.f, bv = 0.f;
+  if (threadIdx.x < rows) {
+    const uint32_t i = r0 + threadIdx.x;
+    ra = P.rp[i];
+    rb = P.rp[i + 1];
+    xo = P.x[i];
+    dg = P.deg[i];
+    bv = P.basev[i];
+    rg = M.row_graph[i];
+  }
+  const uint32_t g0 = M.row_graph[head ? r0 - 1 : r0], g1 = M.row_graph[tail ? r0 + rows : r0 + rows - 1];
+  if (threadIdx.x < kManyLocal) {
+    const uint32_t g = g0 + threadIdx.x;
+    errs[threadIdx.x] = 0ull;
+    done[threadIdx.x] = P.iter > 0 && g <= g1 && fixed_to_err(many_change(P, M, P.iter - 1, g)) < P.threshold;
+  }
+  const bool piece = (threadIdx.x == 0 && head) || (threadIdx.x == 1 && tail);
+  uint32_t h = 0, hp0 = 0, hp1 = 0;
+  if (piece) {
+    h = threadIdx.x == 0 ? r0 - 1 : r0 + rows;
+    hp0 = P.rp[h];
+    hp1 = P.rp[h + 1];
+  }
+  const uint32_t b0 = e0 & ~3u;
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
+  else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
+  if (g0 == g1 && done[0]) return;
+  unsigned long long* const lane =
+      P.lanes + ((uint64_t)(P.iter % 3) * kManyLanes + blockIdx.x % kManyLanes) * M.ngraphs;
+  auto sum = [&](uint32_t a, uint32_t b) { return item_sum(pre, b0, a, b); };
+  auto solved = [&](uint32_t g) {
+    return g - g0 < kManyLocal ? done[g - g0] != 0
+                               : P.iter > 0 && fixed_to_err(many_change(P, M, P.iter - 1, g)) < P.threshold;
+  };
+  unsigned long long err = 0ull;  // with one graph only
+  auto add = [&](uint32_t g, unsigned long long e) {
+    if (g0 == g1) err += e;
+    else if (!e) return;
+    else if (g - g0 < kManyLocal) atomicAdd(&errs[g - g0], e);
+    else atomicAdd(lane + g, e);
+  };
+  if (threadIdx.x < rows && !solved(rg))
+    add(rg, item_update(P, r0 + threadIdx.x, dequantize(sum(ra, rb)), xo, bv, dg));
+  for (uint32_t q = threadIdx.x + kNT; q < rows; q += kNT) {
+    const uint32_t i = r0 + q, g = M.row_graph[i];
+    if (!solved(g)) add(g, item_update(P, i, dequantize(sum(P.rp[i], P.rp[i + 1])), P.x[i], P.basev[i], P.deg[i]));
+  }
+  if (piece) {
+    // all pieces of a row see the same change, so they are all added or none is
+    const uint32_t g = M.row_graph[h];
+    unsigned long long z;
+    uint32_t a;
+    if (!solved(g) && add_piece(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a))
+      add(g, item_update(P, h, dequantize(z), P.x[h], P.basev[h], P.deg[h]));
+  }
+  if (g0 == g1) {
+    err = wave_sum(err);
+    if (lane_id() == 0) wsum[threadIdx.x >> 6] = err;
+    __syncthreads();
+    err = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+    if (threadIdx.x == 0 && err) atomicAdd(lane + g0, err);
+  } else {
+    __syncthreads();
+    if (threadIdx.x < kManyLocal && errs[threadIdx.x]) atomicAdd(lane + g0 + threadIdx.x, errs[threadIdx.x]);
+  }
+}
+
+__global__ __launch_bounds__(256) void item_many_init_kernel(ItemParams P, ManyParams M) {
+  const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < P.count) {
+    P.hsum[i] = 0ull;
+    P.hcnt[i] = 0u;
+  }
+  if (i < 3ull * kManyLanes * M.ngraphs) P.lanes[i] = 0ull;
+}
+
+__global__ __launch_bounds__(256) void item_many_fold_kernel(ItemParams P, ManyParams M, uint32_t k) {
+  const uint32_t g = blockIdx.x * 256 + threadIdx.x;
+  if (g < M.ngraphs) P.acc[(uint64_t)k * M.ngraphs + g] = many_change(P, M, k, g);
+}
+
 // ---- weighted ----
 // The L1 changes of a weighted sweep have no bound (fixed_point.hpp's scale covers row sums), so
 // they stay doubles: every item stores its own and, where a long row starts in it, that row's; every
@@ -537,6 +652,22 @@ void items_enqueue_init(hipStream_t s, const ItemParams& P, float init, float* c
 
 void items_enqueue_sweep(hipStream_t s, const ItemParams& P) {
   pr_item_kernel<<<P.count, kNT, 0, s>>>(P);
+  NWG_LAUNCH_CHECK();
+}
+
+void items_many_enqueue_init(hipStream_t s, const ItemParams& P, const ManyParams& M) {
+  const uint64_t m = std::max<uint64_t>(P.count, 3ull * kManyLanes * M.ngraphs);
+  item_many_init_kernel<<<(uint32_t)ceil_div(m, 256), 256, 0, s>>>(P, M);
+  NWG_LAUNCH_CHECK();
+}
+
+void items_many_enqueue_sweep(hipStream_t s, const ItemParams& P, const ManyParams& M) {
+  pr_item_many_kernel<<<P.count, kNT, 0, s>>>(P, M);
+  NWG_LAUNCH_CHECK();
+}
+
+void items_many_enqueue_fold(hipStream_t s, const ItemParams& P, const ManyParams& M, uint32_t k) {
+  item_many_fold_kernel<<<(uint32_t)ceil_div(M.ngraphs, 256), 256, 0, s>>>(P, M, k);
   NWG_LAUNCH_CHECK();
 }
 

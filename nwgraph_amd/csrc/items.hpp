@@ -37,6 +37,15 @@ struct ItemParams {
   double threshold;
 };
 
+// Many graphs in one block-diagonal CSC: every row has its graph's base (ItemParams::basev), and every
+// graph its own L1 changes and stopping rule.  ItemParams::acc is iters x ngraphs, and lanes are
+// 3 slots of kManyLanes lanes of ngraphs counters (slots as in ItemParams).
+constexpr uint32_t kManyLanes = 8;
+struct ManyParams {
+  const uint32_t* row_graph;  // non-decreasing
+  uint32_t ngraphs;
+};
+
 // Where a segment of weighted sweeps leaves what the host reads: the solve's two words of scales, then
 // err[k] at words[2 + k], k in [first, last] of the segment (words null: nowhere).
 struct WMail {
@@ -104,6 +113,10 @@ void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, ui
 // hsum and hcnt (count each)
 void items_enqueue_init(hipStream_t s, const ItemParams& P, float init, float* c0, uint64_t iters);
 void items_enqueue_sweep(hipStream_t s, const ItemParams& P);
+// Many graphs: hsum, hcnt and the lanes cleared; a sweep; acc of sweep k, the last one launched
+void items_many_enqueue_init(hipStream_t s, const ItemParams& P, const ManyParams& M);
+void items_many_enqueue_sweep(hipStream_t s, const ItemParams& P, const ManyParams& M);
+void items_many_enqueue_fold(hipStream_t s, const ItemParams& P, const ManyParams& M, uint32_t k);
 // Weighted: xin[0] = src (null: v), err[0 .. iters) and the items' counters cleared; a sweep; err[k]
 // of sweep k, the last one launched.
 void witems_enqueue_init(hipStream_t s, const WItemParams& P, const float* src, float v, float* dst, uint64_t iters);

@@ -1,7 +1,9 @@
 // multi.hip -- many independent graphs solved by one persistent launch per sweep.
 //
 // The graphs are concatenated into one block-diagonal CSC (vertex ids offset per
-// graph).  The union is cut into work items (graph, rows [r0, r1)): up to 256
+// graph), swept by the item sweep (items.hip) or, as a plan option, the binned sweep.  Outside
+// 0 <= damping <= 1, where scores may leave the range of the exact sums, the union is cut into
+// work items (graph, rows [r0, r1)): up to 256
 // consecutive rows of one graph whose in-edges total at most kItemNnz, or one row
 // with more in-edges (a hub item).  A persistent grid walks the items round-robin;
 // each sweep:
@@ -11,7 +13,7 @@
 //   hub item     the whole workgroup strides over the row and reduces
 // Each graph keeps the reference's scalars (init = 1/N_g, base = (1-d)/N_g,
 // page_rank.hpp:92-94) and its own stopping rule: the L1 change of graph g in sweep k
-// is accumulated in fixed point in acc[k][g]; items of a converged graph are skipped.
+// is accumulated in fixed point in acc[k][g]; rows of a converged graph are skipped.
 // The init launch and max_iters sweep launches are captured in one HIP graph.
 #include <hip/hip_runtime.h>
 
@@ -114,24 +116,19 @@ __global__ __launch_bounds__(kThreads) void multi_copy_kernel(uint32_t n, uint64
                                                               uint32_t eoff, float init, uint32_t* __restrict__ rp_all,
                                                               uint32_t* __restrict__ col_all,
                                                               uint32_t* __restrict__ deg_all,
-                                                              float* __restrict__ vinit) {
+                                                              float* __restrict__ vinit, uint32_t g,
+                                                              uint32_t* __restrict__ row_graph) {
   const uint64_t t = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
   if (t < n) {
     rp_all[voff + t] = eoff + rp[t];
     deg_all[voff + t] = deg[t];
     vinit[voff + t] = init;
+    row_graph[voff + t] = g;
   }
   if (t < nnz) col_all[eoff + t] = col[t] + voff;
 }
 
-// graph of every row of the union
-__global__ __launch_bounds__(kThreads) void row_graph_kernel(uint32_t n, uint32_t voff, uint32_t g,
-                                                             uint32_t* __restrict__ row_graph) {
-  const uint32_t t = blockIdx.x * kThreads + threadIdx.x;
-  if (t < n) row_graph[voff + t] = g;
-}
-
-// per-row base (1-d)/N_g of the binned sweep
+// per-row base (1-d)/N_g
 __global__ __launch_bounds__(kThreads) void row_base_kernel(uint64_t nv, const uint32_t* __restrict__ row_graph,
                                                             const float* __restrict__ gbase, float* __restrict__ base) {
   const uint64_t t = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
@@ -154,6 +151,11 @@ struct nwg_multigraph {
   nwg::DevBuf<float> vinit, x, c0, c1, gbase;
   nwg::DevBuf<unsigned long long> acc;
   uint32_t n_items = 0;
+  // item sweep of the union
+  nwg::DevBuf<uint4> idesc;
+  nwg::DevBuf<unsigned long long> ihsum, ilanes;
+  nwg::DevBuf<uint32_t> ihcnt;
+  uint32_t n_sweep_items = 0;
   nwg::Captured cap;
   // binned sweep of the union (plan option binned)
   bool binned = false;
@@ -186,21 +188,39 @@ nwg_multigraph* multigraph_create(nwg_ctx* ctx, uint32_t ngraphs, nwg_graph* con
   mg->col.alloc(mg->ne ? mg->ne : 1);
   mg->deg.alloc(mg->nv);
   mg->vinit.alloc(mg->nv);
+  mg->row_graph.alloc(mg->nv);
+  mg->row_base.alloc(mg->nv);
   for (uint32_t g = 0; g < ngraphs; ++g) {
     const nwg_graph* gr = graphs[g];
     multi_copy_kernel<<<grid1(std::max<uint64_t>(gr->n, gr->nnz)), kThreads, 0, s>>>(
         gr->n, gr->nnz, gr->csc_ptr.p, gr->csc_idx.p, gr->outdeg.p, (uint32_t)mg->voff[g], (uint32_t)eoff[g],
-        (float)(1.0 / gr->n), mg->rp.p, mg->col.p, mg->deg.p, mg->vinit.p);
+        (float)(1.0 / gr->n), mg->rp.p, mg->col.p, mg->deg.p, mg->vinit.p, g, mg->row_graph.p);
     NWG_LAUNCH_CHECK();
   }
   const uint32_t ne32 = (uint32_t)mg->ne;
   NWG_HIP(hipMemcpyAsync(mg->rp.p + mg->nv, &ne32, 4, hipMemcpyHostToDevice, s));
-  // work items from the union's row pointers
+  mg->x.alloc(mg->nv);
+  mg->c0.alloc(mg->nv);
+  mg->c1.alloc(mg->nv);
+  mg->gbase.alloc(ngraphs);
+  mg->n_sweep_items = item_count((uint32_t)mg->nv, mg->ne);
+  mg->idesc.alloc(mg->n_sweep_items);
+  mg->ihsum.alloc(mg->n_sweep_items);
+  mg->ihcnt.alloc(mg->n_sweep_items);
+  mg->ilanes.alloc(3ull * kManyLanes * ngraphs);
+  if (mg->n_sweep_items) items_build(s, (uint32_t)mg->nv, mg->ne, mg->rp.p, mg->idesc.p);
+  NWG_HIP(hipStreamSynchronize(s));
+  return mg.release();
+}
+
+// work items of multi_sweep_kernel from the union's row pointers
+static void build_row_items(hipStream_t s, nwg_multigraph* mg) {
+  if (mg->n_items) return;
   std::vector<uint32_t> rp(mg->nv + 1);
   NWG_HIP(hipMemcpyAsync(rp.data(), mg->rp.p, (mg->nv + 1) * 4, hipMemcpyDeviceToHost, s));
   NWG_HIP(hipStreamSynchronize(s));
   std::vector<uint32_t> ig, i0, i1;
-  for (uint32_t g = 0; g < ngraphs; ++g) {
+  for (uint32_t g = 0; g < mg->ngraphs; ++g) {
     uint64_t r = mg->voff[g];
     const uint64_t rend = mg->voff[g + 1];
     while (r < rend) {
@@ -214,35 +234,23 @@ nwg_multigraph* multigraph_create(nwg_ctx* ctx, uint32_t ngraphs, nwg_graph* con
       r = r1;
     }
   }
-  mg->n_items = (uint32_t)ig.size();
   mg->item_graph.alloc(ig.size());
   mg->item_r0.alloc(ig.size());
   mg->item_r1.alloc(ig.size());
   NWG_HIP(hipMemcpyAsync(mg->item_graph.p, ig.data(), ig.size() * 4, hipMemcpyHostToDevice, s));
   NWG_HIP(hipMemcpyAsync(mg->item_r0.p, i0.data(), i0.size() * 4, hipMemcpyHostToDevice, s));
   NWG_HIP(hipMemcpyAsync(mg->item_r1.p, i1.data(), i1.size() * 4, hipMemcpyHostToDevice, s));
-  mg->x.alloc(mg->nv);
-  mg->c0.alloc(mg->nv);
-  mg->c1.alloc(mg->nv);
-  mg->gbase.alloc(ngraphs);
   NWG_HIP(hipStreamSynchronize(s));
-  return mg.release();
+  mg->n_items = (uint32_t)ig.size();
 }
 
-// Selects the schedule of the union's sweeps: the items of multi_sweep_kernel, or the binned
+// Selects the schedule of the union's sweeps: the item sweep (items.hip), or the binned
 // sweep (binned.hip) over a tiled copy of the union with a graph id per row.
 void multigraph_set_binned(nwg_ctx* ctx, nwg_multigraph* mg, bool binned) {
   hipStream_t s = ctx->stream;
   if (binned && !mg->bl.built) {
-    mg->row_graph.alloc(mg->nv ? mg->nv : 1);
-    for (uint32_t g = 0; g < mg->ngraphs; ++g) {
-      const uint32_t n = (uint32_t)(mg->voff[g + 1] - mg->voff[g]);
-      if (n) row_graph_kernel<<<grid1(n), kThreads, 0, s>>>(n, (uint32_t)mg->voff[g], g, mg->row_graph.p);
-    }
-    NWG_LAUNCH_CHECK();
     // no hot tiles: the union's first ids are one graph's, not the union's hubs
     binned_build(s, ActiveCsc{mg->rp.p, mg->col.p, mg->deg.p, nullptr}, (uint32_t)mg->nv, mg->ne, mg->bl, false);
-    mg->row_base.alloc(mg->nv ? mg->nv : 1);
     mg->bvals.alloc(mg->bl.pairs);
     mg->bpart.alloc(std::max<uint64_t>((uint64_t)mg->bl.n_slots << mg->bl.bin_bits, 1));
     NWG_HIP(hipStreamSynchronize(s));
@@ -262,6 +270,9 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   NWG_HIP(hipMemcpyAsync(mg->gbase.p, gb.data(), G * 4ull, hipMemcpyHostToDevice, s));
   mg->acc.ensure(std::max<uint64_t>(max_iters, 1) * G);
 
+  // the item sweep sums scores in fixed point, which holds for those in [0, 1]
+  const bool items = !mg->binned && mg->n_sweep_items && damping >= 0.f && damping <= 1.f;
+  if (!mg->binned && !items) build_row_items(s, mg);
   int dev = 0, cus = 0;
   NWG_HIP(hipGetDevice(&dev));
   NWG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -282,10 +293,30 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   P.acc = mg->acc.p;
   P.threshold = (double)threshold;
 
-  BinParams B{};
-  if (mg->binned) {
+  if (mg->binned || items) {
     row_base_kernel<<<grid1(mg->nv), kThreads, 0, s>>>(mg->nv, mg->row_graph.p, mg->gbase.p, mg->row_base.p);
     NWG_LAUNCH_CHECK();
+  }
+  ItemParams I{};
+  I.desc = mg->idesc.p;
+  I.rp = mg->rp.p;
+  I.col = mg->col.p;
+  I.deg = mg->deg.p;
+  I.x = mg->x.p;
+  I.basev = mg->row_base.p;
+  I.damp = damping;
+  I.n = (uint32_t)mg->nv;
+  I.nnz = (uint32_t)mg->ne;
+  I.count = mg->n_sweep_items;
+  I.hsum = mg->ihsum.p;
+  I.hcnt = mg->ihcnt.p;
+  I.lanes = mg->ilanes.p;
+  I.acc = mg->acc.p;
+  I.threshold = (double)threshold;
+  const ManyParams M{mg->row_graph.p, G};
+
+  BinParams B{};
+  if (mg->binned) {
     const BinnedLayout& L = mg->bl;
     B.brow = L.brow.p;
     B.bsrc = L.bsrc.p;
@@ -322,7 +353,7 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   key.iters = max_iters;
   key.damping = damping;
   key.threshold = threshold;
-  key.extra = grid | (mg->binned ? 0x80000000u : 0u);
+  key.extra = grid | (mg->binned ? 0x80000000u : 0u) | (items ? 0x40000000u : 0u);
   if (!mg->cap.valid || !(mg->cap.key == key)) {
     mg->cap.reset();
     std::lock_guard<std::mutex> capture_lock(capture_mutex());
@@ -331,7 +362,15 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
     try {
       multi_init_kernel<<<grid1(std::max<uint64_t>(mg->nv, max_iters * G)), kThreads, 0, cs>>>(
           mg->nv, mg->deg.p, mg->vinit.p, mg->x.p, mg->c0.p, mg->acc.p, max_iters * G);
+      if (items) items_many_enqueue_init(cs, I, M);
       for (uint64_t k = 0; k < max_iters; ++k) {
+        if (items) {
+          I.iter = (uint32_t)k;
+          I.cin = (k & 1) ? mg->c1.p : mg->c0.p;
+          I.cout = (k & 1) ? mg->c0.p : mg->c1.p;
+          items_many_enqueue_sweep(cs, I, M);
+          continue;
+        }
         if (mg->binned) {
           B.iter = (uint32_t)k;
           binned_enqueue_sweep(cs, B);  // throws on a failed launch
@@ -342,6 +381,7 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
         P.cout = (k & 1) ? mg->c0.p : mg->c1.p;
         multi_sweep_kernel<<<grid, kThreads, 0, cs>>>(P);
       }
+      if (items && max_iters) items_many_enqueue_fold(cs, I, M, (uint32_t)max_iters - 1);
     } catch (...) {
       // leave the capture stream out of capture mode, so that later solves can record again
       hipGraph_t tmp = nullptr;

@@ -340,8 +340,8 @@ class MultiGraph:
         self.offsets = np.concatenate([[0], np.cumsum([g.n for g in self.graphs])]).astype(np.int64)
 
     def set_plan(self, binned):
-        """Schedule of the union's sweeps: the per-item persistent kernel (binned=0) or the
-        binned sweep of the union (binned=1)."""
+        """Schedule of the union's sweeps: the item sweep (binned=0) or the binned sweep of the
+        union (binned=1)."""
         p = PlanParams()
         p.binned = int(binned)
         self.ctx.check(self.ctx.lib.nwg_multigraph_set_plan(self.ctx.handle, self.handle, ctypes.byref(p)))

@@ -127,6 +127,38 @@ def test_resident_items_stop_and_personalise(ctx, n):
     g.close()
 
 
+@pytest.mark.parametrize("kind", ["tiny", "long rows between tiny ones", "one each"])
+def test_items_of_many_graphs(ctx, kind):
+    """Items over rows of several graphs, of more than the 64 whose L1 changes meet in LDS, and rows over
+    several items that end among other graphs' rows: every graph's scores and stopping sweep."""
+    rng = np.random.default_rng(7)
+    if kind == "tiny":
+        sizes = [[int(d) for d in rng.integers(0, 3, n)] for n in list(rng.integers(1, 5, 300)) + [1, 900]]
+    elif kind == "long rows between tiny ones":
+        sizes = []
+        for big in (1019, 1020, 1021, 2040, 5000, 30000):
+            sizes += [[1, 2, 0], [big], [0, big, 1, big + 1, 0], [3]]
+    else:
+        sizes = [[int(d) for d in np.minimum(rng.zipf(1.8, n), 4000)] for n in (300, 1020, 5000, 40001)]
+    parts = [_csc(d, 11 + q) for q, d in enumerate(sizes)]
+    graphs = [ctx.graph_from_csc(ptr, col, deg) for _, ptr, col, deg in parts]
+    mg = ctx.multigraph(graphs)
+    for thr, sweeps in ((0.0, SWEEPS), (1e-4, 60), (1e-4, 60)):
+        got, its, _, _ = mg.pagerank(D, thr, sweeps)
+        for q, (n, ptr, col, deg) in enumerate(parts):
+            want, err = _fp64(n, ptr, col, deg, D, sweeps)
+            bound = 3 * 2.0**-24 / (1 - D) * max(want.sum(), 1.0 / n)
+            # stops that float64 sweeps decide: no change as close to the threshold as both errors
+            clear = [abs(e - thr) > 2 * bound for e in err]
+            stop = next((k + 1 for k, e in enumerate(err) if e < thr), sweeps)
+            if all(clear[:stop]) or thr == 0.0:
+                assert its[q] == (stop if thr else sweeps) or err[int(its[q]) - 1] == 0.0, (q, its[q], stop)
+                want = _fp64(n, ptr, col, deg, D, int(its[q]))[0]
+                assert np.abs(got[mg.offsets[q] : mg.offsets[q + 1]] - want).sum() <= bound, q
+    for g in graphs:
+        g.close()
+
+
 def test_weighted_items_with_a_fold_launch(ctx):
     """More than 1024 items: the L1 change is folded by a launch between the sweeps; stops as the change
     of float64 sweeps says, away from the threshold."""
