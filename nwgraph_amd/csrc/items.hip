@@ -212,8 +212,7 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
   const uint32_t b0 = e0 & ~3u;
   if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
   else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) ch += __shfl_xor(ch, m, 64);
+  ch = wave_sum(ch);
   if (blockIdx.x == 0) {
     if (threadIdx.x < 64) P.lanes[((P.iter + 1) % 3) * kItemLaneSlot + lane * kItemLanePad] = 0ull;
     if (threadIdx.x == 0 && P.iter > 0) P.acc[P.iter - 1] = ch;
