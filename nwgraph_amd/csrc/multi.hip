@@ -14,7 +14,7 @@
 // Each graph keeps the reference's scalars (init = 1/N_g, base = (1-d)/N_g,
 // page_rank.hpp:92-94) and its own stopping rule: the L1 change of graph g in sweep k
 // is accumulated in fixed point in acc[k][g]; rows of a converged graph are skipped.
-// The init launch and max_iters sweep launches are captured in one HIP graph.
+// A repeated solve's launches are one captured HIP graph.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,6 +22,7 @@
 
 #include "device_utils.hpp"
 #include "nwg_internal.hpp"
+#include "small.hpp"
 
 namespace nwg {
 
@@ -156,7 +157,9 @@ struct nwg_multigraph {
   nwg::DevBuf<unsigned long long> ihsum, ilanes;
   nwg::DevBuf<uint32_t> ihcnt;
   uint32_t n_sweep_items = 0;
-  nwg::Captured cap;
+  uint64_t max_n = 0, max_nnz = 0;  // of one graph
+  nwg::DevBuf<uint32_t> voff_dev;
+  std::vector<std::unique_ptr<nwg::Captured>> caps;  // the solve's launches
   // binned sweep of the union (plan option binned)
   bool binned = false;
   nwg::BinnedLayout bl;
@@ -180,6 +183,8 @@ nwg_multigraph* multigraph_create(nwg_ctx* ctx, uint32_t ngraphs, nwg_graph* con
     NWG_REQUIRE(graphs[g] && graphs[g]->device == ctx->device, "graph missing or on another device");
     mg->voff[g + 1] = mg->voff[g] + graphs[g]->n;
     eoff[g + 1] = eoff[g] + graphs[g]->nnz;
+    mg->max_n = std::max<uint64_t>(mg->max_n, graphs[g]->n);
+    mg->max_nnz = std::max<uint64_t>(mg->max_nnz, graphs[g]->nnz);
   }
   mg->nv = mg->voff[ngraphs];
   mg->ne = eoff[ngraphs];
@@ -208,6 +213,9 @@ nwg_multigraph* multigraph_create(nwg_ctx* ctx, uint32_t ngraphs, nwg_graph* con
   mg->ihsum.alloc(mg->n_sweep_items);
   mg->ihcnt.alloc(mg->n_sweep_items);
   mg->ilanes.alloc(3ull * kManyLanes * ngraphs);
+  const std::vector<uint32_t> voff32(mg->voff.begin(), mg->voff.end());
+  mg->voff_dev.alloc(ngraphs + 1);
+  NWG_HIP(hipMemcpyAsync(mg->voff_dev.p, voff32.data(), (ngraphs + 1) * 4ull, hipMemcpyHostToDevice, s));
   if (mg->n_sweep_items) items_build(s, (uint32_t)mg->nv, mg->ne, mg->rp.p, mg->idesc.p);
   NWG_HIP(hipStreamSynchronize(s));
   return mg.release();
@@ -255,7 +263,7 @@ void multigraph_set_binned(nwg_ctx* ctx, nwg_multigraph* mg, bool binned) {
     mg->bpart.alloc(std::max<uint64_t>((uint64_t)mg->bl.n_slots << mg->bl.bin_bits, 1));
     NWG_HIP(hipStreamSynchronize(s));
   }
-  if (mg->binned != binned) mg->cap.reset();
+  if (mg->binned != binned) mg->caps.clear();
   mg->binned = binned;
 }
 
@@ -314,6 +322,20 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   I.acc = mg->acc.p;
   I.threshold = (double)threshold;
   const ManyParams M{mg->row_graph.p, G};
+  // every graph a workgroup of its own, all sweeps in one launch
+  const bool small = items && small_fits(mg->max_n, mg->max_nnz, true) && max_iters <= kSmallSweeps;
+  SmallParams S{};
+  S.rp = mg->rp.p;
+  S.col = mg->col.p;
+  S.deg = mg->deg.p;
+  S.voff = mg->voff_dev.p;
+  S.ngraphs = G;
+  S.basev = mg->row_base.p;
+  S.damp = damping;
+  S.x = mg->x.p;
+  S.out = scores_dev;
+  S.acc = mg->acc.p;
+  S.threshold = (double)threshold;
 
   BinParams B{};
   if (mg->binned) {
@@ -354,57 +376,32 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   key.damping = damping;
   key.threshold = threshold;
   key.extra = grid | (mg->binned ? 0x80000000u : 0u) | (items ? 0x40000000u : 0u);
-  if (!mg->cap.valid || !(mg->cap.key == key)) {
-    mg->cap.reset();
-    std::lock_guard<std::mutex> capture_lock(capture_mutex());
-    hipStream_t cs = ctx->capture_stream;
-    NWG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    try {
-      multi_init_kernel<<<grid1(std::max<uint64_t>(mg->nv, max_iters * G)), kThreads, 0, cs>>>(
-          mg->nv, mg->deg.p, mg->vinit.p, mg->x.p, mg->c0.p, mg->acc.p, max_iters * G);
-      if (items) items_many_enqueue_init(cs, I, M);
-      for (uint64_t k = 0; k < max_iters; ++k) {
-        if (items) {
-          I.iter = (uint32_t)k;
-          I.cin = (k & 1) ? mg->c1.p : mg->c0.p;
-          I.cout = (k & 1) ? mg->c0.p : mg->c1.p;
-          items_many_enqueue_sweep(cs, I, M);
-          continue;
-        }
-        if (mg->binned) {
-          B.iter = (uint32_t)k;
-          binned_enqueue_sweep(cs, B);  // throws on a failed launch
-          continue;
-        }
-        P.iter = (uint32_t)k;
-        P.cin = (k & 1) ? mg->c1.p : mg->c0.p;
-        P.cout = (k & 1) ? mg->c0.p : mg->c1.p;
-        multi_sweep_kernel<<<grid, kThreads, 0, cs>>>(P);
-      }
-      if (items && max_iters) items_many_enqueue_fold(cs, I, M, (uint32_t)max_iters - 1);
-    } catch (...) {
-      // leave the capture stream out of capture mode, so that later solves can record again
-      hipGraph_t tmp = nullptr;
-      (void)hipStreamEndCapture(cs, &tmp);
-      if (tmp) (void)hipGraphDestroy(tmp);
-      mg->cap.reset();
-      throw;
-    }
-    hipGraph_t gr = nullptr;
-    const hipError_t e1 = hipGetLastError();
-    NWG_HIP(hipStreamEndCapture(cs, &gr));
-    mg->cap.graph = gr;
-    NWG_HIP(e1);
-    NWG_HIP(hipGraphInstantiate(&mg->cap.exec, mg->cap.graph, nullptr, nullptr, 0));
-    mg->cap.key = key;
-    mg->cap.valid = true;
-  }
   NWG_HIP(hipEventRecord(ctx->ev0, s));
-  NWG_HIP(hipGraphLaunch(mg->cap.exec, s));
+  if (small) small_enqueue(s, S, mg->max_n, mg->max_nnz, 0, max_iters);
+  else run_segment(ctx, mg->caps, 0, key, [&](hipStream_t t) {
+    multi_init_kernel<<<grid1(std::max<uint64_t>(mg->nv, max_iters * G)), kThreads, 0, t>>>(
+        mg->nv, mg->deg.p, mg->vinit.p, mg->x.p, mg->c0.p, mg->acc.p, max_iters * G);
+    NWG_LAUNCH_CHECK();
+    if (items) items_many_enqueue_init(t, I, M);
+    for (uint64_t k = 0; k < max_iters; ++k) {
+      I.iter = B.iter = P.iter = (uint32_t)k;
+      I.cin = P.cin = (k & 1) ? mg->c1.p : mg->c0.p;
+      I.cout = P.cout = (k & 1) ? mg->c0.p : mg->c1.p;
+      if (items) {
+        items_many_enqueue_sweep(t, I, M);
+      } else if (mg->binned) {
+        binned_enqueue_sweep(t, B);
+      } else {
+        multi_sweep_kernel<<<grid, kThreads, 0, t>>>(P);
+        NWG_LAUNCH_CHECK();
+      }
+    }
+    if (items && max_iters) items_many_enqueue_fold(t, I, M, (uint32_t)max_iters - 1);
+  });
   NWG_HIP(hipEventRecord(ctx->ev1, s));
   std::vector<unsigned long long> acc(std::max<uint64_t>(max_iters, 1) * G);
   NWG_HIP(hipMemcpyAsync(acc.data(), mg->acc.p, max_iters * G * 8ull, hipMemcpyDeviceToHost, s));
-  if (scores_dev) NWG_HIP(hipMemcpyAsync(scores_dev, mg->x.p, mg->nv * 4, hipMemcpyDeviceToDevice, s));
+  if (scores_dev && !small) NWG_HIP(hipMemcpyAsync(scores_dev, mg->x.p, mg->nv * 4, hipMemcpyDeviceToDevice, s));
   NWG_HIP(hipStreamSynchronize(s));
   float ms = 0.f;
   NWG_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));

@@ -29,6 +29,7 @@
 #include "device_utils.hpp"
 #include "items.hpp"
 #include "nwg_internal.hpp"
+#include "small.hpp"
 
 namespace nwg {
 
@@ -246,7 +247,28 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
   // Others, and CSCs of more items than the scratch holds, keep the float row sums.
   const bool items = item_count(n, nnz) <= kNaMaxItems && damping >= 0.f && damping <= 1.f;
   const float init = (float)(1.0 / n);  // page_rank.hpp:93
-  if (items) {
+  if (items && small_fits(n, nnz, false)) {
+    SmallParams S{};
+    S.rp = csc_ptr;
+    S.col = csc_idx;
+    S.deg = deg;
+    S.n = n;
+    S.ngraphs = 1;
+    S.base = P.base;
+    S.damp = damping;
+    S.x = scores;
+    S.acc = acc;
+    S.mail = ctx->mail;
+    S.threshold = P.threshold;
+    NWG_HIP(hipEventRecord(ctx->ev0, s));
+    uint64_t k0 = 0;
+    do {
+      const uint64_t k1 = std::min(k0 + kSmallSweeps, max_iters);
+      small_enqueue(s, S, n, nnz, k0, k1);
+      k0 = k1;
+    } while (k0 < max_iters);
+    NWG_HIP(hipEventRecord(ctx->ev1, s));
+  } else if (items) {
     ItemParams I{};
     uint4* desc = reinterpret_cast<uint4*>(base + kOffDesc);
     I.desc = desc;

@@ -32,6 +32,7 @@
 
 #include "device_utils.hpp"
 #include "nwg_internal.hpp"
+#include "small.hpp"
 
 namespace nwg {
 
@@ -42,8 +43,6 @@ constexpr int kThreads = 256;
 // the plan names a bin size (plan_takes_items)
 constexpr uint64_t kBinnedEdges = 1ull << 18;
 constexpr uint64_t kBinnedMinEdges = 3ull << 21;
-// rounding slack allowed above 1 in the sum of a teleport vector
-constexpr double kTeleportSlack = 1e-4;
 
 struct SweepParams {
   const uint32_t* rp;
@@ -336,13 +335,6 @@ __global__ __launch_bounds__(kThreads) void pr_delta_push_kernel(SweepParams P, 
 // (teleport_ok), and the host after the solve.  (One workgroup per 256 entries adding to one double
 // took 74 us for 1.5 M vertices on MI355X, and the wait some 20.)
 constexpr uint32_t kTeleBlocks = 512;
-struct TeleCheck {
-  double sum;
-  double bad;
-};
-__host__ __device__ __forceinline__ bool teleport_ok(const TeleCheck& c) {
-  return c.bad == 0.0 && c.sum <= 1.0 + kTeleportSlack;
-}
 __global__ __launch_bounds__(kThreads) void pr_teleport_check_kernel(uint32_t n, const float* __restrict__ v,
                                                                      TeleCheck* __restrict__ part) {
   __shared__ double red_d[kThreads / 64];
@@ -1024,6 +1016,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   double sweep_ms = 0.0;
   uint64_t launched = max_iters;
   std::vector<hipEvent_t> evs;
+  const bool small = items && sched == PrSchedule::kJacobi && !timing && small_fits(n, g->nnz, false);
   const bool class_kernels = !items && (!g->plan.bl.built || sched == PrSchedule::kDelta);
   unsigned long long* const mail = !class_kernels && max_iters <= kMailWords ? ctx->mail : nullptr;
   // scores in the caller's numbering
@@ -1043,6 +1036,24 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     NWG_REQUIRE(c.bad == 0.0, "teleport entries must be finite and in [0, 1]");
     NWG_REQUIRE(teleport_ok(c), "teleport entries must sum to at most 1");
   };
+  SmallParams sp{};
+  if (small) {
+    sp.rp = P.rp;
+    sp.col = P.col;
+    sp.deg = P.deg;
+    sp.n = n;
+    sp.ngraphs = 1;
+    sp.basev = P.basev;
+    sp.base = P.base;
+    sp.damp = damping;
+    sp.x = st.x.p;
+    sp.out = scores_dev;
+    sp.order = g->active(g->plan.params.relabel != 0).order;
+    sp.tele = personalised ? reinterpret_cast<const TeleCheck*>(st.tcheck.p) + kTeleBlocks : nullptr;
+    sp.acc = st.acc.p;
+    sp.mail = mail;
+    sp.threshold = (double)threshold;
+  }
   if (!timing) {
     CaptureKey key;
     key.ptrs[0] = st.x.p;
@@ -1072,11 +1083,17 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     // convergence launch only up to a segment's end
     NWG_HIP(hipEventRecord(ctx->ev0, s));
     uint64_t seg = 0;
-    for (uint64_t k0 = 0;; k0 = segment_end(k0, max_iters, first)) {
-      const uint64_t k1 = segment_end(k0, max_iters, first);
-      run_segment(ctx, st.caps, seg++, key, [&](hipStream_t t) {
-        enqueue_solve(t, g, st, P, max_iters, nullptr, sched, k0, k1, mail);
-      });
+    auto end_of = [&](uint64_t k0) {
+      return small ? std::min(k0 + kSmallSweeps, max_iters) : segment_end(k0, max_iters, first);
+    };
+    for (uint64_t k0 = 0;; k0 = end_of(k0)) {
+      const uint64_t k1 = end_of(k0);
+      if (small)
+        small_enqueue(s, sp, n, g->nnz, k0, k1);
+      else
+        run_segment(ctx, st.caps, seg++, key, [&](hipStream_t t) {
+          enqueue_solve(t, g, st, P, max_iters, nullptr, sched, k0, k1, mail);
+        });
       if (k1 >= max_iters) break;
       unsigned long long last = 0ull;
       if (!mail) NWG_HIP(hipMemcpyAsync(&last, st.acc.p + (k1 - 1), sizeof last, hipMemcpyDeviceToHost, s));
@@ -1107,7 +1124,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   std::vector<unsigned long long> acc(std::max<uint64_t>(max_iters, 1));
   if (!mail)
     NWG_HIP(hipMemcpyAsync(acc.data(), st.acc.p, max_iters * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-  copy_out();
+  if (!small) copy_out();
   NWG_HIP(hipStreamSynchronize(s));
   if (timing && personalised) {
     try {
