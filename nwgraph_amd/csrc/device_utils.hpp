@@ -41,6 +41,10 @@ __device__ __forceinline__ unsigned long long dpp_or_zero(unsigned long long v) 
   return ((unsigned long long)dpp_or_zero<Ctrl, Rows>((uint32_t)(v >> 32)) << 32) |
          dpp_or_zero<Ctrl, Rows>((uint32_t)v);
 }
+template <int Ctrl, int Rows>
+__device__ __forceinline__ double dpp_or_zero(double v) {
+  return __longlong_as_double((long long)dpp_or_zero<Ctrl, Rows>((unsigned long long)__double_as_longlong(v)));
+}
 template <class T>
 __device__ __forceinline__ T wave_scan_dpp(T v) {
   v += dpp_or_zero<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8

@@ -38,6 +38,26 @@ struct SmallParams {
   double threshold;
 };
 
+// One weighted solve y <- fma(d, sum w y, b), whose scales are made on the device (WItemParams).
+struct SmallWeighted {
+  const uint32_t* rp;
+  const uint32_t* col;
+  const float* w;         // in the order of col
+  const float* base;
+  const float* y0;        // first iterate; null: uniform
+  float uniform;
+  float damp;
+  uint32_t n;
+  float* state;           // the iterate between launches
+  float* out;             // the last iterate
+  const int* qshift;
+  double* err;            // [k]: L1 change of sweep k; 0 once stopped
+  unsigned long long* mail;         // nullable: the scales' two words, then err
+  const unsigned long long* scale;
+  double threshold;
+  const double* thr_scale;  // nullable: the stop compares with threshold * *thr_scale
+};
+
 // Sweeps per launch: a solve of any length is cut into launches of bounded time.
 constexpr uint64_t kSmallSweeps = 1024;
 
@@ -45,5 +65,6 @@ constexpr uint64_t kSmallSweeps = 1024;
 bool small_fits(uint64_t n, uint64_t nnz, bool many);
 // sweeps [k0, k1) of the solve; n and nnz: the largest graph's
 void small_enqueue(hipStream_t s, const SmallParams& P, uint64_t n, uint64_t nnz, uint64_t k0, uint64_t k1);
+void small_weighted_enqueue(hipStream_t s, const SmallWeighted& P, uint64_t nnz, uint64_t k0, uint64_t k1);
 
 }  // namespace nwg

@@ -32,6 +32,7 @@
 
 #include "device_utils.hpp"
 #include "nwg_internal.hpp"
+#include "small.hpp"
 
 namespace nwg {
 
@@ -545,9 +546,9 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
     return WMail{mail, reinterpret_cast<const unsigned long long*>(st.scale.p), (uint32_t)k0};
   };
   // sweeps [k0, k1) (and the init with k0 = 0) on stream t
+  const float uniform = (float)(1.0 / n);
   auto enqueue = [&](hipStream_t t, uint64_t k0, uint64_t k1) {
     const float* src = q.y0;
-    const float uniform = (float)(1.0 / n);
     if (kind == WSweep::kItems) {
       WItemParams I{};
       I.desc = it->desc.p;
@@ -658,16 +659,42 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
   key.plan_version = L ? L->build_id : grid;
   key.extra = (relative ? 1u : 0u) | (q.y0 ? 0u : 2u) | ((uint32_t)kind << 2);
   const uint64_t first = kind == WSweep::kBinned ? kSegFirstBinned : kSegFirst;
+  // a small graph: all sweeps in one launch
+  const bool small = kind == WSweep::kItems && small_fits(n, g->nnz, false);
+  SmallWeighted sp{};
+  if (small) {
+    sp.rp = q.rp;
+    sp.col = q.col;
+    sp.w = q.w;
+    sp.base = q.base;
+    sp.y0 = q.y0;
+    sp.uniform = uniform;
+    sp.damp = q.damping;
+    sp.n = n;
+    sp.state = st.y0.p;
+    sp.out = q.out;
+    sp.qshift = qshift;
+    sp.err = st.err.p;
+    sp.mail = mail;
+    sp.scale = reinterpret_cast<const unsigned long long*>(st.scale.p);
+    sp.threshold = (double)q.threshold;
+    sp.thr_scale = thr_scale;
+  }
   std::vector<double> h(std::max<uint64_t>(max_iters, 1), 0.0);
   WScale sc{1.0, 0, 1};
   double stop = (double)q.threshold;
   uint64_t iters = max_iters, seg = 0;
   NWG_HIP(hipEventRecord(ctx->ev0, s));
-  for (uint64_t k0 = 0;; k0 = segment_end(k0, max_iters, first), ++seg) {
-    const uint64_t k1 = segment_end(k0, max_iters, first);
-    run_segment(ctx, caps, seg, key, [&](hipStream_t t) { enqueue(t, k0, k1); });
+  auto end_of = [&](uint64_t k0) {
+    return small ? std::min(k0 + kSmallSweeps, max_iters) : segment_end(k0, max_iters, first);
+  };
+  for (uint64_t k0 = 0;; k0 = end_of(k0), ++seg) {
+    const uint64_t k1 = end_of(k0);
+    if (small) small_weighted_enqueue(s, sp, g->nnz, k0, k1);
+    else run_segment(ctx, caps, seg, key, [&](hipStream_t t) { enqueue(t, k0, k1); });
     NWG_HIP(hipEventRecord(ctx->ev1, s));
-    wout_kernel<<<grid1(n), kThreads, 0, s>>>(n, y[0], y[1], st.err.p, (uint32_t)k1, (double)q.threshold, thr_scale,
+    if (!small)
+      wout_kernel<<<grid1(n), kThreads, 0, s>>>(n, y[0], y[1], st.err.p, (uint32_t)k1, (double)q.threshold, thr_scale,
                                              q.out);
     NWG_LAUNCH_CHECK();
     if (eager) then();

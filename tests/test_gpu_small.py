@@ -29,8 +29,9 @@ def _degrees(n, m, kind):
 
 
 @pytest.mark.parametrize("kind", ["skewed", "one row", "few long rows"])
-@pytest.mark.parametrize("n,m", [(1, 3), (2, 4096), (1023, 4095), (1024, 4096), (1025, 4096), (1024, 4097), (4096, 8191),
-                                 (3001, 8192), (3001, 8193), (4096, 16384), (4097, 16384), (4095, 16385)])
+@pytest.mark.parametrize("n,m", [(1, 3), (2, 4096), (1023, 4095), (1024, 4096), (1025, 4096), (1024, 4097),
+                                 (4096, 8191), (3001, 8192), (3001, 8193), (4096, 16384), (4097, 16384),
+                                 (4095, 16385), (4096, 20480), (4096, 20481)])
 def test_scores_and_changes(ctx, n, m, kind):
     n, ptr, col, deg = _csc(_degrees(n, m, kind), n)
     sweeps = 12
@@ -97,3 +98,53 @@ def test_many_graphs_one_workgroup_each(ctx):
                     assert np.abs(got[mg.offsets[q] : mg.offsets[q + 1]] - want).sum() <= bound, q
     for g in graphs:
         g.close()
+
+
+@pytest.mark.parametrize("kind", ["skewed", "one row", "few long rows"])
+@pytest.mark.parametrize("n,m", [(1, 3), (1024, 4096), (1025, 4096), (1024, 4097), (4096, 8192), (3001, 8193),
+                                 (4096, 16384), (4097, 16384), (4095, 16385), (4096, 20480), (4096, 20481)])
+def test_weighted_solves(ctx, n, m, kind):
+    """Forward and adjoint with the bounds of test_weighted_items_match_float64 (u = 2^-24: 72 u of every
+    score after 12 sweeps; the adjoint off by 6 u of the largest |lambda|, damped by d), stops away
+    from the threshold, and a solve over two launches, whose scores have settled to 6 u / (1 - d) of
+    every score."""
+    sweeps, u = 12, 2.0**-24
+    rng = np.random.default_rng(m)
+    src, dst = rng.integers(0, n, m), np.repeat(np.arange(n), _degrees(n, m, kind))
+    g = ctx.graph_from_edges(n, src.astype(np.uint32), dst.astype(np.uint32), clean=False)
+    ptr, col, _ = g.csc()
+    row = np.repeat(np.arange(n), np.diff(ptr.astype(np.int64)))
+    w = rng.uniform(0.1, 1.0, m).astype(np.float32)
+    wn = w / np.bincount(col, weights=w.astype(np.float64), minlength=n)[col]
+    v = rng.random(n).astype(np.float32)
+    g.set_weights(w)
+
+    def iterate(b, x, at, to, count):
+        err = []
+        for _ in range(count):
+            y = b + D * np.bincount(to, weights=wn * x[at], minlength=n)
+            err.append(np.abs(y - x).sum())
+            x = y
+        return x, err
+
+    want, err = iterate((1 - D) * v.astype(np.float64), np.full(n, 1.0 / n), col, row, sweeps)
+    x, fi = g.wpr_forward(v, D, 0.0, sweeps)
+    assert np.all(np.abs(x - want) <= 72 * u * want) and fi["iterations"] == sweeps
+    c = rng.normal(size=n).astype(np.float32)
+    gw, gv, bi = g.wpr_backward(x, c, D, 0.0, sweeps)
+    lam, lmax = c.astype(np.float64), np.abs(c).max()
+    for _ in range(sweeps):
+        lam = c + D * np.bincount(col, weights=wn * lam[row], minlength=n)
+        lmax = max(lmax, np.abs(lam).max())
+    assert np.abs(gv - (1 - D) * lam).max() <= (6 / (1 - D) + 2) * u * lmax
+    for it in (2, 5, 9):
+        if err[it - 1] > 1e-4 * np.abs(want).sum() and err[it - 1] < 0.95 * err[it - 2]:
+            _, info = g.wpr_forward(v, D, float(np.sqrt(err[it - 1] * err[it - 2])), 40)
+            assert info["iterations"] == it
+            thr = float(np.sqrt(err[it - 1] * err[it - 2])) / np.abs(v.astype(np.float64)).sum()
+            _, info = g.wpr_forward(v, D, thr, 40, relative=True)
+            assert info["iterations"] == it
+    settled, _ = iterate((1 - D) * v.astype(np.float64), want, col, row, 200)
+    x, info = g.wpr_forward(v, D, 0.0, 1500)
+    assert info["iterations"] == 1500 and np.all(np.abs(x - settled) <= 6 / (1 - D) * u * settled)
+    g.close()
