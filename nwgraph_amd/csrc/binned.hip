@@ -28,6 +28,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
+#include <functional>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -1024,6 +1026,40 @@ void binned_build(hipStream_t s, const ActiveCsc& a, uint32_t n, uint64_t nnz, B
     if (q && (double)q >= 1.4142 * (double)(1ull << lg)) ++lg;
     lg = std::min<uint32_t>(std::max<uint32_t>(lg, 15u), kItem2Log);
     cap2 = 1u << lg;
+  }
+  // Up to one bin per CU the launch is a few items per CU at most, and both a second round of them and
+  // every partial slot (its rows stored and read again) show.  There the cap is the one of least
+  // cost = the busiest CU's entries, items handed out in order to the first free CU, + 300 entries per slot
+  // of 2^13 rows, 680 per slot of 2^14: weights that put these measured solves in order (MI355X, us with the
+  // caps 2^15 / 2^16 / 100,000 / 180,000 / 2^18, and with this one): RMAT-20 938 / 829 / 795 / 986 / 1149, 832; weighted
+  // 2770 / 2611 / 2400 / 2654 / 3065, 2405; uniform random 500,000 with 10 M edges 338 / 306 / 312 / 327 / 332, 308, and
+  // 1.5 M with 24 M (2^14-row bins) 900 / 660 / 640 / 562 / 630, 540.  With fewer than 2^15 entries per CU 2^15
+  // stays the best (weighted R-MAT, 400,000 rows, 5.5 M edges: 1277 / 1348 / 1512 / 1839 / 2137).
+  if (L.n_bins <= (uint32_t)cus && etotal > (uint64_t)cus << 15) {
+    const uint64_t slot_cost = L.bin_bits >= 14 ? 680 : 300;
+    uint64_t best = ~0ull;
+    for (uint32_t i = 0;; ++i) {
+      const uint32_t cap = (uint32_t)(32768.0 * std::exp2(i / 4.0));
+      if (cap > (1u << kItem2Log)) break;
+      std::vector<uint64_t> load(cus, 0);  // a heap of the CUs' entries, the least first
+      uint64_t most = 0, split = 0;
+      for (uint32_t b = 0; b < L.n_bins; ++b) {
+        const uint64_t len = etp[(uint64_t)(b + 1) * TC] - etp[(uint64_t)b * TC];
+        const uint64_t cnt = std::max<uint64_t>(ceil_div(len, cap), 1);
+        if (cnt > 1) split += cnt;
+        for (uint64_t q = 0; q < cnt; ++q) {
+          std::pop_heap(load.begin(), load.end(), std::greater<>());
+          load.back() += ceil_div(len, cnt);
+          most = std::max(most, load.back());
+          std::push_heap(load.begin(), load.end(), std::greater<>());
+        }
+      }
+      const uint64_t cost = most + split * slot_cost;
+      if (cost < best) {
+        best = cost;
+        cap2 = cap;
+      }
+    }
   }
   std::vector<uint4> it2, it3;
   std::vector<uint32_t> ihe, ihd;
