@@ -459,7 +459,8 @@ void out_degrees_device(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t*
 }
 
 void check_device_csc(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* ptr, const uint32_t* col,
-                      const uint32_t* given, uint32_t* deg, const CscCheckScratch* scratch) {
+                      const uint32_t* given, uint32_t* deg, const CscCheckScratch* scratch, bool wait) {
+  NWG_REQUIRE(wait || scratch, "the check's flags outlive it in the caller's memory only");
   if (given || deg) degrees_aligned(col);
   DevBuf<uint32_t> own_flags, own_part, own_counted;
   uint32_t* flags = scratch ? scratch->flags : (own_flags.alloc(2), own_flags.p);
@@ -487,11 +488,16 @@ void check_device_csc(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* p
       NWG_LAUNCH_CHECK();
     }
   }
+  if (!wait) return;
   uint32_t bad[2] = {0, 0};
   NWG_HIP(hipMemcpyAsync(bad, flags, sizeof bad, hipMemcpyDeviceToHost, s));
   NWG_HIP(hipStreamSynchronize(s));
-  if (bad[0]) throw Error(NWG_EINVAL, kBadCsc);
-  if (bad[1]) throw Error(NWG_EINVAL, "outdeg: some vertex's out-degree is below its number of entries in the CSC");
+  csc_verdict(bad[0], bad[1]);
+}
+
+void csc_verdict(uint64_t bad_csc, uint64_t bad_outdeg) {
+  if (bad_csc) throw Error(NWG_EINVAL, kBadCsc);
+  if (bad_outdeg) throw Error(NWG_EINVAL, "outdeg: some vertex's out-degree is below its number of entries in the CSC");
 }
 
 void build_csc_device(hipStream_t s, uint32_t n, uint64_t ne, const uint32_t* src, const uint32_t* dst, bool clean,

@@ -226,7 +226,13 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
 
   // the contribution arrays, not in use yet, take the partial histograms
   const CscCheckScratch scratch_mem{flag, cdeg, reinterpret_cast<uint32_t*>(c0), kOffDeg - kOffC0};
-  check_device_csc(s, n, nnz, csc_ptr, csc_idx, outdeg, outdeg ? nullptr : cdeg, &scratch_mem);
+  // The item sweep's exact fixed-point sums cover scores in [0, 1]: damping factors in [0, 1].
+  // Others, and CSCs of more items than the scratch holds, keep the float row sums.
+  const bool items = item_count(n, nnz) <= kNaMaxItems && damping >= 0.f && damping <= 1.f;
+  // a small graph's one launch looks at the flags itself (257 vertices, 20 sweeps: 80 to 60 us without
+  // the wait in between)
+  const bool small = items && small_fits(n, nnz, false);
+  check_device_csc(s, n, nnz, csc_ptr, csc_idx, outdeg, outdeg ? nullptr : cdeg, &scratch_mem, !small);
   const uint32_t* deg = outdeg ? outdeg : cdeg;  // counted: build_degrees, common.hpp:110-121
 
   NaParams P{};
@@ -243,11 +249,8 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
   P.threshold = (double)threshold;  // page_rank.hpp:144
   const uint32_t fold_blocks = (uint32_t)ceil_div(P.nblk, kNaFoldChunk);
 
-  // The item sweep's exact fixed-point sums cover scores in [0, 1]: damping factors in [0, 1].
-  // Others, and CSCs of more items than the scratch holds, keep the float row sums.
-  const bool items = item_count(n, nnz) <= kNaMaxItems && damping >= 0.f && damping <= 1.f;
   const float init = (float)(1.0 / n);  // page_rank.hpp:93
-  if (items && small_fits(n, nnz, false)) {
+  if (small) {
     SmallParams S{};
     S.rp = csc_ptr;
     S.col = csc_idx;
@@ -257,6 +260,8 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
     S.base = P.base;
     S.damp = damping;
     S.x = scores;
+    S.bad = flag;
+    S.bad_mail = ctx->mail + kMailWords;
     S.acc = acc;
     S.mail = ctx->mail;
     S.threshold = P.threshold;
@@ -268,6 +273,8 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
       k0 = k1;
     } while (k0 < max_iters);
     NWG_HIP(hipEventRecord(ctx->ev1, s));
+    NWG_HIP(hipStreamSynchronize(s));
+    csc_verdict(ctx->mail[kMailWords], ctx->mail[kMailWords + 1]);
   } else if (items) {
     ItemParams I{};
     uint4* desc = reinterpret_cast<uint4*>(base + kOffDesc);

@@ -238,7 +238,7 @@ inline uint64_t segment_end(uint64_t start, uint64_t max_iters, uint64_t first) 
 }
 
 constexpr uint64_t kMailWords = 8192;  // of nwg_ctx::mail for L1 changes; longer solves copy.  Two
-                                       // more words take the teleport check
+                                       // more words take a solve's check of its inputs
 
 // Identity of a captured sweep loop: re-capture when any of it changes.
 struct CaptureKey {
@@ -468,8 +468,10 @@ struct CscCheckScratch {
 // monotone from 0 to nnz, every entry of col is below n and (with given) no vertex's given
 // out-degree is below its number of entries; without given, deg receives the counted
 // out-degrees (both null: only the structure is checked).  No scratch: allocates.
+// wait: raise what is found; else the flags stay in scratch->flags, for the device and for csc_verdict.
 void check_device_csc(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* ptr, const uint32_t* col,
-                      const uint32_t* given, uint32_t* deg, const CscCheckScratch* scratch = nullptr);
+                      const uint32_t* given, uint32_t* deg, const CscCheckScratch* scratch = nullptr, bool wait = true);
+void csc_verdict(uint64_t bad_csc, uint64_t bad_outdeg);
 
 // ---- primitives (scan.hip / sort.hip) ----
 // exclusive scan of n values; out has n+1 entries (out[n] = total).

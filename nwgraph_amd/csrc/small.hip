@@ -145,6 +145,11 @@ __global__ __launch_bounds__(NT) void small_solve_kernel(SmallParams P, uint64_t
   __shared__ unsigned long long q[H::kRows + 1];  // contributions; the last one is 0, for lanes past the edges
   __shared__ unsigned long long werr[H::kWaves];
   const uint32_t tid = threadIdx.x, g = blockIdx.x;
+  if (P.bad) {
+    const uint32_t b0 = P.bad[0], b1 = P.bad[1];
+    if (g == 0 && tid < 2) P.bad_mail[tid] = tid ? b1 : b0;
+    if (b0 | b1) return;
+  }
   const uint32_t r0 = P.voff ? P.voff[g] : 0u;
   const uint32_t n = P.voff ? P.voff[g + 1] - r0 : P.n;
   if (!n) {

@@ -33,6 +33,8 @@ struct SmallParams {
   float* out;             // nullable: out[order ? order[i] : i] = x[i], unless tele (nullable) failed
   const uint32_t* order;
   const TeleCheck* tele;
+  const uint32_t* bad;       // nullable: two flags that say the graph is not to be looked at; in bad_mail too
+  unsigned long long* bad_mail;
   unsigned long long* acc;   // [k * ngraphs + graph]: L1 change of sweep k, fixed point; 0 once stopped
   unsigned long long* mail;  // nullable, one graph: acc[k] there too
   double threshold;

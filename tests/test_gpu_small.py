@@ -148,3 +148,32 @@ def test_weighted_solves(ctx, n, m, kind):
     x, info = g.wpr_forward(v, D, 0.0, 1500)
     assert info["iterations"] == 1500 and np.all(np.abs(x - settled) <= 6 / (1 - D) * u * settled)
     g.close()
+
+
+@pytest.mark.parametrize("what", ["id", "decreasing", "end", "out-degree"])
+def test_noalloc_refuses_what_its_check_finds(ctx, what):
+    """The solve is queued behind the check and leaves the scores alone when it fails."""
+    import torch
+    from nwgraph_amd import NwgError, _lib
+
+    n, ptr, col, deg = _csc(_degrees(1000, 5000, "skewed"), 3)
+    if what == "id":
+        col[777] = n
+    elif what == "decreasing":
+        ptr[500], ptr[501] = ptr[501] + 1, ptr[500]
+    elif what == "end":
+        ptr[n] -= 1
+    else:
+        deg[col[0]] -= 1
+    dev = [torch.from_numpy(a.astype(np.int32)).cuda() for a in (ptr, col, deg)]
+    x = torch.full((n,), -1.0, device="cuda")
+    torch.cuda.synchronize()
+    for given in (True, False):
+        if what == "out-degree" and not given:
+            continue
+        with pytest.raises(NwgError) as e:
+            ctx.check(ctx.lib.nwg_pagerank_f32_noalloc(ctx.handle, n, col.size, dev[0].data_ptr(), dev[1].data_ptr(),
+                                                       dev[2].data_ptr() if given else None, x.data_ptr(), D, 0.0, 20,
+                                                       None))
+        assert e.value.code == _lib.NWG_EINVAL
+        assert torch.all(x == -1.0)
