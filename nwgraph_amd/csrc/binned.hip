@@ -880,11 +880,12 @@ void binned_build(hipStream_t s, const ActiveCsc& a, uint32_t n, uint64_t nnz, B
   L = BinnedLayout();
   // Bins of 2^14 rows have fewer pairs per entry (0.35 against 0.43 at RMAT-25, so 17 % fewer
   // pair values to store and read), but their 128 KiB of row sums leave one bin-pass
-  // workgroup per CU, which pays once there are enough of them.  Measured on MI355X, us per sweep
-  // with 2^14 / 2^13 rows: RMAT-20 (16 M entries) 50.8 / 43.8, uniform random with 24 M 91.7 / 95.3,
-  // RMAT-22 (65 M) 93.7 / 104.2, 236 M RMAT edges 259 / 289, RMAT-25 (529 M) 622 / 724; the 256-graph
-  // union (213 M, no hot tiles) 390 / 290.
-  L.bin_bits = bin_bits ? bin_bits : nnz >= (hot ? 5ull << 22 : 1ull << 28) ? 14 : 13;
+  // workgroup per CU, which pays once there are enough of them.  Measured on MI355X, us per solve
+  // with 2^14 / 2^13 rows: RMAT-20 (16 M entries) 946 / 831, uniform random with 24 M 520 / 487, R-MAT with
+  // 31 M 1206 / 1086, uniform random with 35 M 917 / 1283, R-MAT with 47 M 1496 / 2116, RMAT-22 (65 M) 1959 / 2148,
+  // 188 M 4653 / 5245; us per sweep of RMAT-25 (529 M) 622 / 724, of the 256-graph union (213 M, no hot
+  // tiles) 390 / 290.
+  L.bin_bits = bin_bits ? bin_bits : nnz >= (hot ? 1ull << 25 : 1ull << 28) ? 14 : 13;
   const uint32_t bin_rows_ = 1u << L.bin_bits;
   L.n_bins = (uint32_t)ceil_div(n, bin_rows_);
   L.n_chunks = (uint32_t)ceil_div(n, kChunkSrc);
@@ -1030,11 +1031,12 @@ void binned_build(hipStream_t s, const ActiveCsc& a, uint32_t n, uint64_t nnz, B
   // Up to one bin per CU the launch is a few items per CU at most, and both a second round of them and
   // every partial slot (its rows stored and read again) show.  There the cap is the one of least
   // cost = the busiest CU's entries, items handed out in order to the first free CU, + 300 entries per slot
-  // of 2^13 rows, 680 per slot of 2^14: weights that put these measured solves in order (MI355X, us with the
-  // caps 2^15 / 2^16 / 100,000 / 180,000 / 2^18, and with this one): RMAT-20 938 / 829 / 795 / 986 / 1149, 832; weighted
-  // 2770 / 2611 / 2400 / 2654 / 3065, 2405; uniform random 500,000 with 10 M edges 338 / 306 / 312 / 327 / 332, 308, and
-  // 1.5 M with 24 M (2^14-row bins) 900 / 660 / 640 / 562 / 630, 540.  With fewer than 2^15 entries per CU 2^15
-  // stays the best (weighted R-MAT, 400,000 rows, 5.5 M edges: 1277 / 1348 / 1512 / 1839 / 2137).
+  // of 2^13 rows, 680 per slot of 2^14: weights that put these measured solves in order (MI355X, us with
+  // the caps 2^15 / 2^16 / 100,000 / 180,000 / 2^18, and with this one): RMAT-20 938 / 829 / 795 / 986 / 1149, 832;
+  // weighted 2770 / 2611 / 2400 / 2654 / 3065, 2405; uniform random 500,000 with 10 M edges 338 / 306 / 312 /
+  // 327 / 332, 308, and 1.5 M with 24 M (2^14-row bins) 900 / 660 / 640 / 562 / 630, 540.  With fewer than 2^15
+  // entries per CU 2^15 stays the best (weighted R-MAT, 400,000 rows, 5.5 M edges: 1277 / 1348 / 1512 /
+  // 1839 / 2137).
   if (L.n_bins <= (uint32_t)cus && etotal > (uint64_t)cus << 15) {
     const uint64_t slot_cost = L.bin_bits >= 14 ? 680 : 300;
     uint64_t best = ~0ull;

@@ -527,17 +527,21 @@ void build_csc_device(hipStream_t s, uint32_t n, uint64_t ne, const uint32_t* sr
   g->nnz = nnz;
   g->outdeg.alloc(n);
   out_degrees_device(s, n, nnz, g->csc_idx.p, g->outdeg.p);
-  note_max_outdeg(s, g);
-  NWG_HIP(hipStreamSynchronize(s));
+  if (g->nnz >= kSkewEdges) note_max_outdeg(s, g);  // waits
+  else NWG_HIP(hipStreamSynchronize(s));
 }
 
 void note_max_outdeg(hipStream_t s, nwg_graph* g) {
-  if (g->nnz < kOrderEdges) return;
+  if (g->nnz < kSkewEdges) return;
   DevBuf<uint32_t> m(1);
   fill_u32_kernel<<<1, 256, 0, s>>>(m.p, 1, 0u);
   max_u32_kernel<<<(uint32_t)std::min<uint64_t>(grid_for(g->n), 1024), 256, 0, s>>>(g->outdeg.p, g->n, m.p);
   NWG_LAUNCH_CHECK();
   g->max_outdeg = read_back_u32(s, m.p);
+}
+
+bool skewed_degrees(const nwg_graph* g) {
+  return (double)g->max_outdeg > 64.0 + 8.0 * (double)g->nnz / (double)std::max<uint32_t>(g->n, 1);
 }
 
 void build_csr_device(hipStream_t s, nwg_graph* g) {

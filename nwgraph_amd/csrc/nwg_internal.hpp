@@ -382,7 +382,7 @@ struct nwg_graph {
   uint32_t n = 0;
   uint64_t nnz = 0;
   nwg::DevBuf<uint32_t> csc_ptr, csc_idx, outdeg;
-  uint32_t max_outdeg = 0;  // largest out-degree, of graphs of kOrderEdges edges and more
+  uint32_t max_outdeg = 0;  // largest out-degree, of graphs of kSkewEdges edges and more
   // optional transposed structure for the adjoint
   bool has_csr = false;
   nwg::DevBuf<uint32_t> csr_ptr, csr_idx, csr_to_csc;
@@ -527,9 +527,11 @@ void build_segments(hipStream_t s, const uint32_t* rp, uint32_t n, uint32_t min_
 nwg_plan_params default_plan_params();
 // edges from which a default plan may order the vertices by degree
 constexpr uint64_t kOrderEdges = 1ull << 23;
-// g->max_outdeg, when the graph is large enough for a plan to look at it; waits for the device
+// g->max_outdeg, when the graph is large enough for a plan to look at it; then waits for the device
+constexpr uint64_t kSkewEdges = 1ull << 21;
 void note_max_outdeg(hipStream_t s, nwg_graph* g);
-// the plan a PageRank solve of g builds on first use (binned sweep and degree ordering by size)
+// whether some vertex has far more out-edges than the average (false below kSkewEdges)
+bool skewed_degrees(const nwg_graph* g);
 nwg_plan_params default_plan_for(const nwg_graph* g);
 // binned sweep (binned.hip)
 // w (device, CSC order of a, nullable): also lay out the entries' weights (L.bw)

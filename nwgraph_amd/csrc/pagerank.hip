@@ -570,15 +570,15 @@ nwg_plan_params default_plan_params() {
 // streams for the last-level cache, nontemporal stores once they no longer stay there either (us per
 // sweep with hints 0 / 1 / 2: uniform random with 24 M edges 92 / 103 / 111, 67 M 242 / 217 / 234, 79 M
 // 253 / 227 / 234, the lattice with 57 M 159 / 141 / 152, RMAT-22 with 65 M 95 / 104 / 103, RMAT with
-// 236 M 279 / 238 / 256, RMAT-25 with 529 M 666 / 694 / 628).  The plan asks for the binned sweep from kBinnedEdges, and leaves the bin
-// size, hence the sweep, to the graph's size (plan_takes_items).  The binned layout indexes
-// entries and pairs with 32 bits (below 2^31 entries and 2^30 pairs with pads), so larger
-// graphs keep the pull sweep.
+// 236 M 279 / 238 / 256, RMAT-25 with 529 M 666 / 694 / 628).  The plan asks for the binned sweep from
+// kBinnedEdges, and leaves the bin size, hence the sweep, to the graph's size and degrees
+// (plan_takes_items).  The binned layout indexes entries and pairs with 32 bits (below 2^31
+// entries and 2^30 pairs with pads), so larger graphs keep the pull sweep.
 nwg_plan_params default_plan_for(const nwg_graph* g) {
   nwg_plan_params p = default_plan_params();
   if (g->nnz >= kBinnedEdges && g->nnz < (1ull << 30) - (1ull << 26)) p.binned = 1;
-  const bool skewed = (double)g->max_outdeg > 64.0 + 8.0 * (double)g->nnz / (double)std::max<uint32_t>(g->n, 1);
-  if (g->nnz >= kOrderEdges && skewed) p.relabel = 1;
+  const bool skewed = g->nnz >= kOrderEdges && skewed_degrees(g);
+  if (skewed) p.relabel = 1;
   const uint64_t pairs = skewed ? g->nnz / 3 : g->nnz;  // about
   if (p.binned) p.stream_hints = pairs >= 3ull << 25 ? 2 : pairs >= 1ull << 25 ? 1 : 0;
   return p;
@@ -603,13 +603,20 @@ static void validate_params(const nwg_plan_params& p) {
 // faster at every size (RMAT-12 6.1 against 27.5 us per sweep, RMAT-18 22 / 105, RMAT-24 2220 /
 // 2495, 4096^2 grid 197 / 199).  A binned plan that leaves the bin size open does from
 // kBinnedEdges to kBinnedMinEdges edges, where the items' one launch a sweep beats the binned
-// sweep's three and the contributions still sit in the L2s (default_plan_for has both sides).
-static bool plan_takes_items(const nwg_plan_params& p, uint64_t nnz) {
+// sweep's three and the contributions still sit in the L2s -- unless no vertex stands out and rows are long:
+// every gather of the items is then a line of its own, while the rows of a bin share their pairs.
+// Measured on MI355X, us per solve, items / binned: R-MAT with 4.5 M edges 487 / 589, 5.7 M 626 / 706, 7.5 M 729 / 705;
+// uniform random with 1.0 M edges (10 per row) 175 / 193, 2.0 M (10) 270 / 248, 2.0 M (20) 256 / 183, 2.4 M (8)
+// 319 / 354, 3.2 M (16) 366 / 224, 6.0 M (12) 650 / 323; lattice with 3.4 M (3.4) 292 / 565.
+static bool plan_takes_items(const nwg_plan_params& p, const nwg_graph* g) {
+  const uint64_t nnz = g->nnz;
   const nwg_plan_params d = default_plan_params();
   if (p.short_max != d.short_max || p.group_max != d.group_max || p.hub_min != d.hub_min ||
       p.hub_segment != d.hub_segment || p.slice_min != d.slice_min)
     return false;
-  return !p.binned || (p.bin_bits == 0 && nnz >= kBinnedEdges && nnz < kBinnedMinEdges);
+  if (!p.binned) return true;
+  if (p.bin_bits != 0 || nnz < kBinnedEdges || nnz >= kBinnedMinEdges) return false;
+  return nnz < kSkewEdges || nnz < 10ull * g->n || skewed_degrees(g);
 }
 
 void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp) {
@@ -620,7 +627,7 @@ void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp) {
   Plan pl;
   pl.params = pp;
   pl.n_tiles = (uint32_t)ceil_div(n, kThreads);
-  if (plan_takes_items(pp, g->nnz)) {
+  if (plan_takes_items(pp, g)) {
     pl.n_items = item_count(n, g->nnz);
     pl.idesc.alloc(pl.n_items);
     items_build(s, n, g->nnz, a.ptr, pl.idesc.p);
