@@ -606,8 +606,9 @@ static void validate_params(const nwg_plan_params& p) {
 // sweep's three and the contributions still sit in the L2s -- unless no vertex stands out and rows are long:
 // every gather of the items is then a line of its own, while the rows of a bin share their pairs.
 // Measured on MI355X, us per solve, items / binned: R-MAT with 4.5 M edges 487 / 589, 5.7 M 626 / 706, 7.5 M 729 / 705;
-// uniform random with 1.0 M edges (10 per row) 175 / 193, 2.0 M (10) 270 / 248, 2.0 M (20) 256 / 183, 2.4 M (8)
-// 319 / 354, 3.2 M (16) 366 / 224, 6.0 M (12) 650 / 323; lattice with 3.4 M (3.4) 292 / 565.
+// uniform random with 1.0 M edges (10 per row) 175 / 193, 2.2 M (9) 300 / 272, 2.0 M (20) 256 / 183, 2.8 M (8) 359 /
+// 369, 3.2 M (16) 366 / 224, 3.5 M (7) 450 / 467, 4.0 M (8) 487 / 407, 4.9 M (7) 594 / 612, 6.0 M (12) 650 / 323;
+// lattice with 3.4 M (3.4) 292 / 565.
 static bool plan_takes_items(const nwg_plan_params& p, const nwg_graph* g) {
   const uint64_t nnz = g->nnz;
   const nwg_plan_params d = default_plan_params();
@@ -616,7 +617,7 @@ static bool plan_takes_items(const nwg_plan_params& p, const nwg_graph* g) {
     return false;
   if (!p.binned) return true;
   if (p.bin_bits != 0 || nnz < kBinnedEdges || nnz >= kBinnedMinEdges) return false;
-  return nnz < kSkewEdges || nnz < 10ull * g->n || skewed_degrees(g);
+  return nnz < kSkewEdges || 2 * nnz < (nnz < 3ull << 20 ? 18ull : 15ull) * g->n || skewed_degrees(g);
 }
 
 void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp) {
