@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <new>
 
 #include "nwg_internal.hpp"
@@ -29,7 +30,7 @@ PoolScope::PoolScope(std::shared_ptr<DevPool> p) : prev_(std::move(t_pool)) { t_
 PoolScope::~PoolScope() { t_pool = std::move(prev_); }
 
 void DevPool::trim_locked() noexcept {
-  for (auto& b : free_) (void)hipFree(b.second);
+  for (auto& b : free_) (void)hipFree(b.second.p);
   free_.clear();
   held_ = 0;
 }
@@ -41,7 +42,7 @@ void* DevPool::take(size_t bytes, size_t* size) {
     std::lock_guard<std::mutex> lk(mu_);
     const auto it = free_.lower_bound(want);
     if (it != free_.end() && it->first <= want + want / 2) {  // the smallest that does, if not much too large
-      void* p = it->second;
+      void* p = it->second.p;
       *size = it->first;
       held_ -= it->first;
       free_.erase(it);
@@ -66,15 +67,16 @@ void DevPool::give(void* p, size_t size) noexcept {
   {
     std::lock_guard<std::mutex> lk(mu_);
     if (size <= limit_) {
-      // room for it: the largest free blocks go first
       while (held_ + size > limit_) {
-        const auto it = std::prev(free_.end());
-        (void)hipFree(it->second);
+        const auto it = std::min_element(free_.begin(), free_.end(), [](const auto& a, const auto& b) {
+          return a.second.given < b.second.given;
+        });
+        (void)hipFree(it->second.p);
         held_ -= it->first;
         free_.erase(it);
       }
       try {
-        free_.emplace(size, p);
+        free_.emplace(size, Free{p, ++gifts_});
         held_ += size;
         return;
       } catch (const std::bad_alloc&) {

@@ -11,11 +11,15 @@
 // their work before they return (also when they fail: guarded()), so a block that comes back
 // after the stream was changed has no work left on it.  Objects that outlive a call are
 // destroyed after the device is idle.  The lists are locked: threads may share a context's
-// objects.  Bounds: the pool keeps at most 1/64 of the device's memory in free blocks, gives all
-// of them back when an allocation fails or the context is destroyed, and keeps nothing after that.
+// objects.  Bounds: the pool keeps at most 1/64 of the device's memory in free blocks, of which those
+// given back longest ago make room for new ones (the largest first instead: once a program has solved
+// graphs of many sizes, every build of the 67 M-edge graph gave its own blocks away, 27 ms against 4),
+// gives all of them back when an allocation fails or the context is destroyed, and keeps nothing
+// after that.
 #pragma once
 
 #include <cstddef>
+#include <cstdint>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -37,7 +41,12 @@ class DevPool {
  private:
   void trim_locked() noexcept;
   std::mutex mu_;
-  std::multimap<size_t, void*> free_;
+  struct Free {
+    void* p;
+    uint64_t given;  // when: blocks given back longest ago go first
+  };
+  std::multimap<size_t, Free> free_;  // by size
+  uint64_t gifts_ = 0;
   size_t held_ = 0, limit_;
 };
 
