@@ -115,13 +115,19 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* __restrict__ p,
   if (i < n) p[i] = v;
 }
 
+// One atomic per workgroup of at most kMaxBlocks: those to one address take some 12 ns each (one per
+// wave of 1024 workgroups took 38 to 53 us).
+constexpr uint64_t kMaxBlocks = 512;
 __global__ __launch_bounds__(256) void max_u32_kernel(const uint32_t* __restrict__ v, uint64_t n,
                                                       uint32_t* __restrict__ out) {
+  __shared__ uint32_t wm[4];
   uint32_t m = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) m = max(m, v[i]);
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
-  if (lane_id() == 0) atomicMax(out, m);
+  if (lane_id() == 0) wm[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicMax(out, max(max(wm[0], wm[1]), max(wm[2], wm[3])));
 }
 
 // Out-degree histogram of the CSC's source ids [build_degrees, common.hpp:110-121].  A
@@ -535,7 +541,7 @@ void note_max_outdeg(hipStream_t s, nwg_graph* g) {
   if (g->nnz < kSkewEdges) return;
   DevBuf<uint32_t> m(1);
   fill_u32_kernel<<<1, 256, 0, s>>>(m.p, 1, 0u);
-  max_u32_kernel<<<(uint32_t)std::min<uint64_t>(grid_for(g->n), 1024), 256, 0, s>>>(g->outdeg.p, g->n, m.p);
+  max_u32_kernel<<<(uint32_t)std::min<uint64_t>(grid_for(g->n), kMaxBlocks), 256, 0, s>>>(g->outdeg.p, g->n, m.p);
   NWG_LAUNCH_CHECK();
   g->max_outdeg = read_back_u32(s, m.p);
 }

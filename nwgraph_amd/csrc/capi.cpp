@@ -99,8 +99,9 @@ int nwg_set_stream(nwg_ctx* ctx, void* stream) {
 const char* nwg_last_error(const nwg_ctx* ctx) { return ctx ? ctx->last_error.c_str() : "null context"; }
 
 // ------------------------------------------------------------------ graphs
-int nwg_graph_create_csc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* csc_ptr, const uint32_t* csc_idx,
-                         const uint32_t* outdeg, int mem_kind, nwg_graph** out) {
+// planned: the graph's first solve may choose its plan (else the caller sets one that looks at no degree)
+static int create_csc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* csc_ptr, const uint32_t* csc_idx,
+                      const uint32_t* outdeg, int mem_kind, bool planned, nwg_graph** out) {
   if (!ctx || !out) return NWG_EINVAL;
   *out = nullptr;
   return guarded(ctx, [&] {
@@ -125,9 +126,14 @@ int nwg_graph_create_csc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t*
     else g->outdeg.alloc(n);
     nwg::check_device_csc(s, n, nnz, g->csc_ptr.p, g->csc_idx.p, outdeg ? g->outdeg.p : nullptr,
                           outdeg ? nullptr : g->outdeg.p);
-    nwg::note_max_outdeg(s, g.get());
+    if (planned) nwg::note_max_outdeg(s, g.get());
     *out = g.release();
   });
+}
+
+int nwg_graph_create_csc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* csc_ptr, const uint32_t* csc_idx,
+                         const uint32_t* outdeg, int mem_kind, nwg_graph** out) {
+  return create_csc(ctx, n, nnz, csc_ptr, csc_idx, outdeg, mem_kind, true, out);
 }
 
 int nwg_graph_build_from_edges(nwg_ctx* ctx, uint32_t n, uint64_t ne, const uint32_t* src, const uint32_t* dst,
@@ -365,7 +371,7 @@ int nwg_pagerank_f32(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* csc
                      nwg_pr_info* info) {
   if (!ctx) return NWG_EINVAL;
   nwg_graph* g = nullptr;
-  int rc = nwg_graph_create_csc(ctx, n, nnz, csc_ptr, csc_idx, outdeg, NWG_MEM_HOST, &g);
+  int rc = create_csc(ctx, n, nnz, csc_ptr, csc_idx, outdeg, NWG_MEM_HOST, false, &g);
   if (rc != NWG_OK) return rc;
   // A graph made for one solve takes the pull sweep on its own numbering: it has nothing to
   // build, while the binned layout and the degree-ordered copy cost more than they save in
