@@ -233,8 +233,8 @@ def run_plain(args, ctx, grid=False):
     if binned:
         kernel_desc = "one sweep (pr_chunk_kernel + pr_bin_kernel + pr_bin_combine_kernel)"
     else:
-        kernel_desc = ("one sweep (pr_tile_kernel + pr_group_kernel<4..64> + pr_sgroup_kernel<4..64> + pr_hubseg_kernel"
-                       " + pr_finish_kernel, those the plan uses)")
+        kernel_desc = ("one sweep (pr_item_kernel; with class cutoffs of the plan's own pr_tile_kernel +"
+                       " pr_group_kernel<4..64> + pr_sgroup_kernel<4..64> + pr_hubseg_kernel + pr_finish_kernel)")
     traffic, traffic_src = args.traffic, "--traffic" if args.traffic else None
     if traffic is None and (grid or args.edge_factor == 16):
         key = ("grid", args.width) if grid else ("rmat", args.scale)

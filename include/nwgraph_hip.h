@@ -90,9 +90,10 @@ typedef struct nwg_plan_params {
   uint32_t relabel;      /* 1: sweep a copy of the CSC renumbered by out-degree (results returned in original ids) */
   uint32_t binned;       /* 1: binned sweep (propagation blocking over a tiled copy of the CSC, 8 bytes per
                             entry; row sums exact in fixed point) instead of the degree-binned pull sweep */
-  uint32_t bin_bits;     /* binned sweep: rows per bin, log2: 13 or 14 (0 = by size: 14 from 2^28 edges; a
+  uint32_t bin_bits;     /* binned sweep: rows per bin, log2: 13 or 14 (0 = by size: 14 from 2^25 edges; a
                             binned plan of 2^18 to 6.3 M edges that leaves it 0 runs the item sweep,
-                            which gives the same scores) */
+                            which gives the same scores, unless no out-degree stands out and
+                            rows are long) */
 } nwg_plan_params;
 
 /* ---------------------------------------------------------------- context */
@@ -229,8 +230,9 @@ int nwg_graph_pagerank_inplace(nwg_ctx* ctx, nwg_graph* g, float* scores, const 
 int nwg_graph_pagerank_delta(nwg_ctx* ctx, nwg_graph* g, float* scores, float damping,
                              float threshold, uint64_t max_iters, int mem_kind, nwg_pr_info* info);
 /* Scheduling plan of the sweep: set explicitly, read back, or autotune.  Without either, the
- * first PageRank solve of a graph builds a plan by size: the binned sweep from 2^18 edges,
- * on the degree-ordered copy from 2^23 edges, else the pull sweep (get_plan reports it).
+ * first PageRank solve of a graph builds a plan by size and degrees: the binned sweep from 2^18
+ * edges, on the degree-ordered copy from 2^23 edges with skewed out-degrees, else the pull sweep
+ * (get_plan reports it).
  * The pull sweep runs over work items of equal numbers of edges, one launch per sweep, unless
  * the plan sets class cutoffs (short_max .. slice_min) of its own; its row sums are exact, as
  * the binned sweep's. */
