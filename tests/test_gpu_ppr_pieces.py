@@ -37,7 +37,7 @@ def _fp64(n, ptr, col, deg, ids):
 
 
 @pytest.mark.parametrize("n,tile,k,relabel", [(6001, 8, 1, 0), (6001, 8, 21, 1), (6001, 16, 18, 0), (6001, 32, 35, 1),
-                                              (6001, 64, 64, 0), (6001, 64, 131, 1), (540001, 64, 64, 0),
+                                              (6001, 64, 64, 0), (6001, 64, 131, 1), (6001, 16, 301, 0), (540001, 64, 64, 0),
                                               (540001, 32, 63, 1)])
 def test_rows_at_the_edges_of_the_split(ctx, n, tile, k, relabel):
     import torch
