@@ -231,7 +231,7 @@ int nwg_graph_pagerank_delta(nwg_ctx* ctx, nwg_graph* g, float* scores, float da
                              float threshold, uint64_t max_iters, int mem_kind, nwg_pr_info* info);
 /* Scheduling plan of the sweep: set explicitly, read back, or autotune.  Without either, the
  * first PageRank solve of a graph builds a plan by size and degrees: the binned sweep from 2^18
- * edges, on the degree-ordered copy from 2^23 edges with skewed out-degrees, else the pull sweep
+ * edges, on the degree-ordered copy from 2^20 edges with skewed out-degrees, else the pull sweep
  * (get_plan reports it).
  * The pull sweep runs over work items of equal numbers of edges, one launch per sweep, unless
  * the plan sets class cutoffs (short_max .. slice_min) of its own; its row sums are exact, as

@@ -525,10 +525,8 @@ void build_segments(hipStream_t s, const uint32_t* rp, uint32_t n, uint32_t min_
                     DevBuf<uint32_t>& rows, DevBuf<uint32_t>& seg_ptr, DevBuf<uint32_t>& seg_row, uint32_t* nrows,
                     uint32_t* nsegs);
 nwg_plan_params default_plan_params();
-// edges from which a default plan may order the vertices by degree
-constexpr uint64_t kOrderEdges = 1ull << 23;
 // g->max_outdeg, when the graph is large enough for a plan to look at it; then waits for the device
-constexpr uint64_t kSkewEdges = 1ull << 21;
+constexpr uint64_t kSkewEdges = 1ull << 20;
 void note_max_outdeg(hipStream_t s, nwg_graph* g);
 // whether some vertex has far more out-edges than the average (false below kSkewEdges)
 bool skewed_degrees(const nwg_graph* g);

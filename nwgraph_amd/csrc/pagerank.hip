@@ -562,10 +562,12 @@ nwg_plan_params default_plan_params() {
 // The plan a PageRank solve builds when none was set or tuned.  Measured on MI355X (edge
 // factor 16, us per sweep, items / binned): RMAT-12 6.1 / 19.6, RMAT-16 9.1 / 19.5, RMAT-18 (3.9 M
 // edges) 21.7 / 26.8, RMAT-19 (8.0 M) 40.6 / 35.7 degree ordered, RMAT-20 79 / 53, uniform random
-// with 2.1 M edges 14.7 / 21.7, with 8.4 M 45.2 / 43.4.  Degree ordering pays from RMAT-19 on where
-// degrees are skewed, and costs where they are not and the numbering has locality of its own
-// (ordered / as given: RMAT-20 43.8 / 51.1, RMAT-22 93.7 / 129.9, uniform random with 79 M edges
-// 241 / 233, the 4096^2 lattice 171 / 151).  Nontemporal loads pay once
+// with 2.1 M edges 14.7 / 21.7, with 8.4 M 45.2 / 43.4.  Degree ordering pays where degrees are
+// skewed (the hubs' contributions then share lines, which the L1s keep: us per solve ordered / as
+// given, items, R-MAT with 0.28 M edges 140 / 151, 1.5 M 190 / 223, 2.8 M 263 / 311, 5.5 M 450 / 539; it takes
+// 0.3 to 0.8 ms to make, so smaller graphs keep their numbering), and costs where they are not and
+// the numbering has locality of its own (per binned sweep: RMAT-20 43.8 / 51.1, RMAT-22 93.7 / 129.9,
+// uniform random with 79 M edges 241 / 233, the 4096^2 lattice 171 / 151).  Nontemporal loads pay once
 // the pair values (some 4 bytes per entry or, with skewed degrees, per three entries) compete with the
 // streams for the last-level cache, nontemporal stores once they no longer stay there either (us per
 // sweep with hints 0 / 1 / 2: uniform random with 24 M edges 92 / 103 / 111, 67 M 242 / 217 / 234, 79 M
@@ -577,7 +579,7 @@ nwg_plan_params default_plan_params() {
 nwg_plan_params default_plan_for(const nwg_graph* g) {
   nwg_plan_params p = default_plan_params();
   if (g->nnz >= kBinnedEdges && g->nnz < (1ull << 30) - (1ull << 26)) p.binned = 1;
-  const bool skewed = g->nnz >= kOrderEdges && skewed_degrees(g);
+  const bool skewed = g->nnz >= kSkewEdges && skewed_degrees(g);
   if (skewed) p.relabel = 1;
   const uint64_t pairs = skewed ? g->nnz / 3 : g->nnz;  // about
   if (p.binned) p.stream_hints = pairs >= 3ull << 25 ? 2 : pairs >= 1ull << 25 ? 1 : 0;
@@ -617,7 +619,7 @@ static bool plan_takes_items(const nwg_plan_params& p, const nwg_graph* g) {
     return false;
   if (!p.binned) return true;
   if (p.bin_bits != 0 || nnz < kBinnedEdges || nnz >= kBinnedMinEdges) return false;
-  return nnz < kSkewEdges || 2 * nnz < (nnz < 3ull << 20 ? 18ull : 15ull) * g->n || skewed_degrees(g);
+  return nnz < 2 * kSkewEdges || 2 * nnz < (nnz < 3ull << 20 ? 18ull : 15ull) * g->n || skewed_degrees(g);
 }
 
 void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp) {
