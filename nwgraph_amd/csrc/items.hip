@@ -243,10 +243,11 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
 // L1 change of graph g in sweep k
 __device__ __forceinline__ unsigned long long many_change(const ItemParams& P, const ManyParams& M, uint32_t k,
                                                           uint32_t g) {
-  const unsigned long long* l = P.lanes + (uint64_t)(k % 3) * kManyLanes * M.ngraphs + g;
+  const uint32_t stride = many_stride(M.ngraphs);
+  const unsigned long long* l = P.lanes + (uint64_t)(k % 3) * kManyLanes * stride + g;
   unsigned long long s = 0ull;
 #pragma unroll
-  for (uint32_t q = 0; q < kManyLanes; ++q) s += l[(uint64_t)q * M.ngraphs];
+  for (uint32_t q = 0; q < kManyLanes; ++q) s += l[(uint64_t)q * stride];
   return s;
 }
 
@@ -266,8 +267,9 @@ __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyPar
   if (P.iter > 0)
     for (uint32_t q = blockIdx.x * kNT + threadIdx.x; q < M.ngraphs; q += gridDim.x * kNT)
       P.acc[(uint64_t)(P.iter - 1) * M.ngraphs + q] = many_change(P, M, P.iter - 1, q);
-  for (uint64_t q = blockIdx.x * kNT + threadIdx.x; q < (uint64_t)kManyLanes * M.ngraphs; q += gridDim.x * kNT)
-    P.lanes[(uint64_t)((P.iter + 1) % 3) * kManyLanes * M.ngraphs + q] = 0ull;
+  const uint64_t slot = (uint64_t)kManyLanes * many_stride(M.ngraphs);
+  for (uint64_t q = blockIdx.x * kNT + threadIdx.x; q < slot; q += gridDim.x * kNT)
+    P.lanes[(P.iter + 1) % 3 * slot + q] = 0ull;
   const uint4 d = P.desc[blockIdx.x];
   const uint32_t e0 = d.x, e1 = d.y, r0 = d.z, rows = d.w & kRowMask;
   const bool head = d.w & kHeadPiece, tail = d.w & kTailPiece;
@@ -301,7 +303,7 @@ __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyPar
   else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
   if (g0 == g1 && done[0]) return;
   unsigned long long* const lane =
-      P.lanes + ((uint64_t)(P.iter % 3) * kManyLanes + blockIdx.x % kManyLanes) * M.ngraphs;
+      P.lanes + P.iter % 3 * slot + (uint64_t)(blockIdx.x % kManyLanes) * many_stride(M.ngraphs);
   auto sum = [&](uint32_t a, uint32_t b) { return item_sum(pre, b0, a, b); };
   auto solved = [&](uint32_t g) {
     return g - g0 < kManyLocal ? done[g - g0] != 0
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(256) void item_many_init_kernel(ItemParams P, ManyP
     P.hsum[i] = 0ull;
     P.hcnt[i] = 0u;
   }
-  if (i < 3ull * kManyLanes * M.ngraphs) P.lanes[i] = 0ull;
+  if (i < 3ull * kManyLanes * many_stride(M.ngraphs)) P.lanes[i] = 0ull;
 }
 
 __global__ __launch_bounds__(256) void item_many_fold_kernel(ItemParams P, ManyParams M, uint32_t k) {
@@ -655,7 +657,7 @@ void items_enqueue_sweep(hipStream_t s, const ItemParams& P) {
 }
 
 void items_many_enqueue_init(hipStream_t s, const ItemParams& P, const ManyParams& M) {
-  const uint64_t m = std::max<uint64_t>(P.count, 3ull * kManyLanes * M.ngraphs);
+  const uint64_t m = std::max<uint64_t>(P.count, 3ull * kManyLanes * many_stride(M.ngraphs));
   item_many_init_kernel<<<(uint32_t)ceil_div(m, 256), 256, 0, s>>>(P, M);
   NWG_LAUNCH_CHECK();
 }

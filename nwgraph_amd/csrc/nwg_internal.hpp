@@ -519,6 +519,15 @@ float stream_probe_device(hipStream_t s, hipEvent_t e0, hipEvent_t e1, uint32_t 
 // ---- PageRank (pagerank.hip) ----
 // (re)build the sweep plan of g with the given parameters; g is unchanged on failure
 void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp);
+// The rows of many graphs in one CSC, each graph ordered (ordered[g] != 0) or as it is, within its rows.
+struct UnionOrder {
+  const uint32_t* row_graph;
+  const uint32_t* ordered;
+  int graph_bits, deg_bits;
+};
+// Degree-ordered copy of a CSC (u null: one graph); false when the ids and degrees exceed its sort keys.
+bool degree_order(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* ptr, const uint32_t* col,
+                  const uint32_t* deg, const UnionOrder* u, Relabeled& rl);
 void relabel_build(hipStream_t s, nwg_graph* g);
 // rows with in-degree >= min_deg (ascending) and their split into `seg`-nonzero segments
 void build_segments(hipStream_t s, const uint32_t* rp, uint32_t n, uint32_t min_deg, uint32_t seg,

@@ -23,18 +23,26 @@ constexpr int kThreads = 256;
 
 inline uint32_t grid1(uint64_t m) { return (uint32_t)ceil_div(m ? m : 1, kThreads); }
 
-// key = (no in-edges << (32 + b)) | ((2^32-1 - outdeg) << b) | id : ascending order = the
-// vertices with in-edges first, each group by out-degree descending, id ascending.  (A vertex
+// key = (graph, no in-edges, largest degree - outdeg, id): ascending order = graph after graph, in each
+// the vertices with in-edges first, each group by out-degree descending, id ascending.  (A vertex
 // without in-edges reaches its fixed point in one sweep; grouping them last leaves the
-// binned sweep whole bins with nothing to add, which it stops visiting.)
+// binned sweep whole bins with nothing to add, which it stops visiting.)  A graph that keeps its
+// numbering has 0 in between.  Degrees from 2^dbits - 1 on count as that.
 __global__ __launch_bounds__(kThreads) void degree_key_kernel(uint32_t n, const uint32_t* __restrict__ deg,
-                                                              const uint32_t* __restrict__ ptr, int b,
+                                                              const uint32_t* __restrict__ ptr, int b, int dbits,
+                                                              const uint32_t* __restrict__ row_graph,
+                                                              const uint32_t* __restrict__ ordered,
                                                               uint64_t* __restrict__ keys) {
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  if (i < n) {
-    const uint64_t no_in = ptr[i + 1] == ptr[i] ? 1ull : 0ull;
-    keys[i] = (no_in << (32 + b)) | ((uint64_t)(0xFFFFFFFFu - deg[i]) << b) | i;
+  if (i >= n) return;
+  const uint64_t g = row_graph ? row_graph[i] : 0u;
+  const uint32_t most = 0xFFFFFFFFu >> (32 - dbits);
+  uint64_t no_in = 0, d = 0;
+  if (!ordered || ordered[g]) {
+    no_in = ptr[i + 1] == ptr[i] ? 1ull : 0ull;
+    d = most - min(deg[i], most);
   }
+  keys[i] = (((((g << 1) | no_in) << dbits) | d) << b) | i;
 }
 
 __global__ __launch_bounds__(kThreads) void order_kernel(uint32_t n, const uint64_t* __restrict__ keys, int b,
@@ -68,37 +76,43 @@ __global__ __launch_bounds__(kThreads) void edge_key_kernel(uint32_t n, uint64_t
 
 }  // namespace
 
-void relabel_build(hipStream_t s, nwg_graph* g) {
-  if (g->rl) return;
-  const uint32_t n = g->n;
-  const uint64_t nnz = g->nnz;
-  const int b = key_bits_for(n);
-  NWG_REQUIRE(b <= 31, "degree ordering needs at most 2^31 vertices");
-  std::unique_ptr<Relabeled> rl(new Relabeled());
-  rl->order.alloc(n);
-  rl->rank.alloc(n);
-  rl->outdeg.alloc(n);
+bool degree_order(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* ptr, const uint32_t* col,
+                  const uint32_t* deg, const UnionOrder* u, Relabeled& rl) {
+  const int b = key_bits_for(n), dbits = u ? u->deg_bits : 32, top = b + dbits + 1 + (u ? u->graph_bits : 0);
+  if (b > 31 || top > 64) return false;
+  rl.order.alloc(n);
+  rl.rank.alloc(n);
+  rl.outdeg.alloc(n);
   {
     DevBuf<uint64_t> keys(n), tmp(n);
-    degree_key_kernel<<<grid1(n), kThreads, 0, s>>>(n, g->outdeg.p, g->csc_ptr.p, b, keys.p);
+    degree_key_kernel<<<grid1(n), kThreads, 0, s>>>(n, deg, ptr, b, dbits, u ? u->row_graph : nullptr,
+                                                    u ? u->ordered : nullptr, keys.p);
     NWG_LAUNCH_CHECK();
-    radix_sort_pairs(s, keys, tmp, nullptr, nullptr, n, 0, 33 + b);
-    order_kernel<<<grid1(n), kThreads, 0, s>>>(n, keys.p, b, g->outdeg.p, rl->order.p, rl->rank.p, rl->outdeg.p);
+    radix_sort_pairs(s, keys, tmp, nullptr, nullptr, n, b, top);  // stable, and the ids ascend
+    order_kernel<<<grid1(n), kThreads, 0, s>>>(n, keys.p, b, deg, rl.order.p, rl.rank.p, rl.outdeg.p);
     NWG_LAUNCH_CHECK();
     NWG_HIP(hipStreamSynchronize(s));
   }
-  rl->csc_ptr.alloc((uint64_t)n + 1);
-  rl->csc_idx.alloc(nnz ? nnz : 1);
+  rl.csc_ptr.alloc((uint64_t)n + 1);
+  rl.csc_idx.alloc(nnz ? nnz : 1);
   {
     DevBuf<uint64_t> keys(nnz ? nnz : 1), tmp(nnz ? nnz : 1);
     if (nnz) {
-      edge_key_kernel<<<grid1(nnz), kThreads, 0, s>>>(n, nnz, g->csc_ptr.p, g->csc_idx.p, rl->rank.p, b, keys.p);
+      edge_key_kernel<<<grid1(nnz), kThreads, 0, s>>>(n, nnz, ptr, col, rl.rank.p, b, keys.p);
       NWG_LAUNCH_CHECK();
       radix_sort_pairs(s, keys, tmp, nullptr, nullptr, nnz, 0, 2 * b);
     }
-    sorted_keys_to_csx(s, keys.p, nnz, n, b, rl->csc_ptr.p, rl->csc_idx.p);
+    sorted_keys_to_csx(s, keys.p, nnz, n, b, rl.csc_ptr.p, rl.csc_idx.p);
     NWG_HIP(hipStreamSynchronize(s));
   }
+  return true;
+}
+
+void relabel_build(hipStream_t s, nwg_graph* g) {
+  if (g->rl) return;
+  std::unique_ptr<Relabeled> rl(new Relabeled());
+  NWG_REQUIRE(degree_order(s, g->n, g->nnz, g->csc_ptr.p, g->csc_idx.p, g->outdeg.p, nullptr, *rl),
+              "degree ordering needs at most 2^31 vertices");
   g->rl = std::move(rl);
 }
 
