@@ -226,9 +226,10 @@ struct BinParams {
 // A solve's sweeps run as captured HIP graphs of kSegFirst sweeps, then kSegNext at a time,
 // with the host checking the last sweep's L1 change between segments: sweeps after
 // convergence still launch (and exit at once), and at a few microseconds per launch, 80 of
-// them cost more than the check.  A check costs about 12 us, an empty sweep 3 with one launch
-// and 7 to 9 with the binned sweeps' three: those are checked from the 8th sweep on
-// (uniform random with 24 M edges, 8 sweeps: 0.75 to 0.63 ms).
+// them cost more than the check.  A check costs 12 to 30 us, an empty sweep 3 with one launch
+// and 7 to 9 with the binned sweeps' three: those are checked from the 8th sweep on where no vertex
+// stands out, as such graphs converge within some 10 sweeps (uniform random with 24 M edges, 8
+// sweeps: 0.75 to 0.63 ms), and from the 20th where one does (R-MAT graphs take 15 to 25).
 constexpr uint64_t kSegFirst = 20;
 constexpr uint64_t kSegFirstBinned = 8;
 constexpr uint64_t kSegNext = 8;

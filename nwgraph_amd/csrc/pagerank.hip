@@ -1087,7 +1087,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     key.damping = damping;
     key.threshold = threshold;
     key.extra = (uint32_t)sched;
-    const uint64_t first = items || class_kernels ? kSegFirst : kSegFirstBinned;
+    const uint64_t first = items || class_kernels || skewed_degrees(g) ? kSegFirst : kSegFirstBinned;
     // the solve runs in segments (first sweeps, then kSegNext at a time); between segments the host
     // reads the last sweep's L1 change and stops once the solve has converged, so sweeps after
     // convergence launch only up to a segment's end
