@@ -151,7 +151,7 @@ int nwg_multigraph_autotune(nwg_ctx* ctx, nwg_multigraph* mg, uint32_t* binned_o
     for (uint32_t b = 0; b <= 1; ++b) {
       nwg::multigraph_set_binned(ctx, mg, b != 0);
       double ms = 1e30;
-      for (int r = 0; r < 2; ++r) {  // the first run of a schedule also captures its graph
+      for (int r = 0; r < 3; ++r) {  // launched one by one, captured, replayed: the last one counts
         nwg_pr_info info{};
         nwg::multigraph_run(ctx, mg, 0.85f, -1.0f, 4, out.p, nullptr, nullptr, &info);
         ms = info.ms_total;

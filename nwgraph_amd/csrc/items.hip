@@ -185,6 +185,9 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
   __shared__ unsigned long long wsum[kNT / 64];
   const uint32_t lane = threadIdx.x & 63u;
   const uint4 d = P.desc[blockIdx.x];
+  // a solve that stopped before the previous sweep gathers nothing more (9 of 20 sweeps, allocation-free:
+  // uniform random with 18 M edges 2.55 to 1.48 ms, with 3 M 0.39 to 0.24; resident, 1.9 M 0.23 to 0.14)
+  if (P.iter > 1 && fixed_to_err(P.acc[P.iter - 2]) < P.threshold) return;
   // the previous sweep's L1 change: loaded now, looked at once the gathers are done (a check
   // first would put its latency in front of theirs)
   unsigned long long ch = 0ull;
@@ -601,9 +604,11 @@ __global__ __launch_bounds__(256) void item_init_kernel(ItemParams P, float init
 
 __global__ __launch_bounds__(64) void item_fold_kernel(const unsigned long long* __restrict__ lanes,
                                                        unsigned long long* __restrict__ acc, uint32_t first,
-                                                       uint32_t k, unsigned long long* __restrict__ mail) {
+                                                       uint32_t k, double threshold,
+                                                       unsigned long long* __restrict__ mail) {
   unsigned long long v = lanes[(k % 3) * kItemLaneSlot + threadIdx.x * kItemLanePad];
   v = wave_sum(v);
+  if (k > 0 && fixed_to_err(acc[k - 1]) < threshold) v = 0ull;  // sweep k did nothing, its lanes are older
   if (threadIdx.x == 0) acc[k] = v;
   if (!mail) return;
   for (uint32_t q = first + threadIdx.x; q < k; q += 64) mail[q] = acc[q];
@@ -673,7 +678,7 @@ void items_many_enqueue_fold(hipStream_t s, const ItemParams& P, const ManyParam
 }
 
 void items_enqueue_fold(hipStream_t s, const ItemParams& P, uint32_t first, uint32_t k, unsigned long long* mail) {
-  item_fold_kernel<<<1, 64, 0, s>>>(P.lanes, P.acc, first, k, mail);
+  item_fold_kernel<<<1, 64, 0, s>>>(P.lanes, P.acc, first, k, P.threshold, mail);
   NWG_LAUNCH_CHECK();
 }
 
