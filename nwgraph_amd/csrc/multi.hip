@@ -195,15 +195,17 @@ struct nwg_multigraph {
 
 namespace nwg {
 
-// Graphs with skewed out-degrees are swept in degree order, as single ones are (default_plan_for): fewer
-// (bin, source) pairs and lines that the L1s keep.  MI355X, 20 sweeps: 256 graphs of 2^10 to 2^18 vertices
-// (213 M edges) binned 5.42 to 4.92 ms; 12 of 2^12 to 2^18 (9.5 M) binned 1.53 to 1.12, items 0.87 to 0.80.
-// Unions below kOrderUnion edges keep their numbering (the copy takes longer than it saves over a few
-// solves), and so do those whose sort would take 16 GiB of keys.
+// Graphs of more than kOrderRows vertices with skewed out-degrees are swept in degree order, as single ones
+// are (default_plan_for): fewer (bin, source) pairs and lines that the L1s keep.  MI355X, 20 sweeps, ordered /
+// as given: 256 graphs of 2^10 to 2^18 vertices (213 M edges) binned 4.92 / 5.42 ms; 12 of 2^12 to 2^18 (9.5 M)
+// binned 1.08 / 1.35, items 0.78 / 0.84.  Smaller graphs gain nothing: 90 of 2^10 to 2^16 (28 M) binned 1.51 /
+// 1.42, 96 of 2^12 (7 M) items 0.55 / 0.53.  Unions below kOrderUnion edges keep their numbering (the copy
+// takes longer than it saves over a few solves), and so do those whose sort would take 16 GiB of keys.
+constexpr uint64_t kOrderRows = 1ull << 16;
 constexpr uint64_t kOrderUnion = 1ull << 20, kOrderUnionMax = 1ull << 30;
 static void order_by_degree(hipStream_t s, nwg_multigraph* mg, const std::vector<uint64_t>& eoff) {
   const uint32_t G = mg->ngraphs;
-  if (mg->ne < kOrderUnion || mg->ne >= kOrderUnionMax || small_fits(mg->max_n, mg->max_nnz, true)) return;
+  if (mg->ne < kOrderUnion || mg->ne >= kOrderUnionMax || mg->max_n <= kOrderRows) return;
   std::vector<uint32_t> most(G, 0u);
   DevBuf<uint32_t> flags(G);
   NWG_HIP(hipMemcpyAsync(flags.p, most.data(), G * 4ull, hipMemcpyHostToDevice, s));
@@ -215,8 +217,8 @@ static void order_by_degree(hipStream_t s, nwg_multigraph* mg, const std::vector
   for (uint32_t g = 0; g < G; ++g) {
     const double n = (double)std::max<uint64_t>(mg->voff[g + 1] - mg->voff[g], 1);
     const bool skewed = (double)most[g] > 64.0 + 8.0 * (double)(eoff[g + 1] - eoff[g]) / n;  // skewed_degrees()
-    most[g] = skewed ? 1u : 0u;
-    any = any || skewed;
+    most[g] = skewed && n > (double)kOrderRows ? 1u : 0u;
+    any = any || most[g];
   }
   if (!any) return;
   NWG_HIP(hipMemcpyAsync(flags.p, most.data(), G * 4ull, hipMemcpyHostToDevice, s));
