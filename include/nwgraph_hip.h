@@ -284,7 +284,9 @@ int nwg_multigraph_autotune(nwg_ctx* ctx, nwg_multigraph* mg, uint32_t* binned_o
 
 /* ------------------------------------------- weighted PageRank and adjoint */
 /* Edge weights in CSC order (weight of edge col[p] -> row).  With normalize=1 each
- * source's outgoing weights are divided by their sum (row-normalised transition). */
+ * source's outgoing weights are divided by their sum (row-normalised transition).  A sum of 0
+ * (or past the largest float) leaves a source's weights undefined: below 2^18 edges, and with a
+ * plan that is not binned, what they reach is NaN; the binned sweep drops the source's mass. */
 int nwg_graph_set_weights(nwg_ctx* ctx, nwg_graph* g, const float* w_csc, int normalize,
                           int mem_kind);
 /* Fill raw weights w(u,v) = 0.1 + 0.9 t, t ~ U[0,1) from Philox (u, v, seed), then set them. */

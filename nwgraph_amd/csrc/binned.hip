@@ -811,7 +811,7 @@ __global__ __launch_bounds__(256) void bin_place_kernel(uint64_t nnz, const uint
       else hi = mid;
     }
     lw = lo & ((1u << bb) - 1u);
-    bw[bin_slot(ne)] = w[p];
+    bw[bin_slot(ne)] = w[p] == w[p] ? w[p] : 0.f;  // undefined (0 / 0): moves nothing, as fixed point has no NaN
   }
   brow[bin_slot(ne)] = (uint16_t)(bin_perm(lw) | (f ? kPairStart : 0u));
   if (f) {

@@ -534,7 +534,8 @@ __device__ __forceinline__ void item_row_sums(const RowSumParams& P, uint32_t b0
 
 __device__ __forceinline__ void row_sum_out(const RowSumParams& P, const RowSumOut& o, uint32_t u, double s) {
   if (!P.gather) {
-    o.out[u] = (float)s;
+    const float f = (float)s;
+    o.out[u] = __builtin_isinf(f) ? __builtin_nanf("") : f;  // past the floats: the weights it divides would be 0
     return;
   }
   const double x = (double)o.x[u], norm = (double)o.norm[u];

@@ -391,6 +391,7 @@ struct nwg_graph {
   bool has_weights = false;
   bool w_normalized = false;
   bool w_nonneg = false;  // every raw weight finite and >= 0
+  bool w_undefined = false;  // some normalised weight is NaN (its source's sum is 0 or no finite float)
   nwg::DevBuf<float> w_csc, w_raw, w_csr, w_rowsum;
   // work items of the weighted sweeps over the CSC (forward) and the CSR (adjoint)
   nwg::DevBuf<uint32_t> w_items_csc_r0, w_items_csc_r1, w_items_csr_r0, w_items_csr_r1;

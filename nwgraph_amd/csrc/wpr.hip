@@ -319,14 +319,19 @@ __global__ __launch_bounds__(kThreads) void row_of_kernel(uint32_t n, uint64_t n
 }
 
 __global__ __launch_bounds__(64) void wclear_kernel(uint32_t* __restrict__ p) {
-  if (threadIdx.x == 0) *p = 0u;
+  if (threadIdx.x < 2) p[threadIdx.x] = 0u;
 }
 
+// *undefined = 1 when some weight is NaN: its source's raw weights sum to 0, or to no finite float
 __global__ __launch_bounds__(kThreads) void normalise_kernel(uint64_t nnz, const uint32_t* __restrict__ col,
                                                              const float* __restrict__ w_raw,
-                                                             const float* __restrict__ s, float* __restrict__ w) {
+                                                             const float* __restrict__ s, float* __restrict__ w,
+                                                             uint32_t* __restrict__ undefined) {
   const uint64_t p = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (p < nnz) w[p] = w_raw[p] / s[col[p]];
+  if (p >= nnz) return;
+  const float v = w_raw[p] / s[col[p]];
+  w[p] = v;
+  if (v != v) *undefined = 1u;
 }
 
 __global__ __launch_bounds__(kThreads) void gather_kernel(uint64_t nnz, const uint32_t* __restrict__ perm,
@@ -449,8 +454,9 @@ void weights_set(hipStream_t s, nwg_graph* g, const float* w_dev, bool normalize
   g->w_csc.ensure(nnz ? nnz : 1);
   g->w_csr.ensure(nnz ? nnz : 1);
   g->w_rowsum.ensure(g->n);
-  // raw weights all finite and >= 0: the fixed-point bound of the exact weighted sweeps holds
-  DevBuf<uint32_t> bad(1);
+  // raw weights all finite and >= 0, and every source's sum finite and above 0: the fixed-point bound of
+  // the exact weighted sweeps holds
+  DevBuf<uint32_t> bad(2);
   wclear_kernel<<<1, 64, 0, s>>>(bad.p);
   if (nnz) weight_copy_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, w_dev, g->w_raw.p, bad.p);
   NWG_LAUNCH_CHECK();
@@ -458,7 +464,9 @@ void weights_set(hipStream_t s, nwg_graph* g, const float* w_dev, bool normalize
     RowSumOut o{};
     o.out = g->w_rowsum.p;
     csr_row_sums(s, g, g->csr_to_csc.p, g->w_raw.p, nullptr, o);
-    if (nnz) normalise_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csc_idx.p, g->w_raw.p, g->w_rowsum.p, g->w_csc.p);
+    if (nnz)
+      normalise_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csc_idx.p, g->w_raw.p, g->w_rowsum.p, g->w_csc.p,
+                                                       bad.p + 1);
     NWG_LAUNCH_CHECK();
   } else {
     std::vector<float> ones(g->n, 1.0f);
@@ -468,12 +476,13 @@ void weights_set(hipStream_t s, nwg_graph* g, const float* w_dev, bool normalize
   }
   if (nnz) gather_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csr_to_csc.p, g->w_csc.p, g->w_csr.p);
   NWG_LAUNCH_CHECK();
-  uint32_t hb = 0;
-  NWG_HIP(hipMemcpyAsync(&hb, bad.p, sizeof hb, hipMemcpyDeviceToHost, s));
+  uint32_t hb[2] = {0, 0};
+  NWG_HIP(hipMemcpyAsync(hb, bad.p, sizeof hb, hipMemcpyDeviceToHost, s));
   NWG_HIP(hipStreamSynchronize(s));
   g->has_weights = true;
   g->w_normalized = normalize;
-  g->w_nonneg = hb == 0;
+  g->w_nonneg = hb[0] == 0;
+  g->w_undefined = hb[1] != 0;
   if (g->wst) {  // the weighted layouts carry the old weights
     g->wst->bl_csc.reset();
     g->wst->bl_csr.reset();
@@ -742,13 +751,14 @@ static WState& wstate(nwg_graph* g) {
 // (RMAT, us per sweep, items / binned): 53 K edges 5.9 / 19.9, 228 K 7.2 / 23.1, 842 K 9.9 / 20.3, 1.9 M 17.7 / 23.5,
 // 3.9 M 32.1 / 26.2.
 // Above, and where the plan names a bin size, the binned sweep when the plan (or, before any plan,
-// its size) asks for it.
+// its size) asks for it.  Weights that are undefined (0 / 0) show as NaN in the pull sweep, which takes the
+// items' place for them; the binned layout carries them as 0, so that its sweeps drop their sources' mass.
 constexpr uint32_t kItemsWeighted = 2560;
 static WSweep weighted_sweep(const nwg_graph* g, float damping) {
   if (!g->w_normalized || !g->w_nonneg || g->nnz == 0) return WSweep::kPull;
   const nwg_plan_params pp = g->plan.built ? g->plan.params : default_plan_for(g);
   if (pp.binned && pp.bin_bits) return WSweep::kBinned;
-  if (item_count(g->n, g->nnz) <= kItemsWeighted && damping >= 0.f && damping < 1.f) return WSweep::kItems;
+  if (!g->w_undefined && item_count(g->n, g->nnz) <= kItemsWeighted && damping >= 0.f && damping < 1.f) return WSweep::kItems;
   return pp.binned ? WSweep::kBinned : WSweep::kPull;
 }
 
