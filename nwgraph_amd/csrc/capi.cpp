@@ -61,7 +61,7 @@ int nwg_create(nwg_ctx** out, int device) {
     NWG_HIP(hipEventCreate(&ctx->ev0));
     NWG_HIP(hipEventCreate(&ctx->ev1));
     nwg::noalloc_setup(device);
-    NWG_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->mail), (nwg::kMailWords + 2) * 8, hipHostMallocDefault));
+    NWG_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->mail), (nwg::kMailCut + 1) * 8, hipHostMallocDefault));
     size_t total_bytes = 0;
     NWG_HIP(hipDeviceTotalMem(&total_bytes, device));
     ctx->pool = std::make_shared<nwg::DevPool>(total_bytes / 64);

@@ -24,6 +24,22 @@ __device__ __forceinline__ unsigned long long quantize(float c) {
   const uint32_t l = (uint32_t)(r * 4294967296.f);  // floor(r * 2^32) < 2^32
   return ((unsigned long long)h << 32) | l;
 }
+// Whether quantize cuts bits of some value off: the smallest magnitude but 0 among the values noted is
+// below 2^-37 (signed: 2^-37 / 2^t).  Kept as twice the bits less 2, of which 0 gives the largest
+// number: one or two integer operations a value.
+struct CutNote {
+  uint32_t least = ~0u;
+  __device__ __forceinline__ void note(float v) { least = min(least, (__float_as_uint(v) << 1) - 2u); }
+  __device__ __forceinline__ bool cuts(int t = 0) const {
+    return least < (__float_as_uint(__builtin_ldexpf(1.f, -37 - t)) << 1) - 2u;
+  }
+};
+// A sum of m such values is short by less than m units of 2^-60 (of 2^(-60 - t) when scaled by 2^t),
+// which is above 2^-26 of a result x only below m * 2^-34: there a float sum would be the more precise,
+// and the sweeps add the row up once more in double.
+__device__ __forceinline__ bool sum_is_coarse(float x, uint32_t m, int t = 0) {
+  return fabsf(x) < __builtin_ldexpf((float)m, -34 - t);
+}
 // v * 2^-60 rounded to the nearest float (ties to even).  Below 2^53 (sums under 2^-7, nearly
 // every row) v is exact as a double, so one rounding to float and an exact scale by 2^-60 give
 // it; above, integer operations do.

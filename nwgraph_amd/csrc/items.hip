@@ -20,7 +20,10 @@
 // running prefix over the item (lane, then wave, then workgroup), and row i's sum is the
 // difference of the prefix at its two ends.  The sums are exact integers, so the difference is
 // the row's exact sum: short and long rows cost the same, nothing diverges, and the result
-// depends on no order (fixed_point.hpp).
+// depends on no order (fixed_point.hpp).  Where cut-off bits could show (scores far below the others:
+// long personalised solves, damping 1), a row is added up once more in double from its gathers.  Noting cut
+// bits and looking at the note takes 1 to 3 % of a sweep where none are (20 sweeps, RMAT-12 100.8 to 102.6 us,
+// RMAT-16 164.4 to 168.9).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -42,6 +45,7 @@ constexpr uint32_t kNT = 256;
 constexpr uint32_t kHeadPiece = 1u << 30;  // the item's first edges belong to a long row begun before it
 constexpr uint32_t kTailPiece = 1u << 31;  // its last edges to a long row that goes on after it
 constexpr uint32_t kRowMask = kHeadPiece - 1;
+constexpr uint32_t kCutRow = 1u << 31;     // in a long row's count of pieces: some value was cut
 
 // units per item; an item stages at most 2 kSpan - 2 edges, and 3 before them for alignment, in
 // the 8 kNT places it has
@@ -119,11 +123,11 @@ __device__ __forceinline__ void item_ids(const uint32_t* __restrict__ ids, uint3
 
 // K values per lane: inclusive fixed-point prefix of the edges [e0, e1), entry q of it for edge
 // b0 + q (b0 = e0 rounded down to 4; entries before e0 are 0).  w null: value cin[id]; else
-// w * cin[id] scaled by 2^qs.
+// w * cin[id] scaled by 2^qs.  cuts: per wave, whether some value lost bits.
 template <int K, bool W>
 __device__ __forceinline__ void item_prefix(const uint32_t* __restrict__ col, const float* w, int qs,
                                             const float* cin, uint32_t nnz, uint32_t b0, uint32_t e0, uint32_t e1,
-                                            unsigned long long* pre, unsigned long long* wsum) {
+                                            unsigned long long* pre, unsigned long long* wsum, uint32_t* cuts) {
   const uint32_t q0 = threadIdx.x * K;
   uint32_t u[K];
   item_ids<K>(col, nnz, b0 + q0, e1, u);
@@ -133,18 +137,29 @@ __device__ __forceinline__ void item_prefix(const uint32_t* __restrict__ col, co
 #pragma unroll
   for (int t = 0; t < K; ++t) c[t] = cin[u[t]];  // ids outside [e0, e1) are ids too, or 0
   unsigned long long v[K], s = 0;
+  CutNote cut;  // entries outside [e0, e1) too: noting one that cuts costs time only
 #pragma unroll
   for (int t = 0; t < K; ++t) {
     const uint32_t p = b0 + q0 + t;
     unsigned long long q;
-    if constexpr (W) q = quantize_signed(__uint_as_float(wt[t]) * c[t], qs);
-    else q = quantize(c[t]);
+    if constexpr (W) {
+      const float f = __uint_as_float(wt[t]) * c[t];
+      q = quantize_signed(f, qs);
+      cut.note(f);
+    } else {
+      q = quantize(c[t]);
+      cut.note(c[t]);
+    }
     s += (p >= e0 && p < e1) ? q : 0ull;
     v[t] = s;
   }
+  const uint64_t any_cut = __ballot(cut.cuts(qs));
   unsigned long long inc = wave_inclusive_scan(s);
   unsigned long long off = inc - s;
-  if (lane_id() == 63) wsum[threadIdx.x >> 6] = inc;
+  if (lane_id() == 63) {
+    wsum[threadIdx.x >> 6] = inc;
+    cuts[threadIdx.x >> 6] = any_cut != 0;
+  }
   __syncthreads();
 #pragma unroll
   for (uint32_t w2 = 0; w2 < kNT / 64 - 1; ++w2) off += w2 < (threadIdx.x >> 6) ? wsum[w2] : 0ull;
@@ -161,28 +176,71 @@ __device__ __forceinline__ unsigned long long item_sum(const unsigned long long*
   return a == b0 ? hi : hi - pre[pos(a - 1 - b0)];
 }
 
+static_assert(kNT == 256, "cuts of four waves");
+__device__ __forceinline__ bool item_cuts(const uint32_t* cuts) { return (cuts[0] | cuts[1] | cuts[2] | cuts[3]) != 0; }
+
+// sum of the entries a, a + step, ... below b of a row, as item_prefix's without the rounding to units
+template <bool W>
+__device__ __forceinline__ double direct_sum(const uint32_t* __restrict__ col, const float* w, const float* cin,
+                                             uint64_t a, uint64_t b, uint32_t step) {
+  double s = 0.0;
+#pragma unroll 4
+  for (uint64_t p = a; p < b; p += step) {
+    const double c = (double)cin[col[p]];
+    if constexpr (W) s += (double)w[p] * c;
+    else s += c;
+  }
+  return s;
+}
+// The sums of the long rows whose lanes ask for them (entries [a, b) each), by the whole wave.
+template <bool W>
+__device__ __forceinline__ void direct_long_sums(const uint32_t* __restrict__ col, const float* w, const float* cin,
+                                                 uint32_t a, uint32_t b, bool ask, float* z) {
+  for (uint64_t m = __ballot(ask); __builtin_expect(m != 0, 0); m &= m - 1) {
+    const int l = __builtin_ctzll(m);
+    const uint32_t ra = (uint32_t)__shfl((int)a, l, 64), rb = (uint32_t)__shfl((int)b, l, 64);
+    const double s = wave_sum(direct_sum<W>(col, w, cin, (uint64_t)ra + lane_id(), rb, 64));
+    if ((int)lane_id() == l) *z = (float)s;
+  }
+}
+
 // Adds a piece of long row h (entries [hp0, hp1), this piece's sum `mine`) to the row's counter, that
 // of the item it starts in; true for the last piece, which gets the row's sum and leaves the
-// counters at 0 for the next sweep.  *start: the item the row starts in.
+// counters at 0 for the next sweep.  *start: the item the row starts in.  cut: in, whether a value of
+// this piece was cut; out, of any piece.
 __device__ __forceinline__ bool add_piece(unsigned long long* hsum, uint32_t* hcnt, uint32_t h, uint32_t hp0,
                                           uint32_t hp1, unsigned long long mine, unsigned long long* z,
-                                          uint32_t* start) {
+                                          uint32_t* start, bool& cut) {
   // the row's pieces are those of the items its edges' units lie in
   const uint32_t a = (uint32_t)(((uint64_t)h + hp0) / kSpan), b = (uint32_t)(((uint64_t)h + hp1 - 1) / kSpan);
   *start = a;
   unsigned long long old = __hip_atomic_fetch_add(hsum + a, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // in the word of the count, so before it
+  if (cut) (void)__hip_atomic_fetch_or(hcnt + a, kCutRow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // the sum has been added (its old value is back) before the piece is counted
   asm volatile("s_waitcnt vmcnt(0)" : "+v"(old) : : "memory");
-  if (__hip_atomic_fetch_add(hcnt + a, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != b - a) return false;
+  const uint32_t counted = __hip_atomic_fetch_add(hcnt + a, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((counted & ~kCutRow) != b - a) return false;
+  cut = counted & kCutRow;
   *z = __hip_atomic_exchange(hsum + a, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(hcnt + a, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return true;
+}
+
+// the sum of a row's entries [a, b): s in fixed point, or in double where that is too coarse for it
+__device__ __forceinline__ float item_row_sum(const ItemParams& P, unsigned long long s, uint32_t a, uint32_t b,
+                                              float base, const uint32_t* cuts) {
+  const float z = dequantize(s);
+  if (__builtin_expect(item_cuts(cuts), 0) && sum_is_coarse(__builtin_fmaf(P.damp, z, base), b - a))
+    return (float)direct_sum<false>(P.col, nullptr, P.cin, a, b, 1);
+  return z;
 }
 
 __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
   static_assert(kItemLanes == 64 && kNT == 256, "one lane counter per wavefront lane, four waves");
   __shared__ unsigned long long pre[9 * kNT];
   __shared__ unsigned long long wsum[kNT / 64];
+  __shared__ uint32_t cuts[kNT / 64];
   const uint32_t lane = threadIdx.x & 63u;
   const uint4 d = P.desc[blockIdx.x];
   // a solve that stopped before the previous sweep gathers nothing more (9 of 20 sweeps, allocation-free:
@@ -213,8 +271,8 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
-  else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
   ch = wave_sum(ch);
   if (blockIdx.x == 0) {
     if (threadIdx.x < 64) P.lanes[((P.iter + 1) % 3) * kItemLaneSlot + lane * kItemLanePad] = 0ull;
@@ -223,17 +281,31 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
   if (P.iter > 0 && fixed_to_err(ch) < P.threshold) return;
   auto sum = [&](uint32_t a, uint32_t b) { return item_sum(pre, b0, a, b); };
   unsigned long long err = 0ull;
-  if (threadIdx.x < rows) err = item_update(P, r0 + threadIdx.x, dequantize(sum(ra, rb)), xo, bv, dg);
-  for (uint32_t q = threadIdx.x + kNT; q < rows; q += kNT) {
+  for (uint32_t q = threadIdx.x; q < rows;) {
+    err += item_update(P, r0 + q, item_row_sum(P, sum(ra, rb), ra, rb, bv, cuts), xo, bv, dg);
+    if ((q += kNT) >= rows) break;
     const uint32_t i = r0 + q;
-    err += item_update(P, i, dequantize(sum(P.rp[i], P.rp[i + 1])), P.x[i], P.basev ? P.basev[i] : P.base, P.deg[i]);
+    ra = P.rp[i];
+    rb = P.rp[i + 1];
+    xo = P.x[i];
+    dg = P.deg[i];
+    if (P.basev) bv = P.basev[i];
   }
+  float hz = 0.f, hb = 0.f;
+  bool last = false, ask = false;
   if (piece) {
     unsigned long long z;
     uint32_t a;
-    if (add_piece(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a))
-      err += item_update(P, h, dequantize(z), P.x[h], P.basev ? P.basev[h] : P.base, P.deg[h]);
+    bool cut = item_cuts(cuts);
+    last = add_piece(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a, cut);
+    if (last) {
+      hz = dequantize(z);
+      hb = P.basev ? P.basev[h] : P.base;
+      ask = cut && sum_is_coarse(__builtin_fmaf(P.damp, hz, hb), hp1 - hp0);
+    }
   }
+  direct_long_sums<false>(P.col, nullptr, P.cin, hp0, hp1, ask, &hz);
+  if (last) err += item_update(P, h, hz, P.x[h], hb, P.deg[h]);
   err = wave_sum(err);
   if (lane == 0) wsum[threadIdx.x >> 6] = err;
   __syncthreads();
@@ -264,6 +336,7 @@ constexpr uint32_t kManyLocal = 64;
 __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyParams M) {
   __shared__ unsigned long long pre[9 * kNT];
   __shared__ unsigned long long wsum[kNT / 64];
+  __shared__ uint32_t cuts[kNT / 64];
   __shared__ unsigned long long errs[kManyLocal];
   __shared__ uint32_t done[kManyLocal];
   // the previous sweep's changes, for the host, and the next sweep's lanes
@@ -302,8 +375,8 @@ __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyPar
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
-  else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum);
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
   if (g0 == g1 && done[0]) return;
   unsigned long long* const lane =
       P.lanes + P.iter % 3 * slot + (uint64_t)(blockIdx.x % kManyLanes) * many_stride(M.ngraphs);
@@ -319,20 +392,35 @@ __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyPar
     else if (g - g0 < kManyLocal) atomicAdd(&errs[g - g0], e);
     else atomicAdd(lane + g, e);
   };
-  if (threadIdx.x < rows && !solved(rg))
-    add(rg, item_update(P, r0 + threadIdx.x, dequantize(sum(ra, rb)), xo, bv, dg));
-  for (uint32_t q = threadIdx.x + kNT; q < rows; q += kNT) {
-    const uint32_t i = r0 + q, g = M.row_graph[i];
-    if (!solved(g)) add(g, item_update(P, i, dequantize(sum(P.rp[i], P.rp[i + 1])), P.x[i], P.basev[i], P.deg[i]));
+  for (uint32_t q = threadIdx.x; q < rows;) {
+    if (!solved(rg)) add(rg, item_update(P, r0 + q, item_row_sum(P, sum(ra, rb), ra, rb, bv, cuts), xo, bv, dg));
+    if ((q += kNT) >= rows) break;
+    const uint32_t i = r0 + q;
+    ra = P.rp[i];
+    rb = P.rp[i + 1];
+    xo = P.x[i];
+    dg = P.deg[i];
+    bv = P.basev[i];
+    rg = M.row_graph[i];
   }
+  float hz = 0.f, hb = 0.f;
+  bool last = false, ask = false;
+  uint32_t hg = 0;
   if (piece) {
     // all pieces of a row see the same change, so they are all added or none is
-    const uint32_t g = M.row_graph[h];
+    hg = M.row_graph[h];
     unsigned long long z;
     uint32_t a;
-    if (!solved(g) && add_piece(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a))
-      add(g, item_update(P, h, dequantize(z), P.x[h], P.basev[h], P.deg[h]));
+    bool cut = item_cuts(cuts);
+    last = !solved(hg) && add_piece(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a, cut);
+    if (last) {
+      hz = dequantize(z);
+      hb = P.basev[h];
+      ask = cut && sum_is_coarse(__builtin_fmaf(P.damp, hz, hb), hp1 - hp0);
+    }
   }
+  direct_long_sums<false>(P.col, nullptr, P.cin, hp0, hp1, ask, &hz);
+  if (last) add(hg, item_update(P, h, hz, P.x[h], hb, P.deg[h]));
   if (g0 == g1) {
     err = wave_sum(err);
     if (lane_id() == 0) wsum[threadIdx.x >> 6] = err;
@@ -383,6 +471,7 @@ __device__ __forceinline__ double witem_change(const WItemParams& P, uint32_t k,
 __global__ __launch_bounds__(kNT) void wpr_item_kernel(WItemParams P) {
   __shared__ unsigned long long pre[9 * kNT];
   __shared__ unsigned long long wsum[kNT / 64];
+  __shared__ uint32_t cuts[kNT / 64];
   __shared__ double red[kNT / 64], red2[kNT / 64];
   const double stop = witem_stop(P);
   // a solve that stopped before the previous sweep: that sweep stored no parts
@@ -407,31 +496,50 @@ __global__ __launch_bounds__(kNT) void wpr_item_kernel(WItemParams P) {
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * kNT) item_prefix<4, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
-  else item_prefix<8, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum);
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  else item_prefix<8, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum, cuts);
   if (P.iter > 0 && !P.folded) {
     const double ch = witem_change(P, P.iter - 1, red);
     if (blockIdx.x == 0 && threadIdx.x == 0) P.err[P.iter - 1] = ch;
     if (ch < stop) return;
   }
-  auto update = [&](uint32_t i, unsigned long long z, float old, float b) -> double {
-    const float xn = __builtin_fmaf(P.damp, dequantize_signed(z, qs), b);
+  auto coarse = [&](float z, float b, uint32_t m) { return sum_is_coarse(__builtin_fmaf(P.damp, z, b), m, qs); };
+  auto update = [&](uint32_t i, float z, float old, float b) -> double {
+    const float xn = __builtin_fmaf(P.damp, z, b);
     P.xout[i] = xn;
     return (double)fabsf(xn - old);
   };
+  auto row_sum = [&](uint32_t a, uint32_t b, float base) -> float {
+    const float z = dequantize_signed(item_sum(pre, b0, a, b), qs);
+    if (__builtin_expect(item_cuts(cuts), 0) && coarse(z, base, b - a)) return (float)direct_sum<true>(P.col, P.w, P.xin, a, b, 1);
+    return z;
+  };
   double e = 0.0;
-  if (threadIdx.x < rows) e = update(r0 + threadIdx.x, item_sum(pre, b0, ra, rb), xo, bv);
-  for (uint32_t q = threadIdx.x + kNT; q < rows; q += kNT) {
+  for (uint32_t q = threadIdx.x; q < rows;) {
+    e += update(r0 + q, row_sum(ra, rb, bv), xo, bv);
+    if ((q += kNT) >= rows) break;
     const uint32_t i = r0 + q;
-    e += update(i, item_sum(pre, b0, P.rp[i], P.rp[i + 1]), P.xin[i], P.basev[i]);
+    ra = P.rp[i];
+    rb = P.rp[i + 1];
+    xo = P.xin[i];
+    bv = P.basev[i];
   }
   double* part = P.part + (uint64_t)(P.iter & 1u) * 2 * P.count;
+  float hz = 0.f, hb = 0.f;
+  uint32_t ha = 0;
+  bool last = false, ask = false;
   if (piece) {
     unsigned long long z;
-    uint32_t a;
-    if (add_piece(P.hsum, P.hcnt, h, hp0, hp1, item_sum(pre, b0, max(hp0, e0), min(hp1, e1)), &z, &a))
-      part[P.count + a] = update(h, z, P.xin[h], P.basev[h]);
+    bool cut = item_cuts(cuts);
+    last = add_piece(P.hsum, P.hcnt, h, hp0, hp1, item_sum(pre, b0, max(hp0, e0), min(hp1, e1)), &z, &ha, cut);
+    if (last) {
+      hz = dequantize_signed(z, qs);
+      hb = P.basev[h];
+      ask = cut && coarse(hz, hb, hp1 - hp0);
+    }
   }
+  direct_long_sums<true>(P.col, P.w, P.xin, hp0, hp1, ask, &hz);
+  if (last) part[P.count + ha] = update(h, hz, P.xin[h], hb);
   e = wave_sum(e);
   if ((threadIdx.x & 63u) == 0) red2[threadIdx.x >> 6] = e;
   __syncthreads();

@@ -392,7 +392,7 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   I.threshold = (double)threshold;
   const ManyParams M{mg->row_graph.p, G};
   // every graph a workgroup of its own, all sweeps in one launch
-  const bool small = items && small_fits(mg->max_n, mg->max_nnz, true) && max_iters <= kSmallSweeps;
+  bool small = items && small_fits(mg->max_n, mg->max_nnz, true) && max_iters <= kSmallSweeps;
   SmallParams S{};
   S.rp = mg->rp.p;
   S.col = mg->col.p;
@@ -404,7 +404,9 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   S.x = mg->x.p;
   S.out = scores_dev;
   S.acc = mg->acc.p;
+  S.cut = ctx->mail + kMailCut;
   S.threshold = (double)threshold;
+  *S.cut = 0ull;
 
   BinParams B{};
   if (mg->binned) {
@@ -445,9 +447,7 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   key.damping = damping;
   key.threshold = threshold;
   key.extra = grid | (mg->binned ? 0x80000000u : 0u) | (items ? 0x40000000u : 0u);
-  NWG_HIP(hipEventRecord(ctx->ev0, s));
-  if (small) small_enqueue(s, S, mg->max_n, mg->max_nnz, 0, max_iters);
-  else run_segment(ctx, mg->caps, 0, key, [&](hipStream_t t) {
+  auto enqueue = [&](hipStream_t t) {
     multi_init_kernel<<<grid1(std::max<uint64_t>(mg->nv, max_iters * G)), kThreads, 0, t>>>(
         mg->nv, mg->deg.p, mg->vinit.p, mg->x.p, mg->c0.p, mg->acc.p, max_iters * G);
     NWG_LAUNCH_CHECK();
@@ -466,17 +466,27 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
       }
     }
     if (items && max_iters) items_many_enqueue_fold(t, I, M, (uint32_t)max_iters - 1);
-  });
-  NWG_HIP(hipEventRecord(ctx->ev1, s));
+  };
   std::vector<unsigned long long> acc(std::max<uint64_t>(max_iters, 1) * G);
-  NWG_HIP(hipMemcpyAsync(acc.data(), mg->acc.p, max_iters * G * 8ull, hipMemcpyDeviceToHost, s));
-  if (scores_dev && !small && mg->rank.p) {
-    multi_out_kernel<<<grid1(mg->nv), kThreads, 0, s>>>(mg->nv, mg->rank.p, mg->x.p, scores_dev);
-    NWG_LAUNCH_CHECK();
-  } else if (scores_dev && !small) {
-    NWG_HIP(hipMemcpyAsync(scores_dev, mg->x.p, mg->nv * 4, hipMemcpyDeviceToDevice, s));
+  auto solve = [&] {
+    NWG_HIP(hipEventRecord(ctx->ev0, s));
+    if (small) small_enqueue(s, S, mg->max_n, mg->max_nnz, 0, max_iters);
+    else run_segment(ctx, mg->caps, 0, key, enqueue);
+    NWG_HIP(hipEventRecord(ctx->ev1, s));
+    NWG_HIP(hipMemcpyAsync(acc.data(), mg->acc.p, max_iters * G * 8ull, hipMemcpyDeviceToHost, s));
+    if (scores_dev && !small && mg->rank.p) {
+      multi_out_kernel<<<grid1(mg->nv), kThreads, 0, s>>>(mg->nv, mg->rank.p, mg->x.p, scores_dev);
+      NWG_LAUNCH_CHECK();
+    } else if (scores_dev && !small) {
+      NWG_HIP(hipMemcpyAsync(scores_dev, mg->x.p, mg->nv * 4, hipMemcpyDeviceToDevice, s));
+    }
+    NWG_HIP(hipStreamSynchronize(s));
+  };
+  solve();
+  if (small && *S.cut) {  // the item sweep adds up what fixed point was too coarse for
+    small = false;
+    solve();
   }
-  NWG_HIP(hipStreamSynchronize(s));
   float ms = 0.f;
   NWG_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   uint64_t max_it = 0;

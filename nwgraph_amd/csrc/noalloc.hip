@@ -231,7 +231,7 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
   const bool items = item_count(n, nnz) <= kNaMaxItems && damping >= 0.f && damping <= 1.f;
   // a small graph's one launch looks at the flags itself (257 vertices, 20 sweeps: 80 to 60 us without
   // the wait in between)
-  const bool small = items && small_fits(n, nnz, false);
+  bool small = items && small_fits(n, nnz, false);
   check_device_csc(s, n, nnz, csc_ptr, csc_idx, outdeg, outdeg ? nullptr : cdeg, &scratch_mem, !small);
   const uint32_t* deg = outdeg ? outdeg : cdeg;  // counted: build_degrees, common.hpp:110-121
 
@@ -264,7 +264,9 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
     S.bad_mail = ctx->mail + kMailWords;
     S.acc = acc;
     S.mail = ctx->mail;
+    S.cut = ctx->mail + kMailCut;
     S.threshold = P.threshold;
+    *S.cut = 0ull;
     NWG_HIP(hipEventRecord(ctx->ev0, s));
     uint64_t k0 = 0;
     do {
@@ -275,7 +277,9 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
     NWG_HIP(hipEventRecord(ctx->ev1, s));
     NWG_HIP(hipStreamSynchronize(s));
     csc_verdict(ctx->mail[kMailWords], ctx->mail[kMailWords + 1]);
-  } else if (items) {
+    small = *S.cut == 0ull;  // else the item sweep adds up what fixed point was too coarse for
+  }
+  if (items && !small) {
     ItemParams I{};
     uint4* desc = reinterpret_cast<uint4*>(base + kOffDesc);
     I.desc = desc;
@@ -304,7 +308,7 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
     }
     if (max_iters) items_enqueue_fold(s, I, 0, (uint32_t)(max_iters - 1), ctx->mail);
     NWG_HIP(hipEventRecord(ctx->ev1, s));
-  } else {
+  } else if (!items) {
     NWG_HIP(hipEventRecord(ctx->ev0, s));
     na_init_kernel<<<(uint32_t)ceil_div(std::max<uint64_t>(n, max_iters), kNaThreads), kNaThreads, 0, s>>>(
         n, deg, init, scores, c0, acc, max_iters);

@@ -239,7 +239,8 @@ inline uint64_t segment_end(uint64_t start, uint64_t max_iters, uint64_t first) 
 }
 
 constexpr uint64_t kMailWords = 8192;  // of nwg_ctx::mail for L1 changes; longer solves copy.  Two
-                                       // more words take a solve's check of its inputs
+                                       // more words take a solve's check of its inputs, and one
+constexpr uint64_t kMailCut = kMailWords + 2;  // whether a one-workgroup solve was cut short of bits
 
 // Identity of a captured sweep loop: re-capture when any of it changes.
 struct CaptureKey {

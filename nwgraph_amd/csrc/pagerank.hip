@@ -1026,7 +1026,7 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
   double sweep_ms = 0.0;
   uint64_t launched = max_iters;
   std::vector<hipEvent_t> evs;
-  const bool small = items && sched == PrSchedule::kJacobi && !timing && small_fits(n, g->nnz, false);
+  bool small = items && sched == PrSchedule::kJacobi && !timing && small_fits(n, g->nnz, false);
   const bool class_kernels = !items && (!g->plan.bl.built || sched == PrSchedule::kDelta);
   unsigned long long* const mail = !class_kernels && max_iters <= kMailWords ? ctx->mail : nullptr;
   // scores in the caller's numbering
@@ -1062,9 +1062,11 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     sp.tele = personalised ? reinterpret_cast<const TeleCheck*>(st.tcheck.p) + kTeleBlocks : nullptr;
     sp.acc = st.acc.p;
     sp.mail = mail;
+    sp.cut = ctx->mail + kMailCut;
     sp.threshold = (double)threshold;
+    *sp.cut = 0ull;
   }
-  if (!timing) {
+  auto solve = [&] {
     CaptureKey key;
     key.ptrs[0] = st.x.p;
     key.ptrs[1] = st.contrib0.p;
@@ -1119,6 +1121,9 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
       }
     }
     NWG_HIP(hipEventRecord(ctx->ev1, s));
+  };
+  if (!timing) {
+    solve();
   } else {
     evs.resize(2 * max_iters + 4);
     for (auto& e : evs) NWG_HIP(hipEventCreate(&e));
@@ -1132,10 +1137,13 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     NWG_HIP(hipEventRecord(ctx->ev1, s));
   }
   std::vector<unsigned long long> acc(std::max<uint64_t>(max_iters, 1));
-  if (!mail)
-    NWG_HIP(hipMemcpyAsync(acc.data(), st.acc.p, max_iters * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-  if (!small) copy_out();
-  NWG_HIP(hipStreamSynchronize(s));
+  auto finish = [&] {
+    if (!mail)
+      NWG_HIP(hipMemcpyAsync(acc.data(), st.acc.p, max_iters * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    if (!small) copy_out();
+    NWG_HIP(hipStreamSynchronize(s));
+  };
+  finish();
   if (timing && personalised) {
     try {
       check_teleport();
@@ -1145,6 +1153,12 @@ void pagerank_run(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float d
     }
   }
   check_teleport();
+  if (small && *sp.cut) {  // the item sweep adds up what fixed point was too coarse for
+    small = false;
+    launched = max_iters;
+    solve();
+    finish();
+  }
   // sweeps that were not launched changed nothing
   if (mail) std::copy(mail, mail + launched, acc.begin());
   NWG_HIP(hipEventElapsedTime(&ms_total, ctx->ev0, ctx->ev1));

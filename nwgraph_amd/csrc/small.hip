@@ -161,6 +161,7 @@ __global__ __launch_bounds__(NT) void small_solve_kernel(SmallParams P, uint64_t
   const float init = (float)(1.0 / n);  // page_rank.hpp:93
   float x[kR], b[kR];
   uint32_t dg[kR];
+  CutNote cut;
 #pragma unroll
   for (uint32_t r = 0; r < kR; ++r) {
     const uint32_t i = tid + r * NT;
@@ -171,7 +172,9 @@ __global__ __launch_bounds__(NT) void small_solve_kernel(SmallParams P, uint64_t
       dg[r] = P.deg[r0 + i];
       b[r] = P.basev ? P.basev[r0 + i] : P.base;
       x[r] = k0 ? P.x[r0 + i] : init;
-      q[i] = quantize(x[r] / (float)dg[r]);
+      const float c = x[r] / (float)dg[r];
+      q[i] = quantize(c);
+      cut.note(c);
     }
   }
   if (tid == 0) q[H::kRows] = 0ull;
@@ -194,7 +197,9 @@ __global__ __launch_bounds__(NT) void small_solve_kernel(SmallParams P, uint64_t
           const float xn = __builtin_fmaf(P.damp, z, b[r]);  // page_rank.hpp:133-135
           err += quantize(fabsf(xn - x[r]));  // in units of 2^-60
           x[r] = xn;
-          q[i] = quantize(xn / (float)dg[r]);
+          const float c = xn / (float)dg[r];
+          q[i] = quantize(c);
+          cut.note(c);
         }
       }
       err = wave_sum(err);
@@ -216,6 +221,7 @@ __global__ __launch_bounds__(NT) void small_solve_kernel(SmallParams P, uint64_t
     P.acc[k * P.ngraphs + g] = 0ull;
     if (P.mail) P.mail[k] = 0ull;
   }
+  if (__syncthreads_or(cut.cuts()) && tid == 0) *P.cut = 1ull;
   const bool write = P.out && !(P.tele && !teleport_ok(*P.tele));
 #pragma unroll
   for (uint32_t r = 0; r < kR; ++r) {
@@ -259,8 +265,13 @@ __global__ __launch_bounds__(NT) void small_weighted_kernel(SmallWeighted P, uin
   typename H::Lane L;
   H::setup(S, L, P.rp, n);
   uint64_t k = k0;
+  CutNote cut;
   while (k < k1) {
-    H::prefix(S, L, [&](uint32_t t) { return quantize_signed(w[t] * H::at(xs, ids, t), qs); });
+    H::prefix(S, L, [&](uint32_t t) {
+      const float f = w[t] * H::at(xs, ids, t);
+      cut.note(f);
+      return quantize_signed(f, qs);
+    });
     __syncthreads();
     double err = 0.0;
 #pragma unroll
@@ -291,6 +302,7 @@ __global__ __launch_bounds__(NT) void small_weighted_kernel(SmallWeighted P, uin
     P.err[k] = 0.0;
     if (P.mail) P.mail[2 + k] = 0ull;
   }
+  if (__syncthreads_or(cut.cuts(qs)) && tid == 0) *P.cut = 1ull;
   if (P.mail && tid < 2) P.mail[tid] = P.scale[tid];
 #pragma unroll
   for (uint32_t r = 0; r < kR; ++r) {

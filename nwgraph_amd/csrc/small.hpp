@@ -37,6 +37,7 @@ struct SmallParams {
   unsigned long long* bad_mail;
   unsigned long long* acc;   // [k * ngraphs + graph]: L1 change of sweep k, fixed point; 0 once stopped
   unsigned long long* mail;  // nullable, one graph: acc[k] there too
+  unsigned long long* cut;   // set to 1 when fixed point cut bits off some contribution
   double threshold;
 };
 
@@ -55,10 +56,13 @@ struct SmallWeighted {
   const int* qshift;
   double* err;            // [k]: L1 change of sweep k; 0 once stopped
   unsigned long long* mail;         // nullable: the scales' two words, then err
+  unsigned long long* cut;          // set to 1 when fixed point cut bits off some product
   const unsigned long long* scale;
   double threshold;
   const double* thr_scale;  // nullable: the stop compares with threshold * *thr_scale
 };
+
+// A solve that reports a cut is no answer: the item sweep is, which adds rows up once more where it shows.
 
 // Sweeps per launch: a solve of any length is cut into launches of bounded time.
 constexpr uint64_t kSmallSweeps = 1024;

@@ -518,11 +518,17 @@ struct WSolve {
 // one graph per segment; base and y0 must be buffers that stay the same from call to call.  st.scale
 // holds the solve's WScale.  Between segments the host reads the sweeps' changes.  `then` queues
 // what follows the solve; with eager it is queued behind every segment before the changes are
-// read, so that a solve that ends in its first segment waits for the device once.  False when b
-// was not finite (an exact sweep is then no answer).
+// read, so that a solve that ends in its first segment waits for the device once.  one: a small graph's
+// solve is one workgroup's.
+enum class WEnd {
+  kDone,
+  kNotFinite,  // b was not finite: an exact sweep is then no answer
+  kCut,        // the one workgroup's fixed point was too coarse: the item sweep is not
+};
 template <class F>
-static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std::unique_ptr<Captured>>& caps,
-                        const WSolve& q, WSweep kind, const BinnedLayout* L, nwg_pr_info* info, bool eager, F&& then) {
+static WEnd fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std::unique_ptr<Captured>>& caps,
+                        const WSolve& q, WSweep kind, const BinnedLayout* L, nwg_pr_info* info, bool one, bool eager,
+                        F&& then) {
   hipStream_t s = ctx->stream;
   const uint32_t n = g->n;
   const uint64_t max_iters = q.max_iters;
@@ -669,7 +675,7 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
   key.extra = (relative ? 1u : 0u) | (q.y0 ? 0u : 2u) | ((uint32_t)kind << 2);
   const uint64_t first = kind == WSweep::kBinned ? kSegFirstBinned : kSegFirst;
   // a small graph: all sweeps in one launch
-  const bool small = kind == WSweep::kItems && small_fits(n, g->nnz, false);
+  const bool small = one && kind == WSweep::kItems && small_fits(n, g->nnz, false);
   SmallWeighted sp{};
   if (small) {
     sp.rp = q.rp;
@@ -685,6 +691,8 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
     sp.qshift = qshift;
     sp.err = st.err.p;
     sp.mail = mail;
+    sp.cut = ctx->mail + kMailCut;
+    *sp.cut = 0ull;
     sp.scale = reinterpret_cast<const unsigned long long*>(st.scale.p);
     sp.threshold = (double)q.threshold;
     sp.thr_scale = thr_scale;
@@ -715,7 +723,8 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
       std::memcpy(&sc, mail, sizeof sc);
       std::memcpy(h.data() + k0, mail + 2 + k0, (k1 - k0) * sizeof(double));
     }
-    if (kind != WSweep::kPull && !sc.finite) return false;
+    if (kind != WSweep::kPull && !sc.finite) return WEnd::kNotFinite;
+    if (small && *sp.cut) return WEnd::kCut;
     if (relative) stop = (double)q.threshold * sc.scale;
     bool ended = k1 >= max_iters;
     for (uint64_t k = k0; k < k1; ++k)
@@ -739,7 +748,7 @@ static bool fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
     if (info->error_trace)
       for (uint64_t k = 0; k < iters && k < info->error_trace_len; ++k) info->error_trace[k] = h[k];
   }
-  return true;
+  return WEnd::kDone;
 }
 
 static WState& wstate(nwg_graph* g) {
@@ -800,8 +809,11 @@ static void weighted_solve(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<s
                            const WSolve& q, nwg_pr_info* info, F&& then) {
   const WSweep kind = weighted_sweep(g, q.damping);
   const BinnedLayout* L = kind == WSweep::kBinned ? weighted_layout(ctx->stream, g, st, q.csr) : nullptr;
-  if (!fixed_point(ctx, g, st, caps, q, kind, L, info, kind == WSweep::kItems, then))
-    (void)fixed_point(ctx, g, st, caps, q, WSweep::kPull, nullptr, info, false, then);
+  const bool eager = kind == WSweep::kItems;
+  WEnd end = fixed_point(ctx, g, st, caps, q, kind, L, info, true, eager, then);
+  if (end == WEnd::kCut) end = fixed_point(ctx, g, st, caps, q, kind, L, info, false, eager, then);
+  if (end == WEnd::kNotFinite)
+    (void)fixed_point(ctx, g, st, caps, q, WSweep::kPull, nullptr, info, false, false, then);
 }
 
 void wpr_forward(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float* x_dev, float damping, float threshold,
