@@ -588,7 +588,7 @@ __device__ __forceinline__ void item_row_sums(const RowSumParams& P, uint32_t b0
     uint32_t wt[K];
     item_ids<K>(reinterpret_cast<const uint32_t*>(P.src), P.nnz, b0 + q0, e1, wt);
 #pragma unroll
-    for (int t = 0; t < K; ++t) val[t] = (double)P.gather[u[t]] * (double)__uint_as_float(wt[t]);
+    for (int t = 0; t < K; ++t) val[t] = (double)(P.d * P.gather[u[t]]) * (double)__uint_as_float(wt[t]);
   } else {
 #pragma unroll
     for (int t = 0; t < K; ++t) val[t] = (double)P.src[u[t]];
@@ -646,9 +646,11 @@ __device__ __forceinline__ void row_sum_out(const RowSumParams& P, const RowSumO
     o.out[u] = __builtin_isinf(f) ? __builtin_nanf("") : f;  // past the floats: the weights it divides would be 0
     return;
   }
-  const double x = (double)o.x[u], norm = (double)o.norm[u];
-  // a source without out-edges has no edge that reads its pair
-  o.ab[u] = make_float2((float)(x / norm), (float)(x * ((double)o.d * s) / norm));
+  // a source without out-edges has no edge that reads its pair; a quotient past the floats stays finite, as
+  // a source of one edge multiplies it by 0
+  float a = o.x[u] / o.norm[u];
+  if (__builtin_isinf(a) && o.norm[u] != 0.f && !__builtin_isinf(o.x[u])) a = __builtin_copysignf(3.402823466e38f, a);
+  o.ab[u] = make_float2(a, (float)s);
   if (o.gv) o.gv[u] = o.omd * P.gather[u];
 }
 

@@ -84,13 +84,14 @@ struct WItemParams {
 
 // Row sums of a compressed structure over its items, s_u = sum of a value per entry q:
 //   gather == null  src[perm[q]]
-//   else            gather[col[q]] * src[q], d times
+//   else            (d gather[col[q]]) * src[q]
 struct RowSumParams {
   const uint4* desc;
   const uint32_t* rp;
   const uint32_t* idx;  // perm or col; 16-byte aligned
   const float* src;     // 16-byte aligned
   const float* gather;
+  float d;
   uint32_t n;
   uint32_t nnz;
   uint32_t count;
@@ -98,14 +99,14 @@ struct RowSumParams {
   double* tail;         // count: and of the one that goes on after it
 };
 // what becomes of s_u: out[u] = s_u, or with gather
-//   ab[u] = {x[u] / norm[u], x[u] * d * s_u / norm[u]} and (nullable) gv[u] = omd * gather[u]
+//   ab[u] = {x[u] / norm[u], s_u} and (nullable) gv[u] = omd * gather[u]
 struct RowSumOut {
   float* out;
   const float* x;
   const float* norm;
   float2* ab;
   float* gv;
-  float d, omd;
+  float omd;
 };
 
 // items of a CSC of n rows and nnz entries

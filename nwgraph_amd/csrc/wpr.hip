@@ -350,9 +350,10 @@ __global__ __launch_bounds__(kThreads) void edge_grad_kernel(uint64_t nnz, const
 }
 
 // The raw-weight gradient of edge p from u = col[p]:
-//   (d lambda_row x_u - t_u) / s_u,  t_u = sum_j d lambda_j x_u w(u->j),
-// as d lambda_row * (x_u / s_u) - t_u / s_u with both quotients made once per source (ab): one
-// gather of 8 bytes per edge.  Edge gradient, row sums over a gathered copy and chain rule as
+//   (d lambda_row x_u - t_u) / s_u,  t_u = x_u m_u,  m_u = sum_j d lambda_j w(u->j),
+// as (x_u / s_u) * (d lambda_row - m_u) with quotient and sum made once per source (ab): one gather of 8
+// bytes per edge, and exactly 0 where the source has no other edge (w = 1, m_u = d lambda_row), as the
+// three passes below gave.  Edge gradient, row sums over a gathered copy and chain rule as
 // three passes took 885 us for 16 M edges on MI355X (the row sums 647: two scattered reads per edge,
 // long rows one load at a time); row sums over items with the products made in place and this
 // pass take 206 us.
@@ -360,10 +361,11 @@ __global__ __launch_bounds__(kThreads) void raw_grad_kernel(uint64_t nnz, const 
                                                             const uint32_t* __restrict__ col, float d,
                                                             const float* __restrict__ lambda,
                                                             const float2* __restrict__ ab, float* __restrict__ gw) {
+#pragma clang fp contract(off)  // the difference is of the rounded products that m_u adds up
   const uint64_t p = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
   if (p >= nnz) return;
   const float2 q = ab[col[p]];
-  gw[p] = __builtin_fmaf(d * lambda[row[p]], q.x, -q.y);
+  gw[p] = q.x * (d * lambda[row[p]] - q.y);
 }
 
 __global__ __launch_bounds__(kThreads) void scale_kernel(uint32_t n, float a, const float* __restrict__ src,
@@ -430,7 +432,7 @@ static const WItems& ensure_items(hipStream_t s, nwg_graph* g, bool csr) {
 
 // s_u over the CSR's rows (items.hip, RowSumParams)
 static void csr_row_sums(hipStream_t s, nwg_graph* g, const uint32_t* idx, const float* src, const float* gather,
-                         const RowSumOut& out) {
+                         float d, const RowSumOut& out) {
   const WItems& it = ensure_items(s, g, true);
   DevBuf<double> pieces(2ull * it.count);
   RowSumParams R{};
@@ -439,6 +441,7 @@ static void csr_row_sums(hipStream_t s, nwg_graph* g, const uint32_t* idx, const
   R.idx = idx;
   R.src = src;
   R.gather = gather;
+  R.d = d;
   R.n = g->n;
   R.nnz = (uint32_t)g->nnz;
   R.count = it.count;
@@ -463,7 +466,7 @@ void weights_set(hipStream_t s, nwg_graph* g, const float* w_dev, bool normalize
   if (normalize) {
     RowSumOut o{};
     o.out = g->w_rowsum.p;
-    csr_row_sums(s, g, g->csr_to_csc.p, g->w_raw.p, nullptr, o);
+    csr_row_sums(s, g, g->csr_to_csc.p, g->w_raw.p, nullptr, 0.f, o);
     if (nnz)
       normalise_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, g->csc_idx.p, g->w_raw.p, g->w_rowsum.p, g->w_csc.p,
                                                        bad.p + 1);
@@ -878,9 +881,8 @@ void wpr_backward(nwg_ctx* ctx, nwg_graph* g, const float* x_dev, const float* g
       o.norm = g->w_rowsum.p;
       o.ab = st.ab.p;
       o.gv = gv_dev;
-      o.d = damping;
       o.omd = 1.0f - damping;
-      csr_row_sums(s, g, g->csr_idx.p, g->w_csr.p, st.lambda.p, o);
+      csr_row_sums(s, g, g->csr_idx.p, g->w_csr.p, st.lambda.p, damping, o);
       raw_grad_kernel<<<grid1(nnz), kThreads, 0, s>>>(nnz, st.row_of.p, g->csc_idx.p, damping, st.lambda.p, st.ab.p,
                                                       gw_dev);
     } else {
