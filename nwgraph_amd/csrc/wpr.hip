@@ -806,13 +806,13 @@ static void prepare_scale(hipStream_t s, WState& st, uint32_t n, const float* v,
 }
 
 // solves q with the graph's sweep, or with the pull sweep when b was not finite (which shows the NaN /
-// infinity as the reference would)
+// infinity as the reference would).  again: `then` can be queued more than once.
 template <class F>
 static void weighted_solve(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std::unique_ptr<Captured>>& caps,
-                           const WSolve& q, nwg_pr_info* info, F&& then) {
+                           const WSolve& q, nwg_pr_info* info, bool again, F&& then) {
   const WSweep kind = weighted_sweep(g, q.damping);
   const BinnedLayout* L = kind == WSweep::kBinned ? weighted_layout(ctx->stream, g, st, q.csr) : nullptr;
-  const bool eager = kind == WSweep::kItems;
+  const bool eager = again && kind == WSweep::kItems;
   WEnd end = fixed_point(ctx, g, st, caps, q, kind, L, info, true, eager, then);
   if (end == WEnd::kCut) end = fixed_point(ctx, g, st, caps, q, kind, L, info, false, eager, then);
   if (end == WEnd::kNotFinite)
@@ -837,7 +837,7 @@ void wpr_forward(nwg_ctx* ctx, nwg_graph* g, const float* teleport_dev, float* x
   q.threshold = threshold;
   q.max_iters = max_iters;
   q.out = x_dev;
-  weighted_solve(ctx, g, st, st.cap_fwd, q, info, [] {});
+  weighted_solve(ctx, g, st, st.cap_fwd, q, info, true, [] {});
   NWG_HIP(hipStreamSynchronize(s));
 }
 
@@ -874,7 +874,7 @@ void wpr_backward(nwg_ctx* ctx, nwg_graph* g, const float* x_dev, const float* g
     NWG_LAUNCH_CHECK();
   }
   if (edges && raw) st.ab.ensure(n);
-  weighted_solve(ctx, g, st, st.cap_adj, q, info, [&] {
+  weighted_solve(ctx, g, st, st.cap_adj, q, info, gv_dev != x_dev, [&] {
     if (edges && raw) {
       RowSumOut o{};
       o.x = x_dev;

@@ -40,3 +40,30 @@ def test_only_out_edge_has_no_gradient(ctx, n, plan):
     a = x.astype(np.float64)[col] / s[col]
     assert np.all(np.abs(gw - a * (dl - mean))[~single] <= (8 * u * size * a)[~single])
     g.close()
+
+
+@pytest.mark.parametrize("raw", [True, False])
+@pytest.mark.parametrize("n", [400, 6000])
+def test_teleport_gradient_over_the_scores(ctx, n, raw):
+    """grad_teleport may be written where the scores were, over one segment of sweeps and over several, and
+    when the solve starts again with another sweep (a gradient of one vertex that is not finite)."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    src, dst = rng.integers(0, n, 6 * n).astype(np.uint32), rng.integers(0, n, 6 * n).astype(np.uint32)
+    g = ctx.graph_from_edges(n, src, dst)
+    g.set_weights(rng.uniform(0.1, 1.0, g.nnz).astype(np.float32))
+    x0, _ = g.wpr_forward(None, D, 0.0, 15)
+    for sweeps, bad in ((10, False), (45, False), (10, True)):
+        c = rng.normal(size=n).astype(np.float32)
+        if bad:
+            c[3] = np.inf
+        want_w, want_v, _ = g.wpr_backward(x0, c, D, 0.0, sweeps, raw_weights=raw)
+        x, cd = torch.from_numpy(x0).cuda(), torch.from_numpy(c).cuda()
+        gw = torch.zeros(g.nnz, device="cuda")
+        torch.cuda.synchronize()
+        g.wpr_backward_device(x.data_ptr(), cd.data_ptr(), gw.data_ptr(), x.data_ptr(), D, 0.0, sweeps,
+                              raw_weights=raw)
+        assert np.array_equal(gw.cpu().numpy(), want_w, equal_nan=True)
+        assert np.array_equal(x.cpu().numpy(), want_v, equal_nan=True)
+    g.close()
