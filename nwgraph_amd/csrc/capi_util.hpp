@@ -11,9 +11,12 @@
 namespace nwg {
 
 // A failed call may leave work in flight on memory its unwinding has put back into the
-// context's pool: wait for it before the next call can take that memory.
+// context's pool: wait for it before the next call can take that memory.  Not on a stream the caller
+// records a graph on: nothing of this call runs there, and a wait would end the recording.
 inline void wait_after_failure(nwg_ctx* ctx) {
   if (!ctx || !ctx->stream) return;
+  hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &recording) == hipSuccess && recording != hipStreamCaptureStatusNone) return;
   (void)hipStreamSynchronize(ctx->stream);
   (void)hipGetLastError();
 }
