@@ -92,6 +92,7 @@ void nwg_destroy(nwg_ctx* ctx) {
 
 int nwg_set_stream(nwg_ctx* ctx, void* stream) {
   if (!ctx) return NWG_EINVAL;
+  std::lock_guard<std::mutex> turn(ctx->mu);
   ctx->stream = stream ? static_cast<hipStream_t>(stream) : ctx->own_stream;
   return NWG_OK;
 }

@@ -21,8 +21,11 @@ inline void wait_after_failure(nwg_ctx* ctx) {
   (void)hipGetLastError();
 }
 
+// Calls on one context take turns: they share its stream, events, recording stream, kept memory and mail.
 template <class F>
 int guarded(nwg_ctx* ctx, F&& f) {
+  std::unique_lock<std::mutex> turn;
+  if (ctx) turn = std::unique_lock<std::mutex>(ctx->mu);
   PoolScope scope(ctx ? ctx->pool : nullptr);
   try {
     f();

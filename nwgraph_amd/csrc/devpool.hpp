@@ -10,8 +10,10 @@
 // calls of that context, whose device work is ordered by the context's stream; calls wait for
 // their work before they return (also when they fail: guarded()), so a block that comes back
 // after the stream was changed has no work left on it.  Objects that outlive a call are
-// destroyed after the device is idle.  The lists are locked: threads may share a context's
-// objects.  Bounds: the pool keeps at most 1/64 of the device's memory in free blocks, of which those
+// destroyed after the device is idle.  The lists are locked: objects are destroyed outside a call's
+// turn on its context.
+//
+// Bounds: the pool keeps at most 1/64 of the device's memory in free blocks, of which those
 // given back longest ago make room for new ones (the largest first instead: once a program has solved
 // graphs of many sizes, every build of the 67 M-edge graph gave its own blocks away, 27 ms against 4),
 // gives all of them back when an allocation fails or the context is destroyed, and keeps nothing

@@ -370,9 +370,9 @@ struct nwg_ctx {
   hipStream_t stream = nullptr;
   hipStream_t capture_stream = nullptr;  // used only to record HIP graphs
   std::string last_error;
-  std::mutex mu;
+  std::mutex mu;  // held by a call on the context (guarded())
   // host memory the device writes: a solve's last kernels leave its L1 changes here, so that the host
-  // reads them after the wait it makes anyway, with no copy
+  // reads them after the wait it makes anyway, with no copy.  One call at a time uses it (mu)
   unsigned long long* mail = nullptr;
   std::shared_ptr<nwg::DevPool> pool;  // device memory kept between this context's calls
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
