@@ -1,11 +1,13 @@
 // autotune.cpp -- picks the sweep plan (degree-bin cutoffs, hub split, cache hints)
 // of a graph by timing candidate plans on the device with HIP events.
 //
-// Search: coordinate descent over the pull sweep's parameters from the default plan, one
+// Search: coordinate descent over the pull sweep's parameters from the default plan (the item
+// sweep; cutoffs of its own ask for the row classes, and only those have cache hints), one
 // parameter at a time, each candidate timed over a few sweeps (launched one by one, each
 // bracketed by events); then the binned sweep in both numberings, with its cache hints and
-// bin size; then the best pull plan and the best binned plan timed again as whole captured
-// 20-sweep solves (median of 7), and the faster one kept.
+// bin size, which is named throughout (left open, the plan may run the item sweep); then the best pull
+// plan and the best binned plan timed again as whole captured 20-sweep solves (median of 7), and
+// the faster one kept.
 // Results are cached per (log2 in-degree histogram, n, nnz, device) for the process
 // and, if NWG_TUNE_CACHE names a file, appended there and reloaded by later processes.
 #include <hip/hip_runtime.h>
@@ -112,13 +114,13 @@ double time_plan_sweeps(nwg_ctx* ctx, nwg_graph* g, uint64_t iters) {
 }
 
 // Median device time per sweep of whole solves (the captured HIP graph of `iters` sweeps,
-// as a caller runs it), after one solve that captures the graph and warms the caches.
+// as a caller runs it), after one solve whose launches go out one by one and one that captures them.
 // Small graphs are launch-bound, where per-sweep event timing of one-by-one launches is
 // noisy and measures launch gaps the captured loop does not have.
 static double time_plan_solve(nwg_ctx* ctx, nwg_graph* g, uint64_t iters, int reps) {
   nwg_pr_info info{};
   DevBuf<float> out(g->n);
-  pagerank_run(ctx, g, nullptr, 0.85f, -1.0f, iters, &info, out.p);
+  for (int r = 0; r < 2; ++r) pagerank_run(ctx, g, nullptr, 0.85f, -1.0f, iters, &info, out.p);
   std::vector<double> t;
   for (int r = 0; r < reps; ++r) {
     pagerank_run(ctx, g, nullptr, 0.85f, -1.0f, iters, &info, out.p);
@@ -165,19 +167,21 @@ nwg_plan_params autotune_plan(nwg_ctx* ctx, nwg_graph* g) {
       }
     }
   };
-  // the pull sweep: numbering, then its row-class cutoffs, hub split, slicing and hints
+  // the pull sweep: numbering, then its row-class cutoffs, hub split and slicing, and the row
+  // classes' hints
   try_field(&nwg_plan_params::relabel, {0, 1});
-  try_field(&nwg_plan_params::stream_hints, {0, 1, 2});
   try_field(&nwg_plan_params::short_max, {0, 2, 4, 8, 16, 32});
   try_field(&nwg_plan_params::group_max, {16, 32, 64, 128, 256, 512, 1024});
   try_field(&nwg_plan_params::hub_min, {2048, 4096, 8192, 16384, 32768, 65536, 262144});
   try_field(&nwg_plan_params::hub_segment, {1024, 2048, 4096, 8192, 16384});
   try_field(&nwg_plan_params::slice_min, {0, 33, 65, 129, 257, 1025});
   try_field(&nwg_plan_params::short_max, {0, 2, 4, 8, 16, 32});
+  if (!plan_takes_items(best, g)) try_field(&nwg_plan_params::stream_hints, {0, 1, 2});
   const nwg_plan_params pull = best;
   // the binned sweep ignores the row-class cutoffs; only the numbering matters
   nwg_plan_params binned = pull, b0 = pull;
   binned.binned = b0.binned = 1;
+  binned.bin_bits = b0.bin_bits = 13;
   binned.relabel = 1;
   b0.relabel = 0;
   if (eval(b0) < eval(binned)) binned = b0;
@@ -199,11 +203,9 @@ nwg_plan_params autotune_plan(nwg_ctx* ctx, nwg_graph* g) {
   // and its bin size (2^14-row bins: fewer pairs, one bin-pass workgroup per CU)
   {
     nwg_plan_params c = binned;
-    c.bin_bits = 13;
-    double b13 = eval(c);
+    const double b13 = eval(c);
     c.bin_bits = 14;
     if (eval(c) < b13) binned = c;
-    else binned.bin_bits = 13;
   }
   // the two winners, timed again as whole captured solves (median of 7)
   plan_build(s, g, pull);

@@ -543,6 +543,8 @@ void note_max_outdeg(hipStream_t s, nwg_graph* g);
 // whether some vertex has far more out-edges than the average (false below kSkewEdges)
 bool skewed_degrees(const nwg_graph* g);
 nwg_plan_params default_plan_for(const nwg_graph* g);
+// whether a plan's sweeps run over items (items.hip)
+bool plan_takes_items(const nwg_plan_params& p, const nwg_graph* g);
 // binned sweep (binned.hip)
 // w (device, CSC order of a, nullable): also lay out the entries' weights (L.bw)
 // bin_bits: rows per bin, log2 (13 or 14; 0 = by size)

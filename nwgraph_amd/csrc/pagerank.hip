@@ -611,7 +611,7 @@ static void validate_params(const nwg_plan_params& p) {
 // uniform random with 1.0 M edges (10 per row) 175 / 193, 2.2 M (9) 300 / 272, 2.0 M (20) 256 / 183, 2.8 M (8) 359 /
 // 369, 3.2 M (16) 366 / 224, 3.5 M (7) 450 / 467, 4.0 M (8) 487 / 407, 4.9 M (7) 594 / 612, 6.0 M (12) 650 / 323;
 // lattice with 3.4 M (3.4) 292 / 565.
-static bool plan_takes_items(const nwg_plan_params& p, const nwg_graph* g) {
+bool plan_takes_items(const nwg_plan_params& p, const nwg_graph* g) {
   const uint64_t nnz = g->nnz;
   const nwg_plan_params d = default_plan_params();
   if (p.short_max != d.short_max || p.group_max != d.group_max || p.hub_min != d.hub_min ||
