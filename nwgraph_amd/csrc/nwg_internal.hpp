@@ -348,6 +348,8 @@ struct PprState {
   uint32_t n_heavy = 0, n_parts = 0;
   uint32_t n_parts_split = 0;  // n_parts with the long rows split by source slice
   bool whole = false;          // built without
+  bool even = false;           // no row has far more in-edges than the average: light rows are longer
+  uint32_t light_max = 0;      // rows of at most so many in-edges take the row path
   uint32_t row_end = 0;  // one past the last row with in-edges (active numbering)
   // heavy rows' in-edges regrouped by (source slice, row), and the pieces they are cut into: first
   // edge, partial sum; each row's partials; each slice's pieces

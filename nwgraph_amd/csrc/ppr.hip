@@ -12,7 +12,7 @@
 //
 // Work split per sweep (one launch + one finishing launch), k-tile after k-tile, with T / 4 lanes of 16
 // bytes per gathered slice (a lane group):
-//   heavy pieces     at most 32 in-edges of one row with more than kLightMax, of one source slice
+//   heavy pieces     at most 32 in-edges of one row with more than light_max, of one source slice
 //                    (an eighth of the sources, one XCD's); the pieces of one row in a
 //                    workgroup leave one partial vector
 //   row workgroups   (1024/T) lane groups x 1 or 4 consecutive rows, over a compacted copy of the
@@ -49,7 +49,6 @@ constexpr uint32_t kErrLanes = 8;
 constexpr uint32_t kPiece = 32;
 struct PprParams {
   const uint32_t* rp;
-  const uint32_t* col;
   const uint32_t* lrp;   // light CSC: rows with in-degree <= light_max, heavy rows empty
   const uint32_t* lcol;
   const uint32_t* degflag;   // out-degree | kSeedFlag when the row is a seed of some vector
@@ -62,9 +61,9 @@ struct PprParams {
   uint32_t n, k;
   uint32_t tiles, kt_shift;  // k-tiles and log2 of their width
   float damp;
-  uint32_t light_max, hub_segment;  // rows with in-degree <= light_max take the row path
+  uint32_t light_max;        // rows with in-degree <= light_max take the row path
   uint32_t row_blocks;       // workgroups of rows per k-tile
-  uint32_t n_hub_rows, n_hub_segs;
+  uint32_t n_hub_rows;
   const uint32_t* hub_rows;
   const uint32_t* part_ptr;    // heavy row h's partials: hub_part rows [part_ptr[h], part_ptr[h + 1])
   const uint32_t* hcol;        // heavy rows' in-edges, source slice by source slice, row by row in each
@@ -184,7 +183,10 @@ __device__ __forceinline__ double slot_reduce(const double (&e)[4], double* lds 
 // k = 64: 142 M line reads, 72 M of them past the L2, 1.6 ms: 81 G lines/s, 9.3 TB/s into the L2s), whatever
 // the tile, the wavefronts in flight or the L2's hit rate.  1.79 ms with one lane per float, rows of
 // up to 256 in-edges on the row path and slices by the low bits of the source.
-template <int T, int kR>
+// kEven: the graph's rows are light up to kLightMaxWhole in-edges, which are added up kU at a time, then
+// these sums (rows of 180, error against 64 bits with one running sum 2.0e-7, so 9.6e-8, in pieces of 32
+// 8.7e-8).  Where light rows end at 32 it gains nothing and costs up to 9 % (RMAT-22, k = 64, 36.9 against 33.6 ms).
+template <int T, int kR, bool kEven>
 __global__ __launch_bounds__(kThreads) void ppr_sweep_kernel(PprParams P) {
   constexpr uint32_t G = T / 4;              // lanes per edge
   constexpr uint32_t kGroups = kThreads / G;
@@ -226,9 +228,11 @@ __global__ __launch_bounds__(kThreads) void ppr_sweep_kernel(PprParams P) {
   const float* __restrict__ ctile = P.cin + (uint64_t)tile * P.n * T;
   // Sum of the contributions of the edges ids[p .. end), in edge order; c: the ids at p + vl, and
   // at the end those at end + vl (up to `last`).  kU gathers in flight, and the next ids with them.
-  // Every lane gathers: lanes of converged vectors share their group's line, and edges past the
-  // end are those of the next row, or source 0.  Loads that a lane condition skipped made the
-  // compiler drain every load in flight before each add.
+  // Every lane gathers: lanes of converged vectors share their group's line, and past the end the last edge
+  // is gathered again, whose line is there or under way (the next row's edges, gathered in its
+  // place, were lines of their own: uniform random, 900,000 rows of 10, k = 64, 5.37 against 5.07 ms, 2 M,
+  // k = 32, 6.21 against 5.89; RMAT-22, k = 64, 33.9 against 33.6).  Loads that a lane condition skipped made
+  // the compiler drain every load in flight before each add.
   auto walk = [&](const uint32_t* __restrict__ ids, uint32_t p, uint32_t end, uint32_t last, uint32_t& c) {
     Four z{{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll 1
@@ -241,11 +245,21 @@ __global__ __launch_bounds__(kThreads) void ppr_sweep_kernel(PprParams P) {
         Four v[kU];
 #pragma unroll
         for (uint32_t t = 0; t < kU; ++t)
-          v[t] = load4(ctile + (uint64_t)(uint32_t)__shfl((int)c, (int)(q0 + t), (int)G) * T + vl * 4);
+          v[t] = load4(ctile + (uint64_t)(uint32_t)__shfl((int)c, (int)min(q0 + t, m - 1), (int)G) * T + vl * 4);
+        if constexpr (kEven) {
+          Four r{{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (uint32_t t = 0; t < kU; ++t)
+          for (uint32_t t = 0; t < kU; ++t)
 #pragma unroll
-          for (int a = 0; a < 4; ++a) z.v[a] += q0 + t < m ? v[t].v[a] : 0.f;
+            for (int a = 0; a < 4; ++a) r.v[a] += q0 + t < m ? v[t].v[a] : 0.f;
+#pragma unroll
+          for (int a = 0; a < 4; ++a) z.v[a] += r.v[a];
+        } else {
+#pragma unroll
+          for (uint32_t t = 0; t < kU; ++t)
+#pragma unroll
+            for (int a = 0; a < 4; ++a) z.v[a] += q0 + t < m ? v[t].v[a] : 0.f;
+        }
       }
       c = cn;
     }
@@ -642,11 +656,30 @@ __global__ __launch_bounds__(kThreads) void light_len_kernel(uint32_t n, const u
   }
 }
 
-// *end = one past the last row with in-edges
-__global__ __launch_bounds__(kThreads) void row_end_kernel(uint32_t n, const uint32_t* __restrict__ rp,
-                                                           uint32_t* __restrict__ end) {
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  if (i < n && rp[i + 1] > rp[i]) atomicMax(end, i + 1);
+// out[0] = one past the last row with in-edges, out[1] = most in-edges of a row.  One atomic each per workgroup.
+__global__ __launch_bounds__(kThreads) void row_stats_kernel(uint32_t n, const uint32_t* __restrict__ rp,
+                                                             uint32_t* __restrict__ out) {
+  __shared__ uint32_t ends[kThreads / 64], mosts[kThreads / 64];
+  uint32_t end = 0, most = 0;
+  for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kThreads) {
+    const uint32_t d = rp[i + 1] - rp[i];
+    if (d) end = (uint32_t)i + 1;
+    most = max(most, d);
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    end = max(end, (uint32_t)__shfl_xor((int)end, o, 64));
+    most = max(most, (uint32_t)__shfl_xor((int)most, o, 64));
+  }
+  if (lane_id() == 0) {
+    ends[threadIdx.x / 64] = end;
+    mosts[threadIdx.x / 64] = most;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicMax(out, max(max(ends[0], ends[1]), max(ends[2], ends[3])));
+    atomicMax(out + 1, max(max(mosts[0], mosts[1]), max(mosts[2], mosts[3])));
+  }
 }
 
 __global__ __launch_bounds__(kThreads) void light_copy_kernel(uint32_t n, const uint32_t* __restrict__ rp,
@@ -729,7 +762,11 @@ static void build_heavy_slices(hipStream_t s, const ActiveCsc& a, uint32_t n, ui
 // 0.56 / 0.60 / 0.71 / 1.1, uniform random 20,000 with k = 33 0.77 / 0.60 / 0.60 / 0.60, RMAT-20 with k = 10
 // 5.8 / 5.8 / 6.5 / 13.3 and with k = 64 7.4 / 8.0 / 9.2 / 12.5, RMAT-22 in degree order with k = 64 35.1 /
 // 34.7 / 34.2 / 34.8: a lane group walks its rows in rounds of 8 gathers, and the longest light row
-// decides where the graph is small or not in degree order.
+// decides where the graph is small or not in degree order.  Where no row stands out (most in-edges at
+// most 64 + 8 times the average) light rows go up to kLightMaxWhole: the pieces would be nearly all rows
+// (uniform random, ms with the cut at 32 / 256: 200,000 rows of 40, k = 64, 3.08 / 2.52, 100,000 of 200, k = 32,
+// 1.96 / 1.67, 900,000 of 20, k = 40, 6.80 / 6.71, 20,000 of 16, k = 33, 0.39 / 0.37) -- but for tiles of 8,
+// where a light row is two lanes' (50,000 of 100, k = 8, 0.38 / 0.40).
 // Rows of fewer than kSplitMin in-edges stay in one slice (64 / 128 / 256: RMAT-20, k = 10, 5.8 / 6.5 / 8.3; all
 // rows whole 10).  Denser graphs split longer rows only, so that the partial vectors take no more
 // than some three times a contribution array, and a solve whose partials would take more than
@@ -741,7 +778,7 @@ constexpr uint64_t kPartBytes = 16ull << 30;
 
 static void build_rows(hipStream_t s, const ActiveCsc& a, uint32_t n, uint64_t nnz, uint32_t tile, bool whole,
                        PprState& st) {
-  const uint32_t light_max = whole ? kLightMaxWhole : kLightMax;
+  const uint32_t light_max = whole || st.even ? kLightMaxWhole : kLightMax;
   const uint32_t big = whole ? ~0u : (uint32_t)std::max<uint64_t>(kSplitMin, 4 * nnz / n);
   build_heavy_slices(s, a, n, light_max + 1, big, tile, kSlices, st);
   DevBuf<uint32_t> len(n);
@@ -757,6 +794,7 @@ static void build_rows(hipStream_t s, const ActiveCsc& a, uint32_t n, uint64_t n
   NWG_LAUNCH_CHECK();
   NWG_HIP(hipStreamSynchronize(s));
   st.whole = whole;
+  st.light_max = light_max;
 }
 
 // A lane group's light rows: 4 (their ids and old contributions loaded ahead) once that leaves the
@@ -781,14 +819,17 @@ void ppr_run(nwg_ctx* ctx, nwg_graph* g, uint32_t k, const std::vector<uint32_t>
   const uint32_t kq = (uint32_t)ceil_div(k, 4);
   if (st.seg_version != g->plan_version || st.seg_tile != tile) {
     st.seg_version = 0;
+    DevBuf<uint32_t> stats(2);
+    uint32_t h[2] = {0, 0};
+    NWG_HIP(hipMemsetAsync(stats.p, 0, 8, s));
+    row_stats_kernel<<<std::min(grid1(n), 512u), kThreads, 0, s>>>(n, a.ptr, stats.p);
+    NWG_LAUNCH_CHECK();
+    NWG_HIP(hipMemcpyAsync(h, stats.p, 8, hipMemcpyDeviceToHost, s));
+    NWG_HIP(hipStreamSynchronize(s));
+    st.row_end = h[0];
+    st.even = tile >= 16 && (double)h[1] <= 64.0 + 8.0 * (double)g->nnz / n;
     build_rows(s, a, n, g->nnz, tile, false, st);
     st.n_parts_split = st.n_parts;
-    DevBuf<uint32_t> end(1);
-    NWG_HIP(hipMemsetAsync(end.p, 0, 4, s));
-    row_end_kernel<<<grid1(n), kThreads, 0, s>>>(n, a.ptr, end.p);
-    NWG_LAUNCH_CHECK();
-    NWG_HIP(hipMemcpyAsync(&st.row_end, end.p, 4, hipMemcpyDeviceToHost, s));
-    NWG_HIP(hipStreamSynchronize(s));
     st.seg_version = g->plan_version;
     st.seg_tile = tile;
   }
@@ -798,7 +839,6 @@ void ppr_run(nwg_ctx* ctx, nwg_graph* g, uint32_t k, const std::vector<uint32_t>
     build_rows(s, a, n, g->nnz, tile, whole, st);
     st.seg_version = g->plan_version;
   }
-  const uint32_t light_max = whole ? kLightMaxWhole : kLightMax;
   const uint32_t n_heavy = st.n_heavy;
   // seed entries sorted by (row, vector); rows in the active numbering
   std::vector<std::pair<uint32_t, uint32_t>> ent;
@@ -865,7 +905,6 @@ void ppr_run(nwg_ctx* ctx, nwg_graph* g, uint32_t k, const std::vector<uint32_t>
 
   PprParams P{};
   P.rp = a.ptr;
-  P.col = a.idx;
   P.lrp = st.lrp.p;
   P.lcol = st.lcol.p;
   P.degflag = st.degflag.p;
@@ -878,7 +917,7 @@ void ppr_run(nwg_ctx* ctx, nwg_graph* g, uint32_t k, const std::vector<uint32_t>
   P.tiles = tiles;
   P.kt_shift = (uint32_t)__builtin_ctz(tile);
   P.damp = damping;
-  P.light_max = light_max;
+  P.light_max = st.light_max;
   P.row_blocks = row_blocks;
   P.n_hub_rows = n_heavy;
   P.hub_rows = st.heavy_rows.p;
@@ -929,8 +968,10 @@ void ppr_run(nwg_ctx* ctx, nwg_graph* g, uint32_t k, const std::vector<uint32_t>
     const uint32_t grid = P.tile_blocks * tiles;  // 0 only for a graph without edges
     auto sweep = [&](auto t) {
       constexpr int T = decltype(t)::value;
-      if (grid && kr == 4) ppr_sweep_kernel<T, 4><<<grid, kThreads, 0, s>>>(P);
-      else if (grid) ppr_sweep_kernel<T, 1><<<grid, kThreads, 0, s>>>(P);
+      if (grid && !st.even && kr == 4) ppr_sweep_kernel<T, 4, false><<<grid, kThreads, 0, s>>>(P);
+      else if (grid && !st.even) ppr_sweep_kernel<T, 1, false><<<grid, kThreads, 0, s>>>(P);
+      else if (grid && kr == 4) ppr_sweep_kernel<T, 4, true><<<grid, kThreads, 0, s>>>(P);
+      else if (grid) ppr_sweep_kernel<T, 1, true><<<grid, kThreads, 0, s>>>(P);
       ppr_finish_kernel<T><<<fin, kThreads, 0, s>>>(P, tiles);
     };
     if (tile == 8) sweep(std::integral_constant<int, 8>());
