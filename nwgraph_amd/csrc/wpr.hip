@@ -718,7 +718,8 @@ static WEnd fixed_point(nwg_ctx* ctx, nwg_graph* g, WState& st, std::vector<std:
                                              q.out);
     NWG_LAUNCH_CHECK();
     if (eager) then();
-    if (!mail && k0 == 0) NWG_HIP(hipMemcpyAsync(&sc, st.scale.p, sizeof sc, hipMemcpyDeviceToHost, s));
+    if (!mail && k0 == 0 && (relative || kind != WSweep::kPull))
+      NWG_HIP(hipMemcpyAsync(&sc, st.scale.p, sizeof sc, hipMemcpyDeviceToHost, s));
     if (!mail && k1 > k0)
       NWG_HIP(hipMemcpyAsync(h.data() + k0, st.err.p + k0, (k1 - k0) * sizeof(double), hipMemcpyDeviceToHost, s));
     NWG_HIP(hipStreamSynchronize(s));
