@@ -50,17 +50,17 @@ void* DevPool::take(size_t bytes, size_t* size) {
     }
   }
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, want);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    {
-      std::lock_guard<std::mutex> lk(mu_);
-      trim_locked();
-    }
-    e = hipMalloc(&p, want);
+  if (hipMalloc(&p, want) == hipSuccess) return p;
+  (void)hipGetLastError();
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    trim_locked();
   }
-  NWG_HIP(e);
-  return p;
+  const hipError_t e = hipMalloc(&p, want);
+  if (e == hipSuccess) return p;
+  (void)hipGetLastError();  // reported here; a caller may go on without the block
+  throw Error(e == hipErrorOutOfMemory ? NWG_ENOMEM : NWG_EHIP,
+              "hipMalloc of " + std::to_string(want) + " bytes failed: " + hipGetErrorString(e));
 }
 
 void DevPool::give(void* p, size_t size) noexcept {

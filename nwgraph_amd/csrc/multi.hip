@@ -200,7 +200,8 @@ namespace nwg {
 // as given: 256 graphs of 2^10 to 2^18 vertices (213 M edges) binned 4.92 / 5.42 ms; 12 of 2^12 to 2^18 (9.5 M)
 // binned 1.08 / 1.35, items 0.78 / 0.84.  Smaller graphs gain nothing: 90 of 2^10 to 2^16 (28 M) binned 1.51 /
 // 1.42, 96 of 2^12 (7 M) items 0.55 / 0.53.  Unions below kOrderUnion edges keep their numbering (the copy
-// takes longer than it saves over a few solves), and so do those whose sort would take 16 GiB of keys.
+// takes longer than it saves over a few solves), and so do those whose sort would take 16 GiB of keys
+// or finds no memory.
 constexpr uint64_t kOrderRows = 1ull << 16;
 constexpr uint64_t kOrderUnion = 1ull << 20, kOrderUnionMax = 1ull << 30;
 static void order_by_degree(hipStream_t s, nwg_multigraph* mg, const std::vector<uint64_t>& eoff) {
@@ -272,7 +273,11 @@ nwg_multigraph* multigraph_create(nwg_ctx* ctx, uint32_t ngraphs, nwg_graph* con
   }
   const uint32_t ne32 = (uint32_t)mg->ne;
   NWG_HIP(hipMemcpyAsync(mg->rp.p + mg->nv, &ne32, 4, hipMemcpyHostToDevice, s));
-  order_by_degree(s, mg.get(), eoff);
+  try {
+    order_by_degree(s, mg.get(), eoff);
+  } catch (const Error& e) {
+    if (e.code != NWG_ENOMEM) throw;
+  }
   mg->x.alloc(mg->nv);
   mg->c0.alloc(mg->nv);
   mg->c1.alloc(mg->nv);
