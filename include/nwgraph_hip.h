@@ -100,7 +100,8 @@ typedef struct nwg_plan_params {
 int nwg_version(void);
 /* Create a context on HIP device `device`.  Creates its own stream.  Calls on one context from
  * several threads take turns.  The context keeps device memory that its calls have released, up
- * to 1/64 of the device's, for later calls; nwg_destroy gives it back. */
+ * to 1/64 of the device's, for later calls; it is given back by nwg_destroy, and when an allocation
+ * of any context on the device fails. */
 int nwg_create(nwg_ctx** out, int device);
 void nwg_destroy(nwg_ctx* ctx);
 /* Run subsequent work on `stream` (a hipStream_t; NULL = the context's own stream). */

@@ -64,7 +64,7 @@ int nwg_create(nwg_ctx** out, int device) {
     NWG_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->mail), (nwg::kMailCut + 1) * 8, hipHostMallocDefault));
     size_t total_bytes = 0;
     NWG_HIP(hipDeviceTotalMem(&total_bytes, device));
-    ctx->pool = std::make_shared<nwg::DevPool>(total_bytes / 64);
+    ctx->pool = std::make_shared<nwg::DevPool>(device, total_bytes / 64);
   });
   if (rc != NWG_OK) {
     nwg_destroy(ctx);

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <new>
+#include <vector>
 
 #include "nwg_internal.hpp"
 
@@ -13,6 +14,10 @@ namespace nwg {
 namespace {
 
 thread_local std::shared_ptr<DevPool> t_pool;
+
+// every pool, for trim_all
+std::mutex g_pools_mu;
+std::vector<DevPool*> g_pools;
 
 // below 1 MiB powers of two, from there whole MiB: few sizes, little waste
 size_t block_size(size_t bytes) {
@@ -28,6 +33,30 @@ size_t block_size(size_t bytes) {
 const std::shared_ptr<DevPool>& current_pool() { return t_pool; }
 PoolScope::PoolScope(std::shared_ptr<DevPool> p) : prev_(std::move(t_pool)) { t_pool = std::move(p); }
 PoolScope::~PoolScope() { t_pool = std::move(prev_); }
+
+DevPool::DevPool(int device, size_t limit) : device_(device), limit_(limit) {
+  std::lock_guard<std::mutex> lk(g_pools_mu);
+  g_pools.push_back(this);
+}
+
+DevPool::~DevPool() {
+  {
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    g_pools.erase(std::find(g_pools.begin(), g_pools.end(), this));
+  }
+  close();
+}
+
+// hipFree waits for the device, which must not happen while another thread records a graph
+void DevPool::trim_all(int device) {
+  std::lock_guard<std::mutex> recording(capture_mutex());
+  std::lock_guard<std::mutex> lk(g_pools_mu);
+  for (DevPool* p : g_pools) {
+    if (p->device_ != device) continue;
+    std::lock_guard<std::mutex> own(p->mu_);
+    p->trim_locked();
+  }
+}
 
 void DevPool::trim_locked() noexcept {
   for (auto& b : free_) (void)hipFree(b.second.p);
@@ -52,10 +81,7 @@ void* DevPool::take(size_t bytes, size_t* size) {
   void* p = nullptr;
   if (hipMalloc(&p, want) == hipSuccess) return p;
   (void)hipGetLastError();
-  {
-    std::lock_guard<std::mutex> lk(mu_);
-    trim_locked();
-  }
+  trim_all(device_);
   const hipError_t e = hipMalloc(&p, want);
   if (e == hipSuccess) return p;
   (void)hipGetLastError();  // reported here; a caller may go on without the block

@@ -16,8 +16,8 @@
 // Bounds: the pool keeps at most 1/64 of the device's memory in free blocks, of which those
 // given back longest ago make room for new ones (the largest first instead: once a program has solved
 // graphs of many sizes, every build of the 67 M-edge graph gave its own blocks away, 27 ms against 4),
-// gives all of them back when an allocation fails or the context is destroyed, and keeps nothing
-// after that.
+// gives all of them back when an allocation of any context on the device fails or its own is destroyed,
+// and keeps nothing after that.
 #pragma once
 
 #include <cstddef>
@@ -30,8 +30,8 @@ namespace nwg {
 
 class DevPool {
  public:
-  explicit DevPool(size_t limit) : limit_(limit) {}
-  ~DevPool() { close(); }
+  DevPool(int device, size_t limit);
+  ~DevPool();
   DevPool(const DevPool&) = delete;
   DevPool& operator=(const DevPool&) = delete;
   // a block of at least bytes (> 0) on the current device; *size receives its size.  Throws Error.
@@ -42,7 +42,9 @@ class DevPool {
 
  private:
   void trim_locked() noexcept;
+  static void trim_all(int device);
   std::mutex mu_;
+  const int device_;
   struct Free {
     void* p;
     uint64_t given;  // when: blocks given back longest ago go first

@@ -1,6 +1,8 @@
 """Memory that only makes a call faster is no reason to refuse it: with too little left for the sort of a union's
-degree order the union keeps its numbering.  The device's memory is taken by one allocation that is
-never written."""
+degree order the union keeps its numbering, and what one context keeps for later calls goes to another that
+needs it.  The device's memory is taken by allocations that are never written."""
+import time
+
 import numpy as np
 import pytest
 
@@ -17,8 +19,12 @@ class _Taken:
 
         torch.cuda.synchronize()
         torch.cuda.empty_cache()
-        free, _ = torch.cuda.mem_get_info()
-        self.block = torch.empty(free - leave, dtype=torch.uint8, device="cuda")
+        self.blocks = []
+        for _ in range(8):  # what was freed before comes back after a while
+            free, _ = torch.cuda.mem_get_info()
+            if free > leave:
+                self.blocks.append(torch.empty(free - leave, dtype=torch.uint8, device="cuda"))
+            time.sleep(0.1)
 
     def __enter__(self):
         return self
@@ -26,7 +32,7 @@ class _Taken:
     def __exit__(self, *exc):
         import torch
 
-        self.block = None
+        self.blocks = None
         torch.cuda.empty_cache()
 
 
@@ -48,3 +54,21 @@ def test_union_without_room_for_its_degree_order():
     c.close()
     for g in graphs:
         g.close()
+
+
+def test_memory_kept_by_another_context():
+    a, b = nwgraph_amd.Context(0), nwgraph_amd.Context(0)
+    m = 80 << 20
+    ptr = np.full(1001, m, np.uint32)
+    ptr[0] = 0
+    col = np.zeros(m, np.uint32)
+    with _Taken(1290 << 20):
+        a.rmat(21, 16, seed=1).close()  # leaves 1130 MB of temporaries with a
+        g = b.graph_from_csc(ptr, col)  # 320 MB of ids
+        assert g.nnz == m and g.csc()[2][0] == m
+        g.close()
+    x = a.rmat(12, 16, seed=1)
+    assert abs(x.pagerank()[0].sum() - 1) < 0.5
+    x.close()
+    a.close()
+    b.close()
