@@ -15,9 +15,12 @@ namespace {
 
 thread_local std::shared_ptr<DevPool> t_pool;
 
-// every pool, for trim_all
+// every pool, for trim_all (never destroyed: a context may outlive this file's statics)
 std::mutex g_pools_mu;
-std::vector<DevPool*> g_pools;
+std::vector<DevPool*>& pools() {
+  static auto* all = new std::vector<DevPool*>();
+  return *all;
+}
 
 // below 1 MiB powers of two, from there whole MiB: few sizes, little waste
 size_t block_size(size_t bytes) {
@@ -36,13 +39,13 @@ PoolScope::~PoolScope() { t_pool = std::move(prev_); }
 
 DevPool::DevPool(int device, size_t limit) : device_(device), limit_(limit) {
   std::lock_guard<std::mutex> lk(g_pools_mu);
-  g_pools.push_back(this);
+  pools().push_back(this);
 }
 
 DevPool::~DevPool() {
   {
     std::lock_guard<std::mutex> lk(g_pools_mu);
-    g_pools.erase(std::find(g_pools.begin(), g_pools.end(), this));
+    pools().erase(std::find(pools().begin(), pools().end(), this));
   }
   close();
 }
@@ -51,7 +54,7 @@ DevPool::~DevPool() {
 void DevPool::trim_all(int device) {
   std::lock_guard<std::mutex> recording(capture_mutex());
   std::lock_guard<std::mutex> lk(g_pools_mu);
-  for (DevPool* p : g_pools) {
+  for (DevPool* p : pools()) {
     if (p->device_ != device) continue;
     std::lock_guard<std::mutex> own(p->mu_);
     p->trim_locked();

@@ -1,10 +1,10 @@
 // items.hip -- PageRank sweep over edge-balanced work items, one launch per sweep.
 //
 // The sweep is the reference's (include/nwgraph/algorithms/page_rank.hpp:121-147, Jacobi form
-// experimental/algorithms/page_rank.hpp:397-430).  It serves graphs whose contributions stay in
-// L2, where a sweep is bound by launches, by load latency and by its longest rows, not by bytes:
-// row classes with a launch each take up to seven launches per sweep, and one wave on a row of
-// thousands of in-edges outlasts everything else.
+// experimental/algorithms/page_rank.hpp:397-430).  It is the pull sweep of every size, and made for graphs
+// whose contributions stay in L2, where a sweep is bound by launches, by load latency and by its longest
+// rows, not by bytes: row classes with a launch each take up to seven launches per sweep, and one wave
+// on a row of thousands of in-edges outlasts everything else.
 //
 // Row i starts at unit D(i) = i + rp[i] of n + nnz units (one per edge, one per row), and item c
 // owns the units [c S, (c + 1) S), S = kSpan = 1020:
@@ -65,7 +65,7 @@ __device__ __forceinline__ uint32_t first_row_from(const uint32_t* __restrict__ 
 // One thread per item.  desc = {e0, e1, r0, rows | flags}: rows [r0, r0 + rows) are finished by
 // the item, their edges lie in [e0, e1) after the head piece (of row r0 - 1) and before the
 // tail piece (of row r0 + rows).
-__global__ __launch_bounds__(256) void item_desc_kernel(uint32_t n, uint64_t nnz, const uint32_t* __restrict__ rp,
+__global__ __launch_bounds__(256) void item_desc_kernel(uint32_t n, const uint32_t* __restrict__ rp,
                                                         uint32_t count, uint4* __restrict__ desc) {
   const uint32_t c = blockIdx.x * 256 + threadIdx.x;
   if (c >= count) return;
@@ -757,7 +757,7 @@ void row_sums_enqueue(hipStream_t s, const RowSumParams& P, const RowSumOut& o) 
 
 void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, uint4* desc) {
   const uint32_t count = item_count(n, nnz);
-  item_desc_kernel<<<(uint32_t)ceil_div(count, 256), 256, 0, s>>>(n, nnz, rp, count, desc);
+  item_desc_kernel<<<(uint32_t)ceil_div(count, 256), 256, 0, s>>>(n, rp, count, desc);
   NWG_LAUNCH_CHECK();
 }
 

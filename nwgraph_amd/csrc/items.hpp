@@ -92,7 +92,6 @@ struct RowSumParams {
   const float* src;     // 16-byte aligned
   const float* gather;
   float d;
-  uint32_t n;
   uint32_t nnz;
   uint32_t count;
   double* head;         // count: an item's piece of the long row begun before it

@@ -8,8 +8,11 @@
 //   err += |x_i' - x_i|  (float difference, double sum) (page_rank.hpp:134)
 //   contrib'_i = x_i' / (float)outdeg_i                 (page_rank.hpp:116,135)
 // contrib is double-buffered (read contrib[k&1], write contrib[(k+1)&1]); x is
-// updated in place (each row owns its entry).  One sweep is a short sequence of
-// launches, one per row class (degree-binned schedule):
+// updated in place (each row owns its entry).  Plans run the item sweep (items.hip), the binned sweep
+// (binned.hip) or, for small graphs, whole solves in one workgroup (small.hip).  The kernels here
+// serve plans with class cutoffs of their own, the delta schedule, and damping factors outside
+// [0, 1], which the exact sums of the others do not cover.  Their sweep is a short sequence
+// of launches, one per row class (degree-binned schedule):
 //   pr_tile_kernel    256 consecutive rows, one lane per row with in-degree <= short_max
 //   pr_group_kernel   rows listed per class, 4/8/16/32/64 lanes per row, butterfly reduction
 //   pr_sgroup_kernel  source-sliced rows (slice_min <= d < hub_min): workgroup b gathers

@@ -12,14 +12,17 @@
 // and, for raw weights normalised per source (w = w~ / s_u, s_u = sum_k w~(u->k)),
 //   dL/dw~(u->k) = (dL/dw(u->k) - sum_j dL/dw(u->j) w(u->j)) / s_u.
 //
-// Sweep schedule: the rows are cut into work items of up to 256 consecutive rows with at
-// most kItemNnz nonzeros (values staged in LDS; one lane per short row, one wave per row of
-// more than kLaneRow nonzeros) or one longer row
-// (whole-workgroup reduction); a persistent grid walks the items round-robin.
+// Sweeps (weighted_sweep): one workgroup for small graphs (small.hip), the item sweep (items.hip), the
+// binned sweep (binned.hip), all with exact fixed-point row sums; and the pull sweep here, in float, for
+// what their bound does not cover: weights that are negative, not normalised or undefined, a teleport or
+// gradient that is not finite, and large graphs whose plan is not binned.
 //
-// The L1 change of a sweep is summed in double with a fixed order: every workgroup stores
-// its partial, and the last workgroup to finish (a counter per sweep) adds all partials
-// in workgroup order and stores err[k].  The adjoint's changes have no a-priori bound (a
+// The pull sweep: the rows are cut into work items of up to 256 consecutive rows with at most
+// kItemNnz nonzeros (values staged in LDS; one lane per short row, one wave per row of more than
+// kLaneRow nonzeros) or one longer row (whole-workgroup reduction); a persistent grid walks the
+// items round-robin.  Its L1 change is summed in double with a fixed order: every workgroup stores
+// its partial, and the last workgroup to finish (a counter per sweep) adds all partials in
+// workgroup order and stores err[k] (the other sweeps' changes are doubles too).  The adjoint's changes have no a-priori bound (a
 // loss such as -sum log x gives |grad_x| ~ n), so a fixed-point accumulator of bounded
 // range could wrap; this sum cannot, and it does not depend on completion order, so the
 // sweep count is reproducible.
@@ -442,7 +445,6 @@ static void csr_row_sums(hipStream_t s, nwg_graph* g, const uint32_t* idx, const
   R.src = src;
   R.gather = gather;
   R.d = d;
-  R.n = g->n;
   R.nnz = (uint32_t)g->nnz;
   R.count = it.count;
   R.head = pieces.p;
