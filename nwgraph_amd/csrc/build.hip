@@ -469,8 +469,8 @@ void check_device_csc(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* p
   NWG_REQUIRE(wait || scratch, "the check's flags outlive it in the caller's memory only");
   if (given || deg) degrees_aligned(col);
   DevBuf<uint32_t> own_flags, own_part, own_counted;
-  uint32_t* flags = scratch ? scratch->flags : (own_flags.alloc(2), own_flags.p);
-  fill_u32_kernel<<<1, 256, 0, s>>>(flags, 2, 0u);
+  uint32_t* flags = scratch ? scratch->flags : (own_flags.alloc(3), own_flags.p);
+  fill_u32_kernel<<<1, 256, 0, s>>>(flags, 3, 0u);
   csc_check_kernel<<<grid_for(std::max<uint64_t>(nnz, n)), 256, 0, s>>>(n, nnz, ptr, col, flags);
   NWG_LAUNCH_CHECK();
   // the histograms count ids >= n nowhere, so they need not wait for the check above

@@ -21,9 +21,9 @@
 // difference of the prefix at its two ends.  The sums are exact integers, so the difference is
 // the row's exact sum: short and long rows cost the same, nothing diverges, and the result
 // depends on no order (fixed_point.hpp).  Where cut-off bits could show (scores far below the others:
-// long personalised solves, damping 1), a row is added up once more in double from its gathers.  Noting cut
-// bits and looking at the note takes 1 to 3 % of a sweep where none are (20 sweeps, RMAT-12 100.8 to 102.6 us,
-// RMAT-16 164.4 to 168.9).
+// long personalised solves, damping 1), a row is added up once more in double from its gathers.  The form
+// that looks for them takes 1 to 3 % longer (20 sweeps, RMAT-12 101.3 / 102.9 us, RMAT-16 @@ / 168.2), so it runs
+// where the base does not rule them out.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -66,7 +66,8 @@ __device__ __forceinline__ uint32_t first_row_from(const uint32_t* __restrict__ 
 // the item, their edges lie in [e0, e1) after the head piece (of row r0 - 1) and before the
 // tail piece (of row r0 + rows).
 __global__ __launch_bounds__(256) void item_desc_kernel(uint32_t n, const uint32_t* __restrict__ rp,
-                                                        uint32_t count, uint4* __restrict__ desc) {
+                                                        uint32_t count, uint4* __restrict__ desc,
+                                                        uint32_t* __restrict__ longest) {
   const uint32_t c = blockIdx.x * 256 + threadIdx.x;
   if (c >= count) return;
   const uint64_t u0 = (uint64_t)c * kSpan, u1 = u0 + kSpan;
@@ -83,6 +84,7 @@ __global__ __launch_bounds__(256) void item_desc_kernel(uint32_t n, const uint32
     --rows;
     flags |= kTailPiece;
     e1 = (uint32_t)(u1 - (r1 - 1));
+    if (longest) atomicMax(longest, p1 - rp[r1 - 1]);
   }
   desc[c] = make_uint4(e0, e1, r0, rows | flags);
 }
@@ -123,8 +125,8 @@ __device__ __forceinline__ void item_ids(const uint32_t* __restrict__ ids, uint3
 
 // K values per lane: inclusive fixed-point prefix of the edges [e0, e1), entry q of it for edge
 // b0 + q (b0 = e0 rounded down to 4; entries before e0 are 0).  w null: value cin[id]; else
-// w * cin[id] scaled by 2^qs.  cuts: per wave, whether some value lost bits.
-template <int K, bool W>
+// w * cin[id] scaled by 2^qs.  kLook: cuts, per wave, whether some value lost bits.
+template <int K, bool W, bool kLook>
 __device__ __forceinline__ void item_prefix(const uint32_t* __restrict__ col, const float* w, int qs,
                                             const float* cin, uint32_t nnz, uint32_t b0, uint32_t e0, uint32_t e1,
                                             unsigned long long* pre, unsigned long long* wsum, uint32_t* cuts) {
@@ -145,20 +147,21 @@ __device__ __forceinline__ void item_prefix(const uint32_t* __restrict__ col, co
     if constexpr (W) {
       const float f = __uint_as_float(wt[t]) * c[t];
       q = quantize_signed(f, qs);
-      cut.note(f);
+      if constexpr (kLook) cut.note(f);
     } else {
       q = quantize(c[t]);
-      cut.note(c[t]);
+      if constexpr (kLook) cut.note(c[t]);
     }
     s += (p >= e0 && p < e1) ? q : 0ull;
     v[t] = s;
   }
-  const uint64_t any_cut = __ballot(cut.cuts(qs));
+  uint64_t any_cut = 0;
+  if constexpr (kLook) any_cut = __ballot(cut.cuts(qs));
   unsigned long long inc = wave_inclusive_scan(s);
   unsigned long long off = inc - s;
   if (lane_id() == 63) {
     wsum[threadIdx.x >> 6] = inc;
-    cuts[threadIdx.x >> 6] = any_cut != 0;
+    if constexpr (kLook) cuts[threadIdx.x >> 6] = any_cut != 0;
   }
   __syncthreads();
 #pragma unroll
@@ -208,6 +211,7 @@ __device__ __forceinline__ void direct_long_sums(const uint32_t* __restrict__ co
 // of the item it starts in; true for the last piece, which gets the row's sum and leaves the
 // counters at 0 for the next sweep.  *start: the item the row starts in.  cut: in, whether a value of
 // this piece was cut; out, of any piece.
+template <bool kLook>
 __device__ __forceinline__ bool add_piece(unsigned long long* hsum, uint32_t* hcnt, uint32_t h, uint32_t hp0,
                                           uint32_t hp1, unsigned long long mine, unsigned long long* z,
                                           uint32_t* start, bool& cut) {
@@ -216,26 +220,30 @@ __device__ __forceinline__ bool add_piece(unsigned long long* hsum, uint32_t* hc
   *start = a;
   unsigned long long old = __hip_atomic_fetch_add(hsum + a, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // in the word of the count, so before it
-  if (cut) (void)__hip_atomic_fetch_or(hcnt + a, kCutRow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (kLook && cut) (void)__hip_atomic_fetch_or(hcnt + a, kCutRow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // the sum has been added (its old value is back) before the piece is counted
   asm volatile("s_waitcnt vmcnt(0)" : "+v"(old) : : "memory");
   const uint32_t counted = __hip_atomic_fetch_add(hcnt + a, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if ((counted & ~kCutRow) != b - a) return false;
-  cut = counted & kCutRow;
+  cut = kLook && (counted & kCutRow);
   *z = __hip_atomic_exchange(hsum + a, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(hcnt + a, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return true;
 }
 
 // the sum of a row's entries [a, b): s in fixed point, or in double where that is too coarse for it
+template <bool kLook>
 __device__ __forceinline__ float item_row_sum(const ItemParams& P, unsigned long long s, uint32_t a, uint32_t b,
                                               float base, const uint32_t* cuts) {
   const float z = dequantize(s);
-  if (__builtin_expect(item_cuts(cuts), 0) && sum_is_coarse(__builtin_fmaf(P.damp, z, base), b - a))
-    return (float)direct_sum<false>(P.col, nullptr, P.cin, a, b, 1);
+  if constexpr (kLook)
+    if (__builtin_expect(item_cuts(cuts), 0) && sum_is_coarse(__builtin_fmaf(P.damp, z, base), b - a))
+      return (float)direct_sum<false>(P.col, nullptr, P.cin, a, b, 1);
   return z;
 }
 
+// kLook: rows may be too small for the fixed point (looks)
+template <bool kLook>
 __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
   static_assert(kItemLanes == 64 && kNT == 256, "one lane counter per wavefront lane, four waves");
   __shared__ unsigned long long pre[9 * kNT];
@@ -271,8 +279,8 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
-  else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, false, kLook>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  else item_prefix<8, false, kLook>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
   ch = wave_sum(ch);
   if (blockIdx.x == 0) {
     if (threadIdx.x < 64) P.lanes[((P.iter + 1) % 3) * kItemLaneSlot + lane * kItemLanePad] = 0ull;
@@ -282,7 +290,7 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
   auto sum = [&](uint32_t a, uint32_t b) { return item_sum(pre, b0, a, b); };
   unsigned long long err = 0ull;
   for (uint32_t q = threadIdx.x; q < rows;) {
-    err += item_update(P, r0 + q, item_row_sum(P, sum(ra, rb), ra, rb, bv, cuts), xo, bv, dg);
+    err += item_update(P, r0 + q, item_row_sum<kLook>(P, sum(ra, rb), ra, rb, bv, cuts), xo, bv, dg);
     if ((q += kNT) >= rows) break;
     const uint32_t i = r0 + q;
     ra = P.rp[i];
@@ -296,15 +304,15 @@ __global__ __launch_bounds__(kNT) void pr_item_kernel(ItemParams P) {
   if (piece) {
     unsigned long long z;
     uint32_t a;
-    bool cut = item_cuts(cuts);
-    last = add_piece(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a, cut);
+    bool cut = kLook && item_cuts(cuts);
+    last = add_piece<kLook>(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a, cut);
     if (last) {
       hz = dequantize(z);
       hb = P.basev ? P.basev[h] : P.base;
       ask = cut && sum_is_coarse(__builtin_fmaf(P.damp, hz, hb), hp1 - hp0);
     }
   }
-  direct_long_sums<false>(P.col, nullptr, P.cin, hp0, hp1, ask, &hz);
+  if constexpr (kLook) direct_long_sums<false>(P.col, nullptr, P.cin, hp0, hp1, ask, &hz);
   if (last) err += item_update(P, h, hz, P.x[h], hb, P.deg[h]);
   err = wave_sum(err);
   if (lane == 0) wsum[threadIdx.x >> 6] = err;
@@ -333,6 +341,7 @@ __device__ __forceinline__ unsigned long long many_change(const ItemParams& P, c
 // vertices (0.4 M edges) 0.17 / 0.42 / 0.39, 12 of 2^12 to 2^18 (9.5 M) 0.87 / 4.7 / 1.53, 80 of 2^12 to 2^16
 // (18.7 M) 1.47 / 4.5 / 1.63.
 constexpr uint32_t kManyLocal = 64;
+template <bool kLook>
 __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyParams M) {
   __shared__ unsigned long long pre[9 * kNT];
   __shared__ unsigned long long wsum[kNT / 64];
@@ -375,8 +384,8 @@ __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyPar
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * kNT) item_prefix<4, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
-  else item_prefix<8, false>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, false, kLook>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  else item_prefix<8, false, kLook>(P.col, nullptr, 0, P.cin, P.nnz, b0, e0, e1, pre, wsum, cuts);
   if (g0 == g1 && done[0]) return;
   unsigned long long* const lane =
       P.lanes + P.iter % 3 * slot + (uint64_t)(blockIdx.x % kManyLanes) * many_stride(M.ngraphs);
@@ -393,7 +402,7 @@ __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyPar
     else atomicAdd(lane + g, e);
   };
   for (uint32_t q = threadIdx.x; q < rows;) {
-    if (!solved(rg)) add(rg, item_update(P, r0 + q, item_row_sum(P, sum(ra, rb), ra, rb, bv, cuts), xo, bv, dg));
+    if (!solved(rg)) add(rg, item_update(P, r0 + q, item_row_sum<kLook>(P, sum(ra, rb), ra, rb, bv, cuts), xo, bv, dg));
     if ((q += kNT) >= rows) break;
     const uint32_t i = r0 + q;
     ra = P.rp[i];
@@ -411,15 +420,15 @@ __global__ __launch_bounds__(kNT) void pr_item_many_kernel(ItemParams P, ManyPar
     hg = M.row_graph[h];
     unsigned long long z;
     uint32_t a;
-    bool cut = item_cuts(cuts);
-    last = !solved(hg) && add_piece(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a, cut);
+    bool cut = kLook && item_cuts(cuts);
+    last = !solved(hg) && add_piece<kLook>(P.hsum, P.hcnt, h, hp0, hp1, sum(max(hp0, e0), min(hp1, e1)), &z, &a, cut);
     if (last) {
       hz = dequantize(z);
       hb = P.basev[h];
       ask = cut && sum_is_coarse(__builtin_fmaf(P.damp, hz, hb), hp1 - hp0);
     }
   }
-  direct_long_sums<false>(P.col, nullptr, P.cin, hp0, hp1, ask, &hz);
+  if constexpr (kLook) direct_long_sums<false>(P.col, nullptr, P.cin, hp0, hp1, ask, &hz);
   if (last) add(hg, item_update(P, h, hz, P.x[h], hb, P.deg[h]));
   if (g0 == g1) {
     err = wave_sum(err);
@@ -496,8 +505,8 @@ __global__ __launch_bounds__(kNT) void wpr_item_kernel(WItemParams P) {
     hp1 = P.rp[h + 1];
   }
   const uint32_t b0 = e0 & ~3u;
-  if (e1 - b0 <= 4u * kNT) item_prefix<4, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum, cuts);
-  else item_prefix<8, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  if (e1 - b0 <= 4u * kNT) item_prefix<4, true, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum, cuts);
+  else item_prefix<8, true, true>(P.col, P.w, qs, P.xin, P.nnz, b0, e0, e1, pre, wsum, cuts);
   if (P.iter > 0 && !P.folded) {
     const double ch = witem_change(P, P.iter - 1, red);
     if (blockIdx.x == 0 && threadIdx.x == 0) P.err[P.iter - 1] = ch;
@@ -531,7 +540,7 @@ __global__ __launch_bounds__(kNT) void wpr_item_kernel(WItemParams P) {
   if (piece) {
     unsigned long long z;
     bool cut = item_cuts(cuts);
-    last = add_piece(P.hsum, P.hcnt, h, hp0, hp1, item_sum(pre, b0, max(hp0, e0), min(hp1, e1)), &z, &ha, cut);
+    last = add_piece<true>(P.hsum, P.hcnt, h, hp0, hp1, item_sum(pre, b0, max(hp0, e0), min(hp1, e1)), &z, &ha, cut);
     if (last) {
       hz = dequantize_signed(z, qs);
       hb = P.basev[h];
@@ -755,9 +764,9 @@ void row_sums_enqueue(hipStream_t s, const RowSumParams& P, const RowSumOut& o) 
   NWG_LAUNCH_CHECK();
 }
 
-void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, uint4* desc) {
+void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, uint4* desc, uint32_t* longest) {
   const uint32_t count = item_count(n, nnz);
-  item_desc_kernel<<<(uint32_t)ceil_div(count, 256), 256, 0, s>>>(n, rp, count, desc);
+  item_desc_kernel<<<(uint32_t)ceil_div(count, 256), 256, 0, s>>>(n, rp, count, desc, longest);
   NWG_LAUNCH_CHECK();
 }
 
@@ -767,8 +776,14 @@ void items_enqueue_init(hipStream_t s, const ItemParams& P, float init, float* c
   NWG_LAUNCH_CHECK();
 }
 
+// A row's result is at least its base, and no row of m entries is too small for the fixed point where that is
+// m * 2^-34 or more (sum_is_coarse): with the uniform teleport at damping 0.85, rows of an item's span in
+// graphs of up to 2.5 M vertices, rows of 65,536 in graphs of 39,000.
+static bool looks(float base, uint32_t longest) { return !(base >= (float)std::max(kSpan, longest) * 0x1p-34f); }
+
 void items_enqueue_sweep(hipStream_t s, const ItemParams& P) {
-  pr_item_kernel<<<P.count, kNT, 0, s>>>(P);
+  if (P.basev || looks(P.base, P.longest)) pr_item_kernel<true><<<P.count, kNT, 0, s>>>(P);
+  else pr_item_kernel<false><<<P.count, kNT, 0, s>>>(P);
   NWG_LAUNCH_CHECK();
 }
 
@@ -779,7 +794,8 @@ void items_many_enqueue_init(hipStream_t s, const ItemParams& P, const ManyParam
 }
 
 void items_many_enqueue_sweep(hipStream_t s, const ItemParams& P, const ManyParams& M) {
-  pr_item_many_kernel<<<P.count, kNT, 0, s>>>(P, M);
+  if (looks(M.least_base, P.longest)) pr_item_many_kernel<true><<<P.count, kNT, 0, s>>>(P, M);
+  else pr_item_many_kernel<false><<<P.count, kNT, 0, s>>>(P, M);
   NWG_LAUNCH_CHECK();
 }
 

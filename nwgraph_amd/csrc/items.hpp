@@ -35,6 +35,7 @@ struct ItemParams {
   unsigned long long* acc;   // per sweep: L1 change, fixed point
   uint32_t iter;
   double threshold;
+  uint32_t longest;          // in-edges of the longest row above an item's span (items_build), or 0
 };
 
 // Many graphs in one block-diagonal CSC: every row has its graph's base (ItemParams::basev), and every
@@ -47,6 +48,7 @@ __host__ __device__ constexpr uint32_t many_stride(uint32_t ngraphs) { return (n
 struct ManyParams {
   const uint32_t* row_graph;  // non-decreasing
   uint32_t ngraphs;
+  float least_base;           // of ItemParams::basev
 };
 
 // Where a segment of weighted sweeps leaves what the host reads: the solve's two words of scales, then
@@ -110,8 +112,9 @@ struct RowSumOut {
 
 // items of a CSC of n rows and nnz entries
 uint32_t item_count(uint32_t n, uint64_t nnz);
-// their descriptions (item_count of them) from the row pointers
-void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, uint4* desc);
+// their descriptions (item_count of them) from the row pointers; longest (nullable, 0 before): the most
+// in-edges of a row above an item's span.  Reads within rp[0 .. n] whatever it holds.
+void items_build(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* rp, uint4* desc, uint32_t* longest);
 // x = init, c0 (nullable) = init / outdeg, and the solve's counters cleared: acc[0 .. iters), the lanes,
 // hsum and hcnt (count each)
 void items_enqueue_init(hipStream_t s, const ItemParams& P, float init, float* c0, uint64_t iters);

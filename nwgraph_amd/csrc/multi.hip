@@ -182,6 +182,7 @@ struct nwg_multigraph {
   nwg::DevBuf<unsigned long long> ihsum, ilanes;
   nwg::DevBuf<uint32_t> ihcnt;
   uint32_t n_sweep_items = 0;
+  uint32_t longest = 0;  // ItemParams::longest
   uint64_t max_n = 0, max_nnz = 0;  // of one graph
   nwg::DevBuf<uint32_t> voff_dev;
   std::vector<std::unique_ptr<nwg::Captured>> caps;  // the solve's launches
@@ -290,7 +291,10 @@ nwg_multigraph* multigraph_create(nwg_ctx* ctx, uint32_t ngraphs, nwg_graph* con
   const std::vector<uint32_t> voff32(mg->voff.begin(), mg->voff.end());
   mg->voff_dev.alloc(ngraphs + 1);
   NWG_HIP(hipMemcpyAsync(mg->voff_dev.p, voff32.data(), (ngraphs + 1) * 4ull, hipMemcpyHostToDevice, s));
-  if (mg->n_sweep_items) items_build(s, (uint32_t)mg->nv, mg->ne, mg->rp.p, mg->idesc.p);
+  DevBuf<uint32_t> longest(1);
+  NWG_HIP(hipMemcpyAsync(longest.p, &mg->longest, 4, hipMemcpyHostToDevice, s));
+  if (mg->n_sweep_items) items_build(s, (uint32_t)mg->nv, mg->ne, mg->rp.p, mg->idesc.p, longest.p);
+  NWG_HIP(hipMemcpyAsync(&mg->longest, longest.p, 4, hipMemcpyDeviceToHost, s));
   NWG_HIP(hipStreamSynchronize(s));
   return mg.release();
 }
@@ -390,12 +394,13 @@ void multigraph_run(nwg_ctx* ctx, nwg_multigraph* mg, float damping, float thres
   I.n = (uint32_t)mg->nv;
   I.nnz = (uint32_t)mg->ne;
   I.count = mg->n_sweep_items;
+  I.longest = mg->longest;
   I.hsum = mg->ihsum.p;
   I.hcnt = mg->ihcnt.p;
   I.lanes = mg->ilanes.p;
   I.acc = mg->acc.p;
   I.threshold = (double)threshold;
-  const ManyParams M{mg->row_graph.p, G};
+  const ManyParams M{mg->row_graph.p, G, *std::min_element(gb.begin(), gb.end())};
   // every graph a workgroup of its own, all sweeps in one launch
   bool small = items && small_fits(mg->max_n, mg->max_nnz, true) && max_iters <= kSmallSweeps;
   SmallParams S{};

@@ -232,7 +232,15 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
   // a small graph's one launch looks at the flags itself (257 vertices, 20 sweeps: 80 to 60 us without
   // the wait in between)
   bool small = items && small_fits(n, nnz, false);
-  check_device_csc(s, n, nnz, csc_ptr, csc_idx, outdeg, outdeg ? nullptr : cdeg, &scratch_mem, !small);
+  check_device_csc(s, n, nnz, csc_ptr, csc_idx, outdeg, outdeg ? nullptr : cdeg, &scratch_mem, false);
+  uint4* const desc = reinterpret_cast<uint4*>(base + kOffDesc);
+  uint32_t found[3] = {0, 0, ~0u};  // the check's flags, and the longest row (a small graph's solve does not ask)
+  if (!small) {
+    if (items) items_build(s, n, nnz, csc_ptr, desc, flag + 2);  // in bounds whatever the CSC holds
+    NWG_HIP(hipMemcpyAsync(found, flag, sizeof found, hipMemcpyDeviceToHost, s));
+    NWG_HIP(hipStreamSynchronize(s));
+    csc_verdict(found[0], found[1]);
+  }
   const uint32_t* deg = outdeg ? outdeg : cdeg;  // counted: build_degrees, common.hpp:110-121
 
   NaParams P{};
@@ -277,11 +285,11 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
     NWG_HIP(hipEventRecord(ctx->ev1, s));
     NWG_HIP(hipStreamSynchronize(s));
     csc_verdict(ctx->mail[kMailWords], ctx->mail[kMailWords + 1]);
-    small = *S.cut == 0ull;  // else the item sweep adds up what fixed point was too coarse for
+    small = *S.cut == 0ull;
+    if (!small) items_build(s, n, nnz, csc_ptr, desc, nullptr);  // which adds up what fixed point was too coarse for
   }
   if (items && !small) {
     ItemParams I{};
-    uint4* desc = reinterpret_cast<uint4*>(base + kOffDesc);
     I.desc = desc;
     I.rp = csc_ptr;
     I.col = csc_idx;
@@ -297,7 +305,7 @@ void pagerank_noalloc(nwg_ctx* ctx, uint32_t n, uint64_t nnz, const uint32_t* cs
     I.lanes = reinterpret_cast<unsigned long long*>(base + kOffLanes);
     I.acc = acc;
     I.threshold = P.threshold;
-    items_build(s, n, nnz, csc_ptr, desc);
+    I.longest = found[2];
     NWG_HIP(hipEventRecord(ctx->ev0, s));
     items_enqueue_init(s, I, init, c0, max_iters);
     for (uint64_t k = 0; k < max_iters; ++k) {

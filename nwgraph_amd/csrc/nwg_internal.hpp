@@ -155,6 +155,7 @@ struct Plan {
   bool built = false;
   uint32_t n_items = 0;   // item sweep (items.hip): its items (0: not used)
   DevBuf<uint4> idesc;
+  uint32_t longest = 0;   // ItemParams::longest
   // row classes of the class kernels: built by the first solve that runs them
   bool classes = false;
   uint32_t n_tiles = 0;
@@ -464,7 +465,7 @@ void sorted_keys_to_csx(hipStream_t s, const uint64_t* keys, uint64_t m, uint32_
 void out_degrees_device(hipStream_t s, uint32_t n, uint64_t nnz, const uint32_t* col, uint32_t* deg);
 // Device memory check_device_csc works in when its caller cannot allocate.
 struct CscCheckScratch {
-  uint32_t* flags;    // 2 words
+  uint32_t* flags;    // 3 words, of which the last is only cleared
   uint32_t* counted;  // n words
   uint32_t* part;     // part_bytes of partial histograms
   uint64_t part_bytes;

@@ -633,10 +633,14 @@ void plan_build(hipStream_t s, nwg_graph* g, const nwg_plan_params& pp) {
   Plan pl;
   pl.params = pp;
   pl.n_tiles = (uint32_t)ceil_div(n, kThreads);
+  DevBuf<uint32_t> longest;
   if (plan_takes_items(pp, g)) {
     pl.n_items = item_count(n, g->nnz);
     pl.idesc.alloc(pl.n_items);
-    items_build(s, n, g->nnz, a.ptr, pl.idesc.p);
+    longest.alloc(1);
+    NWG_HIP(hipMemcpyAsync(longest.p, &pl.longest, 4, hipMemcpyHostToDevice, s));
+    items_build(s, n, g->nnz, a.ptr, pl.idesc.p, longest.p);
+    NWG_HIP(hipMemcpyAsync(&pl.longest, longest.p, 4, hipMemcpyDeviceToHost, s));
   } else if (pp.binned) {
     binned_build(s, a, n, g->nnz, pl.bl, true, nullptr, (int)pp.bin_bits);
   }
@@ -871,6 +875,7 @@ static ItemParams make_item_params(nwg_graph* g, PrState& st, const SweepParams&
   I.n = P.n;
   I.nnz = (uint32_t)g->nnz;
   I.count = g->plan.n_items;
+  I.longest = g->plan.longest;
   I.hsum = st.ihsum.p;
   I.hcnt = st.ihcnt.p;
   I.lanes = st.ilanes.p;

@@ -428,7 +428,7 @@ static const WItems& ensure_items(hipStream_t s, nwg_graph* g, bool csr) {
   if (!it.desc.n) {
     it.count = item_count(g->n, g->nnz);
     it.desc.alloc(it.count);
-    items_build(s, g->n, g->nnz, csr ? g->csr_ptr.p : g->csc_ptr.p, it.desc.p);
+    items_build(s, g->n, g->nnz, csr ? g->csr_ptr.p : g->csc_ptr.p, it.desc.p, nullptr);
   }
   return it;
 }

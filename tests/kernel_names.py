@@ -4,7 +4,7 @@ import re
 
 
 def kernels(call):
-    """{kernel name with template arguments: launches} of a call"""
+    """{kernel name: launches} of a call, with and without its template arguments"""
     import torch
     from torch.profiler import ProfilerActivity, profile
 
@@ -16,5 +16,7 @@ def kernels(call):
     for e in p.key_averages():
         m = re.search(r"nwg::\(anonymous namespace\)::(\w+(<[^(]*>)?)\(", e.key)
         if m:
-            names[m.group(1).replace(" ", "")] += e.count
+            name = m.group(1).replace(" ", "")
+            for k in {name, name.split("<")[0]}:
+                names[k] += e.count
     return names

@@ -96,3 +96,27 @@ def test_weighted_sweep_by_size(ctx, n, m, want):
     for call in (lambda: g.wpr_forward(None, 0.85, 1e-4, 30), lambda: g.wpr_backward(c, c, 0.85, 1e-2, 30)):
         assert {k for k in names if any(s.split("<")[0] == k for s in kernels(call))} == {want}
     g.close()
+
+
+@pytest.mark.parametrize("row,look", [(12000, False), (13500, True)])  # 2^34 * 0.15 / 200,001 is 12,885
+def test_small_rows_are_looked_for_where_the_base_allows_them(ctx, row, look):
+    n = 200001
+    rng = np.random.default_rng(row)
+    src, dst = rng.integers(0, n, 3 * n).astype(np.uint32), rng.integers(0, n, 3 * n).astype(np.uint32)
+    dst[:row] = 9
+    g = ctx.graph_from_edges(n, src, dst, clean=False)
+    form = lambda call: {k for k in kernels(call) if k.startswith(("pr_item_kernel<", "pr_item_many_kernel<"))}
+    name = "pr_item_kernel<true>" if look else "pr_item_kernel<false>"
+    for _ in range(2):
+        assert form(lambda: g.pagerank(0.85, 1e-4, 20)) == {name}
+    v = np.full(n, 1.0 / n, np.float32)
+    assert form(lambda: g.pagerank(0.85, 1e-4, 20, teleport=v)) == {"pr_item_kernel<true>"}
+    assert form(lambda: g.pagerank(1.0, 1e-4, 20)) == {"pr_item_kernel<true>"}
+    assert form(lambda: g.pagerank(0.85, 1e-4, 20)) == {name}
+    t = ctx.rmat(14, 8, seed=1)
+    mg = ctx.multigraph([t, g])
+    mg.set_plan(0)
+    assert form(lambda: mg.pagerank(0.85, 1e-4, 20)) == {name.replace("item", "item_many")}
+    assert form(lambda: mg.pagerank(1.0, 1e-4, 20)) == {"pr_item_many_kernel<true>"}
+    for h in (mg, t, g):
+        h.close()
