@@ -255,6 +255,9 @@ int nwg_graph_autotune(nwg_ctx* ctx, nwg_graph* g, nwg_plan_params* chosen /*nul
  * contribution as (x / deg) * deg, within 1 ulp of x, so a vector's L1 change can differ from a
  * single-vector solve's by up to ~2^-23 * sum(x) (< 1.2e-7 for scores summing to 1), and a
  * vector whose change lands that close to the threshold may stop one sweep apart from it.
+ * The graph keeps the solve's device memory until it is destroyed: two contribution arrays (n x k
+ * floats) and, for rows whose in-edges are added up in parts, partial sums of about three more at
+ * most.  Where those would pass 16 GiB, parts are longer (one sum per 512 in-edges of long rows).
  * iterations: [host] k counts, nullable. */
 int nwg_ppr_batched(nwg_ctx* ctx, nwg_graph* g, uint32_t k, const uint32_t* seed_ptr,
                     const uint32_t* seeds, float* scores, float damping, float threshold,
